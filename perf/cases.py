@@ -1,0 +1,305 @@
+"""The work that is timed when the speed of this framework is looked at.
+
+Listed are training steps of whole layers - what fine-tuning a model with compressed activations consists of, one
+layer at a time - and the operators of the compression path called by themselves, at the sizes of this
+repository's configurations, tests and benchmark.  `draw` gives further cases of the same ranges.
+
+A layer case is one forward and backward of a fused layer whose calibration is over (the steady state of a run: five
+calibrating steps against thousands), entered as a model enters it: hidden states that require gradients, frozen
+weights, LoRA adapters, an additive attention mask where the layer takes one."""
+import math
+from types import SimpleNamespace
+
+import torch
+
+from hyclora_amd.models import llama, llama_flash_attn, mistral, roberta
+from hyclora_amd.operators import (compress_function, nf4, softmax_kernels, triton_fuse_lora_silu_hadamard_backward_kernels,
+                                   triton_fuse_lora_silu_hadamard_forward_kernels)
+
+BF16 = torch.bfloat16
+RANK = 16
+SOFTMAX_RATIO, NORM_RATIO = 0.05, 0.005          # kept share of an attention map, share of outlier channels
+
+
+# ---- the cases --------------------------------------------------------------------------------------------------
+def _decoder(**kw):
+    return {"kind": "decoder", "weights": "bf16", "padded": False, **kw}
+
+
+def listed():
+    return [
+        # one activation in front of a norm, kept with its outlier channels split off: the smallest call
+        {"name": "outlier_activation_2x512x4096", "kind": "activation", "form": "outlier", "B": 2, "M": 512, "N": 4096, "q_bit": 4},
+        # a projection's output in an MLP of 7B size, kept and restored: the headline round trip of bench.py
+        {"name": "activation_4x1024x11008", "kind": "activation", "form": "plain", "B": 4, "M": 1024, "N": 11008, "q_bit": 4},
+        # queries or keys of a map-free layer (zero points), 13B width, a batch padded to its longest sequence
+        {"name": "zero_point_activation_3x777x5120", "kind": "activation", "form": "zero_point", "B": 3, "M": 777, "N": 5120, "q_bit": 2},
+        # the gated product of a 7B MLP, forward and backward
+        {"name": "gated_mlp_4x1024x11008", "kind": "gated", "T": 4096, "N": 11008, "q_bit": 4},
+        # an attention map kept sparse, then its softmax backward
+        {"name": "attention_map_4x32x1024", "kind": "map", "B": 4, "H": 32, "S": 1024},
+        # the layer that most runs are made of: 7B, batch 4, 1024 tokens
+        _decoder(name="llama7b_b4_s1024", family="llama", mode="intra_inter_full_fuse", B=4, S=1024, hidden=4096, heads=32, kv=32, inter=11008, q_bit=4),
+        # grouped key / value heads, longer sequences, 8-bit codes
+        _decoder(name="mistral7b_b2_s2048", family="mistral", mode="intra_inter_full_fuse", B=2, S=2048, hidden=4096, heads=32, kv=8, inter=14336, q_bit=8),
+        # long-sequence training: no attention map, the largest step
+        _decoder(name="mapfree7b_b1_s8192", family="llama_flash_attn", mode="intra_inter", B=1, S=8192, hidden=4096, heads=32, kv=32, inter=11008, q_bit=4),
+        # the memory / throughput harness: 4-bit frozen weights, 2-bit activations
+        dict(_decoder(name="nf4_llama7b_b4_s512", family="llama", mode="intra_inter", B=4, S=512, hidden=4096, heads=32, kv=32, inter=11008, q_bit=2), weights="nf4"),
+        # 13B width, a ragged batch left-padded to its longest sequence, every activation kept as it is
+        dict(_decoder(name="padded13b_b3_s680", family="llama", mode="intra", B=3, S=680, hidden=5120, heads=40, kv=40, inter=13824, q_bit=8), padded=True),
+        # one short sample: latency of the host path and of small launches
+        _decoder(name="short7b_b1_s96", family="llama", mode="intra_inter_full_fuse", B=1, S=96, hidden=4096, heads=32, kv=32, inter=11008, q_bit=4),
+        # sentence classification with an encoder of base size: many short, padded sequences
+        {"name": "encoder_b32_s128", "kind": "encoder", "mode": "intra_inter", "B": 32, "S": 128, "hidden": 768, "heads": 12, "inter": 3072, "q_bit": 4},
+    ]
+
+
+def _log(rng, lo, hi, multiple=1):
+    return max(lo, int(math.exp(rng.uniform(math.log(lo), math.log(hi)))) // multiple * multiple)
+
+
+def draw(rng):
+    kind = rng.choice(["activation", "gated", "map", "decoder", "decoder", "decoder", "mapfree", "encoder"])
+    bits = rng.choice([2, 4, 8])
+    if kind == "activation":
+        n = 32 * _log(rng, 32, 448)
+        rows = _log(rng, 64, 8192)
+        b = rng.choice([b for b in (1, 2, 3, 4) if rows // b >= 1])
+        return {"kind": kind, "form": rng.choice(["plain", "zero_point", "outlier"]), "B": b, "M": rows // b, "N": n, "q_bit": bits}
+    if kind == "gated":
+        return {"kind": kind, "T": _log(rng, 64, 8192), "N": 128 * _log(rng, 16, 112), "q_bit": bits}
+    if kind == "map":
+        s = _log(rng, 64, 2048, 8)
+        return {"kind": kind, "B": rng.choice([1, 2]) if s > 1024 else rng.choice([1, 2, 3, 4]), "H": rng.choice([12, 16, 32]), "S": s}
+    if kind == "encoder":
+        hidden, heads = rng.choice([(768, 12), (1024, 16)])
+        s = _log(rng, 32, 256, 8)
+        return {"kind": kind, "mode": rng.choice(["intra", "intra_inter"]), "B": rng.randint(8, max(8, min(64, 8192 // s))), "S": s,
+                "hidden": hidden, "heads": heads, "inter": 4 * hidden, "q_bit": bits}
+    hidden, heads, inter = rng.choice([(2048, 16, 5504), (4096, 32, 11008), (4096, 32, 14336), (5120, 40, 13824)])
+    if kind == "mapfree":
+        return _decoder(family="llama_flash_attn", mode="intra_inter", B=1, S=_log(rng, 256, 6144, 8), hidden=hidden, heads=heads, kv=heads,
+                        inter=inter, q_bit=bits)
+    family = rng.choice(["llama", "mistral"])
+    s = _log(rng, 64, 2048, 8)
+    return dict(_decoder(family=family, mode=rng.choice(["intra", "intra_inter", "intra_inter_full_fuse", "intra_inter_full_fuse"]),
+                         B=rng.randint(1, max(1, min(8, 4096 // s))), S=s, hidden=hidden, heads=heads, kv=heads // 4 if family == "mistral" else heads,
+                         inter=inter, q_bit=bits),
+                weights=rng.choice(["bf16", "bf16", "nf4"]), padded=rng.random() < 0.3)
+
+
+# ---- inputs -----------------------------------------------------------------------------------------------------
+class _Linear:
+    """What the layers read of a linear: the weight, and the quantisation state of a 4-bit one."""
+
+    def __init__(self, weight, quant_state=None):
+        self.weight, self.bias = weight, None
+        if quant_state is not None:
+            self.weight.quant_state = quant_state
+
+
+def _activations(shape, gen, spread=10.0):
+    """Hidden states as a transformer has them: unit normal, half a percent of the channels much larger."""
+    x = torch.randn(shape, generator=gen, device="cuda")
+    n = shape[-1]
+    big = torch.randperm(n, generator=gen, device="cuda")[:max(1, int(n * NORM_RATIO))]
+    x[..., big] *= spread
+    return x.to(BF16)
+
+
+def _weight(out_f, in_f, gen, scale, form):
+    if form == "bf16":
+        return _Linear((torch.randn(out_f, in_f, generator=gen, device="cuda") * scale).to(BF16))
+    # bitsandbytes' nested NF4: normal codes, block maxima about 2.5 standard deviations
+    n = out_f * in_f
+    level = torch.tensor(nf4.NF4_TABLE, device="cuda")
+    codes = torch.bucketize(torch.randn(n, generator=gen, device="cuda") / 2.5, (level[1:] + level[:-1]) / 2).to(torch.uint8)
+    packed = (codes[0::2] * 16 + codes[1::2]).reshape(-1, 1)
+    code2 = torch.linspace(-1, 1, 256, device="cuda")
+    absmax = torch.randint(0, 256, (n // 64,), generator=gen, device="cuda", dtype=torch.uint8)
+    state2 = SimpleNamespace(absmax=torch.full((-(-(n // 64) // 256),), 0.3 * scale, device="cuda"), code=code2, blocksize=256)
+    qs = nf4.make_quant_state(absmax, (out_f, in_f), offset=torch.tensor(2.5 * scale, device="cuda"), state2=state2)
+    return _Linear(packed, qs)
+
+
+def _projections(dims, gen, form, scale):
+    out = {}
+    for name, (o_f, i_f) in dims.items():
+        a = (torch.rand(RANK, i_f, generator=gen, device="cuda") * 2 - 1) / math.sqrt(i_f)      # kaiming-uniform
+        b = torch.randn(o_f, RANK, generator=gen, device="cuda") * 1e-3
+        out[name] = (_weight(o_f, i_f, gen, scale, form), _Linear(a.to(BF16).requires_grad_()), _Linear(b.to(BF16).requires_grad_()))
+    return out
+
+
+def _lengths(batch, s, gen):
+    """Lengths of the samples of a padded batch: the longest fills it, the others half of it and up."""
+    n = torch.randint(s // 2, s + 1, (batch,), generator=gen, device="cuda")
+    n[0] = s
+    return n
+
+
+def _config(case):
+    return SimpleNamespace(use_hyclora=True, layer_type=case["mode"], iteration_threshold=1, softmax_outlier_ratio=SOFTMAX_RATIO,
+                           layernorm_outlier_ratio=NORM_RATIO, q_bit=case["q_bit"])
+
+
+def _prepare_decoder(case, gen):
+    b, s, hidden, heads, kv, inter = (case[k] for k in ("B", "S", "hidden", "heads", "kv", "inter"))
+    hd = hidden // heads
+    dims = dict(q=(hidden, hidden), k=(kv * hd, hidden), v=(kv * hd, hidden), o=(hidden, hidden), gate=(inter, hidden), up=(inter, hidden),
+                down=(hidden, inter))
+    p = _projections(dims, gen, case["weights"], 0.02)
+    norms = [(1 + 0.1 * torch.randn(hidden, generator=gen, device="cuda")).to(BF16) for _ in range(2)]
+    pos = torch.arange(s, device="cuda", dtype=torch.float32)
+    theta = 1e6 if case["family"] == "mistral" else 1e4
+    angle = torch.cat([pos[:, None] / theta ** (torch.arange(0, hd, 2, device="cuda", dtype=torch.float32) / hd)] * 2, dim=-1)
+    cos, sin = angle.cos().to(BF16)[None], angle.sin().to(BF16)[None]
+    mask = None
+    if case["family"] != "llama_flash_attn":
+        hidden_from = torch.ones(s, s, dtype=torch.bool, device="cuda").triu(1)[None].expand(b if case["padded"] else 1, s, s)
+        if case["padded"]:                                                                       # left-padded, as batches for causal models are
+            hidden_from = hidden_from | (pos[None, None, :] < (s - _lengths(b, s, gen))[:, None, None])
+        mask = torch.zeros(hidden_from.shape, device="cuda", dtype=BF16).masked_fill_(hidden_from, torch.finfo(BF16).min)[:, None]
+    family = {"llama": llama, "mistral": mistral, "llama_flash_attn": llama_flash_attn}[case["family"]]
+    maker = {"llama": "make_fused_llama_layer", "mistral": "make_fused_mistral_layer", "llama_flash_attn": "make_fused_llama_layer"}[case["family"]]
+    layer = getattr(family, maker)(_config(case))
+    args = [norms[0], None, cos, sin, *p["q"], *p["k"], *p["v"], *p["o"], norms[1], None, *p["gate"], *p["up"], *p["down"], mask, heads, hd, kv]
+    return layer, args, p, (b, s, hidden)
+
+
+def _prepare_encoder(case, gen):
+    b, s, hidden, heads, inter = (case[k] for k in ("B", "S", "hidden", "heads", "inter"))
+    dims = dict(q=(hidden, hidden), k=(hidden, hidden), v=(hidden, hidden), o=(hidden, hidden), up=(inter, hidden), down=(hidden, inter))
+    p = _projections(dims, gen, "bf16", 1.28 / math.sqrt(hidden))
+    for base, _, _ in p.values():
+        base.bias = (0.02 * torch.randn(base.weight.shape[0], generator=gen, device="cuda")).to(BF16)
+    norms = [((1 + 0.1 * torch.randn(hidden, generator=gen, device="cuda")).to(BF16), (0.1 * torch.randn(hidden, generator=gen, device="cuda")).to(BF16))
+             for _ in range(2)]
+    padding = torch.arange(s, device="cuda")[None, :] >= _lengths(b, s, gen)[:, None]
+    mask = torch.zeros((b, s), device="cuda", dtype=BF16).masked_fill_(padding, torch.finfo(BF16).min)[:, None, None]
+    layer = roberta.make_fused_roberta_layer(_config(case))
+    args = [*p["q"], *p["k"], *p["v"], *p["o"], *norms[0], *p["up"], *p["down"], *norms[1], mask, heads, hidden // heads]
+    return layer, args, p, (b, s, hidden)
+
+
+def prepare(case, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    kind = case["kind"]
+    if kind in ("decoder", "encoder"):
+        layer, args, p, shape = (_prepare_decoder if kind == "decoder" else _prepare_encoder)(case, gen)
+        with torch.no_grad():
+            layer(_activations(shape, gen), *args)                        # the calibrating step: statistics frozen from here on
+        x = _activations(shape, gen).requires_grad_()
+        adapters = [m.weight for parts in p.values() for m in parts[1:]]
+        return SimpleNamespace(kind=kind, layer=layer, args=args, x=x, adapters=adapters, grad=torch.randn(shape, generator=gen, device="cuda").to(BF16))
+    q_bit = case.get("q_bit")
+    if kind == "activation":
+        shape = (case["B"], case["M"], case["N"])
+        first = _activations(shape, gen) if case["form"] == "outlier" else torch.randn(shape, generator=gen, device="cuda").to(BF16)
+        st = SimpleNamespace(kind=kind, form=case["form"], q_bit=q_bit, static={})
+        if case["form"] == "outlier":
+            st.static["outlier_channel_index"], st.static["scale"] = compress_function.get_statistics_channel_base(first, NORM_RATIO, q_bit, "per-channel")
+            st.x = torch.randn(shape, generator=gen, device="cuda").to(BF16)
+            st.x[..., st.static["outlier_channel_index"]] *= 10
+        elif case["form"] == "zero_point":
+            shift = torch.randn(shape[-1], generator=gen, device="cuda").to(BF16)
+            st.static["scale"], st.static["zero_point"] = compress_function.get_statistics_only_quant_zero_point(first + shift, q_bit, "per-channel")
+            st.x = torch.randn(shape, generator=gen, device="cuda").to(BF16) + shift
+        else:
+            st.static["scale"] = compress_function.get_statistics_only_quant(first, q_bit, "per-channel")
+            st.x = torch.randn(shape, generator=gen, device="cuda").to(BF16)
+        return st
+    if kind == "gated":
+        t, n = case["T"], case["N"]
+        rn = lambda *size: torch.randn(size, generator=gen, device="cuda")                                            # noqa: E731
+        st = SimpleNamespace(kind=kind, q_bit=q_bit)
+        st.xa1, st.xa2 = (0.6 * rn(1, t, RANK)).to(BF16), (0.6 * rn(1, t, RANK)).to(BF16)
+        st.b1, st.b2 = ((1e-3 * rn(n, RANK)).to(BF16).T for _ in range(2))
+        st.x1, st.x2, st.grad = (1.3 * rn(1, t, n)).to(BF16), (1.3 * rn(1, t, n)).to(BF16), rn(1, t, n).to(BF16)
+        st.s1, st.s2 = (compress_function.get_statistics_only_quant(x, q_bit, "per-channel") for x in (st.x1, st.x2))
+        return st
+    b, h, s = case["B"], case["H"], case["S"]
+    logits = (torch.randn(b, h, s, s, generator=gen, device="cuda") * (8 / math.sqrt(128))).to(BF16)
+    logits.masked_fill_(torch.ones(s, s, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    amap = torch.softmax(logits, dim=-1)
+    threshold = compress_function.get_statistics_softmax(amap, SOFTMAX_RATIO)
+    capacity = int(amap.numel() * SOFTMAX_RATIO * (1 + 1 / 16)) + 64      # the room that a layer gives its lists
+    return SimpleNamespace(kind=kind, map=amap, threshold=threshold, capacity=capacity, grad=torch.randn(b, h, s, s, generator=gen, device="cuda").to(BF16))
+
+
+# ---- one pass ---------------------------------------------------------------------------------------------------
+def run(state):
+    if state.kind in ("decoder", "encoder"):
+        state.x.grad = None
+        for a in state.adapters:
+            a.grad = None
+        y = state.layer(state.x, *state.args)
+        y.backward(state.grad)
+        return [y.detach(), state.x.grad] + [a.grad for a in state.adapters]
+    if state.kind == "activation":
+        c, st = compress_function, state.static
+        if state.form == "outlier":
+            kept, q, idx, scale = c.compression_pack_channel_base(state.x, NORM_RATIO, state.q_bit, "per-channel", 1, 1, st)
+            return [kept, q, c.outlier_addition_fuse_decompression_dequantization(q, scale, kept, idx, state.q_bit)]
+        if state.form == "zero_point":
+            q, scale, zero = c.compression_pack_quant_zp_base(state.x, state.q_bit, "per-channel", 1, 1, st)
+            return [q, c.decompression_dequantization_with_zero_point(q, scale, zero, state.q_bit)]
+        q, scale = c.compression_pack_quant_base(state.x, state.q_bit, "per-channel", 1, 1, st)
+        return [q, c.decompression_dequantization(q, scale, state.q_bit)]
+    if state.kind == "gated":
+        s = state
+        q1, q2, o = triton_fuse_lora_silu_hadamard_forward_kernels.triton_fuse_silu_forward(
+            s.xa1, s.b1, s.x1, s.s1, s.xa2, s.b2, s.x2, s.s2, s.q_bit)
+        again, grad_gate, grad_up = triton_fuse_lora_silu_hadamard_backward_kernels.triton_fuse_silu_backward(
+            s.xa1, s.b1, q1, s.s1, s.xa2, s.b2, q2, s.s2, s.grad, s.q_bit)
+        return [q1, q2, o, again, grad_gate, grad_up]
+    idx, val, seg, count = compress_function.compress_attention_map(state.map, state.threshold, capacity=state.capacity)
+    if count.value() > state.capacity:                                    # as the layers do when a map keeps more than the steps before it
+        idx, val, seg = compress_function.compress_attention_map(state.map, state.threshold, seg)
+    amap, grad = softmax_kernels.softmax_backward_from_compressed(idx, val, seg, state.grad)
+    return [seg, amap, grad]                                              # the restored map holds every kept entry in its place
+
+
+# ---- what a pass cannot do without ------------------------------------------------------------------------------
+def work(case):
+    kind = case["kind"]
+    if kind == "activation":
+        e = case["B"] * case["M"] * case["N"]
+        return {"bytes": e * (4 + case["q_bit"] / 4), "flops": 8 * e}
+    if kind == "gated":
+        e = case["T"] * case["N"]
+        return {"bytes": e * (14 + case["q_bit"] / 2), "flops": e * (8 * RANK + 40)}
+    if kind == "map":
+        e = case["B"] * case["H"] * case["S"] ** 2
+        return {"bytes": e * (2 + 6 + 2 * 10 * SOFTMAX_RATIO), "flops": 8 * e}
+    tokens, hidden, inter = case["B"] * case["S"], case["hidden"], case["inter"]
+    if kind == "encoder":
+        params, kept = 4 * hidden * hidden + 2 * hidden * inter, 8 * hidden + inter
+        pairs = case["B"] * case["S"] ** 2
+    else:
+        kv = case["kv"] * (hidden // case["heads"])
+        params, kept = 2 * hidden * hidden + 2 * hidden * kv + 3 * hidden * inter, 6 * hidden + 2 * kv + 2 * inter
+        pairs = case["B"] * case["S"] * (case["S"] + 1) / 2                                      # causal
+    weight_bytes = 2 * params * (2 if case.get("weights", "bf16") == "bf16" else 0.52)           # read in both directions
+    # hidden states, their gradients and the output; the kept codes written and read; a kept map likewise
+    data = tokens * hidden * 2 * 4 + 2 * tokens * kept * case["q_bit"] / 8
+    if case.get("family") != "llama_flash_attn":
+        data += 2 * 10 * SOFTMAX_RATIO * case["B"] * case["heads"] * case["S"] ** 2
+    return {"bytes": weight_bytes + data, "flops": 4 * tokens * params + 14 * pairs * hidden}
+
+
+def tolerance(case):
+    kind = case["kind"]
+    if kind == "activation":
+        return "exact"                                     # codes and the values that they stand for
+    if kind == "map":
+        return {"rel": 2e-3}                               # bf16 results of row sums in 32 bits
+    if kind == "gated":
+        return {"rel": 4e-3}                               # a rank-16 product in another order moves a bf16 result by a unit now and then
+    # Layers: the attention products once with 32-bit operands, rounded to bf16 like the layer's own, moved the gradients
+    # by 0.63 to 0.71 % of their norm at 4 and 8 bits, 1.1 % at 2 bits (a value that moves by a bf16 unit takes another
+    # code now and then, a step of which is larger than the unit) and single elements by up to 0.56; the encoder's by 0.32 %.
+    if kind == "encoder":
+        return {"rel": 0.02 if case["q_bit"] == 2 else 0.013, "max": 0.9}
+    return {"rel": 0.03 if case["q_bit"] == 2 else 0.028, "max": 0.99}
