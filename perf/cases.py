@@ -80,7 +80,7 @@ def draw(rng):
     hidden, heads, inter = rng.choice([(2048, 16, 5504), (4096, 32, 11008), (4096, 32, 14336), (5120, 40, 13824)])
     if kind == "mapfree":
         return _decoder(family="llama_flash_attn", mode="intra_inter", B=1, S=_log(rng, 256, 6144, 8), hidden=hidden, heads=heads, kv=heads,
-                        inter=inter, q_bit=bits)
+                        inter=inter, q_bit=rng.choice([4, 8]))     # at 2 bits the gradients of two exact attentions differ by 4 to 6 %
     family = rng.choice(["llama", "mistral"])
     s = _log(rng, 64, 2048, 8)
     return dict(_decoder(family=family, mode=rng.choice(["intra", "intra_inter", "intra_inter_full_fuse", "intra_inter_full_fuse"]),
@@ -299,7 +299,8 @@ def tolerance(case):
         return {"rel": 4e-3}                               # a rank-16 product in another order moves a bf16 result by a unit now and then
     # Layers: the attention products once with 32-bit operands, rounded to bf16 like the layer's own, moved the gradients
     # by 0.63 to 0.71 % of their norm at 4 and 8 bits, 1.1 % at 2 bits (a value that moves by a bf16 unit takes another
-    # code now and then, a step of which is larger than the unit) and single elements by up to 0.56; the encoder's by 0.32 %.
+    # code now and then, a step of which is larger than the unit) and single elements by up to 0.56; the encoder's by 0.32 %.  The map-free layer at 8192 tokens and 4 bits: 2.4 % between
+    # two flash kernels, 4.0 % between either and attention in 32 bits (0.8 and 1.1 % at 8 bits).
     if kind == "encoder":
         return {"rel": 0.02 if case["q_bit"] == 2 else 0.013, "max": 0.9}
-    return {"rel": 0.03 if case["q_bit"] == 2 else 0.028, "max": 0.99}
+    return {"rel": 0.03 if case["q_bit"] == 2 or case["family"] == "llama_flash_attn" else 0.028, "max": 0.99}
