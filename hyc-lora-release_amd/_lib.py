@@ -27,7 +27,7 @@ class HycError(RuntimeError):
 
 
 # name -> (restype, argtypes)
-ABI_VERSION = 11          # hyc_abi_version() of the library these signatures describe
+ABI_VERSION = 12          # hyc_abi_version() of the library these signatures describe
 _P, _I, _L = c_void_p, c_int, c_int64
 
 
@@ -93,6 +93,8 @@ _SIGNATURES = {
     "hyc_lora_add_restore": (_I, [_P, _P, _I] + [_P] * 4 + [_L, _L, _L, _I, _P]),
     "hyc_lora_add_quant_rope": (_I, [_P, _P, _I] + [_P] * 7 + [_I, _L, _L, _L, _L, _L, _L, _I, _P]),
     "hyc_lora_add_restore_rope": (_I, [_P, _P, _I] + [_P] * 6 + [_I, _L, _L, _L, _L, _L, _L, _I, _P]),
+    "hyc_flash_fwd": (_I, [_P] * 5 + [_L] * 5 + [ctypes.c_float, _I, _P]),
+    "hyc_flash_bwd": (_I, [_P] * 10 + [_L] * 5 + [ctypes.c_float, _I, _P]),
     "hyc_lora_add_sum": (_I, [_P, _I, _P, _L, _L, _L, _P]),
     "hyc_lora_add_quant_group": (_I, [_P, _I, _L, _L, _I, _P]),
     "hyc_lora_add_restore_group": (_I, [_P, _I, _L, _L, _I, _P]),

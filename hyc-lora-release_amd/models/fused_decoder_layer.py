@@ -60,6 +60,7 @@ from ..operators.softmax_kernels import softmax_backward, softmax_backward_from_
 from ..operators.triton_fuse_lora_silu_hadamard_backward_kernels import triton_fuse_silu_backward
 from ..operators.triton_fuse_lora_silu_hadamard_forward_kernels import triton_fuse_silu_forward
 from ..operators import lora_kernels
+from ..operators.flash_kernels import flash_backward, flash_forward, flash_supported
 from .compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum, lora_parts,
                             repeat_kv, repeat_kv_backward, rope_backward, rope_forward)
 
@@ -295,8 +296,8 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             q = rope_forward(q.transpose(1, 2), cos, sin).transpose(1, 2)
         if not k_rotated:
             k = rope_forward(k.transpose(1, 2), cos, sin).transpose(1, 2)
-        k = repeat_kv(k, n_rep)
-        v = repeat_kv(v, n_rep)
+        if whole or spec.attention == "map":
+            k, v = repeat_kv(k, n_rep), repeat_kv(v, n_rep)
         if whole:
             (quant_zp if spec.attention == "sdpa" else quant)("q_rope", q, "q")
             (quant_zp if spec.attention == "sdpa" else quant)("k_rope", k, "k")
@@ -345,18 +346,30 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             o = heads_matmul(a, v, out_hidden=True)
             del a, v
         else:
-            # causal attention without a map: the flash kernel behind torch's SDPA, called through its
-            # aten entry point so that the row log-sum-exps come back and backward needs no second
-            # forward (the reference keeps flash-attn's softmax_lse the same way,
-            # llama_flash_attn/fused_llama_layer_intra_inter.py:169-180, :459-468)
-            ctx.flash = None
+            # causal attention without a map: the row log-sum-exps come back with the output and backward needs
+            # no second forward (the reference keeps flash-attn's softmax_lse the same way,
+            # llama_flash_attn/fused_llama_layer_intra_inter.py:169-180, :459-468).  Heads of 64 and 128 dims run on
+            # this package's kernels, which read grouped keys and values as they are; other head sizes take the
+            # flash kernel behind torch's SDPA through its aten entry point.
+            ctx.flash, ctx.own_flash = None, False
             query_keep = ctx.key_padding = None
             if attention_mask is not None and attention_mask.dim() == 2:      # the reference's key-padding mask
                 key_padding = attention_mask if attention_mask.device == q.device else attention_mask.to(q.device)
                 attention_mask, query_keep = key_padding_attention_mask(key_padding, q.dtype)
                 if query_keep is not None:
                     ctx.key_padding = key_padding      # backward builds the [B, 1, S, S] mask again instead of keeping it
-            if KEEP_ATTENTION_LSE and attention_mask is None and q.is_cuda:
+            if attention_mask is None and flash_supported(q, k, v):
+                o, lse = flash_forward(q, k, v)
+                ctx.own_flash = True
+                if KEEP_ATTENTION_LSE:
+                    # beside the log-sum-exps, the rest of what torch's flash backward takes: a random state that is not
+                    # used without dropout, and no cumulative lengths
+                    saved["sdpa_lse"] = lse
+                    saved["sdpa_rng"] = saved["sdpa_unused"] = torch.empty((), device=q.device, dtype=torch.int64)
+                    ctx.flash = (None, None, q.shape[2], q.shape[2])
+            else:
+                k, v = repeat_kv(k, q.shape[1] // k.shape[1]), repeat_kv(v, q.shape[1] // v.shape[1])
+            if not ctx.own_flash and KEEP_ATTENTION_LSE and attention_mask is None and q.is_cuda:
                 try:
                     res = torch.ops.aten._scaled_dot_product_flash_attention(q, k, v, 0.0, True, False)
                     o, saved["sdpa_lse"] = res[0], res[1]
@@ -364,7 +377,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                     ctx.flash = tuple(res[2:6])
                 except RuntimeError:
                     ctx.flash = None
-            if ctx.flash is None:
+            if not ctx.own_flash and ctx.flash is None:
                 o = F.scaled_dot_product_attention(q, k, v, attn_mask=attention_mask, is_causal=attention_mask is None)
                 if query_keep is not None:
                     o = o * query_keep
@@ -612,7 +625,9 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 if name != "v" and not rotated:
                     t = rope_forward(t.transpose(1, 2), cos, sin).transpose(1, 2)
                 return t
-            q, k, v = rebuilt("q", H), repeat_kv(rebuilt("k", KV), n_rep), repeat_kv(rebuilt("v", KV), n_rep)
+            q, k, v = rebuilt("q", H), rebuilt("k", KV), rebuilt("v", KV)
+            if not (spec.attention == "sdpa" and ctx.own_flash):
+                k, v = repeat_kv(k, n_rep), repeat_kv(v, n_rep)
             del qkv
 
         if spec.attention == "map":
@@ -632,6 +647,12 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             grad_k = heads_matmul(grad_s.transpose(-2, -1), q, out_hidden=True)
             grad_q = heads_matmul(grad_s, k, out_hidden=True)
             del grad_s, q, k
+        elif ctx.own_flash:
+            # the attention output handed to the backward kernel is the dequantised one, as in the
+            # reference (…intra_inter.py:450-461); grouped keys and values give grouped gradients
+            out, lse = (hidden_to_head_shape(deq("o"), H), S["sdpa_lse"]) if ctx.flash is not None else flash_forward(q, k, v)
+            grad_q, grad_k, grad_v = flash_backward(grad_o, q, k, v, out, lse)
+            del q, k, v, out, grad_o
         elif ctx.flash is not None:
             # the attention output handed to the backward kernel is the dequantised one, as in the
             # reference (…intra_inter.py:450-461)
@@ -652,8 +673,8 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                     o_ = o_ * query_keep
                 grad_q, grad_k, grad_v = torch.autograd.grad(o_, (q_, k_, v_), grad_o)
             del q, k, v, q_, k_, v_, o_, grad_o
-        grad_v = repeat_kv_backward(grad_v, n_rep)
-        grad_k = repeat_kv_backward(grad_k, n_rep)
+        grad_v = repeat_kv_backward(grad_v, grad_v.shape[1] // KV)
+        grad_k = repeat_kv_backward(grad_k, grad_k.shape[1] // KV)
         grad_q = rope_backward(grad_q.transpose(1, 2), cos, sin).transpose(1, 2)
         grad_k = rope_backward(grad_k.transpose(1, 2), cos, sin).transpose(1, 2)
         grad_q, grad_k, grad_v = (head_to_hidden_shape(t) for t in (grad_q, grad_k, grad_v))

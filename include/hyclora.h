@@ -629,6 +629,27 @@ int hyc_lora_add_sum(const hyc_lora_sum_member *members, int count, void *y, int
                      void *stream);
 
 /* ---------------------------------------------------------------------------------------
+ * Attention without a map: o = softmax(q k^T * scale) v, causal or not, and its backward.
+ *
+ * Replaces _flash_attn_varlen_forward / _flash_attn_varlen_backward in the map-free layers
+ * (models/llama_flash_attn/fused_llama_layer_intra_inter.py:169-180, :459-468) and the repeat_kv copies around them.
+ *   q, o, grad_o, grad_q  bf16 [B, S, H, D] contiguous;   k, v, grad_k, grad_v  bf16 [B, S, KV, D] contiguous, H % KV == 0:
+ *                         query head h reads key / value head h / (H / KV); grad_k and grad_v are summed over the heads
+ *                         of a group in fp32 and rounded once;
+ *   lse                   fp32 [B, H, S]: natural log of the row sums of exp(score * scale); output of the forward;
+ *   delta                 fp32 [B, H, S] scratch of the backward (row sums of grad_o * o; o may differ from the forward's,
+ *                         the layers pass the dequantised one).
+ *   D 64 or 128, any S (up to 2^20, S*H*D <= 2^30), all pointers 16-byte aligned.  Scores, softmax and all sums are fp32, the
+ *   probabilities and score gradients are rounded to bf16 for the matrix cores.  Fixed summation order: the same bits on
+ *   every run.
+ */
+int hyc_flash_fwd(const void *q, const void *k, const void *v, void *o, float *lse, int64_t B, int64_t S, int64_t H,
+                  int64_t KV, int64_t D, float scale, int causal, void *stream);
+int hyc_flash_bwd(const void *grad_o, const void *q, const void *k, const void *v, const void *o, const float *lse,
+                  float *delta, void *grad_q, void *grad_k, void *grad_v, int64_t B, int64_t S, int64_t H, int64_t KV,
+                  int64_t D, float scale, int causal, void *stream);
+
+/* ---------------------------------------------------------------------------------------
  * Memory-only probe, FOR BENCHMARKING: loads n_reads and stores n_writes bf16 [T, N] tensors (1..3 each,
  * arrays of device pointers in host memory, 16-byte aligned, N % 8 == 0) with the access shape of the
  * kernels of this library and no arithmetic of the path, so that the rate the memory system gives a

@@ -1,0 +1,50 @@
+"""Map-free attention on the GPU against float64 of the same formulas."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def reference(q, k, v, g, causal):
+    """Output, log-sum-exps and gradients in float64, from the bf16 operands."""
+    n_rep = q.shape[1] // k.shape[1]
+    q, k, v, g = (t.double() for t in (q, k, v, g))
+    kr, vr = k.repeat_interleave(n_rep, 1), v.repeat_interleave(n_rep, 1)
+    s = (q @ kr.transpose(-1, -2).contiguous()) / math.sqrt(q.shape[-1])
+    if causal:
+        n = s.shape[-1]
+        s = s.masked_fill(torch.ones(n, n, dtype=torch.bool, device=s.device).triu(1), float("-inf"))
+    lse = torch.logsumexp(s, -1)
+    p = (s - lse[..., None]).exp()
+    o = p @ vr
+    dp = g @ vr.transpose(-1, -2).contiguous()
+    ds = p * (dp - (g * o).sum(-1, keepdim=True)) / math.sqrt(q.shape[-1])
+    group = lambda t: t.unflatten(1, (k.shape[1], n_rep)).sum(2)                      # noqa: E731
+    return o, lse, ds @ kr, group(ds.transpose(-1, -2).contiguous() @ q), group(p.transpose(-1, -2).contiguous() @ g)
+
+
+# sizes around the tiles: 32 query rows a wave, 128 a workgroup, 64 keys a step
+@pytest.mark.parametrize("s", [1, 31, 64, 65, 127, 128, 129, 200, 385])
+@pytest.mark.parametrize("b,h,kv,d", [(1, 2, 2, 128), (2, 8, 2, 128), (3, 3, 1, 64), (1, 16, 8, 64)])
+@pytest.mark.parametrize("causal", [True, False])
+def test_flash_attention(b, h, kv, d, s, causal):
+    from hyclora_amd.operators.flash_kernels import flash_backward, flash_forward
+    gen = torch.Generator(device="cuda").manual_seed(s * 7 + h + d)
+    hidden = lambda heads: torch.randn(b, s, heads, d, generator=gen, device="cuda").to(BF16).transpose(1, 2)      # noqa: E731
+    q, k, v, g = hidden(h), hidden(kv), hidden(kv), hidden(h)
+    q = (q * 2).to(BF16)
+    want = reference(q, k, v, g, causal)
+    o, lse = flash_forward(q, k, v, causal)
+    grads = flash_backward(g, q, k, v, o, lse, causal)
+    assert (lse.double() - want[1]).abs().max() < 1e-4              # fp32 sums of exponentials of fp32 scores
+    # bf16 probabilities and score gradients (relative 2^-9 each, random in sign) and one bf16 rounding of the result:
+    # 2-norm relative errors of about 2^-9 * sqrt(2); four times that is allowed
+    for got, ref, name in zip((o,) + grads, (want[0],) + want[2:], ("o", "grad_q", "grad_k", "grad_v")):
+        assert got.shape == ref.shape
+        err = (got.double() - ref).norm() / ref.norm().clamp_min(1e-30) if ref.norm() > 1e-6 else (got.double() - ref).norm()
+        assert err < 4 * 2 ** -8.5, (name, err.item())
+    again = flash_backward(g, q, k, v, o, lse, causal)
+    assert all(torch.equal(x, y) for x, y in zip(grads, again))
