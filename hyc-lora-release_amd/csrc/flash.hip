@@ -1,15 +1,17 @@
 // Attention without a map, forward and backward, on the gfx950 matrix cores (causal or not, grouped key / value heads).
 // q, o, grad_o, grad_q: bf16 [B, S, H, D]; k, v, grad_k, grad_v: bf16 [B, S, KV, D]; lse, delta: fp32 [B, H, S].
 //
-// Bound by the matrix cores and the vector units beside them (one exponential per score).  A wave owns 32 rows of one axis
-// (their operands stay in registers) and walks the other axis in tiles of 64 rows that its workgroup of four waves stages in
-// LDS, double-buffered, copied asynchronously while the previous tile is worked on: two workgroups (128 KB) and two waves per
-// SIMD are resident, one wave's exponentials beside the other's products.  Scores are formed transposed (a lane holds one row
-// of the softmax), so the row sums need one exchange between the two halves of a wave and the probabilities are the next
-// product's operand as they stand.  The backward runs as two kernels, one per owned axis, and forms scores twice instead of
-// adding query gradients with atomics: the same bits on every run.
-// [1, 8192, 32 heads, 128], causal: forward 615 us (0.89 PFLOP/s), backward 2400 us (0.80 of its seven products; 0.57 counting
-// five); the library kernels behind torch's scaled_dot_product_attention took 1280 and 5330.
+// Bound by the matrix cores and the vector units beside them (one exponential per score; 46 % and 60 % busy in the forward).
+// A wave owns 32 rows of one axis (their operands stay in registers) and walks the other axis in tiles of 64 rows that its
+// workgroup of four waves stages in LDS, double-buffered, copied asynchronously while the previous tile is worked on: two
+// workgroups (128 KB) and two waves per SIMD are resident, one wave's exponentials beside the other's products.  Scores are
+// formed transposed (a lane holds one row of the softmax), so the row sums need one exchange between the two halves of a wave
+// and the probabilities are the next product's operand as they stand.  The backward runs as two kernels, one per owned axis,
+// and forms scores twice instead of adding query gradients with atomics: the same bits on every run.
+// [1, 8192, 32 heads, 128], causal: forward 590 us (0.93 PFLOP/s), backward 1680 us (1.15 PFLOP/s of its seven products, 0.82
+// counting five); the library kernels behind torch's scaled_dot_product_attention took 1280 and 5330.  The first version of
+// the tile (rows of whole 256 bytes, addresses formed per read, every product waiting for the operand read right before it)
+// took 615 and 2400 us.
 #include "hyc_attn_tile.hpp"
 
 namespace hyc {
@@ -20,6 +22,9 @@ constexpr int kFlashTile = 64;         // rows of the tile the workgroup walks a
 // Head of a workgroup: consecutive workgroups go to the 8 XCDs in turn, so heads that share keys and values (and all
 // blocks of one head) are given numbers that meet on one XCD's L2.
 __device__ __forceinline__ int head_of(int j, int heads) { return heads % 8 ? j : (j % 8) * (heads / 8) + j / 8; }
+
+// whether a step has to look for masked entries: steps in the middle of a sequence are compiled without
+template <bool B> struct Edge { static constexpr bool value = B; };
 
 struct FlashArgs {
     const uint16_t *q, *k, *v, *o, *grad_o;
@@ -32,6 +37,7 @@ struct FlashArgs {
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(const FlashArgs A) {
     using Tile = AttnTile<D, kFlashTile>;
+    constexpr int kOther = 2 * Tile::kBytes;                    // the second tensor's pair of tiles
     __shared__ __attribute__((aligned(1024))) char lds[4 * Tile::kBytes];       // two of keys, two of values
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int heads = A.B * A.H, nblk = (int)gridDim.x / heads;
@@ -48,32 +54,31 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(const FlashArgs A) {
 
     const int kend = CAUSAL ? min(A.S, blk * kFlashRows + kFlashRows) : A.S;
     const int tiles = (kend + kFlashTile - 1) / kFlashTile;
+    const int full = CAUSAL ? blk * (kFlashRows / kFlashTile) : A.S / kFlashTile;    // tiles without an edge for any wave
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(lds));
-    Tile::request(kbase, 0, A.S - 1, ldk, lds0, wave, lane);
-    Tile::request(vbase, 0, A.S - 1, ldk, lds0 + 2 * Tile::kBytes, wave, lane);
+    const typename Tile::Lane at(lane);
+    auto request = [&](int it) {
+        Tile::request(kbase, it * kFlashTile, A.S - 1, ldk, lds0 + (it & 1) * Tile::kBytes, wave, lane);
+        Tile::request(vbase, it * kFlashTile, A.S - 1, ldk, lds0 + (2 + (it & 1)) * Tile::kBytes, wave, lane);
+    };
+    request(0);
 
     f32x16 O[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) O[db] = f32x16{};
     float m = -INFINITY, l = 0.0f;
-    for (int it = 0; it < tiles; ++it) {
-        wait_copies_and_barrier();
-        const int k0 = it * kFlashTile, buf = it & 1;
-        if (it + 1 < tiles) {
-            Tile::request(kbase, k0 + kFlashTile, A.S - 1, ldk, lds0 + (buf ^ 1) * Tile::kBytes, wave, lane);
-            Tile::request(vbase, k0 + kFlashTile, A.S - 1, ldk, lds0 + (2 + (buf ^ 1)) * Tile::kBytes, wave, lane);
-        }
-        if (CAUSAL && k0 > q0 + 31) continue;                  // nothing for this wave's rows; the barriers stay shared
-        const char* K = lds + buf * Tile::kBytes;
-        const char* V = lds + (2 + buf) * Tile::kBytes;
+    auto step = [&](int it, auto edge) {
+        const int k0 = it * kFlashTile;
+        const typename Tile::Lane in = Tile::in_tile(at, lds0 + (it & 1) * Tile::kBytes);
         f32x16 s[2];
         s[0] = f32x16{}; s[1] = f32x16{};
 #pragma unroll
         for (int t = 0; t < D / 16; ++t) {
-            s[0] = mfma32(Tile::rows_operand(K, 0, t, lane), Q[t], s[0]);
-            s[1] = mfma32(Tile::rows_operand(K, 32, t, lane), Q[t], s[1]);
+            s[0] = mfma32(Tile::rows_operand(in, 0, 0, t), Q[t], s[0]);
+            s[1] = mfma32(Tile::rows_operand(in, 0, 32, t), Q[t], s[1]);
         }
-        if ((CAUSAL && k0 + kFlashTile - 1 > q0) || k0 + kFlashTile > A.S) {
+        order_products<D / 8, 1, 6>();
+        if (edge.value) {
             const int last = CAUSAL ? min(qrow, A.S - 1) : A.S - 1;
 #pragma unroll
             for (int kb = 0; kb < 2; ++kb)
@@ -112,8 +117,20 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(const FlashArgs A) {
         for (int t = 0; t < 4; ++t) {
             const bf16x8 P = c_as_operand(s[t >> 1], t & 1);
 #pragma unroll
-            for (int db = 0; db < D / 32; ++db) O[db] = mfma32(Tile::cols_operand(V, 16 * t, 32 * db, lane), P, O[db]);
+            for (int db = 0; db < D / 32; ++db) O[db] = mfma32(Tile::cols_operand(in, kOther, 16 * t, 32 * db), P, O[db]);
         }
+        order_products<D / 8, 2, 4>();
+    };
+    int it = 0;
+    for (; it < full; ++it) {
+        wait_copies_and_barrier();
+        if (it + 1 < tiles) request(it + 1);
+        step(it, Edge<false>{});
+    }
+    for (; it < tiles; ++it) {
+        wait_copies_and_barrier();
+        if (it + 1 < tiles) request(it + 1);
+        if (!CAUSAL || it * kFlashTile <= q0 + 31) step(it, Edge<true>{});      // else nothing for this wave's rows; the barriers stay shared
     }
     l = half_sum(l);
     if (qrow < A.S) {
@@ -122,10 +139,12 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_kernel(const FlashArgs A) {
     }
 }
 
-// grad_q of 128 query rows, and delta = sum_d grad_o * o of these rows for the key / value kernel
+// grad_q of 128 query rows; leaves -delta = -sum_d grad_o * o and the log-sum-exps to base 2 of these rows for the key /
+// value kernel
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, 2) void flash_bwd_q_kernel(const FlashArgs A) {
     using Tile = AttnTile<D, kFlashTile>;
+    constexpr int kOther = 2 * Tile::kBytes;                    // the second tensor's pair of tiles
     __shared__ __attribute__((aligned(1024))) char lds[4 * Tile::kBytes];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
     const int heads = A.B * A.H, nblk = (int)gridDim.x / heads;
@@ -142,8 +161,12 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_q_kernel(const FlashArgs A) 
     load_row_operands<D>(A.q + row_off, h, Q);
     load_row_operands<D>(A.grad_o + row_off, h, G);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(lds));
-    Tile::request(kbase, 0, A.S - 1, ldk, lds0, wave, lane);
-    Tile::request(vbase, 0, A.S - 1, ldk, lds0 + 2 * Tile::kBytes, wave, lane);
+    const typename Tile::Lane at(lane);
+    auto request = [&](int it) {
+        Tile::request(kbase, it * kFlashTile, A.S - 1, ldk, lds0 + (it & 1) * Tile::kBytes, wave, lane);
+        Tile::request(vbase, it * kFlashTile, A.S - 1, ldk, lds0 + (2 + (it & 1)) * Tile::kBytes, wave, lane);
+    };
+    request(0);
 
     float delta = 0.0f;
 #pragma unroll
@@ -156,35 +179,32 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_q_kernel(const FlashArgs A) 
     }
     delta = half_sum(delta);
     const int64_t stat = ((int64_t)b * A.H + head) * A.S + qsafe;
-    if (qrow < A.S && h == 0) A.delta[stat] = delta;
     const float lse2 = A.lse[stat] * kLog2e;
+    if (qrow < A.S && h == 0) {
+        A.delta[stat] = -delta;
+        A.delta[(int64_t)heads * A.S + stat] = lse2;
+    }
 
     const int kend = CAUSAL ? min(A.S, blk * kFlashRows + kFlashRows) : A.S;
     const int tiles = (kend + kFlashTile - 1) / kFlashTile;
+    const int full = CAUSAL ? blk * (kFlashRows / kFlashTile) : A.S / kFlashTile;
     f32x16 dq[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) dq[db] = f32x16{};
-    for (int it = 0; it < tiles; ++it) {
-        wait_copies_and_barrier();
-        const int k0 = it * kFlashTile, buf = it & 1;
-        if (it + 1 < tiles) {
-            Tile::request(kbase, k0 + kFlashTile, A.S - 1, ldk, lds0 + (buf ^ 1) * Tile::kBytes, wave, lane);
-            Tile::request(vbase, k0 + kFlashTile, A.S - 1, ldk, lds0 + (2 + (buf ^ 1)) * Tile::kBytes, wave, lane);
-        }
-        if (CAUSAL && k0 > q0 + 31) continue;
-        const char* K = lds + buf * Tile::kBytes;
-        const char* V = lds + (2 + buf) * Tile::kBytes;
-        const bool edge = (CAUSAL && k0 + kFlashTile - 1 > q0) || k0 + kFlashTile > A.S;
+    auto step = [&](int it, auto edge) {
+        const int k0 = it * kFlashTile;
+        const typename Tile::Lane in = Tile::in_tile(at, lds0 + (it & 1) * Tile::kBytes);
         const int last = CAUSAL ? min(qrow, A.S - 1) : A.S - 1;
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {
             f32x16 s = f32x16{}, dp = f32x16{};
 #pragma unroll
             for (int t = 0; t < D / 16; ++t) {
-                s = mfma32(Tile::rows_operand(K, 32 * kb, t, lane), Q[t], s);
-                dp = mfma32(Tile::rows_operand(V, 32 * kb, t, lane), G[t], dp);
+                s = mfma32(Tile::rows_operand(in, 0, 32 * kb, t), Q[t], s);
+                dp = mfma32(Tile::rows_operand(in, kOther, 32 * kb, t), G[t], dp);
             }
-            if (edge) {
+            order_products<D / 8, 1, 6>();
+            if (edge.value) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     if (k0 + 32 * kb + 8 * (r / 4) + 4 * h + r % 4 > last) s[r] = -INFINITY;
@@ -197,9 +217,21 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_q_kernel(const FlashArgs A) 
                 const bf16x8 dS = c_as_operand(s, t);
 #pragma unroll
                 for (int db = 0; db < D / 32; ++db)
-                    dq[db] = mfma32(Tile::cols_operand(K, 32 * kb + 16 * t, 32 * db, lane), dS, dq[db]);
+                    dq[db] = mfma32(Tile::cols_operand(in, 0, 32 * kb + 16 * t, 32 * db), dS, dq[db]);
             }
+            order_products<D / 16, 2, 3>();
         }
+    };
+    int it = 0;
+    for (; it < full; ++it) {
+        wait_copies_and_barrier();
+        if (it + 1 < tiles) request(it + 1);
+        step(it, Edge<false>{});
+    }
+    for (; it < tiles; ++it) {
+        wait_copies_and_barrier();
+        if (it + 1 < tiles) request(it + 1);
+        if (!CAUSAL || it * kFlashTile <= q0 + 31) step(it, Edge<true>{});
     }
     if (qrow < A.S) store_rows<D>(A.grad_q + row_off, h, dq, A.scale);
 }
@@ -208,6 +240,7 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_q_kernel(const FlashArgs A) 
 template <int D, bool CAUSAL>
 __global__ __launch_bounds__(256, 2) void flash_bwd_kv_kernel(const FlashArgs A) {
     using Tile = AttnTile<D, kFlashTile>;
+    constexpr int kOther = 2 * Tile::kBytes;                    // the second tensor's pair of tiles
     constexpr int kStat = 256;                                  // bytes of 64 row statistics
     __shared__ __attribute__((aligned(1024))) char lds[4 * Tile::kBytes + 4 * kStat];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
@@ -223,60 +256,58 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_kv_kernel(const FlashArgs A)
     load_row_operands<D>(A.k + row_off, h, K);
     load_row_operands<D>(A.v + row_off, h, V);
     const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(lds));
+    const typename Tile::Lane at(lane);
     const int first = CAUSAL ? blk * kFlashRows / kFlashTile : 0;             // first query tile that sees these keys
     const int per_head = (A.S + kFlashTile - 1) / kFlashTile - first;
     const int tiles = per_head * group;
     const uint16_t* qb = A.q + (int64_t)b * A.S * ldq + kvh * group * D;
     const uint16_t* gb = A.grad_o + (int64_t)b * A.S * ldq + kvh * group * D;
-    const float* lb = A.lse + ((int64_t)b * A.H + kvh * group) * A.S;
-    const float* tb = A.delta + ((int64_t)b * A.H + kvh * group) * A.S;
+    const float* delta_b = A.delta + ((int64_t)b * A.H + kvh * group) * A.S;
+    const float* lse_b = delta_b + (int64_t)A.B * A.H * A.S;
 
     auto request = [&](int g, int q0, int buf) {
         Tile::request(qb + g * D, q0, A.S - 1, ldq, lds0 + buf * Tile::kBytes, wave, lane);
         Tile::request(gb + g * D, q0, A.S - 1, ldq, lds0 + (2 + buf) * Tile::kBytes, wave, lane);
-        const uint32_t at = (uint32_t)(q0 + lane < A.S ? q0 + lane : A.S - 1) * 4u;
-        if (wave == 0) copy_to_lds4(lb + (int64_t)g * A.S, at, lds0 + 4 * Tile::kBytes + buf * kStat);
-        if (wave == 1) copy_to_lds4(tb + (int64_t)g * A.S, at, lds0 + 4 * Tile::kBytes + (2 + buf) * kStat);
+        const uint32_t row = (uint32_t)(q0 + lane < A.S ? q0 + lane : A.S - 1) * 4u;
+        if (wave == 0) copy_to_lds4(lse_b + (int64_t)g * A.S, row, lds0 + 4 * Tile::kBytes + buf * kStat);
+        if (wave == 1) copy_to_lds4(delta_b + (int64_t)g * A.S, row, lds0 + 4 * Tile::kBytes + (2 + buf) * kStat);
     };
     request(0, first * kFlashTile, 0);
     f32x16 dk[D / 32], dv[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) dk[db] = dv[db] = f32x16{};
-    int g = 0, tile = 0;                                        // the tile being worked on
-    for (int it = 0; it < tiles; ++it) {
-        wait_copies_and_barrier();
-        const int q0 = (first + tile) * kFlashTile, buf = it & 1;
-        if (++tile == per_head) { tile = 0; ++g; }
-        if (it + 1 < tiles) request(g, (first + tile) * kFlashTile, buf ^ 1);
-        if (CAUSAL && q0 + kFlashTile - 1 < key0) continue;
-        const char* Q = lds + buf * Tile::kBytes;
-        const char* G = lds + (2 + buf) * Tile::kBytes;
-        const char* stat = lds + 4 * Tile::kBytes + buf * kStat;
-        const bool edge = (CAUSAL && q0 < key0 + 31) || q0 + kFlashTile > A.S;
+    auto step = [&](int q0, int buf, bool edge) {
+        const typename Tile::Lane in = Tile::in_tile(at, lds0 + buf * Tile::kBytes);
+        const uint32_t stat = lds0 + 4 * Tile::kBytes + buf * kStat + 16 * h;
+        typedef const __attribute__((address_space(3))) f32x4 lds_f32x4;
 #pragma unroll
-        for (int qb2 = 0; qb2 < 2; ++qb2) {
-            f32x16 s = f32x16{}, dp = f32x16{};
+        for (int half = 0; half < 2; ++half) {
+            f32x16 s = f32x16{}, dp;
+#pragma unroll
+            for (int b4 = 0; b4 < 4; ++b4) {                    // grad_o v^T - delta: the sums start from -delta
+                const f32x4 del = *(lds_f32x4*)(stat + 2 * kStat + (32 * half + 8 * b4) * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dp[4 * b4 + e] = del[e];
+            }
 #pragma unroll
             for (int t = 0; t < D / 16; ++t) {
-                s = mfma32(Tile::rows_operand(Q, 32 * qb2, t, lane), K[t], s);
-                dp = mfma32(Tile::rows_operand(G, 32 * qb2, t, lane), V[t], dp);
+                s = mfma32(Tile::rows_operand(in, 0, 32 * half, t), K[t], s);
+                dp = mfma32(Tile::rows_operand(in, kOther, 32 * half, t), V[t], dp);
             }
 #pragma unroll
             for (int b4 = 0; b4 < 4; ++b4) {
-                const f32x4 lse = *reinterpret_cast<const f32x4*>(stat + (32 * qb2 + 8 * b4 + 4 * h) * 4);
-                const f32x4 del = *reinterpret_cast<const f32x4*>(stat + 2 * kStat + (32 * qb2 + 8 * b4 + 4 * h) * 4);
+                const f32x4 lse = *(lds_f32x4*)(stat + (32 * half + 8 * b4) * 4);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int r = 4 * b4 + e;
-                    const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale2, -lse[e] * kLog2e));
-                    s[r] = p;
-                    dp[r] = p * (dp[r] - del[e]);
+                    s[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], scale2, -lse[e]));
+                    dp[r] = s[r] * dp[r];
                 }
             }
             if (edge) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    const int row = q0 + 32 * qb2 + 8 * (r / 4) + 4 * h + r % 4;
+                    const int row = q0 + 32 * half + 8 * (r / 4) + 4 * h + r % 4;
                     if (row >= A.S || (CAUSAL && row < key)) s[r] = dp[r] = 0.0f;
                 }
             }
@@ -285,11 +316,21 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_kv_kernel(const FlashArgs A)
                 const bf16x8 P = c_as_operand(s, t), dS = c_as_operand(dp, t);
 #pragma unroll
                 for (int db = 0; db < D / 32; ++db) {
-                    dv[db] = mfma32(Tile::cols_operand(G, 32 * qb2 + 16 * t, 32 * db, lane), P, dv[db]);
-                    dk[db] = mfma32(Tile::cols_operand(Q, 32 * qb2 + 16 * t, 32 * db, lane), dS, dk[db]);
+                    dv[db] = mfma32(Tile::cols_operand(in, kOther, 32 * half + 16 * t, 32 * db), P, dv[db]);
+                    dk[db] = mfma32(Tile::cols_operand(in, 0, 32 * half + 16 * t, 32 * db), dS, dk[db]);
                 }
             }
+            order_products<D / 8, 2, 3>();
         }
+    };
+    int g = 0, tile = 0;                                        // the tile being worked on
+    for (int it = 0; it < tiles; ++it) {
+        wait_copies_and_barrier();
+        const int q0 = (first + tile) * kFlashTile, buf = it & 1;
+        if (++tile == per_head) { tile = 0; ++g; }
+        if (it + 1 < tiles) request(g, (first + tile) * kFlashTile, buf ^ 1);
+        if (CAUSAL && q0 + kFlashTile - 1 < key0) continue;    // nothing for this wave's keys; the barriers stay shared
+        step(q0, buf, (CAUSAL && q0 < key0 + 31) || q0 + kFlashTile > A.S);
     }
     if (key < A.S) {
         store_rows<D>(A.grad_k + row_off, h, dk, A.scale);

@@ -46,52 +46,87 @@ __device__ __forceinline__ void wait_copies_and_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
-// A tile of ROWS rows of D bf16 in LDS.  The 16-byte chunks of a row are permuted so that neither read form meets bank
-// conflicts: chunk c of row r lies at slot c ^ swz(r), which keeps pairs of chunks together (a transposing read takes
-// 32 bytes of each of its 4 rows) and spreads 8 consecutive rows over different banks.  The copies write LDS in lane
-// order, so the permutation is made by which chunk a lane fetches.
+// A tile of ROWS rows of D bf16 in LDS, as 1 KB blocks of 16 rows x 4 chunks (of 16 bytes): block (row / 16, chunk / 4),
+// inside it chunk % 4 major, and the 16 rows of a chunk in the order row ^ 4 * (chunk % 4).  An operand of 32 rows reads 16
+// rows of a chunk as 256 contiguous bytes; a transposing read takes 4 rows (64 bytes) of each of 4 chunks, which the order
+// puts on different banks.  Everything that varies inside a kernel's loops (k step, column block, buffer) moves the address
+// by a multiple of a block, an immediate offset: four registers of addresses serve all reads.  A wave's copy fills one
+// block: 64 bytes of each of 16 rows of memory.
 template <int D, int ROWS>
 struct AttnTile {
     static constexpr int kChunks = D / 8;                       // 16-byte chunks of a row
-    static constexpr int kPitch = D * 2;
-    static constexpr int kBytes = ROWS * kPitch;
-    static constexpr int kRowsPerCopy = 64 / kChunks;           // rows one wave instruction covers
-    static constexpr int kCopies = ROWS / (kRowsPerCopy * 4);   // instructions of each of 4 waves
-
-    __device__ static __forceinline__ int swz(int row) { return D == 128 ? 2 * (row & 7) : 2 * ((row >> 1) & 3); }
+    static constexpr int kBlocksAcross = kChunks / 4;
+    static constexpr int kBytes = ROWS * D * 2;
+    static constexpr int kCopies = kBytes / 4096;               // block copies of each of 4 waves
 
     // Requests rows row0 .. row0 + ROWS - 1 (past row_last: row_last again) of a tensor whose rows are `ld` elements
     // apart; called by the 4 waves of a workgroup.
     __device__ static __forceinline__ void request(const uint16_t* base, int row0, int row_last, int ld, uint32_t lds, int wave, int lane) {
-        const int r_in = lane / kChunks, slot = lane % kChunks;
+        const int c = lane >> 4, r = (lane & 15) ^ (4 * c);
 #pragma unroll
         for (int i = 0; i < kCopies; ++i) {
-            const int row = (i * 4 + wave) * kRowsPerCopy + r_in;
+            const int blk = i * 4 + wave, row = (blk / kBlocksAcross) * 16 + r;
             const int src = row0 + row < row_last ? row0 + row : row_last;
-            const uint32_t voff = ((uint32_t)src * (uint32_t)ld + (uint32_t)((slot ^ swz(row)) * 8)) * 2u;
-            copy_to_lds16(base, voff, lds + (uint32_t)((i * 4 + wave) * 1024));
+            const uint32_t voff = ((uint32_t)src * (uint32_t)ld + (uint32_t)((blk % kBlocksAcross) * 32 + c * 8)) * 2u;
+            copy_to_lds16(base, voff, lds + (uint32_t)(blk * 1024));
         }
     }
 
-    // A operand of rows r0 .. r0+31 (r0 a multiple of 32), k = columns 16t .. 16t+15
-    __device__ static __forceinline__ bf16x8 rows_operand(const char* tile, int r0, int t, int lane) {
-        const int row = lane & 31, h = lane >> 5;
-        return as_bf16x8(*reinterpret_cast<const u32x4*>(tile + (r0 + row) * kPitch + (((2 * t + h) ^ swz(row)) * 16)));
+    // What a lane adds to a tile's LDS address for the two read forms
+    struct Lane {
+        uint32_t rows[2], cols[2];
+        __device__ __forceinline__ explicit Lane(int lane) {
+            const int h = lane >> 5, r16 = lane & 15, rb = (lane >> 4) & 1;
+#pragma unroll
+            for (int odd = 0; odd < 2; ++odd) {
+                const int c = 2 * odd + h;
+                rows[odd] = (uint32_t)(rb * kBlocksAcross * 1024 + c * 256 + (r16 ^ (4 * c)) * 16);
+                const int row = 4 * h + (r16 >> 2) + 8 * odd, cc = 2 * rb + ((r16 & 3) >> 1);
+                cols[odd] = (uint32_t)(cc * 256 + (row ^ (4 * cc)) * 16 + (r16 & 1) * 8);
+            }
+        }
+    };
+    // The lane's addresses in one tile, opaque so that what a read adds to them stays an immediate offset instead of an
+    // addition each (a third of the forward kernel's integer instructions)
+    __device__ static __forceinline__ Lane in_tile(const Lane& at, uint32_t tile) {
+        Lane v(at);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            v.rows[i] += tile; v.cols[i] += tile;
+            asm("" : "+v"(v.rows[i]), "+v"(v.cols[i]));
+        }
+        return v;
     }
-    // A operand of the transposed tile: rows = columns d0 .. d0+31 of the tile, k = tile rows k0 .. k0+15 (k0 a multiple
-    // of 16) in the order 4h + {0..3}, 8 + 4h + {0..3}
-    __device__ static __forceinline__ bf16x8 cols_operand(const char* tile, int k0, int d0, int lane) {
-        const int i = lane & 15, g = (lane >> 4) & 1, h = lane >> 5;
-        const int row = 4 * h + (i >> 2);                       // swz has period 8 in rows
-        const int chunk = (d0 >> 3) + 2 * g + ((i & 3) >> 1);
-        const char* p = tile + (k0 + row) * kPitch + (chunk ^ swz(row)) * 16 + (i & 1) * 8;
+    // A operand of tile rows r0 .. r0+31 (r0 a multiple of 32), k = columns 16t .. 16t+15; `off`: constant bytes past the tile
+    __device__ static __forceinline__ bf16x8 rows_operand(const Lane& at, int off, int r0, int t) {
+        typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
+        return as_bf16x8(*(lds_u32x4*)(at.rows[t & 1] + (uint32_t)(off + ((r0 / 16) * kBlocksAcross + t / 2) * 1024)));
+    }
+    // A operand of the transposed tile: rows = columns d0 .. d0+31 of the tile (d0 a multiple of 32), k = tile rows
+    // k0 .. k0+15 (k0 a multiple of 16) in the order 4h + {0..3}, 8 + 4h + {0..3}
+    __device__ static __forceinline__ bf16x8 cols_operand(const Lane& at, int tile, int k0, int d0) {
         typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 8 * kPitch));
+        const uint32_t off = (uint32_t)(tile + ((k0 / 16) * kBlocksAcross + d0 / 32) * 1024);
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at.cols[0] + off));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at.cols[1] + off));
         const u32x2 a = __builtin_bit_cast(u32x2, lo), b = __builtin_bit_cast(u32x2, hi);
         return as_bf16x8(u32x4{a.x, a.y, b.x, b.y});
     }
 };
+
+// Order of a straight run of matrix instructions and the LDS reads that feed them: `ahead` operands are requested before
+// the first product, then one more per product, so that no product waits for the read just issued (left alone, the compiler
+// reads each operand right before its use and waits out the latency every time).  READS: LDS instructions per operand.
+template <int PRODUCTS, int READS, int AHEAD>
+__device__ __forceinline__ void order_products() {
+    __builtin_amdgcn_sched_group_barrier(0x100, READS * AHEAD, 0);
+#pragma unroll
+    for (int i = 0; i < PRODUCTS - AHEAD; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, READS, 0);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x008, AHEAD, 0);
+}
 
 // B operands of 32 rows of a row-major tensor (lane l: row l % 32), all D / 16 k steps
 template <int D>

@@ -57,7 +57,7 @@ def flash_backward(grad_o, q, k, v, o, lse, causal=True):
     grad_o, q, k, v, o = _hidden(grad_o), _hidden(q), _hidden(k), _hidden(v), _hidden(o)
     lse = lse.contiguous()
     gq, gk, gv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-    delta = torch.empty((B, H, S), device=q.device, dtype=torch.float32)
+    delta = torch.empty((2, B, H, S), device=q.device, dtype=torch.float32)
     _lib.call("hyc_flash_bwd", grad_o.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(),
               delta.data_ptr(), gq.data_ptr(), gk.data_ptr(), gv.data_ptr(), B, S, H, k.shape[2], D, 1.0 / math.sqrt(D), int(causal),
               _lib.stream_of(q))

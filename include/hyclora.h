@@ -637,8 +637,8 @@ int hyc_lora_add_sum(const hyc_lora_sum_member *members, int count, void *y, int
  *                         query head h reads key / value head h / (H / KV); grad_k and grad_v are summed over the heads
  *                         of a group in fp32 and rounded once;
  *   lse                   fp32 [B, H, S]: natural log of the row sums of exp(score * scale); output of the forward;
- *   delta                 fp32 [B, H, S] scratch of the backward (row sums of grad_o * o; o may differ from the forward's,
- *                         the layers pass the dequantised one).
+ *   delta                 fp32 [2, B, H, S] scratch of the backward (row sums of grad_o * o, and the log-sum-exps to base 2).
+ *                         The backward's o may differ from the forward's: the layers pass the dequantised one.
  *   D 64 or 128, any S (up to 2^20, S*H*D <= 2^30), all pointers 16-byte aligned.  Scores, softmax and all sums are fp32, the
  *   probabilities and score gradients are rounded to bf16 for the matrix cores.  Fixed summation order: the same bits on
  *   every run.
