@@ -61,6 +61,7 @@ from ..operators.triton_fuse_lora_silu_hadamard_backward_kernels import triton_f
 from ..operators.triton_fuse_lora_silu_hadamard_forward_kernels import triton_fuse_silu_forward
 from ..operators import lora_kernels
 from ..operators.flash_kernels import flash_backward, flash_forward, flash_supported
+from ..operators.map_kernels import MapAttention, map_backward, map_supported
 from .compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum, lora_parts,
                             repeat_kv, repeat_kv_backward, rope_backward, rope_forward)
 
@@ -296,7 +297,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             q = rope_forward(q.transpose(1, 2), cos, sin).transpose(1, 2)
         if not k_rotated:
             k = rope_forward(k.transpose(1, 2), cos, sin).transpose(1, 2)
-        if whole or spec.attention == "map":
+        if whole:
             k, v = repeat_kv(k, n_rep), repeat_kv(v, n_rep)
         if whole:
             (quant_zp if spec.attention == "sdpa" else quant)("q_rope", q, "q")
@@ -305,46 +306,46 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
 
         map_pending = None
         if spec.attention == "map":
-            s = heads_matmul(q, k.transpose(-2, -1))
-            del q, k
-            # scale, mask and softmax in one pass over the scores, in place; once the threshold is
-            # frozen the same pass also counts the entries the compaction keeps
+            # scores, scale, mask, softmax and the output without a dense map in memory; the kept entries follow from a
+            # second walk over the scores.  While calibrating (the threshold is a statistic of the whole map) and in the
+            # uncompressed layer the same kernel writes the map as well.
             m = attention_mask
-            if m is not None and not (m.dim() == 4 and m.shape[1] == 1 and m.shape[0] in (1, s.shape[0])
-                                      and tuple(m.shape[2:]) == tuple(s.shape[2:])):
-                m = m.expand(s.shape[0], 1, *s.shape[2:]) if m.dim() == 4 and m.shape[1] == 1 else None
-            seg = None
-            if s.dtype == torch.bfloat16 and s.shape[-1] % 8 == 0 and s.shape[-1] <= 8192 and \
-                    (attention_mask is None or m is not None):
-                if calib or raw:
-                    a = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, inplace=True)
-                else:
-                    a, seg = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, threshold=sv['a']['outlier'], inplace=True)
+            if m is not None and not (m.dim() == 4 and m.shape[1] == 1 and m.shape[0] in (1, q.shape[0])
+                                      and tuple(m.shape[2:]) == (q.shape[2], k.shape[2])):
+                m = m.expand(q.shape[0], 1, q.shape[2], k.shape[2]) if m.dim() == 4 and m.shape[1] == 1 else None
+            frozen = not (calib or raw)
+            att = a = seg = None
+            if (attention_mask is None or m is not None) and map_supported(q, k, v, m):
+                att = MapAttention(q, k, v, m, threshold=sv['a']['outlier'] if frozen else None, want_map=not frozen)
+                a, o = att.map, att.o
             else:
-                s = s / math.sqrt(head_dim)
-                if attention_mask is not None:
-                    s = s + attention_mask
-                a = torch.softmax(s, dim=-1, dtype=v.dtype)
-            del s
+                k, v = repeat_kv(k, q.shape[1] // k.shape[1]), repeat_kv(v, q.shape[1] // v.shape[1])
+                s = heads_matmul(q, k.transpose(-2, -1))
+                if s.dtype == torch.bfloat16 and s.shape[-1] % 8 == 0 and s.shape[-1] <= 8192 and \
+                        (attention_mask is None or m is not None):
+                    if frozen:
+                        a, seg = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, threshold=sv['a']['outlier'], inplace=True)
+                    else:
+                        a = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, inplace=True)
+                else:
+                    s = s / math.sqrt(head_dim)
+                    if attention_mask is not None:
+                        s = s + attention_mask
+                    a = torch.softmax(s, dim=-1, dtype=v.dtype)
+                del s
+            del q, k
             if raw:
                 saved["a_raw"] = a
             else:
-                thr = get_statistics_softmax(a, softmax_outlier_ratio) if calib else sv['a']['outlier']
+                thr = sv['a']['outlier'] if frozen else get_statistics_softmax(a, softmax_outlier_ratio)
                 stats[("a", "outlier")] = thr
-                capacity = None if (calib or host_state is None) else host_state.get("map_capacity")
-                if capacity is None:
-                    # sizes the lists from nnz read back from the device, as to_sparse() does
-                    saved["a_idx"], saved["a_val"], saved["a_seg"] = compress_attention_map(a, thr, seg)
-                    if host_state is not None:
-                        _note_map_entries(host_state, saved["a_idx"].numel())
-                else:
-                    # frozen threshold: the lists get room for a little more than the recent steps
-                    # needed and nothing is read back here; whether they fitted is looked at after the
-                    # o projection has been enqueued (the map is kept until then)
-                    saved["a_idx"], saved["a_val"], saved["a_seg"], count = compress_attention_map(a, thr, seg, capacity=capacity)
-                    map_pending = (a, thr, count, capacity)
-            o = heads_matmul(a, v, out_hidden=True)
-            del a, v
+                map_pending = keep_map_entries(saved, a if att is None or not frozen else att, thr, seg,
+                                               host_state if frozen else None)
+                if not frozen and host_state is not None:
+                    _note_map_entries(host_state, saved["a_idx"].numel())
+            if att is None:
+                o = heads_matmul(a, v, out_hidden=True)
+            del a, v, att
         else:
             # causal attention without a map: the row log-sum-exps come back with the output and backward needs
             # no second forward (the reference keeps flash-attn's softmax_lse the same way,
@@ -387,15 +388,9 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
         quant("o", o)
         del o
         if map_pending is not None:
-            # The dense map (B*H*S*S bf16, 537 MB at 2 x 32 x 2048^2) is let go before the MLP block allocates
-            # its gate / up tensors.  The wait is for the compaction only, which was enqueued before the two
-            # attention products and the o projection the device still has to run.
-            a, thr, count, capacity = map_pending
-            nnz = count.value()
-            if nnz > capacity:                    # did not fit: write the lists again at their exact size
-                saved["a_idx"], saved["a_val"], saved["a_seg"] = compress_attention_map(a, thr, saved["a_seg"])
-            _note_map_entries(host_state, nnz)
-            del a, map_pending
+            # What the lists are written from (a dense map or q and k) is let go before the MLP block allocates its gate /
+            # up tensors.  The wait is for the kept entries only, which were enqueued before the o projection.
+            check_map_entries(saved, map_pending, host_state)
             map_pending = None
 
         # ---- MLP block ---------------------------------------------------------------------------
@@ -474,7 +469,6 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
         W = {n: (rest[4 * i], rest[4 * i + 1], ctx.quant_states[n], rest[4 * i + 2], rest[4 * i + 3])
              for i, n in enumerate(_PROJ)}
         H, KV, D = ctx.num_heads, ctx.num_key_value_heads, ctx.head_dim
-        n_rep = H // KV
         G = {}                                           # LoRA gradients
 
         def deq(name, **kw):
@@ -626,11 +620,15 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                     t = rope_forward(t.transpose(1, 2), cos, sin).transpose(1, 2)
                 return t
             q, k, v = rebuilt("q", H), rebuilt("k", KV), rebuilt("v", KV)
-            if not (spec.attention == "sdpa" and ctx.own_flash):
-                k, v = repeat_kv(k, n_rep), repeat_kv(v, n_rep)
             del qkv
+        own_map = spec.attention == "map" and "a_raw" not in S and map_supported(q, k, v)
+        if not (own_map or (spec.attention == "sdpa" and ctx.own_flash)):
+            k, v = repeat_kv(k, H // k.shape[1]), repeat_kv(v, H // v.shape[1])
 
-        if spec.attention == "map":
+        if own_map:
+            grad_q, grad_k, grad_v = map_backward(grad_o, q, k, v, S["a_idx"], S["a_val"], S["a_seg"])
+            del q, k, v, grad_o
+        elif spec.attention == "map":
             # grad_a first, then the restored map and the softmax backward come out of one pass over
             # the compressed map (the reference restores, then reads the dense map twice more)
             grad_a = heads_matmul(grad_o, v.transpose(-2, -1))
@@ -695,6 +693,40 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 + (grad_nw2, None)
                 + lora_grads("gate") + lora_grads("up") + lora_grads("down")
                 + (None,) * 12)
+
+
+def keep_map_entries(saved, source, thr, seg, host_state):
+    """Keeps the entries of the attention map above `thr` in `saved`; `source` is the dense map (with its segment offsets
+    `seg`, if the softmax pass counted them) or a MapAttention.  Without a host state that knows the recent counts the lists
+    are sized from a count read back from the device, as to_sparse() does.  With one they get room for a little more than
+    the recent steps needed and nothing is read back here; whether they fitted is looked at later, by check_map_entries
+    with what is returned."""
+    capacity = None if host_state is None else host_state.get("map_capacity")
+    own = isinstance(source, MapAttention)
+    if capacity is None:
+        if own:
+            seg = source.entries(0)[2]
+            saved["a_idx"], saved["a_val"], saved["a_seg"] = source.entries(int(seg[-1].item()), seg)
+        else:
+            saved["a_idx"], saved["a_val"], saved["a_seg"] = compress_attention_map(source, thr, seg)
+        if host_state is not None:
+            _note_map_entries(host_state, saved["a_idx"].numel())
+        return None
+    if own:
+        saved["a_idx"], saved["a_val"], saved["a_seg"], count = source.bounded_entries(capacity)
+    else:
+        saved["a_idx"], saved["a_val"], saved["a_seg"], count = compress_attention_map(source, thr, seg, capacity=capacity)
+    return source, thr, count, capacity
+
+
+def check_map_entries(saved, pending, host_state):
+    """Writes the lists of keep_map_entries again at their exact size if they did not fit."""
+    source, thr, count, capacity = pending
+    nnz = count.value()
+    if nnz > capacity:
+        saved["a_idx"], saved["a_val"], saved["a_seg"] = source.entries(nnz, saved["a_seg"]) if isinstance(source, MapAttention) else \
+            compress_attention_map(source, thr, saved["a_seg"])
+    _note_map_entries(host_state, nnz)
 
 
 MAP_HISTORY = 8            # steps whose kept-entry counts size the next step's attention-map lists

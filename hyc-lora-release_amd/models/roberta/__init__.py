@@ -25,7 +25,8 @@ from ...operators.softmax_kernels import softmax_backward, softmax_backward_from
 from ...operators import lora_kernels
 from ..compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum,
                             lora_parts)
-from ..fused_decoder_layer import _note_map_entries, lora_linear_parts
+from ...operators.map_kernels import MapAttention, map_backward, map_supported
+from ..fused_decoder_layer import _note_map_entries, check_map_entries, keep_map_entries, lora_linear_parts
 
 MODES = ("baseline", "intra", "intra_inter")
 _PROJ = ("q", "k", "v", "o", "up", "down")
@@ -120,45 +121,42 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
         if whole:
             quant("q", q)
             quant("k", k)
-        s = heads_matmul(q, k.transpose(-2, -1))
-        del q, k
         m = attention_mask
-        fits = m is None or (m.dim() == 4 and m.shape[1] == 1 and m.shape[0] in (1, s.shape[0]) and
-                             m.shape[-1] == s.shape[-1] and m.shape[2] in (1, s.shape[2]))
-        if s.dtype == torch.bfloat16 and s.shape[-1] % 8 == 0 and s.shape[-1] <= 8192 and fits:
-            if m is not None and m.shape[2] == 1:                # padding mask [B,1,1,S]: one row for all queries
-                m = m.expand(m.shape[0], 1, s.shape[2], s.shape[3])
-            seg = None
-            if calib or raw:
-                a = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, inplace=True)
-            else:
-                a, seg = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, threshold=sv['a']['outlier'], inplace=True)
+        fits = m is None or (m.dim() == 4 and m.shape[1] == 1 and m.shape[0] in (1, q.shape[0]) and
+                             m.shape[-1] == k.shape[2] and m.shape[2] in (1, q.shape[2]))
+        frozen = not (calib or raw)
+        att = a = seg = None
+        if fits and map_supported(q, k, v, m):
+            # scores to output without a dense map in memory (with it while calibrating and in the uncompressed layer)
+            att = MapAttention(q, k, v, m, threshold=sv['a']['outlier'] if frozen else None, want_map=not frozen)
+            a, o = att.map, att.o
         else:
-            seg = None
-            s = s / math.sqrt(head_dim)
-            if attention_mask is not None:
-                s = s + attention_mask
-            a = torch.softmax(s, dim=-1, dtype=v.dtype)
-        del s
-        o = heads_matmul(a, v, out_hidden=True)
+            s = heads_matmul(q, k.transpose(-2, -1))
+            if s.dtype == torch.bfloat16 and s.shape[-1] % 8 == 0 and s.shape[-1] <= 8192 and fits:
+                if m is not None and m.shape[2] == 1:                # padding mask [B,1,1,S]: one row for all queries
+                    m = m.expand(m.shape[0], 1, s.shape[2], s.shape[3])
+                if frozen:
+                    a, seg = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, threshold=sv['a']['outlier'], inplace=True)
+                else:
+                    a = softmax_forward(s, 1.0 / math.sqrt(head_dim), m, inplace=True)
+            else:
+                s = s / math.sqrt(head_dim)
+                if attention_mask is not None:
+                    s = s + attention_mask
+                a = torch.softmax(s, dim=-1, dtype=v.dtype)
+            del s
+            o = heads_matmul(a, v, out_hidden=True)
+        del q, k
         map_pending = None
         if raw:
             saved["a_raw"] = a
         else:
-            thr = get_statistics_softmax(a, softmax_outlier_ratio) if calib else sv['a']['outlier']
+            thr = sv['a']['outlier'] if frozen else get_statistics_softmax(a, softmax_outlier_ratio)
             stats[("a", "outlier")] = thr
-            capacity = None if (calib or host_state is None) else host_state.get("map_capacity")
-            if capacity is None:
-                # sizes the lists from nnz read back from the device, as to_sparse() does
-                saved["a_idx"], saved["a_val"], saved["a_seg"] = compress_attention_map(a, thr, seg)
-                if host_state is not None:
-                    _note_map_entries(host_state, saved["a_idx"].numel())
-            else:
-                # frozen threshold: lists with room for a little more than the recent steps needed, nothing read
-                # back here; whether they fitted is looked at once the o projection has been enqueued
-                saved["a_idx"], saved["a_val"], saved["a_seg"], count = compress_attention_map(a, thr, seg, capacity=capacity)
-                map_pending = (a, thr, count, capacity)
-        del a
+            map_pending = keep_map_entries(saved, a if att is None or not frozen else att, thr, seg, host_state if frozen else None)
+            if not frozen and host_state is not None:
+                _note_map_entries(host_state, saved["a_idx"].numel())
+        del a, att
         if whole:
             quant("v", v)
         del v
@@ -167,12 +165,8 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
         quant("o", o)
         del o
         if map_pending is not None:
-            a, thr, count, capacity = map_pending
-            nnz = count.value()                   # waits for the compaction only, enqueued before the projection
-            if nnz > capacity:                    # did not fit: write the lists again at their exact size
-                saved["a_idx"], saved["a_val"], saved["a_seg"] = compress_attention_map(a, thr, saved["a_seg"])
-            _note_map_entries(host_state, nnz)
-            del a, map_pending
+            check_map_entries(saved, map_pending, host_state)      # waits for the kept entries only, enqueued before the projection
+            del map_pending
 
         # ---- first LayerNorm (post-norm: on the residual sum) ----------------------------------
         x_medium, saved["mean_1"], saved["rstd_1"], _, _ = layernorm_forward(o_final, norm_weight_1, norm_bias_1, _EPS)
@@ -279,24 +273,26 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
             v = deq("v", is_head=True, num_heads=H)
         else:
             v = hidden_to_head_shape(rebuilt("v"), H)
-        grad_a = heads_matmul(grad_o, v.transpose(-2, -1))
-        del v
-        if "a_raw" in S:
-            a = S["a_raw"]
-            grad_s = softmax_backward(a, grad_a) / math.sqrt(D)
-        else:
-            a, grad_s = softmax_backward_from_compressed(S["a_idx"], S["a_val"], S["a_seg"], grad_a,
-                                                         out_scale=1.0 / math.sqrt(D))
-        del grad_a
-        grad_v = heads_matmul(a.transpose(-2, -1), grad_o, out_hidden=True)
-        del a, grad_o
         if whole:
             q, k = deq("q", is_head=True, num_heads=H), deq("k", is_head=True, num_heads=H)
         else:
             q, k = hidden_to_head_shape(rebuilt("q"), H), hidden_to_head_shape(rebuilt("k"), H)
-        grad_k = heads_matmul(grad_s.transpose(-2, -1), q, out_hidden=True)
-        grad_q = heads_matmul(grad_s, k, out_hidden=True)
-        del grad_s, q, k
+        if "a_raw" not in S and map_supported(q, k, v):
+            grad_q, grad_k, grad_v = map_backward(grad_o, q, k, v, S["a_idx"], S["a_val"], S["a_seg"])
+        else:
+            grad_a = heads_matmul(grad_o, v.transpose(-2, -1))
+            if "a_raw" in S:
+                a = S["a_raw"]
+                grad_s = softmax_backward(a, grad_a) / math.sqrt(D)
+            else:
+                a, grad_s = softmax_backward_from_compressed(S["a_idx"], S["a_val"], S["a_seg"], grad_a,
+                                                             out_scale=1.0 / math.sqrt(D))
+            del grad_a
+            grad_v = heads_matmul(a.transpose(-2, -1), grad_o, out_hidden=True)
+            grad_k = heads_matmul(grad_s.transpose(-2, -1), q, out_hidden=True)
+            grad_q = heads_matmul(grad_s, k, out_hidden=True)
+            del a, grad_s
+        del q, k, v, grad_o
         grad_q, grad_k, grad_v = (head_to_hidden_shape(t) for t in (grad_q, grad_k, grad_v))
 
         # q, k and v share their input: their input gradients are added up in one pass

@@ -650,6 +650,43 @@ int hyc_flash_bwd(const void *grad_o, const void *q, const void *k, const void *
                   int64_t D, float scale, int causal, void *stream);
 
 /* ---------------------------------------------------------------------------------------
+ * Attention through a softmax map of which only the largest entries are kept: the products, the softmax and the compaction
+ * without a dense map in memory, and the backward straight from the kept entries.
+ *     t = bf16(bf16(bf16(q k^T) * scale) + mask);   p = bf16(softmax_fp32(t));   o = bf16(p v)
+ *     kept: p > bf16(threshold) and p != 0, or NaN (the rule and the list of hyc_sparse_count / hyc_sparse_write)
+ *     g = bf16(grad_o v^T);  ds = bf16(bf16((g - sum_row bf16(a * g)) * a) * scale)  with a = the kept p, else 0
+ *     grad_q = bf16(ds k);   grad_k = bf16(ds^T q);   grad_v = bf16(a^T grad_o)
+ *
+ * Replaces q @ k^T / sqrt(d) + mask, softmax, a @ v, (a * (a > threshold)).to_sparse() and, in backward, to_dense(), the four
+ * attention products, softmax_backward and the repeat_kv copies (models/llama/fused_llama_layer_intra_inter_full_fuse.py:153-180,
+ * :403-447; operators/compress_function.py:309-317; operators/softmax_kernels.py:7-38).
+ *   q, o, grad_o, grad_q  bf16 [B, S, H, D] contiguous;  k, v, grad_k, grad_v  bf16 [B, S, KV, D] contiguous, H % KV == 0
+ *                (grad_k, grad_v: each query head's rounded to bf16, a group's added in fp32 and rounded); D 64 or 128; S % 8 == 0, S <= 4096;
+ *   mask         bf16 or NULL, added to every head: entry (b, i, j) at b * mask_stride_b + i * mask_stride_row + j (strides
+ *                multiples of 8, 0 broadcasts).  Keys at or below -1e30 cost nothing where 32 rows x 64 keys are all so;
+ *   map          bf16 [B, H, S, S] or NULL: the dense p as well (calibration, uncompressed layers);
+ *   threshold    fp32 on the device or NULL: hyc_map_fwd then leaves in `workspace` what hyc_map_emit needs;
+ *   workspace    hyc_map_workspace(B, S, H) bytes, 16-byte aligned, kept unchanged between hyc_map_fwd and hyc_map_emit.
+ * hyc_map_emit   writes indices int64 / values bf16 [capacity] (entries past `capacity` are not written, as in
+ *                hyc_sparse_write_bounded) and seg_offsets int64 [hyc_sparse_num_segments(B*H*S*S) + 1], whose last element is
+ *                the number of kept entries; same q, k, mask, threshold and scale as the forward.
+ * hyc_map_bwd    takes complete lists of `capacity` >= kept entries (< 2^31); workspace hyc_map_bwd_workspace(...) bytes.
+ * Fixed summation orders, no floating-point atomics: the same bits on every run.
+ */
+int64_t hyc_map_workspace(int64_t B, int64_t S, int64_t H);
+int hyc_map_fwd(const void *q, const void *k, const void *v, const void *mask, int64_t mask_stride_b, int64_t mask_stride_row,
+                void *o, void *map, const float *threshold, void *workspace, int64_t workspace_bytes, int64_t B, int64_t S,
+                int64_t H, int64_t KV, int64_t D, float scale, void *stream);
+int hyc_map_emit(const void *q, const void *k, const void *mask, int64_t mask_stride_b, int64_t mask_stride_row,
+                 const float *threshold, const void *workspace, int64_t workspace_bytes, int64_t capacity, int64_t *indices,
+                 void *values, int64_t *seg_offsets, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D, float scale,
+                 void *stream);
+int64_t hyc_map_bwd_workspace(int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D, int64_t capacity);
+int hyc_map_bwd(const void *grad_o, const void *q, const void *k, const void *v, const int64_t *indices, const void *values,
+                const int64_t *seg_offsets, int64_t capacity, void *workspace, int64_t workspace_bytes, void *grad_q,
+                void *grad_k, void *grad_v, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D, float scale, void *stream);
+
+/* ---------------------------------------------------------------------------------------
  * Memory-only probe, FOR BENCHMARKING: loads n_reads and stores n_writes bf16 [T, N] tensors (1..3 each,
  * arrays of device pointers in host memory, 16-byte aligned, N % 8 == 0) with the access shape of the
  * kernels of this library and no arithmetic of the path, so that the rate the memory system gives a

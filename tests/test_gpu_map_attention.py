@@ -1,0 +1,100 @@
+"""Attention through a sparsely kept map against the separate operators it replaces: the kept entries bit for bit those of the
+compaction of the dense map it writes itself, everything else against float64 of the same formulas."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF16 = torch.bfloat16
+
+
+def operands(b, h, kv, s, d, seed):
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    hidden = lambda heads: (1.4 * torch.randn(b, s, heads, d, generator=gen, device="cuda")).to(BF16).transpose(1, 2)     # noqa: E731
+    return hidden(h), hidden(kv), hidden(kv), hidden(h)
+
+
+def masks(kind, b, s):
+    low = torch.finfo(BF16).min
+    causal = torch.ones(s, s, dtype=torch.bool, device="cuda").triu(1)[None]
+    left = torch.arange(s, device="cuda")[None] < torch.tensor([(s * i) // (b + 1) for i in range(b)], device="cuda")[:, None]
+    if kind == "none":
+        return None
+    if kind == "causal":
+        return torch.zeros(1, 1, s, s, device="cuda", dtype=BF16).masked_fill_(causal, float("-inf"))
+    if kind == "padded":          # left-padded causal batch with a finite mask value: the padded rows attend to nothing of their own
+        return torch.zeros(b, 1, s, s, device="cuda", dtype=BF16).masked_fill_((causal | left[:, None, :])[:, None], low)
+    if kind == "keys":            # one mask row for all queries
+        return torch.zeros(b, 1, 1, s, device="cuda", dtype=BF16).masked_fill_(left.flip(1)[:, None, None], low)
+    return torch.randn(1, 1, s, s, generator=torch.Generator(device="cuda").manual_seed(5), device="cuda").to(BF16)      # a bias
+
+
+def dense(q, k, mask):
+    """The map with the layers' roundings, from float64 scores."""
+    n_rep = q.shape[1] // k.shape[1]
+    kt = k.repeat_interleave(n_rep, 1).double().transpose(-1, -2).contiguous()
+    t = (q.double() @ kt).to(BF16)
+    t = (t.float() * (1.0 / math.sqrt(q.shape[-1]))).to(BF16)
+    if mask is not None:
+        t = (t.float() + mask.float()).to(BF16)
+    return torch.softmax(t.double(), -1)
+
+
+def rel(got, want):
+    return ((got.double() - want.double()).norm() / want.double().norm().clamp_min(1e-30)).item()
+
+
+@pytest.mark.parametrize("kind", ["none", "causal", "padded", "keys", "bias"])
+@pytest.mark.parametrize("b,h,kv,s,d", [(1, 2, 2, 8, 64), (2, 4, 4, 32, 128), (2, 3, 1, 72, 64), (3, 8, 2, 136, 128), (1, 4, 2, 200, 128),
+                                        (2, 2, 2, 256, 64), (1, 2, 1, 520, 128), (1, 1, 1, 4096, 64)])
+def test_forward_and_kept_entries(b, h, kv, s, d, kind):
+    from hyclora_amd.operators.compress_function import compress_attention_map, get_statistics_softmax
+    from hyclora_amd.operators.map_kernels import MapAttention
+    q, k, v, _ = operands(b, h, kv, s, d, seed=s + h)
+    mask = masks(kind, b, s)
+    full = MapAttention(q, k, v, mask, want_map=True)
+    want = dense(q, k, mask)
+    # one bf16 rounding of a value that a score's last bit may move (2^-9 of a score of a few units): a few 2^-9 in the 2-norm
+    assert rel(full.map, want) < 8 * 2 ** -9
+    o = full.map.double() @ v.repeat_interleave(h // kv, 1).double().contiguous()
+    assert rel(full.o, o) < 2 ** -8
+    thr = get_statistics_softmax(full.map, 0.05)
+    for threshold in (thr, torch.zeros((), device="cuda"), torch.full((), -1.0, device="cuda"), torch.full((), 2.0, device="cuda")):
+        idx, val, seg = compress_attention_map(full.map, threshold)
+        part = MapAttention(q, k, v, mask, threshold=threshold)
+        assert torch.equal(part.o, full.o)
+        n = idx.numel()
+        for capacity in (n, n + 100, n // 2):
+            idx2, val2, seg2, count = part.bounded_entries(capacity)
+            assert count.value() == n and torch.equal(seg2, seg)
+            m = min(n, capacity)
+            assert torch.equal(idx2[:m], idx[:m]) and torch.equal(val2[:m], val[:m])
+
+
+@pytest.mark.parametrize("ratio", [0.0, 0.05, 1.0])
+@pytest.mark.parametrize("b,h,kv,s,d", [(1, 2, 2, 8, 64), (2, 4, 4, 32, 128), (2, 3, 1, 72, 64), (3, 8, 2, 136, 128), (1, 4, 2, 200, 128),
+                                        (2, 2, 2, 256, 64), (1, 2, 1, 520, 128), (1, 1, 1, 4096, 64)])
+def test_backward_from_kept_entries(b, h, kv, s, d, ratio):
+    from hyclora_amd.operators.compress_function import compress_attention_map, get_statistics_softmax, restore_attention_map
+    from hyclora_amd.operators.map_kernels import MapAttention, map_backward
+    q, k, v, go = operands(b, h, kv, s, d, seed=s + h)
+    full = MapAttention(q, k, v, masks("causal", b, s), want_map=True)
+    thr = torch.full((), 2.0, device="cuda") if ratio == 0 else torch.zeros((), device="cuda") if ratio == 1 else \
+        get_statistics_softmax(full.map, ratio)
+    idx, val, seg = compress_attention_map(full.map, thr)
+    got = map_backward(go, q, k, v, idx, val, seg)
+    a = restore_attention_map(idx, val, seg, (b, h, s, s))
+    n_rep = h // kv
+    kr, vr = (t.repeat_interleave(n_rep, 1).double().contiguous() for t in (k, v))
+    g = (go.double() @ vr.transpose(-1, -2).contiguous()).to(BF16)
+    dsum = (a.float() * g.float()).to(BF16).double().sum(-1, keepdim=True)
+    ds = (((g.double() - dsum) * a.double()).to(BF16).float() / math.sqrt(d)).to(BF16).double()
+    group = lambda t: t.unflatten(1, (kv, n_rep)).sum(2)                              # noqa: E731
+    want = (ds @ kr, group(ds.transpose(-1, -2).contiguous() @ q.double()), group(a.double().transpose(-1, -2).contiguous() @ go.double()))
+    for x, w, name in zip(got, want, ("grad_q", "grad_k", "grad_v")):
+        assert x.shape == w.shape
+        # the same bf16 operands on both sides, up to last bits of g; fp32 sums and one rounding
+        assert (rel(x, w) < 2 ** -8 if w.norm() > 0 else x.abs().max() == 0), (name, rel(x, w))
+    again = map_backward(go, q, k, v, torch.cat([idx, idx.new_full((7,), -1)]), torch.cat([val, val.new_zeros(7)]), seg)
+    assert all(torch.equal(x, y) for x, y in zip(got, again))          # room past the entries is not read
