@@ -42,6 +42,43 @@ def heads_matmul(a: torch.Tensor, b: torch.Tensor, out_hidden: bool = False):
     return out
 
 
+_GEMM_TILE, _COMPUTE_UNITS = 256, 256
+
+
+def _whole_rounds(rows: int, cols: int) -> int:
+    """Columns of a [rows, cols] product to hand to the library first, 0 = all in one call.
+
+    Its bf16 kernels work on 256 x 256 tiles, one per compute unit and round.  Where the tiles fill whole rounds and a
+    remainder, one call spreads the remainder over all units along the contraction, which costs up to half of the time again;
+    the whole rounds in one call and the remaining columns in another do not.  Measured with the frozen weight as it lies
+    (forward) and transposed (backward), [rows, contraction] x cols:  4096 x 4096 x 11008: 413 -> 271 and 347 -> 307 us;
+    2048 x 4096 x 11008: 160 -> 148, 280 -> 176;  8192 x 4096 x 11008: 645 -> 506, 672 -> 579;  8192 x 5120 x 5120: 447 -> 302,
+    460 -> 339;  8192 x 5120 x 13824: 953 -> 786, 1008 -> 883;  4096 x 2048 x 5504: 90 -> 78, 99 -> 99;  4096 x 4096 x 14336: 333 ->
+    335, 384 -> 378.  Left in one call: a single whole round with more than half of another behind it (2048 x 5120 x 13824: 207 ->
+    218, 232 -> 244), and row counts whose tiles do not divide a round (6144 x 4096 x 14336: 547 -> 668)."""
+    down, across = -(-rows // _GEMM_TILE), -(-cols // _GEMM_TILE)
+    rest = down * across % _COMPUTE_UNITS
+    if _COMPUTE_UNITS % down or down * across <= _COMPUTE_UNITS or rest == 0:
+        return 0
+    if down * across < 2 * _COMPUTE_UNITS and rest > _COMPUTE_UNITS // 2:
+        return 0
+    return (across - rest // down) * _GEMM_TILE
+
+
+def frozen_matmul(x: torch.Tensor, w: torch.Tensor):
+    """x @ w for a frozen weight (or its transposed view) w [K, N]: the library product, in the calls that suit its tiles."""
+    k, n = w.shape
+    rows = x.numel() // max(k, 1)
+    cut = _whole_rounds(rows, n) if x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and not torch.is_grad_enabled() else 0
+    if cut == 0:
+        return x @ w
+    x2 = x.reshape(rows, k)
+    out = torch.empty(rows, n, device=x.device, dtype=x.dtype)
+    torch.mm(x2, w[:, :cut], out=out[:, :cut])
+    torch.mm(x2, w[:, cut:], out=out[:, cut:])
+    return out.view(*x.shape[:-1], n)
+
+
 def dense_weight(w: torch.Tensor, quant_state):
     """Frozen weight as a dense [out, in] matrix.  quant_state None = already dense (the benchmark
     configurations); otherwise a bitsandbytes-format NF4 weight, dequantised by the HIP kernel (the
@@ -70,7 +107,7 @@ def lora_parts(w, w_quant_state, w_lora_a, b, x, x_lora_a=None):
     from `x_lora_a` when the caller has it already (the fused norm kernel forms it)."""
     wt = dense_weight(w, w_quant_state).t()
     x = x.to(wt.dtype)
-    x_main = x @ wt
+    x_main = frozen_matmul(x, wt)
     if b is not None:
         x_main = x_main + b.to(wt.dtype)
     if x_lora_a is None:
@@ -119,7 +156,7 @@ def lora_backward(w, w_quant_state, w_lora_a, w_lora_b, x, x_lora_a, grad_y, x_c
             grad_a = lora_kernels.lora_products(x, u=grad_mid)[0].t()
         else:
             grad_a = x.to(dt).mT @ grad_mid
-    grad_x = grad_y @ wd
+    grad_x = frozen_matmul(grad_y, wd)
     if defer_input:
         return grad_a, grad_b, (grad_x, grad_mid, w_lora_a.mT)
     if lora_kernels.supported(grad_x, grad_mid, w_lora_a.mT) and (accumulate is None or accumulate.dtype == dt):

@@ -62,7 +62,7 @@ from ..operators.triton_fuse_lora_silu_hadamard_forward_kernels import triton_fu
 from ..operators import lora_kernels
 from ..operators.flash_kernels import flash_backward, flash_forward, flash_supported
 from ..operators.map_kernels import MapAttention, map_backward, map_supported
-from .compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum, lora_parts,
+from .compute_utils import (frozen_matmul, head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum, lora_parts,
                             repeat_kv, repeat_kv_backward, rope_backward, rope_forward)
 
 MODES = ("baseline", "intra", "intra_inter", "intra_inter_full_fuse")
@@ -399,8 +399,8 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             from .compute_utils import dense_weight
             wg, wu = dense_weight(w_gate, qs_gate).t(), dense_weight(w_up, qs_up).t()
             x_norm_2 = x_norm_2.to(wg.dtype)
-            gate_main = x_norm_2 @ wg if b_gate is None else x_norm_2 @ wg + b_gate.to(wg.dtype)
-            up_main = x_norm_2 @ wu if b_up is None else x_norm_2 @ wu + b_up.to(wu.dtype)
+            gate_main = frozen_matmul(x_norm_2, wg) if b_gate is None else x_norm_2 @ wg + b_gate.to(wg.dtype)
+            up_main = frozen_matmul(x_norm_2, wu) if b_up is None else x_norm_2 @ wu + b_up.to(wu.dtype)
             gate_lora_a = xa_ready.pop("gate", None)
             up_lora_a = xa_ready.pop("up", None)
             if gate_lora_a is None:
@@ -558,7 +558,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             else:
                 grad_b_down = S["down_lora_a"].to(wd.dtype).mT @ g
                 grad_mid = g @ lb.mT
-            grad_down = g @ wd
+            grad_down = frozen_matmul(g, wd)
             if lora_kernels.supported(grad_down, grad_mid, la.mT):
                 grad_down = lora_kernels.lora_add(grad_down, grad_mid, la.mT, inplace=True)
             else:

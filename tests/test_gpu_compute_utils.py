@@ -104,3 +104,21 @@ def test_attention_products_on_hidden_layout_views(CU, dev, B, n_rep):
     gk = CU.heads_matmul(s.transpose(-2, -1), q, out_hidden=True)
     want = (s.double().transpose(-2, -1) @ q.double()).reshape(B, KV, n_rep, S, D).sum(2)
     assert_close_bf16(CU.repeat_kv_backward(gk, n_rep), want, what="repeat_kv_backward on a strided view")
+
+
+@pytest.mark.parametrize("rows,n,k", [(2048, 2816 + 8192, 128), (1024, 17152, 96), (8192, 2304, 64), (2000, 8448, 64), (256, 65792, 32), (2048, 13824, 64)])
+@pytest.mark.parametrize("transposed", [True, False])
+def test_frozen_matmul_in_whole_rounds(rows, n, k, transposed):
+    """The product in one or two library calls, at sizes on both sides of the rule: the calls' columns meet exactly."""
+    import hyclora_amd  # noqa: F401
+    from hyclora_amd.models import compute_utils as CU
+    g = torch.Generator(device="cuda").manual_seed(rows + n)
+    x = torch.randn(1, rows, k, generator=g, device="cuda").to(torch.bfloat16)
+    w = torch.randn(*((n, k) if transposed else (k, n)), generator=g, device="cuda").to(torch.bfloat16)
+    w = w.t() if transposed else w
+    with torch.no_grad():
+        got = CU.frozen_matmul(x, w)
+    want = x.float() @ w.float()
+    assert got.shape == want.shape and got.is_contiguous()
+    # one bf16 rounding (half a unit of 2^-8) and the order of up to 128 fp32 additions
+    assert ((got.float() - want).abs() <= 2 ** -8 * want.abs() + 1e-4).all()
