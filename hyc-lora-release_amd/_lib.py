@@ -6,6 +6,7 @@ code, an exception is raised — there is no CPU or torch fallback.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import weakref
 from ctypes import c_char_p, c_int, c_int64, c_void_p
 from pathlib import Path
@@ -14,6 +15,7 @@ import torch
 
 _HERE = Path(__file__).resolve().parent
 LIB_PATH = _HERE / "libhyclora.so"
+NATIVE_PATH = _HERE / "_native.so"
 
 _lib = None
 
@@ -131,6 +133,27 @@ def lib() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = handle
     return _lib
+
+
+_native = None
+
+
+def native():
+    """The host side of the operators in native code (csrc/host/native.cpp), loaded once; it has no fallback either."""
+    global _native
+    if _native is None:
+        lib()                                      # the kernel library first: _native.so is linked against it
+        if not NATIVE_PATH.exists():
+            raise RuntimeError(f"{NATIVE_PATH} not found: build it with `python {(_HERE / 'build.py')}`")
+        spec = importlib.util.spec_from_file_location("hyclora_amd._native", NATIVE_PATH)
+        module = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(module)
+        _native = module
+    return _native
+
+
+def raise_error(name: str, code: int):
+    raise HycError(name, code, error_string(code))
 
 
 def error_string(code: int) -> str:

@@ -1,4 +1,5 @@
-"""Build recipe for the gfx950 kernel library (libhyclora.so, next to this file).
+"""Build recipe for the gfx950 kernel library (libhyclora.so, next to this file) and the host side of its operators
+(_native.so).
 
     python hyc-lora-release_amd/build.py            # compile every .hip under csrc/
 
@@ -21,6 +22,10 @@ CSRC = HERE / "csrc"
 OBJ = CSRC / "_obj"
 LIB = HERE / "libhyclora.so"
 
+HOST_SRC = CSRC / "host" / "native.cpp"
+NATIVE = HERE / "_native.so"
+
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -61,7 +66,25 @@ def build(verbose: bool = True, only=None) -> Path:
     with ThreadPoolExecutor(jobs) as pool:
         list(pool.map(lambda c: _run(c, verbose), todo))
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(LIB), *objects], verbose)
+    if only is None or HOST_SRC.name in only or not NATIVE.exists():
+        build_native(verbose)
     return LIB
+
+
+def build_native(verbose: bool = True) -> Path:
+    """Compile the host side of the operators (csrc/host/native.cpp, plain C++) into _native.so, a Python module that is
+    linked against torch and libhyclora.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    include = [f"-I{p}" for p in [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], ROCM + "/include"]]
+    libs = [f"-L{p}" for p in [*cpp_extension.library_paths(), str(HERE)]]
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    _run([os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-DTORCH_API_INCLUDE_EXTENSION_H", *include, str(HOST_SRC), "-o", str(NATIVE), *libs,
+          "-lc10", "-ltorch_cpu", "-ltorch", "-ltorch_python", "-lc10_hip", "-l:libhyclora.so", "-Wl,-rpath,$ORIGIN"], verbose)
+    return NATIVE
 
 
 if __name__ == "__main__":

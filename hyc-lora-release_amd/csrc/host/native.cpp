@@ -1,0 +1,511 @@
+// The host side of the operators in native code: argument checks, output and workspace allocation, the library products and
+// the launches that one Python wrapper makes, in one call.  A layer step on a short sequence is bound by the host (7B widths,
+// one sample of 96 tokens: 1.7 ms of Python, ctypes and torch calls for 0.7 ms of kernels), so what the wrappers do per call
+// matters as much as the kernels there.
+//
+// Every function takes the operands the layers hand over - bf16, contiguous, 16-byte aligned, on the device, of matching
+// shapes - and returns nothing when they are anything else; the Python wrapper then converts, copies or refuses them.  No
+// state is kept.
+#include <torch/extension.h>
+
+#include <c10/hip/HIPStream.h>
+
+#include <optional>
+#include <tuple>
+#include <vector>
+
+#include "../../../include/hyclora.h"
+
+namespace {
+
+using at::Tensor;
+using OptT = std::optional<Tensor>;
+
+void check(const char* fn, int rc) {
+    if (rc != HYC_OK) {
+        pybind11::gil_scoped_acquire gil;
+        pybind11::module_::import("hyclora_amd._lib").attr("raise_error")(fn, rc);
+    }
+}
+void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+bool aligned(const Tensor& t, uintptr_t a = 16) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % a == 0; }
+bool is_bf(const Tensor& t) { return t.defined() && t.is_cuda() && t.scalar_type() == at::kBFloat16; }
+bool plain(const Tensor& t) { return is_bf(t) && t.is_contiguous() && aligned(t); }
+bool plain_or_none(const OptT& t) { return !t || plain(*t); }
+bool vec(const Tensor& t, int64_t n) { return plain(t) && t.numel() == n; }            // per-channel vector
+void* ptr(const OptT& t) { return t ? t->data_ptr() : nullptr; }
+bool bits_ok(int64_t b) { return b == 2 || b == 4 || b == 8; }
+bool packed(const Tensor& q, int64_t numel, int64_t bits) {
+    return q.defined() && q.is_cuda() && q.scalar_type() == at::kByte && q.is_contiguous() && q.numel() * 8 == numel * bits;
+}
+Tensor bytes_like(const Tensor& x, int64_t n, int64_t bits) {                            // packed codes of a [B, M, n] tensor
+    auto s = x.sizes().vec();
+    s.back() = n * bits / 8;
+    return at::empty(s, x.options().dtype(at::kByte));
+}
+
+// A LoRA operand [R, N]: as it lies, or as the transposed view of an [N, R] weight
+struct Lora {
+    const void* p = nullptr;
+    int transposed = 0;
+    int64_t r = 0, n = 0;
+    bool ok = false;
+    explicit Lora(const Tensor& b) {
+        if (!is_bf(b) || b.dim() != 2) return;
+        r = b.size(0);
+        n = b.size(1);
+        if (b.is_contiguous()) ok = aligned(b);
+        else if (b.stride(0) == 1 && b.stride(1) == r) { transposed = 1; ok = aligned(b, 8); }
+        p = b.data_ptr();
+    }
+    bool fits(int64_t width) const { return ok && n == width && n % 32 == 0 && r % 4 == 0 && r >= 4 && r <= 64; }
+};
+
+// ---- LoRA adds ----------------------------------------------------------------------------------------------------
+OptT lora_add(const Tensor& x, const Tensor& xa, const Tensor& b, const OptT& residual, bool inplace) {
+    const Lora B(b);
+    if (!plain(x) || x.dim() < 1 || !B.fits(x.size(-1)) || x.numel() == 0) return std::nullopt;
+    const int64_t rows = x.numel() / B.n;
+    if (!plain(xa) || xa.dim() < 1 || xa.size(-1) != B.r || xa.numel() != rows * B.r) return std::nullopt;
+    if (residual && (!plain(*residual) || residual->sizes() != x.sizes())) return std::nullopt;
+    Tensor y = inplace ? x : at::empty_like(x);
+    check("hyc_lora_add", hyc_lora_add(xa.data_ptr(), B.p, B.transposed, x.data_ptr(), ptr(residual), y.data_ptr(), rows, B.n, B.r, stream_of(x)));
+    return y;
+}
+
+using Term = std::tuple<Tensor, Tensor, Tensor>;          // x, xa, b
+OptT lora_add_sum(const std::vector<Term>& terms) {
+    if (terms.size() < 2 || terms.size() > 3) return std::nullopt;
+    const Tensor& first = std::get<0>(terms[0]);
+    if (!plain(first) || first.dim() < 1 || first.numel() == 0) return std::nullopt;
+    hyc_lora_sum_member m[3];
+    int64_t r = 0, n = first.size(-1), rows = 0;
+    for (size_t i = 0; i < terms.size(); ++i) {
+        const auto& [x, xa, b] = terms[i];
+        const Lora B(b);
+        if (!plain(x) || x.sizes() != first.sizes() || !B.fits(n) || B.r > 16 || (i && B.r != r)) return std::nullopt;
+        r = B.r;
+        rows = x.numel() / n;
+        if (!plain(xa) || xa.size(-1) != r || xa.numel() != rows * r) return std::nullopt;
+        m[i] = {xa.data_ptr(), B.p, B.transposed, x.data_ptr()};
+    }
+    check("hyc_lora_add_sum", hyc_lora_add_sum(m, (int)terms.size(), first.data_ptr(), rows, n, r, stream_of(first)));
+    return first;
+}
+
+struct Rope {                                              // the two angle tables of a rotation
+    Tensor cos, sin;
+    bool ok = false, fp32 = false;
+    Rope(const Tensor& c, const Tensor& s, int64_t seq, int64_t half) {
+        auto table = [&](const Tensor& t) {
+            Tensor v = t.dim() == 3 && t.size(0) == 1 ? t.squeeze(0) : t;
+            const bool good = v.is_cuda() && v.dim() == 2 && v.size(0) > 1 && v.size(0) >= seq && v.size(1) >= half && v.stride(1) == 1 &&
+                              v.stride(0) % 8 == 0 && aligned(v);
+            return good ? v : Tensor();
+        };
+        cos = table(c);
+        sin = table(s);
+        ok = cos.defined() && sin.defined() && cos.scalar_type() == sin.scalar_type() &&
+             (cos.scalar_type() == at::kBFloat16 || cos.scalar_type() == at::kFloat);
+        fp32 = ok && cos.scalar_type() == at::kFloat;
+    }
+};
+
+// (x or codes, xa, b, scale, zero point, cos, sin)
+using Item = std::tuple<Tensor, Tensor, Tensor, Tensor, OptT, OptT, OptT>;
+bool member(const Item& it, int64_t B, int64_t M, int64_t bits, bool restore, bool with_zero, int64_t& rank, std::vector<Rope>& ropes,
+            hyc_lora_add_member& m) {
+    const auto& [x, xa, b, scale, zero, cos, sin] = it;
+    const Lora L(b);
+    if (x.dim() != 3 || x.size(0) != B || x.size(1) != M || x.numel() == 0 || !L.fits(L.n)) return false;
+    if (restore ? !(packed(x, B * M * L.n, bits) && aligned(x)) : !(plain(x) && x.size(2) == L.n)) return false;
+    if (rank && L.r != rank) return false;
+    rank = L.r;
+    if (!plain(xa) || xa.size(-1) != L.r || xa.numel() != B * M * L.r || !vec(scale, L.n)) return false;
+    if (zero.has_value() != with_zero || (zero && !vec(*zero, L.n))) return false;
+    m = {};
+    m.xa = xa.data_ptr(); m.b = L.p; m.b_transposed = L.transposed; m.scale = scale.data_ptr(); m.zero_point = ptr(zero); m.N = L.n;
+    if (restore) m.q = x.data_ptr();
+    else m.x = x.data_ptr();
+    if (cos) {
+        if (!sin || L.n % 128) return false;
+        ropes.emplace_back(*cos, *sin, M, 64);
+        const Rope& R = ropes.back();
+        if (!R.ok) return false;
+        m.cos_t = R.cos.data_ptr(); m.sin_t = R.sin.data_ptr(); m.table_is_fp32 = R.fp32;
+        m.seq_len = M; m.stride_cos = R.cos.stride(0); m.stride_sin = R.sin.stride(0);
+    }
+    return true;
+}
+
+std::optional<std::vector<std::tuple<Tensor, Tensor>>> lora_add_quant_group(const std::vector<Item>& items, int64_t bits, bool inplace) {
+    if (items.empty() || items.size() > 4 || !bits_ok(bits) || std::get<0>(items[0]).dim() != 3) return std::nullopt;
+    const int64_t B = std::get<0>(items[0]).size(0), M = std::get<0>(items[0]).size(1);
+    const bool with_zero = std::get<4>(items[0]).has_value();
+    hyc_lora_add_member m[4];
+    std::vector<Rope> ropes;
+    ropes.reserve(4);
+    int64_t rank = 0;
+    for (size_t i = 0; i < items.size(); ++i)
+        if (!member(items[i], B, M, bits, false, with_zero, rank, ropes, m[i])) return std::nullopt;
+    std::vector<std::tuple<Tensor, Tensor>> out;
+    for (size_t i = 0; i < items.size(); ++i) {
+        const Tensor& x = std::get<0>(items[i]);
+        Tensor y = inplace ? x : at::empty_like(x), q = bytes_like(x, m[i].N, bits);
+        m[i].q = q.data_ptr();
+        m[i].y = y.data_ptr();
+        out.emplace_back(q, y);
+    }
+    check("hyc_lora_add_quant_group", hyc_lora_add_quant_group(m, (int)items.size(), B * M, rank, (int)bits, stream_of(std::get<0>(items[0]))));
+    return out;
+}
+
+std::optional<std::vector<Tensor>> lora_add_restore_group(const std::vector<Item>& items, int64_t bits) {
+    if (items.empty() || items.size() > 4 || !bits_ok(bits) || std::get<0>(items[0]).dim() != 3) return std::nullopt;
+    const int64_t B = std::get<0>(items[0]).size(0), M = std::get<0>(items[0]).size(1);
+    const bool with_zero = std::get<4>(items[0]).has_value();
+    hyc_lora_add_member m[4];
+    std::vector<Rope> ropes;
+    ropes.reserve(4);
+    int64_t rank = 0;
+    for (size_t i = 0; i < items.size(); ++i)
+        if (!member(items[i], B, M, bits, true, with_zero, rank, ropes, m[i])) return std::nullopt;
+    std::vector<Tensor> out;
+    for (size_t i = 0; i < items.size(); ++i) {
+        out.push_back(at::empty({B, M, m[i].N}, std::get<1>(items[i]).options()));
+        m[i].y = out.back().data_ptr();
+    }
+    check("hyc_lora_add_restore_group", hyc_lora_add_restore_group(m, (int)items.size(), B * M, rank, (int)bits, stream_of(out[0])));
+    return out;
+}
+
+// ---- rank-R products ----------------------------------------------------------------------------------------------
+// (u^T x, x v^T) of a dense x [.., N] or, the first only, of packed codes [B, M, N * bits / 8]
+std::optional<std::tuple<OptT, OptT>> contract(const OptT& x, const OptT& q, const OptT& scale, const OptT& zero, int64_t bits, const OptT& u,
+                                               const OptT& v, int64_t n, bool p1_transposed) {
+    if (!u && !v) return std::nullopt;
+    const Tensor& src = x ? *x : *q;
+    if (n <= 0 || n % 32) return std::nullopt;
+    int64_t T = 0;
+    if (x) {
+        if (!plain(*x) || x->size(-1) != n || x->numel() == 0) return std::nullopt;
+        T = x->numel() / n;
+    } else {
+        if (!bits_ok(bits) || !q->is_contiguous() || q->numel() == 0 || (q->numel() * 8) % (n * bits)) return std::nullopt;
+        T = q->numel() * 8 / (n * bits);
+        if (!packed(*q, T * n, bits) || !aligned(*q) || v || !scale || !vec(*scale, n) || (zero && !vec(*zero, n))) return std::nullopt;
+    }
+    int64_t r = u ? u->size(-1) : v->size(0);
+    if (r % 2 || r < 2 || r > 64) return std::nullopt;
+    if (u && (!plain(*u) || u->numel() != T * r)) return std::nullopt;
+    const void* vp = nullptr;
+    int vt = 0;
+    if (v) {
+        const Lora V(*v);
+        if (!V.ok || V.r != r || V.n != n) return std::nullopt;
+        vp = V.p;
+        vt = V.transposed;
+    }
+    const auto o = src.options().dtype(at::kBFloat16);
+    const int64_t bytes = hyc_lora_contract_workspace(T, n, r, u.has_value(), v.has_value());
+    Tensor ws = at::empty({std::max<int64_t>(bytes, 16)}, src.options().dtype(at::kByte));
+    OptT p1, p2;
+    if (u) p1 = p1_transposed ? at::empty({n, r}, o) : at::empty({r, n}, o);
+    if (v) {
+        auto s = src.sizes().vec();
+        s.back() = r;
+        p2 = at::empty(s, o);
+    }
+    check("hyc_lora_contract", hyc_lora_contract(ptr(x), x ? nullptr : q->data_ptr(), x ? nullptr : scale->data_ptr(), x ? nullptr : ptr(zero),
+                                                 x ? 0 : (int)bits, ptr(u), vp, vt, ptr(p1), p1_transposed, ptr(p2), ws.data_ptr(), ws.numel(), T,
+                                                 n, r, stream_of(src)));
+    return std::make_tuple(p1, p2);
+}
+
+// ---- products with a frozen weight --------------------------------------------------------------------------------
+// Columns to hand to the library first (0: all in one call); the rule and its figures stand at _whole_rounds in
+// models/compute_utils.py.
+int64_t whole_rounds(int64_t rows, int64_t cols) {
+    constexpr int64_t tile = 256, units = 256;
+    const int64_t down = (rows + tile - 1) / tile, across = (cols + tile - 1) / tile, rest = down * across % units;
+    if (units % down || down * across <= units || rest == 0 || (down * across < 2 * units && rest > units / 2)) return 0;
+    return (across - rest / down) * tile;
+}
+Tensor frozen_product(const Tensor& x, const Tensor& w) {          // x [.., K] contiguous, w [K, N]
+    const int64_t k = w.size(0), n = w.size(1), rows = x.numel() / k;
+    auto shape = x.sizes().vec();
+    shape.back() = n;
+    const Tensor x2 = x.view({rows, k});
+    const int64_t cut = whole_rounds(rows, n);
+    if (cut == 0) return at::mm(x2, w).view(shape);
+    Tensor out = at::empty({rows, n}, x.options());
+    Tensor a = out.narrow(1, 0, cut), b = out.narrow(1, cut, n - cut);
+    at::mm_out(a, x2, w.narrow(1, 0, cut));
+    at::mm_out(b, x2, w.narrow(1, cut, n - cut));
+    return out.view(shape);
+}
+bool weight_ok(const Tensor& w, int64_t in) { return is_bf(w) && w.dim() == 2 && w.size(1) == in && w.is_contiguous(); }
+
+// -> (x W^T, x A)
+std::optional<std::tuple<Tensor, Tensor>> lora_parts(const Tensor& w, const Tensor& la, const Tensor& x, const OptT& xa) {
+    if (at::GradMode::is_enabled() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !weight_ok(w, x.size(-1))) return std::nullopt;
+    if (!is_bf(la) || la.dim() != 2 || la.size(0) != x.size(-1) || (xa && !is_bf(*xa))) return std::nullopt;
+    Tensor main = frozen_product(x, w.t());
+    if (xa) return std::make_tuple(main, *xa);
+    auto shape = x.sizes().vec();
+    shape.back() = la.size(1);
+    return std::make_tuple(main, at::mm(x.view({-1, la.size(0)}), la).view(shape));
+}
+
+// -> (x W^T + (x A) B [+ residual], x W^T, x A)
+std::optional<std::tuple<Tensor, Tensor, Tensor>> lora_forward(const Tensor& w, const Tensor& la, const Tensor& lb, const Tensor& x,
+                                                               const OptT& residual, const OptT& xa) {
+    const Lora L(lb);
+    if (w.dim() != 2 || !L.fits(w.size(0)) || !plain(x) || x.dim() < 2 || x.numel() == 0 || !is_bf(la) || la.dim() != 2 || la.size(1) != L.r)
+        return std::nullopt;
+    auto shape = x.sizes().vec();
+    const int64_t rows = x.numel() / shape.back();
+    shape.back() = L.n;
+    if ((residual && !(plain(*residual) && residual->sizes() == at::IntArrayRef(shape))) ||
+        (xa && !(plain(*xa) && xa->size(-1) == L.r && xa->numel() == rows * L.r)))
+        return std::nullopt;
+    auto parts = lora_parts(w, la, x, xa);
+    if (!parts) return std::nullopt;
+    auto& [main, a] = *parts;
+    OptT y = lora_add(main, a, lb, residual, false);
+    TORCH_CHECK(y.has_value(), "LoRA operands do not match: x A is ", a.sizes(), ", B is ", lb.sizes(), ", x W^T is ", main.sizes());
+    return std::make_tuple(*y, main, a);
+}
+
+// lora_backward of models/compute_utils.py: -> (grad A, grad B, grad x) or, deferred, (grad A, grad B, (grad_y W, grad_y B^T, A^T))
+pybind11::object lora_backward(const Tensor& w, const Tensor& la, const Tensor& lb, const OptT& x, const OptT& q, const OptT& scale,
+                               const OptT& zero, int64_t bits, const Tensor& xa, const Tensor& grad_y, const OptT& accumulate, bool defer) {
+    const pybind11::object none = pybind11::none();
+    const Lora L(lb);
+    if (at::GradMode::is_enabled() || !plain(grad_y) || grad_y.numel() == 0 || !is_bf(w) || w.dim() != 2 || !w.is_contiguous() ||
+        w.size(0) != grad_y.size(-1) || !L.fits(w.size(0)) || !plain(xa) || !is_bf(la) || la.dim() != 2 || la.size(0) != w.size(1) ||
+        la.size(1) != L.r || w.size(1) % 32)
+        return none;
+    const Tensor at_ = la.t();                                     // A^T [R, in]
+    if (!Lora(at_).fits(w.size(1)) || !plain_or_none(accumulate)) return none;
+    if (x ? !(plain(*x) && x->size(-1) == w.size(1)) : !(q && scale && vec(*scale, w.size(1)) && (!zero || vec(*zero, w.size(1))))) return none;
+    auto both = contract(grad_y, std::nullopt, std::nullopt, std::nullopt, 0, xa, lb, w.size(0), true);
+    if (!both) return none;
+    const Tensor grad_b = std::get<0>(*both)->t(), grad_mid = *std::get<1>(*both);
+    auto ga = x ? contract(x, std::nullopt, std::nullopt, std::nullopt, 0, grad_mid, std::nullopt, w.size(1), false)
+                : contract(std::nullopt, q, scale, zero, bits, grad_mid, std::nullopt, w.size(1), false);
+    if (!ga) return none;
+    const Tensor grad_a = std::get<0>(*ga)->t();
+    Tensor grad_x = frozen_product(grad_y, w);
+    if (defer) return pybind11::make_tuple(grad_a, grad_b, pybind11::make_tuple(grad_x, grad_mid, at_));
+    OptT sum = lora_add(grad_x, grad_mid, at_, accumulate, true);
+    TORCH_CHECK(sum.has_value(), "LoRA operands do not match: grad x is ", grad_x.sizes(), ", A^T is ", at_.sizes());
+    return pybind11::make_tuple(grad_a, grad_b, *sum);
+}
+
+// ---- quantise / dequantise ----------------------------------------------------------------------------------------
+std::optional<std::tuple<OptT, Tensor>> quantize(const Tensor& x, const Tensor& s, const OptT& z, const OptT& channel, int64_t bits) {
+    if (!plain(x) || x.dim() != 3 || x.numel() == 0 || !bits_ok(bits)) return std::nullopt;
+    const int64_t B = x.size(0), M = x.size(1), N = x.size(2);
+    if (N % 32 || !vec(s, N) || (z && !vec(*z, N))) return std::nullopt;
+    if (channel && !(channel->is_cuda() && channel->scalar_type() == at::kLong && channel->is_contiguous())) return std::nullopt;
+    const int64_t k = channel ? channel->numel() : 0;
+    Tensor q = bytes_like(x, N, bits);
+    OptT kept;
+    if (channel) kept = at::zeros({B, M, k}, x.options());         // a list position without a column reads as zeros
+    check("hyc_quant_pack", hyc_quant_pack(x.data_ptr(), s.data_ptr(), ptr(z), q.data_ptr(), k ? (const int64_t*)channel->data_ptr() : nullptr, k,
+                                           k ? kept->data_ptr() : nullptr, 0, B, M, N, M * N, N, N, 0, (int)bits, stream_of(x)));
+    return std::make_tuple(kept, q);
+}
+
+OptT dequantize(const Tensor& q, const Tensor& s, const OptT& z, const OptT& kept, const OptT& channel, int64_t bits) {
+    if (!bits_ok(bits) || q.dim() != 3 || q.numel() == 0 || s.dim() < 1) return std::nullopt;
+    const int64_t B = q.size(0), M = q.size(1), N = s.size(-1);
+    if (N % 32 || !packed(q, B * M * N, bits) || !aligned(q) || !vec(s, N) || (z && !vec(*z, N))) return std::nullopt;
+    int64_t k = 0;
+    if (channel) {
+        k = channel->numel();
+        if (!channel->is_cuda() || channel->scalar_type() != at::kLong || !channel->is_contiguous() || !kept || !is_bf(*kept) ||
+            !kept->is_contiguous() || kept->dim() != 3 || kept->size(0) != B || kept->size(1) != M || kept->size(2) != k)
+            return std::nullopt;
+    }
+    Tensor x = at::empty({B, M, N}, s.options());
+    check("hyc_unpack_dequant", hyc_unpack_dequant(q.data_ptr(), s.data_ptr(), ptr(z), x.data_ptr(), k ? (const int64_t*)channel->data_ptr() : nullptr,
+                                                   k, k ? kept->data_ptr() : nullptr, B, M, N, M * N, N, N, 0, (int)bits, stream_of(x)));
+    return x;
+}
+
+// ---- norms --------------------------------------------------------------------------------------------------------
+bool table_ok(const OptT& table, int64_t n) {
+    return table && table->is_cuda() && table->scalar_type() == at::kShort && table->numel() == n && table->is_contiguous();
+}
+
+// -> (y, rstd, q_y, q_x, x_outlier, [y @ a]) of rmsnorm_forward_compress; k outlier channels, in `table`
+using Normed = std::tuple<Tensor, Tensor, OptT, OptT, OptT, std::vector<Tensor>>;
+std::optional<Normed> norm_compress(const Tensor& x, const Tensor& w, double eps, int64_t bits, const OptT& scale_y, const OptT& scale_x,
+                                    const OptT& table, int64_t k, const std::vector<Tensor>& lora_a) {
+    if (!plain(x) || x.dim() != 3 || x.numel() == 0 || !bits_ok(bits) || !plain(w)) return std::nullopt;
+    const int64_t n = x.size(2), rows = x.numel() / n;
+    if (n % 32 || n > 8192 || w.numel() != n || (scale_y && !vec(*scale_y, n)) || (scale_x && !vec(*scale_x, n))) return std::nullopt;
+    if (!scale_x) k = 0;
+    if (k && !table_ok(table, n)) return std::nullopt;
+    const size_t g = lora_a.size();
+    const void* weights[4];
+    int64_t ranks[4], blocks = 0;
+    if (g) {
+        if (g > 4 || n % 512 || rows % 2) return std::nullopt;
+        for (size_t i = 0; i < g; ++i) {
+            const Tensor& a = lora_a[i];                           // the [N, R] view of a contiguous [R, N] weight
+            if (!is_bf(a) || a.dim() != 2 || a.size(0) != n || a.stride(0) != 1 || a.stride(1) != n || a.size(1) < 1 || a.size(1) > 64 || !aligned(a))
+                return std::nullopt;
+            weights[i] = a.data_ptr();
+            ranks[i] = a.size(1);
+            blocks += (ranks[i] + 15) / 16;
+        }
+        if (blocks > 4) return std::nullopt;
+    }
+    Tensor y = at::empty_like(x), rstd = at::empty({rows}, x.options().dtype(at::kFloat));
+    OptT qy, qx, kept;
+    if (scale_y) qy = bytes_like(x, n, bits);
+    if (scale_x) {
+        qx = bytes_like(x, n, bits);
+        kept = at::empty({x.size(0), x.size(1), k}, x.options());
+    }
+    const uint16_t* tab = k ? (const uint16_t*)table->data_ptr() : nullptr;
+    void* kp = k ? kept->data_ptr() : nullptr;
+    std::vector<Tensor> outs;
+    if (g) {
+        void* out_p[4];
+        for (size_t i = 0; i < g; ++i) {
+            outs.push_back(at::empty({x.size(0), x.size(1), ranks[i]}, x.options()));
+            out_p[i] = outs.back().data_ptr();
+        }
+        check("hyc_rmsnorm_fwd_compress_lora",
+              hyc_rmsnorm_fwd_compress_lora(x.data_ptr(), w.data_ptr(), y.data_ptr(), (float*)rstd.data_ptr(), rows, n, (float)eps, (int)bits,
+                                            ptr(scale_y), ptr(qy), ptr(scale_x), ptr(qx), tab, k, kp, (int)g, weights, ranks, out_p, stream_of(x)));
+    } else {
+        check("hyc_rmsnorm_fwd_compress",
+              hyc_rmsnorm_fwd_compress(x.data_ptr(), w.data_ptr(), 0, y.data_ptr(), (float*)rstd.data_ptr(), rows, n, (float)eps, (int)bits,
+                                       ptr(scale_y), ptr(qy), ptr(scale_x), ptr(qx), tab, k, kp, stream_of(x)));
+    }
+    return Normed(y, rstd, qy, qx, kept, outs);
+}
+
+OptT norm_backward_codes(const Tensor& dy, const Tensor& q, const Tensor& scale, const OptT& kept, const OptT& table, int64_t k, int64_t bits,
+                         const Tensor& w, const Tensor& rstd, const OptT& residual) {
+    if (!plain(dy) || dy.numel() == 0 || !bits_ok(bits)) return std::nullopt;
+    const int64_t n = dy.size(-1), rows = dy.numel() / n;
+    if (n % 512 || n > 8192 || rows % 2 || !packed(q, rows * n, bits) || !vec(scale, n) || !plain(w) || w.numel() != n) return std::nullopt;
+    if (!rstd.is_cuda() || rstd.scalar_type() != at::kFloat || !rstd.is_contiguous() || rstd.numel() != rows) return std::nullopt;
+    if (k && (!table_ok(table, n) || !kept || !is_bf(*kept) || !kept->is_contiguous() || kept->numel() != rows * k)) return std::nullopt;
+    if (residual && (!plain(*residual) || residual->sizes() != dy.sizes())) return std::nullopt;
+    Tensor dx = at::empty_like(dy);
+    check("hyc_rmsnorm_bwd_codes",
+          hyc_rmsnorm_bwd_codes(dy.data_ptr(), q.data_ptr(), scale.data_ptr(), k ? (const uint16_t*)table->data_ptr() : nullptr, k,
+                                k ? kept->data_ptr() : nullptr, (int)bits, w.data_ptr(), 0, (const float*)rstd.data_ptr(), ptr(residual),
+                                dx.data_ptr(), rows, n, stream_of(dy)));
+    return dx;
+}
+
+// ---- element-wise, rotation, gated product ------------------------------------------------------------------------
+OptT binary(const std::string& name, const Tensor& a, const Tensor& b) {
+    if (!plain(a) || !plain(b) || a.sizes() != b.sizes()) return std::nullopt;
+    auto* fn = name == "hyc_silu_bwd" ? hyc_silu_bwd : name == "hyc_silu_mul" ? hyc_silu_mul : name == "hyc_silu_once_mul" ? hyc_silu_once_mul :
+               name == "hyc_gelu_bwd" ? hyc_gelu_bwd : nullptr;
+    if (!fn) return std::nullopt;
+    Tensor o = at::empty_like(a);
+    check(name.c_str(), fn(a.data_ptr(), b.data_ptr(), o.data_ptr(), a.numel(), stream_of(a)));
+    return o;
+}
+
+OptT rope(const Tensor& x, const Tensor& cos, const Tensor& sin, bool backward) {
+    if (!is_bf(x) || x.dim() != 4 || x.size(3) % 16 || x.stride(3) != 1 || x.stride(0) % 8 || x.stride(1) % 8 || x.stride(2) % 8 || !aligned(x))
+        return std::nullopt;
+    const Rope R(cos, sin, x.size(1), x.size(3) / 2);
+    if (!R.ok) return std::nullopt;
+    check("hyc_rope", hyc_rope(x.data_ptr(), R.cos.data_ptr(), R.sin.data_ptr(), R.fp32, x.size(0), x.size(1), x.size(2), x.size(3), x.stride(0),
+                               x.stride(1), x.stride(2), R.cos.stride(0), R.sin.stride(0), backward, stream_of(x)));
+    return x;
+}
+
+struct Gated {                                             // operands the fused gated product shares between its directions
+    bool ok = false;
+    int64_t rows = 0, n = 0, r = 0;
+    const void *b1 = nullptr, *b2 = nullptr;
+    int bt = 0;
+    Gated(const Tensor& like, const Tensor& xa1, const Tensor& b1_, const Tensor& s1, const Tensor& xa2, const Tensor& b2_, const Tensor& s2) {
+        if (!plain(like) || like.dim() != 3 || like.numel() == 0) return;
+        n = like.size(2);
+        rows = like.numel() / n;
+        const Lora A(b1_), B(b2_);
+        if (!A.fits(n) || !B.fits(n) || A.r != B.r || A.transposed != B.transposed) return;
+        r = A.r;
+        b1 = A.p; b2 = B.p; bt = A.transposed;
+        ok = plain(xa1) && plain(xa2) && xa1.size(-1) == r && xa2.size(-1) == r && xa1.numel() == rows * r && xa2.numel() == rows * r && vec(s1, n) &&
+             vec(s2, n);
+    }
+};
+std::optional<std::tuple<Tensor, Tensor, Tensor>> gated_forward(const Tensor& xa1, const Tensor& b1, const Tensor& x1, const Tensor& s1,
+                                                                const Tensor& xa2, const Tensor& b2, const Tensor& x2, const Tensor& s2, int64_t bits) {
+    const Gated G(x1, xa1, b1, s1, xa2, b2, s2);
+    if (!G.ok || !plain(x2) || x2.sizes() != x1.sizes() || !bits_ok(bits)) return std::nullopt;
+    Tensor q1 = bytes_like(x1, G.n, bits), q2 = bytes_like(x1, G.n, bits), o = at::empty_like(x1);
+    check("hyc_lora_silu_mul_fwd", hyc_lora_silu_mul_fwd(xa1.data_ptr(), G.b1, x1.data_ptr(), s1.data_ptr(), xa2.data_ptr(), G.b2, x2.data_ptr(),
+                                                         s2.data_ptr(), q1.data_ptr(), q2.data_ptr(), o.data_ptr(), G.rows, G.n, G.r, (int)bits, G.bt,
+                                                         stream_of(x1)));
+    return std::make_tuple(q1, q2, o);
+}
+std::optional<std::tuple<Tensor, Tensor, Tensor>> gated_backward(const Tensor& xa1, const Tensor& b1, const Tensor& q1, const Tensor& s1,
+                                                                 const Tensor& xa2, const Tensor& b2, const Tensor& q2, const Tensor& s2,
+                                                                 const Tensor& grad_o, int64_t bits) {
+    const Gated G(grad_o, xa1, b1, s1, xa2, b2, s2);
+    if (!G.ok || !bits_ok(bits) || !packed(q1, G.rows * G.n, bits) || !packed(q2, G.rows * G.n, bits) || !aligned(q1) || !aligned(q2) ||
+        q1.dim() != 3 || q2.dim() != 3 || q1.size(1) != grad_o.size(1) || q2.size(1) != grad_o.size(1))
+        return std::nullopt;
+    Tensor o = at::empty_like(grad_o), gg = at::empty_like(grad_o), gu = at::empty_like(grad_o);
+    check("hyc_lora_silu_mul_bwd", hyc_lora_silu_mul_bwd(xa1.data_ptr(), G.b1, q1.data_ptr(), s1.data_ptr(), xa2.data_ptr(), G.b2, q2.data_ptr(),
+                                                         s2.data_ptr(), grad_o.data_ptr(), o.data_ptr(), gg.data_ptr(), gu.data_ptr(), G.rows, G.n,
+                                                         G.r, (int)bits, G.bt, stream_of(grad_o)));
+    return std::make_tuple(o, gg, gu);
+}
+
+// ---- NF4 weights --------------------------------------------------------------------------------------------------
+OptT nf4_dequant(const Tensor& packed_w, const Tensor& absmax, const Tensor& code2, const Tensor& absmax2, const OptT& offset, const Tensor& table,
+                 int64_t rows, int64_t cols, int64_t blocksize, int64_t blocksize2) {
+    const int64_t n = rows * cols;
+    auto f32 = [](const Tensor& t) { return t.is_cuda() && t.scalar_type() == at::kFloat && t.is_contiguous(); };
+    auto u8 = [](const Tensor& t) { return t.is_cuda() && t.scalar_type() == at::kByte && t.is_contiguous(); };
+    if (n <= 0 || blocksize <= 0 || blocksize2 <= 0 || !u8(packed_w) || packed_w.numel() * 2 != n || !u8(absmax) || !f32(code2) || code2.numel() != 256 ||
+        !f32(absmax2) || !f32(table) || table.numel() != 16 || (offset && (!f32(*offset) || offset->numel() != 1)))
+        return std::nullopt;
+    const int64_t blocks = (n + blocksize - 1) / blocksize;
+    if (absmax.numel() < blocks || absmax2.numel() < (blocks + blocksize2 - 1) / blocksize2) return std::nullopt;
+    Tensor out = at::empty({rows, cols}, packed_w.options().dtype(at::kBFloat16));
+    check("hyc_nf4_dequant", hyc_nf4_dequant(packed_w.data_ptr(), absmax.data_ptr(), 1, (const float*)code2.data_ptr(), (const float*)absmax2.data_ptr(),
+                                             offset ? (const float*)offset->data_ptr() : nullptr, blocksize2, (const float*)table.data_ptr(), out.data_ptr(),
+                                             n, blocksize, stream_of(packed_w)));
+    return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(_native, m) {
+    m.def("stream_of", [](const Tensor& t) { return (uintptr_t)stream_of(t); });
+    m.def("lora_add", &lora_add);
+    m.def("lora_add_sum", &lora_add_sum);
+    m.def("lora_add_quant_group", &lora_add_quant_group);
+    m.def("lora_add_restore_group", &lora_add_restore_group);
+    m.def("contract", &contract);
+    m.def("lora_parts", &lora_parts);
+    m.def("lora_forward", &lora_forward);
+    m.def("lora_backward", &lora_backward);
+    m.def("quantize", &quantize);
+    m.def("dequantize", &dequantize);
+    m.def("norm_compress", &norm_compress);
+    m.def("norm_backward_codes", &norm_backward_codes);
+    m.def("binary", &binary);
+    m.def("rope", &rope);
+    m.def("gated_forward", &gated_forward);
+    m.def("gated_backward", &gated_backward);
+    m.def("nf4_dequant", &nf4_dequant);
+}

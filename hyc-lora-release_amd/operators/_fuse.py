@@ -55,6 +55,9 @@ def _common(xa1, b1, s1, xa2, b2, s2, quantize_bit, n):
 def fuse_forward(xa1, b1, x1, s1, xa2, b2, x2, s2, quantize_bit=8):
     if x1.dim() != 3 or x2.shape != x1.shape:
         raise ValueError(f"x1 and x2 must be [B, M, N] of one shape, got {tuple(x1.shape)} and {tuple(x2.shape)}")
+    done = _lib.native().gated_forward(xa1, b1, x1, s1, xa2, b2, x2, s2, quantize_bit)
+    if done is not None:
+        return done
     B, M, N = x1.shape
     _validate(xa1, b1, s1, xa2, b2, s2, quantize_bit, B * M, N)
     _lib.require_gpu(xa1, b1, x1, s1, xa2, b2, x2, s2)
@@ -74,6 +77,9 @@ def fuse_forward(xa1, b1, x1, s1, xa2, b2, x2, s2, quantize_bit=8):
 def fuse_backward(xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, quantize_bit=8):
     if grad_o.dim() != 3:
         raise ValueError(f"grad_o must be [B, M, N], got shape {tuple(grad_o.shape)}")
+    done = _lib.native().gated_backward(xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, quantize_bit)
+    if done is not None:
+        return done
     B, M, N = grad_o.shape
     _validate(xa1, b1, s1, xa2, b2, s2, quantize_bit, B * M, N)
     want = (B, M, N * quantize_bit // 8)

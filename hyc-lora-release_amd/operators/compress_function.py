@@ -208,6 +208,10 @@ def _quantize(x, s, z, channel, quantize_bit, dtype, zero_input=False):
     if dtype != BF16:
         raise NotImplementedError("the gfx950 kernels compute in bfloat16 only")
     epp = _check_bits(quantize_bit)
+    if not zero_input:
+        done = _lib.native().quantize(x, s, z if z is None or z.dtype == BF16 or not z.is_cuda else _lib.bf16_vector(z), channel, quantize_bit)
+        if done is not None:
+            return done
     _lib.require_gpu(x, s, z, channel)
     if x.dtype != BF16:
         x = x.to(BF16)
@@ -240,6 +244,10 @@ def _dequantize(q, s, z, x_outlier, channel, quantize_bit, is_head, num_heads, d
     if dtype != BF16:
         raise NotImplementedError("the gfx950 kernels compute in bfloat16 only")
     epp = _check_bits(quantize_bit)
+    x = _lib.native().dequantize(q, s, z if z is None or z.dtype == BF16 or not z.is_cuda else _lib.bf16_vector(z), x_outlier, channel,
+                                 quantize_bit)
+    if x is not None:
+        return hidden_to_head_shape(x, num_heads=num_heads) if is_head else x
     _lib.require_gpu(q, s, z, x_outlier, channel)
     B, M, nbytes = q.shape
     N = s.shape[-1]

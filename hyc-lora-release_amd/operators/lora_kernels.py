@@ -64,6 +64,9 @@ def _lora_b(b):
 def lora_add(x_main, xa, b, inplace=False, residual=None):
     """bf16(x_main + bf16(xa @ b)), then - with a residual of x_main's shape - bf16(residual + that);
     `inplace` overwrites x_main (contiguous bf16) and returns it."""
+    y = _lib.native().lora_add(x_main, xa, b, residual, inplace)
+    if y is not None:
+        return y
     n = x_main.shape[-1]
     r = _check(xa, b, n, x_main.numel() // max(n, 1))
     if residual is not None and residual.shape != x_main.shape:
@@ -100,6 +103,9 @@ def lora_add_sum(terms):
     bits of lora_add(x_0, ...), lora_add(x_1, ..., residual=that), lora_add(x_2, ..., residual=that), in one
     pass.  terms: (x_main, xa, b) triples of one shape; the result overwrites the first x_main when that is a
     contiguous bf16 tensor, and is returned."""
+    y = _lib.native().lora_add_sum(terms)
+    if y is not None:
+        return y
     if not 2 <= len(terms) <= 3:
         raise ValueError(f"lora_add_sum takes two or three terms, got {len(terms)}")
     shape = terms[0][0].shape
@@ -124,6 +130,14 @@ def lora_add_sum(terms):
     arr = (_lib.LoraSumMember * len(members))(*members)
     _lib.call("hyc_lora_add_sum", arr, len(members), y.data_ptr(), rows, n, rank, _lib.stream_of(y))
     return y
+
+
+def _bf16_or_none(t):
+    return t if t is None or t.dtype == BF16 else _lib.bf16_vector(t)
+
+
+def _bf16_vectors(*vectors):
+    return all(t is None or t.is_cuda for t in vectors)
 
 
 def _vec_ok(t, n, name):
@@ -157,6 +171,11 @@ def lora_add_quant(x_main, xa, b, scale, zero_point=None, quantize_bit=8, inplac
     if x_main.dim() != 3:
         raise ValueError(f"x_main must be [B, M, N], got shape {tuple(x_main.shape)}")
     B, M, n = x_main.shape
+    if _bf16_vectors(scale, zero_point):
+        done = _lib.native().lora_add_quant_group([_item(dict(xa=xa, b=b, scale=scale, zero_point=zero_point, rope=rope), x_main)],
+                                                  quantize_bit, inplace)
+        if done is not None:
+            return done[0]
     r = _check(xa, b, n, B * M)
     _vec_ok(scale, n, "scale")
     _vec_ok(zero_point, n, "zero point")
@@ -191,6 +210,10 @@ def lora_add_restore(q, scale, xa, b, zero_point=None, quantize_bit=8, rope=None
     n = scale.numel()
     if nbytes * 8 != n * quantize_bit or q.dtype != torch.uint8:
         raise ValueError(f"packed codes must be uint8 of width {n * quantize_bit // 8}, got {q.dtype} {nbytes}")
+    if _bf16_vectors(scale, zero_point):
+        done = _lib.native().lora_add_restore_group([_item(dict(xa=xa, b=b, scale=scale, zero_point=zero_point, rope=rope), q)], quantize_bit)
+        if done is not None:
+            return done[0]
     r = _check(xa, b, n, B * M)
     _vec_ok(zero_point, n, "zero point")
     _lib.require_gpu(q, scale, xa, b, zero_point)
@@ -226,10 +249,19 @@ def _member(xa, b, bt, x, s, z, q, y, rope_tables, n):
     return m
 
 
+def _item(it, x):
+    """A group member as the native call takes it."""
+    zp, rope = _bf16_or_none(it.get("zero_point")), it.get("rope")
+    return (x, it["xa"], it["b"], it["scale"], zp, None, None) if rope is None else (x, it["xa"], it["b"], it["scale"], zp, *rope)
+
+
 def lora_add_quant_group(items, quantize_bit=8, inplace=False):
     """lora_add_quant for up to GROUP_MAX operand sets in one launch -> [(q, y), ...], each pair the same bits
     as its own call.  items: dicts with x_main [B, M, N_i], xa [B, M, R], b [R, N_i], scale, and optionally
     zero_point (all items or none) and rope=(cos, sin); B, M and R are shared."""
+    outs = _lib.native().lora_add_quant_group([_item(it, it["x_main"]) for it in items], quantize_bit, inplace)
+    if outs is not None:
+        return outs
     if quantize_bit not in (2, 4, 8):
         raise ValueError(f"quantize_bit must be 2, 4 or 8, got {quantize_bit}")
     if not 1 <= len(items) <= GROUP_MAX:
@@ -273,6 +305,9 @@ def lora_add_quant_group(items, quantize_bit=8, inplace=False):
 def lora_add_restore_group(items, quantize_bit=8):
     """lora_add_restore for up to GROUP_MAX operand sets in one launch -> [y, ...].  items: dicts with q
     [B, M, N_i*bits/8], scale, xa, b and optionally zero_point (all or none) and rope=(cos, sin)."""
+    outs = _lib.native().lora_add_restore_group([_item(it, it["q"]) for it in items], quantize_bit)
+    if outs is not None:
+        return outs
     if quantize_bit not in (2, 4, 8):
         raise ValueError(f"quantize_bit must be 2, 4 or 8, got {quantize_bit}")
     if not 1 <= len(items) <= GROUP_MAX:
@@ -345,6 +380,9 @@ def lora_products(x, u=None, v=None, p1_transposed=False):
     if u is None and v is None:
         raise ValueError("nothing to compute: pass u, v or both")
     n = x.shape[-1]
+    done = _lib.native().contract(x, None, None, None, 0, u, v, n, p1_transposed)
+    if done is not None:
+        return done
     r = u.shape[-1] if u is not None else v.shape[0]
     if n % 32 or r % 2 or not 2 <= r <= 64:
         raise ValueError(f"width must be a multiple of 32 and the rank even within 2..64, got {n}, {r}")
@@ -371,6 +409,9 @@ def lora_product_from_codes(q, scale, u, zero_point=None, quantize_bit=8):
     n = scale.numel()
     if nbytes * 8 != n * quantize_bit or q.dtype != torch.uint8:
         raise ValueError(f"packed codes must be uint8 of width {n * quantize_bit // 8}, got {q.dtype} {nbytes}")
+    done = _lib.native().contract(None, q, scale, _bf16_or_none(zero_point), quantize_bit, u, None, n, False)
+    if done is not None:
+        return done[0]
     r = u.shape[-1]
     if n % 32 or r % 2 or not 2 <= r <= 64:
         raise ValueError(f"width must be a multiple of 32 and the rank even within 2..64, got {n}, {r}")

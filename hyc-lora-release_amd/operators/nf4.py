@@ -45,6 +45,14 @@ def dequantize_nf4(w, quant_state):
     if getattr(qs, "dtype", torch.bfloat16) != torch.bfloat16:
         raise NotImplementedError("dequantize_nf4 produces bfloat16 weights")
     dev = w.device
+    nested = bool(getattr(qs, "nested", False))
+    if nested and len(qs.shape) == 2:                    # what a double-quantised checkpoint holds, statistics as they lie
+        code = getattr(qs, "code", None)
+        done = _lib.native().nf4_dequant(w, qs.absmax, qs.state2.code, qs.state2.absmax, qs.offset if torch.is_tensor(qs.offset) else None,
+                                         _default_table(dev) if code is None else code, *qs.shape, int(qs.blocksize), int(qs.state2.blocksize)) \
+            if qs.offset is None or torch.is_tensor(qs.offset) else None
+        if done is not None:
+            return done
     n = 1
     for d in qs.shape:
         n *= int(d)
@@ -56,7 +64,6 @@ def dequantize_nf4(w, quant_state):
     if table.numel() != 16:
         raise ValueError("the 4-bit code book must have 16 entries")
     out = torch.empty(n, device=dev, dtype=torch.bfloat16)
-    nested = bool(getattr(qs, "nested", False))
     if nested:
         absmax = qs.absmax.reshape(-1).contiguous()
         s2 = qs.state2

@@ -114,6 +114,12 @@ def rmsnorm_backward_from_codes(dy, q_x, scale_x, x_outlier, outlier_idx, q_bit,
     (fused_llama_layer_intra_inter_full_fuse.py:386-393), with `residual` added like there."""
     _lib.require_gpu(dy, q_x, scale_x, w, rstd, residual)
     n = dy.shape[-1]
+    k = 0 if outlier_idx is None else int(outlier_idx.numel())
+    if k and table is None and outlier_idx.is_cuda:
+        table = outlier_table(outlier_idx, n, cached=True)
+    dx = _lib.native().norm_backward_codes(dy, q_x, scale_x, x_outlier, table, k, q_bit, w, rstd, residual)
+    if dx is not None:
+        return dx
     if not backward_from_codes_supported(dy, n, False):
         raise NotImplementedError("rmsnorm_backward_from_codes: bfloat16 gradient, N a multiple of 512 up to 8192, even row count")
     dy = dy.contiguous()
@@ -232,6 +238,12 @@ def rmsnorm_forward_compress(x, weight, eps, q_bit, scale_y=None, scale_x=None, 
     [B, M, R] bf16 - lora_forward's `x @ w_lora_a` (models/utils/compute_utils.py:22) for each of them,
     formed while y is still on the chip instead of by one library GEMM each over y in memory
     (see lora_a_supported for the shapes this takes)."""
+    k = 0 if outlier_idx is None or scale_x is None else outlier_idx.numel()
+    if k and table is None and outlier_idx.is_cuda:
+        table = outlier_table(outlier_idx, x.shape[-1], cached=True)
+    done = _lib.native().norm_compress(x, weight, eps, q_bit, scale_y, scale_x, table, k, lora_a or [])
+    if done is not None:
+        return done if lora_a else done[:5]
     _lib.require_gpu(x, weight)
     if x.dtype != torch.bfloat16 or x.dim() != 3:
         raise NotImplementedError("rmsnorm_forward_compress takes bfloat16 [batch, seq, hidden] activations")

@@ -27,6 +27,9 @@ def _table(t, seq_len, half):
 
 
 def _rotate(x, cos, sin, backward):
+    done = _lib.native().rope(x, cos, sin, backward)
+    if done is not None:
+        return done
     _lib.require_gpu(x, cos, sin)
     if x.dtype != torch.bfloat16 or x.dim() != 4:
         raise NotImplementedError("rope rotates a bfloat16 [batch, seq, heads, head_dim] tensor")
