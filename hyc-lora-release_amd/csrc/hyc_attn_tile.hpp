@@ -47,11 +47,12 @@ __device__ __forceinline__ void wait_copies_and_barrier() {
 }
 
 // A tile of ROWS rows of D bf16 in LDS, as 1 KB blocks of 16 rows x 4 chunks (of 16 bytes): block (row / 16, chunk / 4),
-// inside it chunk % 4 major, and the 16 rows of a chunk in the order row ^ 4 * (chunk % 4).  An operand of 32 rows reads 16
-// rows of a chunk as 256 contiguous bytes; a transposing read takes 4 rows (64 bytes) of each of 4 chunks, which the order
-// puts on different banks.  Everything that varies inside a kernel's loops (k step, column block, buffer) moves the address
-// by a multiple of a block, an immediate offset: four registers of addresses serve all reads.  A wave's copy fills one
-// block: 64 bytes of each of 16 rows of memory.
+// inside it the 64 bytes of a row together, its chunks in the order chunk ^ (row / 4).  A wave's copy fills one block, four
+// neighbouring lanes 64 contiguous bytes of memory: with the lanes of a row 16 apart (chunk-major blocks) the copies found 64
+// lines instead of 16 per instruction and moved 28 bytes per ns and unit, a quarter of what L2 gives.  An operand of 32
+// rows reads a chunk of 16 rows, a transposing read 4 rows of 4 chunks; both meet 256 bytes of different banks.  Everything
+// that varies inside a kernel's loops (k step, column block, buffer) moves the address by a multiple of a block, an immediate
+// offset: four registers of addresses serve all reads.
 template <int D, int ROWS>
 struct AttnTile {
     static constexpr int kChunks = D / 8;                       // 16-byte chunks of a row
@@ -59,31 +60,39 @@ struct AttnTile {
     static constexpr int kBytes = ROWS * D * 2;
     static constexpr int kCopies = kBytes / 4096;               // block copies of each of 4 waves
 
+    // Bytes of chunk c (0..3) of row r (0..15) in a block
+    __device__ static __forceinline__ int in_block(int r, int c) { return r * 64 + ((c ^ (r >> 2)) * 16); }
+
     // Requests rows row0 .. row0 + ROWS - 1 (past row_last: row_last again) of a tensor whose rows are `ld` elements
     // apart; called by the 4 waves of a workgroup.
     __device__ static __forceinline__ void request(const uint16_t* base, int row0, int row_last, int ld, uint32_t lds, int wave, int lane) {
-        const int c = lane >> 4, r = (lane & 15) ^ (4 * c);
 #pragma unroll
         for (int i = 0; i < kCopies; ++i) {
-            const int blk = i * 4 + wave, row = (blk / kBlocksAcross) * 16 + r;
-            const int src = row0 + row < row_last ? row0 + row : row_last;
-            const uint32_t voff = ((uint32_t)src * (uint32_t)ld + (uint32_t)((blk % kBlocksAcross) * 32 + c * 8)) * 2u;
-            copy_to_lds16(base, voff, lds + (uint32_t)(blk * 1024));
+            const int blk = i * 4 + wave;
+            copy_to_lds16(base, source(blk, row0, row_last, ld, lane), lds + (uint32_t)(blk * 1024));
         }
+    }
+    // Bytes from the tensor's base to what a lane copies into block `blk`
+    __device__ static __forceinline__ uint32_t source(int blk, int row0, int row_last, int ld, int lane) {
+        const int r = lane >> 2, c = (lane & 3) ^ (r >> 2), row = (blk / kBlocksAcross) * 16 + r;
+        const int src = row0 + row < row_last ? row0 + row : row_last;
+        return ((uint32_t)src * (uint32_t)ld + (uint32_t)((blk % kBlocksAcross) * 32 + c * 8)) * 2u;
     }
 
     // What a lane adds to a tile's LDS address for the two read forms
     struct Lane {
-        uint32_t rows[2], cols[2];
+        uint32_t rows[2], cols[2], order[4];
         __device__ __forceinline__ explicit Lane(int lane) {
             const int h = lane >> 5, r16 = lane & 15, rb = (lane >> 4) & 1;
 #pragma unroll
             for (int odd = 0; odd < 2; ++odd) {
                 const int c = 2 * odd + h;
-                rows[odd] = (uint32_t)(rb * kBlocksAcross * 1024 + c * 256 + (r16 ^ (4 * c)) * 16);
+                rows[odd] = (uint32_t)(rb * kBlocksAcross * 1024 + in_block(r16, c));
                 const int row = 4 * h + (r16 >> 2) + 8 * odd, cc = 2 * rb + ((r16 & 3) >> 1);
-                cols[odd] = (uint32_t)(cc * 256 + (row ^ (4 * cc)) * 16 + (r16 & 1) * 8);
+                cols[odd] = (uint32_t)(in_block(row, cc) + (r16 & 1) * 8);
             }
+#pragma unroll
+            for (int c = 0; c < 4; ++c) order[c] = (uint32_t)(rb * kBlocksAcross * 1024 + in_block(r16, c) + h * 8);
         }
     };
     // The lane's addresses in one tile, opaque so that what a read adds to them stays an immediate offset instead of an
@@ -95,12 +104,21 @@ struct AttnTile {
             v.rows[i] += tile; v.cols[i] += tile;
             asm("" : "+v"(v.rows[i]), "+v"(v.cols[i]));
         }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v.order[i] += tile;
         return v;
     }
     // A operand of tile rows r0 .. r0+31 (r0 a multiple of 32), k = columns 16t .. 16t+15; `off`: constant bytes past the tile
     __device__ static __forceinline__ bf16x8 rows_operand(const Lane& at, int off, int r0, int t) {
         typedef const __attribute__((address_space(3))) u32x4 lds_u32x4;
         return as_bf16x8(*(lds_u32x4*)(at.rows[t & 1] + (uint32_t)(off + ((r0 / 16) * kBlocksAcross + t / 2) * 1024)));
+    }
+    // The same rows and k in the order 4h + {0..3}, 8 + 4h + {0..3}: the other operand of a product with cols_operand
+    __device__ static __forceinline__ bf16x8 rows_in_c_order(const Lane& at, int r0, int t) {
+        typedef const __attribute__((address_space(3))) u32x2 lds_u32x2;
+        const uint32_t off = (uint32_t)(((r0 / 16) * kBlocksAcross + t / 2) * 1024);
+        const u32x2 a = *(lds_u32x2*)(at.order[2 * (t & 1)] + off), b = *(lds_u32x2*)(at.order[2 * (t & 1) + 1] + off);
+        return as_bf16x8(u32x4{a.x, a.y, b.x, b.y});
     }
     // A operand of the transposed tile: rows = columns d0 .. d0+31 of the tile (d0 a multiple of 32), k = tile rows
     // k0 .. k0+15 (k0 a multiple of 16) in the order 4h + {0..3}, 8 + 4h + {0..3}
