@@ -29,7 +29,7 @@ class HycError(RuntimeError):
 
 
 # name -> (restype, argtypes)
-ABI_VERSION = 13          # hyc_abi_version() of the library these signatures describe
+ABI_VERSION = 14          # hyc_abi_version() of the library these signatures describe
 _P, _I, _L = c_void_p, c_int, c_int64
 
 
@@ -102,6 +102,8 @@ _SIGNATURES = {
     "hyc_map_emit": (_I, [_P] * 3 + [_L] * 2 + [_P] * 2 + [_L] * 2 + [_P] * 3 + [_L] * 5 + [ctypes.c_float, _P]),
     "hyc_map_bwd_workspace": (_L, [_L] * 6),
     "hyc_map_bwd": (_I, [_P] * 7 + [_L, _P, _L] + [_P] * 3 + [_L] * 5 + [ctypes.c_float, _P]),
+    "hyc_few_rows_workspace": (_L, [_L] * 3),
+    "hyc_few_rows": (_I, [_P, _P, _I, _P, _P] + [_L] * 4 + [_P]),
     "hyc_lora_add_sum": (_I, [_P, _I, _P, _L, _L, _L, _P]),
     "hyc_lora_add_quant_group": (_I, [_P, _I, _L, _L, _I, _P]),
     "hyc_lora_add_restore_group": (_I, [_P, _I, _L, _L, _I, _P]),

@@ -67,8 +67,13 @@ def _whole_rounds(rows: int, cols: int) -> int:
 
 
 def frozen_matmul(x: torch.Tensor, w: torch.Tensor):
-    """x @ w for a frozen weight (or its transposed view) w [K, N]: the library product, in the calls that suit its tiles."""
+    """x @ w for a frozen weight (or its transposed view) w [K, N]: the kernel for a few rows (csrc/few_rows.hip) where that is the
+    faster one, else the library product, in the calls that suit its tiles."""
     k, n = w.shape
+    if x.is_cuda:
+        done = _lib.native().few_rows(x, w)
+        if done is not None:
+            return done
     rows = x.numel() // max(k, 1)
     cut = _whole_rounds(rows, n) if x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and not torch.is_grad_enabled() else 0
     if cut == 0:

@@ -687,6 +687,17 @@ int hyc_map_bwd(const void *grad_o, const void *q, const void *k, const void *v,
                 void *grad_k, void *grad_v, int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D, float scale, void *stream);
 
 /* ---------------------------------------------------------------------------------------
+ * A product of a few rows with a frozen weight: out = x w^T (w_is_nk: w bf16 [N, K]) or x w (w bf16 [K, N]), summed in fp32
+ * in an order that depends on the shape alone.  Stands for the frozen-weight GEMMs of short batches
+ * (models/utils/compute_utils.py:18-36).
+ *   x bf16 [T, K], out bf16 [T, N], contiguous;  T <= 128, N % 128 == 0, K % 64 == 0, N * K < 2^31;
+ *   workspace: hyc_few_rows_workspace(T, N, K) bytes (0: shape not taken).  All pointers 16-byte aligned.
+ */
+int64_t hyc_few_rows_workspace(int64_t T, int64_t N, int64_t K);
+int hyc_few_rows(const void *x, const void *w, int w_is_nk, void *out, void *workspace, int64_t workspace_bytes, int64_t T,
+                 int64_t N, int64_t K, void *stream);
+
+/* ---------------------------------------------------------------------------------------
  * Memory-only probe, FOR BENCHMARKING: loads n_reads and stores n_writes bf16 [T, N] tensors (1..3 each,
  * arrays of device pointers in host memory, 16-byte aligned, N % 8 == 0) with the access shape of the
  * kernels of this library and no arithmetic of the path, so that the rate the memory system gives a
