@@ -480,15 +480,16 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> gated_forward(const Tensor& xa
 }
 std::optional<std::tuple<Tensor, Tensor, Tensor>> gated_backward(const Tensor& xa1, const Tensor& b1, const Tensor& q1, const Tensor& s1,
                                                                  const Tensor& xa2, const Tensor& b2, const Tensor& q2, const Tensor& s2,
-                                                                 const Tensor& grad_o, int64_t bits) {
+                                                                 const Tensor& grad_o, int64_t bits, bool once) {
     const Gated G(grad_o, xa1, b1, s1, xa2, b2, s2);
     if (!G.ok || !bits_ok(bits) || !packed(q1, G.rows * G.n, bits) || !packed(q2, G.rows * G.n, bits) || !aligned(q1) || !aligned(q2) ||
         q1.dim() != 3 || q2.dim() != 3 || q1.size(1) != grad_o.size(1) || q2.size(1) != grad_o.size(1))
         return std::nullopt;
     Tensor o = at::empty_like(grad_o), gg = at::empty_like(grad_o), gu = at::empty_like(grad_o);
-    check("hyc_lora_silu_mul_bwd", hyc_lora_silu_mul_bwd(xa1.data_ptr(), G.b1, q1.data_ptr(), s1.data_ptr(), xa2.data_ptr(), G.b2, q2.data_ptr(),
-                                                         s2.data_ptr(), grad_o.data_ptr(), o.data_ptr(), gg.data_ptr(), gu.data_ptr(), G.rows, G.n,
-                                                         G.r, (int)bits, G.bt, stream_of(grad_o)));
+    auto* fn = once ? hyc_lora_silu_once_mul_bwd : hyc_lora_silu_mul_bwd;
+    check(once ? "hyc_lora_silu_once_mul_bwd" : "hyc_lora_silu_mul_bwd",
+          fn(xa1.data_ptr(), G.b1, q1.data_ptr(), s1.data_ptr(), xa2.data_ptr(), G.b2, q2.data_ptr(), s2.data_ptr(), grad_o.data_ptr(), o.data_ptr(),
+             gg.data_ptr(), gu.data_ptr(), G.rows, G.n, G.r, (int)bits, G.bt, stream_of(grad_o)));
     return std::make_tuple(o, gg, gu);
 }
 

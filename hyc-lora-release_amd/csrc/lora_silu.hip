@@ -308,7 +308,9 @@ HYC_FUSE_KERNEL(HYC_FWD_DEEP) void lora_silu_fwd_kernel(const FuseArgs a) {
 }
 
 // ------------------------------------------------------------------------------------
-template <int QBIT, int KSTEPS>
+// ONCE: silu(y1) = y1 * sigmoid(y1) rounded once, as torch's F.silu (the layers that recompute it so), instead of with the
+// sigmoid rounded first.  The gradient of the gate uses the rounded sigmoid in both.
+template <int QBIT, int KSTEPS, bool ONCE>
 HYC_FUSE_KERNEL(HYC_BWD_DEEP) void lora_silu_bwd_kernel(const FuseArgs a) {
     constexpr int CT = kFuseColTiles<QBIT>, RS = kFuseWaves / CT;
     const int lane = threadIdx.x & (kWave - 1);
@@ -355,8 +357,8 @@ HYC_FUSE_KERNEL(HYC_BWD_DEEP) void lora_silu_bwd_kernel(const FuseArgs a) {
             const float x2 = QBIT == 2 ? d2 : rbf(d2);
             const float y1 = rbf(x1 + lora_elem(La, j));
             const float y2 = rbf(x2 + lora_elem(Lb, j));
-            const float sig = rbf(sigmoidf_(y1));
-            const float sil = rbf(y1 * sig);
+            const float sigma = sigmoidf_(y1), sig = rbf(sigma);
+            const float sil = rbf(y1 * (ONCE ? sigma : sig));
             of[j] = sil * y2;
             const float gh1 = rbf(gf[j] * y2);
             gu[j] = gf[j] * sil;
@@ -487,21 +489,21 @@ static int fuse_check(const FuseArgs& a, int64_t T, int64_t N, int64_t R, int q_
     return 1;
 }
 
-#define HYC_FUSE_LAUNCH_K(KERNEL, QB)                                                                     \
-    do {                                                                                                  \
-        if (ksteps == 1) hipLaunchKernelGGL((KERNEL<QB, 1>), grid, block, 0, st, a);                      \
-        else if (ksteps == 2) hipLaunchKernelGGL((KERNEL<QB, 2>), grid, block, 0, st, a);                 \
-        else if (ksteps == 3) hipLaunchKernelGGL((KERNEL<QB, 3>), grid, block, 0, st, a);                 \
-        else hipLaunchKernelGGL((KERNEL<QB, 4>), grid, block, 0, st, a);                                  \
+#define HYC_FUSE_LAUNCH_K(KERNEL, QB, ...)                                                                 \
+    do {                                                                                                   \
+        if (ksteps == 1) hipLaunchKernelGGL((KERNEL<QB, 1, ##__VA_ARGS__>), grid, block, 0, st, a);        \
+        else if (ksteps == 2) hipLaunchKernelGGL((KERNEL<QB, 2, ##__VA_ARGS__>), grid, block, 0, st, a);   \
+        else if (ksteps == 3) hipLaunchKernelGGL((KERNEL<QB, 3, ##__VA_ARGS__>), grid, block, 0, st, a);   \
+        else hipLaunchKernelGGL((KERNEL<QB, 4, ##__VA_ARGS__>), grid, block, 0, st, a);                    \
     } while (0)
-#define HYC_FUSE_LAUNCH(KERNEL)                                  \
-    do {                                                         \
-        if (q_bit == 8) HYC_FUSE_LAUNCH_K(KERNEL, 8);            \
-        else if (q_bit == 4) HYC_FUSE_LAUNCH_K(KERNEL, 4);       \
-        else HYC_FUSE_LAUNCH_K(KERNEL, 2);                       \
+#define HYC_FUSE_LAUNCH(KERNEL, ...)                                  \
+    do {                                                              \
+        if (q_bit == 8) HYC_FUSE_LAUNCH_K(KERNEL, 8, ##__VA_ARGS__);  \
+        else if (q_bit == 4) HYC_FUSE_LAUNCH_K(KERNEL, 4, ##__VA_ARGS__); \
+        else HYC_FUSE_LAUNCH_K(KERNEL, 2, ##__VA_ARGS__);             \
     } while (0)
 
-static int fuse_launch(FuseArgs& a, int64_t T, int64_t N, int64_t R, int q_bit, bool fwd, void* stream) {
+static int fuse_launch(FuseArgs& a, int64_t T, int64_t N, int64_t R, int q_bit, bool fwd, void* stream, bool once = false) {
     const int rc = fuse_check(a, T, N, R, q_bit, fwd);
     if (rc <= 0) return rc;
     a.T = T;
@@ -517,7 +519,8 @@ static int fuse_launch(FuseArgs& a, int64_t T, int64_t N, int64_t R, int q_bit, 
     const int ksteps = (int)cdiv(R, 16);
     hipStream_t st = (hipStream_t)stream;
     if (fwd) HYC_FUSE_LAUNCH(lora_silu_fwd_kernel);
-    else HYC_FUSE_LAUNCH(lora_silu_bwd_kernel);
+    else if (once) HYC_FUSE_LAUNCH(lora_silu_bwd_kernel, true);
+    else HYC_FUSE_LAUNCH(lora_silu_bwd_kernel, false);
     return check_launch();
 }
 
@@ -551,7 +554,7 @@ extern "C" int hyc_lora_silu_mul_fwd(const void* xa1, const void* b1, const void
     return fuse_launch(a, T, N, R, q_bit, true, stream);
 }
 
-extern "C" int hyc_lora_silu_mul_bwd(const void* xa1, const void* b1, const void* q1, const void* s1,
+static int gated_bwd(bool once, const void* xa1, const void* b1, const void* q1, const void* s1,
                                      const void* xa2, const void* b2, const void* q2, const void* s2,
                                      const void* grad_o, void* o, void* grad_gate, void* grad_up, int64_t T,
                                      int64_t N, int64_t R, int q_bit, int b_transposed, void* stream) {
@@ -561,5 +564,19 @@ extern "C" int hyc_lora_silu_mul_bwd(const void* xa1, const void* b1, const void
     a.xa2 = (const uint16_t*)xa2; a.b2 = (const uint16_t*)b2; a.s2 = (const uint16_t*)s2;
     a.q1 = (uint8_t*)q1; a.q2 = (uint8_t*)q2;
     a.g = (const uint16_t*)grad_o; a.o = (uint16_t*)o; a.gg = (uint16_t*)grad_gate; a.gu = (uint16_t*)grad_up;
-    return fuse_launch(a, T, N, R, q_bit, false, stream);
+    return fuse_launch(a, T, N, R, q_bit, false, stream, once);
+}
+
+extern "C" int hyc_lora_silu_mul_bwd(const void* xa1, const void* b1, const void* q1, const void* s1,
+                                     const void* xa2, const void* b2, const void* q2, const void* s2,
+                                     const void* grad_o, void* o, void* grad_gate, void* grad_up, int64_t T,
+                                     int64_t N, int64_t R, int q_bit, int b_transposed, void* stream) {
+    return gated_bwd(false, xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, o, grad_gate, grad_up, T, N, R, q_bit, b_transposed, stream);
+}
+
+extern "C" int hyc_lora_silu_once_mul_bwd(const void* xa1, const void* b1, const void* q1, const void* s1,
+                                     const void* xa2, const void* b2, const void* q2, const void* s2,
+                                     const void* grad_o, void* o, void* grad_gate, void* grad_up, int64_t T,
+                                     int64_t N, int64_t R, int q_bit, int b_transposed, void* stream) {
+    return gated_bwd(true, xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, o, grad_gate, grad_up, T, N, R, q_bit, b_transposed, stream);
 }

@@ -74,10 +74,11 @@ def fuse_forward(xa1, b1, x1, s1, xa2, b2, x2, s2, quantize_bit=8):
     return q1, q2, o
 
 
-def fuse_backward(xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, quantize_bit=8):
+def fuse_backward(xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, quantize_bit=8, round_once=False):
+    """round_once: silu(y1) rounded once, as F.silu, instead of with the sigmoid rounded first."""
     if grad_o.dim() != 3:
         raise ValueError(f"grad_o must be [B, M, N], got shape {tuple(grad_o.shape)}")
-    done = _lib.native().gated_backward(xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, quantize_bit)
+    done = _lib.native().gated_backward(xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, quantize_bit, round_once)
     if done is not None:
         return done
     B, M, N = grad_o.shape
@@ -93,7 +94,7 @@ def fuse_backward(xa1, b1, q1, s1, xa2, b2, q2, s2, grad_o, quantize_bit=8):
     o = torch.empty((B, M, N), device=grad_o.device, dtype=BF16)
     gg = torch.empty_like(o)
     gu = torch.empty_like(o)
-    _lib.call("hyc_lora_silu_mul_bwd", xa1.data_ptr(), b1.data_ptr(), q1.data_ptr(), s1.data_ptr(),
+    _lib.call("hyc_lora_silu_once_mul_bwd" if round_once else "hyc_lora_silu_mul_bwd", xa1.data_ptr(), b1.data_ptr(), q1.data_ptr(), s1.data_ptr(),
               xa2.data_ptr(), b2.data_ptr(), q2.data_ptr(), s2.data_ptr(), grad_o.data_ptr(), o.data_ptr(),
               gg.data_ptr(), gu.data_ptr(), B * M, N, R, quantize_bit, bt, _lib.stream_of(grad_o))
     return o, gg, gu

@@ -496,6 +496,12 @@ int hyc_lora_silu_mul_bwd(const void *xa1, const void *b1, const void *q1, const
                           const void *xa2, const void *b2, const void *q2, const void *s2,
                           const void *grad_o, void *o, void *grad_gate, void *grad_up,
                           int64_t T, int64_t N, int64_t R, int q_bit, int b_transposed, void *stream);
+/* The same with silu(y1) = bf16(y1 * sigmoid(y1)) rounded once, as torch's F.silu: what the layers that do not fuse recompute
+ * (models/llama/fused_llama_layer_intra_inter.py:362-381).  grad_gate is that of hyc_lora_silu_mul_bwd. */
+int hyc_lora_silu_once_mul_bwd(const void *xa1, const void *b1, const void *q1, const void *s1,
+                               const void *xa2, const void *b2, const void *q2, const void *s2,
+                               const void *grad_o, void *o, void *grad_gate, void *grad_up,
+                               int64_t T, int64_t N, int64_t R, int q_bit, int b_transposed, void *stream);
 
 /* ---------------------------------------------------------------------------------------
  * LoRA add around the compressed copy of a projection's frozen part:
