@@ -316,7 +316,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 m = m.expand(q.shape[0], 1, q.shape[2], k.shape[2]) if m.dim() == 4 and m.shape[1] == 1 else None
             frozen = not (calib or raw)
             att = a = seg = None
-            if (attention_mask is None or m is not None) and map_supported(q, k, v, m):
+            if (attention_mask is None or m is not None) and map_kernels_fit(q, k, v, m, None if raw else q_bit):
                 att = MapAttention(q, k, v, m, threshold=sv['a']['outlier'] if frozen else None, want_map=not frozen)
                 a, o = att.map, att.o
             else:
@@ -722,6 +722,17 @@ def gated_product_fits(x, gate, up):
 
 def fuse_backward_round_once(*operands):
     return fuse_backward(*operands, round_once=True)
+
+
+SHORT_2BIT_TOKENS = 1024
+
+
+def map_kernels_fit(q, k, v, mask, q_bit):
+    """Whether the forward attention of a decoder layer that keeps `q_bit` codes (None: none) runs on the map kernels.  Short
+    steps at 2 bits stay with the library's products: a step of a 2-bit code is as large as the values, so an attention
+    output one bf16 unit off takes another code now and then, and where few tokens are summed one such code moved single
+    gradient entries by up to 1.5 times their size (64 to 512 tokens, 5120 wide; 0.7 at 1024 and 2048, 0.4 at 4 bits and 64)."""
+    return map_supported(q, k, v, mask) and (q_bit != 2 or q.shape[0] * q.shape[2] >= SHORT_2BIT_TOKENS)
 
 
 def keep_map_entries(saved, source, thr, seg, host_state):

@@ -98,3 +98,12 @@ def test_backward_from_kept_entries(b, h, kv, s, d, ratio):
         assert (rel(x, w) < 2 ** -8 if w.norm() > 0 else x.abs().max() == 0), (name, rel(x, w))
     again = map_backward(go, q, k, v, torch.cat([idx, idx.new_full((7,), -1)]), torch.cat([val, val.new_zeros(7)]), seg)
     assert all(torch.equal(x, y) for x, y in zip(got, again))          # room past the entries is not read
+
+
+@pytest.mark.parametrize("q_bit,b,s,fits", [(2, 1, 1016, False), (2, 1, 1024, True), (2, 2, 512, True), (2, 3, 64, False), (4, 1, 64, True), (8, 1, 8, True),
+                                            (None, 1, 64, True)])
+def test_short_two_bit_steps_stay_with_the_library(monkeypatch, q_bit, b, s, fits):
+    from hyclora_amd.models import fused_decoder_layer as L
+    monkeypatch.setattr(L, "map_supported", lambda *a: True)
+    q = torch.empty(b, 2, s, 64)
+    assert L.map_kernels_fit(q, q, q, None, q_bit) is fits
