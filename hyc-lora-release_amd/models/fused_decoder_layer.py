@@ -22,8 +22,8 @@ as one function with three switches:
               'sdpa'  no map is saved; the flash kernel's log-sum-exps are, and its backward gets the
                       dequantised attention output; q/k main use a zero point
                       (llama_flash_attn/fused_llama_layer_intra_inter.py:118-180, :450-468 - the
-                      flash-attn kernels themselves are replaced by the ones behind torch's
-                      scaled_dot_product_attention)
+                      flash-attn kernels are replaced by operators/flash_kernels.py, or the ones
+                      behind torch's scaled_dot_product_attention where those do not fit)
   norm weights receive gradients when they require grad (rmsnorm_updatable_kernels.py:173-220).
 
 Deliberate differences from the reference:
