@@ -194,6 +194,22 @@ __device__ __forceinline__ void walk_tiles(uint64_t todo, int& buf, Request requ
 
 __device__ __forceinline__ float prob(float t, float m, float inv) { return __builtin_amdgcn_exp2f((t - m) * kLog2e) * inv; }
 
+// Probabilities of a tile's 64 keys, in place.  Keys past the row get 0, whatever the row's sum is: in a row of NaN scores or of
+// nothing but -inf, `inv` is not finite and prob(-inf) is NaN, which counts as kept.
+__device__ __forceinline__ void map_probs(const MapArgs& A, int k0, int h, float m, float inv, f32x16 (&s)[2]) {
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[kb][r] = prob(s[kb][r], m, inv);
+    if (k0 + kMapTile > A.S) {
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                if (k0 + 32 * kb + 8 * (r / 4) + 4 * h + r % 4 >= A.S) s[kb][r] = 0.0f;
+    }
+}
+
 // Row maxima and sums in a first walk over the keys, the probabilities, their count and the output in a second: a
 // probability is rounded to bf16 relative to its row's final sum, so an online softmax cannot form it.
 template <int D>
@@ -270,13 +286,12 @@ __global__ __launch_bounds__(256, 2) void map_fwd_kernel(const MapArgs A) {
         f32x16 s[2];
         const typename Tile::Lane in = Tile::in_tile(at, lds0 + b * Tile::kBytes);
         map_scores<D, Tile>(A, R, in, Q, k0, (R.plain >> t) & 1, h, s);
+        map_probs(A, k0, h, m, inv, s);
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[kb][r] = prob(s[kb][r], m, inv);
+            for (int r = 0; r < 16; ++r)
                 if (!(s[kb][r] <= limit)) ++count;
-            }
         bf16x8 P[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) P[i] = c_as_operand(s[i >> 1], i & 1);
@@ -348,14 +363,12 @@ __global__ __launch_bounds__(256, 2) void map_emit_kernel(const MapArgs A) {
         const int k0 = t * kMapTile;
         f32x16 s[2];
         map_scores<D, Tile>(A, R, Tile::in_tile(at, lds0 + b * Tile::kBytes), Q, k0, (R.plain >> t) & 1, h, s);
+        map_probs(A, k0, h, m, inv, s);
         uint32_t own[2] = {0, 0};
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                s[kb][r] = prob(s[kb][r], m, inv);
-                own[kb] |= !(s[kb][r] <= limit) ? 1u << (8 * (r / 4) + r % 4) : 0u;
-            }
+            for (int r = 0; r < 16; ++r) own[kb] |= !(s[kb][r] <= limit) ? 1u << (8 * (r / 4) + r % 4) : 0u;
         uint32_t full[2];
 #pragma unroll
         for (int kb = 0; kb < 2; ++kb) {

@@ -72,6 +72,33 @@ def test_forward_and_kept_entries(b, h, kv, s, d, kind):
             assert torch.equal(idx2[:m], idx[:m]) and torch.equal(val2[:m], val[:m])
 
 
+def same_bits(a, b):
+    return torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+@pytest.mark.parametrize("s", [8, 72, 96, 128, 200])
+def test_rows_without_a_finite_sum_keep_nothing_past_their_end(s):
+    """Rows of nothing but -inf and rows of NaN scores: every one of their S entries is kept (NaN is), none past the row."""
+    from hyclora_amd.operators.compress_function import compress_attention_map
+    from hyclora_amd.operators.map_kernels import MapAttention
+    b, h = 2, 3
+    q, k, v, _ = operands(b, h, h, s, 64, seed=s)
+    mask = torch.zeros(b, 1, s, s, device="cuda", dtype=BF16)
+    mask[0, :, 0] = mask[1, :, s - 1] = mask[1, :, s // 2] = float("-inf")
+    q = q.clone()
+    q[0, 1, s - 1] = q[1, 2, 3] = float("nan")
+    empty = mask.isinf().all(-1).expand(b, h, s) | q.isnan().any(-1)
+    full = MapAttention(q, k, v, mask, want_map=True)
+    assert torch.equal(full.map.isnan(), empty[..., None].expand(b, h, s, s))
+    for threshold in (0.05, 0.0, -1.0, 2.0):
+        threshold = torch.full((), threshold, device="cuda")
+        idx, val, seg = compress_attention_map(full.map, threshold)
+        part = MapAttention(q, k, v, mask, threshold=threshold)
+        idx2, val2, seg2, count = part.bounded_entries(idx.numel() + 100)
+        assert count.value() == idx.numel() and torch.equal(seg2, seg)
+        assert torch.equal(idx2[:idx.numel()], idx) and same_bits(val2[:idx.numel()], val)
+
+
 @pytest.mark.parametrize("ratio", [0.0, 0.05, 1.0])
 @pytest.mark.parametrize("b,h,kv,s,d", [(1, 2, 2, 8, 64), (2, 4, 4, 32, 128), (2, 3, 1, 72, 64), (3, 8, 2, 136, 128), (1, 4, 2, 200, 128),
                                         (2, 2, 2, 256, 64), (1, 2, 1, 520, 128), (1, 1, 1, 4096, 64)])
