@@ -30,6 +30,8 @@ struct MapArgs {
     float *row_max, *row_inv;          // per row of the map
     uint32_t* counts;
     const uint64_t* classes;           // per mask batch and 32 rows: tiles with a live entry, tiles without a mask entry but 0
+    const uint32_t* wild;              // per key / value head 64 words, a byte per 16 rows of a tile: not 0 if one is not finite
+    uint32_t* walked_all;              // per workgroup of the forward: whether it walked every tile after all
     const int64_t* row_offsets;
     int64_t *indices, *seg_offsets;
     uint16_t* values;
@@ -38,15 +40,47 @@ struct MapArgs {
     float scale;
 };
 
-// Which tiles of the mask matter: bit t of classes[..][0] is set when some entry of the 32 rows x 64 keys is above kDead, of
+// 16 rows of a tile of keys and of values, looked at by one wave: is an element infinite or NaN?
+template <int D>
+__device__ __forceinline__ bool any_wild(const uint16_t* k, const uint16_t* v, int ld, int row0, int row_last, int lane) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    constexpr int kLanes = D / 8, kRows = 64 / kLanes, kLoads = 16 / kRows;      // lanes of a row, rows of a load
+    u32x4 e[2 * kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int64_t at = (int64_t)min(row0 + i * kRows + lane / kLanes, row_last) * ld + lane % kLanes * 8;
+        e[2 * i] = ld16(k + at);
+        e[2 * i + 1] = ld16(v + at);
+    }
+    u16x2 most = {0, 0};
+#pragma unroll
+    for (int i = 0; i < 2 * kLoads; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, e[i][j] & 0x7fff7fffu));
+    return __any(most.x >= 0x7f80 || most.y >= 0x7f80);
+}
+
+// Which tiles matter.  Of the mask: bit t of classes[..][0] is set when some entry of the 32 rows x 64 keys is above kDead, of
 // classes[..][1] when all are zero.  A wave looks at 8 tiles (a byte of either word), a lane at 8 keys of the 32 rows; a
-// causal mask lets half of the tiles go.
-__global__ __launch_bounds__(256) void map_classes_kernel(const uint16_t* mask, int64_t sb, int64_t sr, int S, int blocks, uint8_t* classes) {
-    const int lane = threadIdx.x & 63, bytes = (S + 511) / 512;
-    const int unit = blockIdx.x * 4 + (threadIdx.x >> 6);
+// causal mask lets half of the tiles go.  Of the keys and values: tiles may only go where all of a head's are finite, since a
+// weight of 0 times an infinite value, or an infinite score under a mask of -inf, is NaN (one read of both, 6 us of 117 at
+// [4, 1024, 32 heads, 128]).
+template <int D>
+__global__ __launch_bounds__(256) void map_classes_kernel(const MapArgs A, int mask_wgs, int mask_batches) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = A.S, bytes = (S + 511) / 512, blocks = (S + 31) / 32;
+    if ((int)blockIdx.x >= mask_wgs * mask_batches) {
+        const int i = (int)blockIdx.x - mask_wgs * mask_batches, nt = (S + kMapTile - 1) / kMapTile;
+        const int kvh = i % A.KV, t = i / A.KV % nt, b = i / A.KV / nt;
+        const int64_t at = ((int64_t)b * S * A.KV + kvh) * D;
+        const bool w = any_wild<D>(A.k + at, A.v + at, A.KV * D, t * kMapTile + wave * 16, S - 1, lane);
+        if (lane == 0) reinterpret_cast<uint8_t*>(const_cast<uint32_t*>(A.wild))[((int64_t)(b * A.KV + kvh) * 64 + t) * 4 + wave] = w;
+        return;
+    }
+    const int mb = (int)blockIdx.x / mask_wgs, unit = (int)blockIdx.x % mask_wgs * 4 + wave;
     if (unit >= blocks * bytes) return;
     const int rb = unit / bytes, step = unit % bytes, key = step * 512 + lane * 8;
-    const uint16_t* base = mask + (int64_t)blockIdx.y * sb + (int64_t)rb * 32 * sr;
+    const int64_t sr = A.mask_sr;
+    const uint16_t* base = A.mask + (int64_t)mb * A.mask_sb + (int64_t)rb * 32 * sr;
     const int rows = sr == 0 ? 1 : min(32, S - rb * 32);
     bool any = false, zero = true;
     if (key < S) {
@@ -71,7 +105,7 @@ __global__ __launch_bounds__(256) void map_classes_kernel(const uint16_t* mask, 
         if (!((z >> (8 * t)) & 0xff)) plain |= 1u << t;
     }
     if (lane == 0) {
-        uint8_t* out = classes + ((int64_t)blockIdx.y * blocks + rb) * 16 + step;
+        uint8_t* out = reinterpret_cast<uint8_t*>(const_cast<uint64_t*>(A.classes)) + ((int64_t)mb * blocks + rb) * 16 + step;
         out[0] = (uint8_t)live;
         out[8] = (uint8_t)plain;
     }
@@ -127,6 +161,8 @@ __device__ __forceinline__ MapRows map_rows(const MapArgs& A, int lane, int wave
         R.wg_live = 0;
         for (int w = 0; w < 4; ++w) R.wg_live |= c[2 * min(blk * 4 + w, nrb - 1)] & all;
         R.wg_live = uniform64(R.wg_live);
+        const uint32_t* w = A.wild + (int64_t)(R.b * A.KV + R.kvh) * 64;
+        if (__any(lane < (A.S + kMapTile - 1) / kMapTile && w[lane] != 0)) R.live = R.wg_live = all;
         R.mrow = A.mask + (int64_t)R.b * A.mask_sb + (int64_t)R.row_in * A.mask_sr;
     }
     return R;
@@ -254,8 +290,12 @@ __global__ __launch_bounds__(256, 2) void map_fwd_kernel(const MapArgs A) {
             m = mn;
         });
         // A row none of whose live tiles holds a live entry of its own (a padded query: all its keys are masked) needs the
-        // entries that were left out: with a finite mask value they all weigh the same.
-        if (attempt == 1 || !A.mask || !__syncthreads_or(m <= 0.5f * kDead)) break;
+        // entries that were left out: with a finite mask value they all weigh the same.  So does a row whose sum is NaN: its
+        // weights are NaN at every key.
+        if (attempt == 1 || !A.mask) break;
+        const bool again = __syncthreads_or(m <= 0.5f * kDead || l != l);
+        if (A.threshold && threadIdx.x == 0) A.walked_all[blockIdx.x] = again;
+        if (!again) break;
         R.live = R.wg_live = tiles_of(A.S);
         m = -INFINITY;
         l = 0.0f;
@@ -344,7 +384,7 @@ __global__ __launch_bounds__(256, 2) void map_emit_kernel(const MapArgs A) {
     const float row_max = A.row_max[R.flat], m = row_max == -INFINITY ? 0.0f : row_max;
     const float inv = A.row_inv[R.flat], limit = keep_limit(*A.threshold);
     const bool valid = R.qrow < A.S;
-    if (A.mask && __syncthreads_or(row_max <= 0.5f * kDead)) R.live = R.wg_live = tiles_of(A.S);
+    if (A.mask && A.walked_all[blockIdx.x]) R.live = R.wg_live = tiles_of(A.S);
     int64_t at_out = A.row_offsets[R.flat];
     const int64_t elem0 = R.flat * A.S;
     const int64_t total = A.row_offsets[(int64_t)A.B * A.H * A.S];
@@ -791,7 +831,7 @@ static MapBwdWorkspace map_bwd_workspace(int64_t B, int64_t S, int64_t H, int64_
 }
 
 struct MapWorkspace {                   // offsets in bytes
-    int64_t row_max, row_inv, counts, row_offsets, classes, bytes;
+    int64_t row_max, row_inv, counts, row_offsets, classes, wild, walked_all, bytes;
 };
 static MapWorkspace map_workspace(int64_t B, int64_t S, int64_t H) {
     const int64_t rows = B * H * S, nrb = cdiv(S, 32);
@@ -802,7 +842,9 @@ static MapWorkspace map_workspace(int64_t B, int64_t S, int64_t H) {
     w.counts = w.row_inv + up(rows * 4);
     w.row_offsets = w.counts + up(rows * 4);
     w.classes = w.row_offsets + up((rows + 1) * 8);
-    w.bytes = w.classes + up(B * nrb * 16);
+    w.wild = w.classes + up(B * nrb * 16);
+    w.walked_all = w.wild + up(B * H * 64 * 4);
+    w.bytes = w.walked_all + up(cdiv(S, kMapRows) * B * H * 4);
     return w;
 }
 
@@ -829,6 +871,7 @@ static MapArgs map_args(const void* q, const void* k, const void* mask, int64_t 
     A.threshold = threshold;
     A.row_max = (float*)(ws + w.row_max); A.row_inv = (float*)(ws + w.row_inv); A.counts = (uint32_t*)(ws + w.counts);
     A.row_offsets = (const int64_t*)(ws + w.row_offsets); A.classes = (const uint64_t*)(ws + w.classes);
+    A.wild = (const uint32_t*)(ws + w.wild); A.walked_all = (uint32_t*)(ws + w.walked_all);
     A.B = (int)B; A.S = (int)S; A.H = (int)H; A.KV = (int)KV; A.scale = scale;
     return A;
 }
@@ -848,9 +891,10 @@ extern "C" int hyc_map_fwd(const void* q, const void* k, const void* v, const vo
     A.v = (const uint16_t*)v; A.o = (uint16_t*)o; A.map = (uint16_t*)map;
     hipStream_t st = (hipStream_t)stream;
     if (mask) {
-        const int nrb = (int)cdiv(S, 32);
-        map_classes_kernel<<<dim3((unsigned)cdiv(nrb * cdiv(S, 512), 4), mask_stride_b ? (unsigned)B : 1u), 256, 0, st>>>(
-            A.mask, mask_stride_b, mask_stride_row, (int)S, nrb, (uint8_t*)const_cast<uint64_t*>(A.classes));
+        const int mask_wgs = (int)cdiv(cdiv(S, 32) * cdiv(S, 512), 4), batches = mask_stride_b ? (int)B : 1;
+        const dim3 wgs((unsigned)(mask_wgs * batches + cdiv(S, kMapTile) * B * KV));
+        if (D == 128) map_classes_kernel<128><<<wgs, 256, 0, st>>>(A, mask_wgs, batches);
+        else map_classes_kernel<64><<<wgs, 256, 0, st>>>(A, mask_wgs, batches);
     }
     const dim3 grid((unsigned)(cdiv(S, kMapRows) * B * H));
     if (D == 128) map_fwd_kernel<128><<<grid, 256, 0, st>>>(A);

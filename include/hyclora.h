@@ -669,7 +669,9 @@ int hyc_flash_bwd(const void *grad_o, const void *q, const void *k, const void *
  *   q, o, grad_o, grad_q  bf16 [B, S, H, D] contiguous;  k, v, grad_k, grad_v  bf16 [B, S, KV, D] contiguous, H % KV == 0
  *                (grad_k, grad_v: each query head's rounded to bf16, a group's added in fp32 and rounded); D 64 or 128; S % 8 == 0, S <= 4096;
  *   mask         bf16 or NULL, added to every head: entry (b, i, j) at b * mask_stride_b + i * mask_stride_row + j (strides
- *                multiples of 8, 0 broadcasts).  Keys at or below -1e30 cost nothing where 32 rows x 64 keys are all so;
+ *                multiples of 8, 0 broadcasts).  Keys at or below -1e30 cost nothing where 32 rows x 64 keys are all so, all
+ *                keys and values of the head are finite and no row of the 128 has a NaN sum or only such keys; otherwise they
+ *                are worked through, so NaN and infinities spread as over a dense map (finite scores are taken to be below 1e30);
  *   map          bf16 [B, H, S, S] or NULL: the dense p as well (calibration, uncompressed layers);
  *   threshold    fp32 on the device or NULL: hyc_map_fwd then leaves in `workspace` what hyc_map_emit needs;
  *   workspace    hyc_map_workspace(B, S, H) bytes, 16-byte aligned, kept unchanged between hyc_map_fwd and hyc_map_emit.

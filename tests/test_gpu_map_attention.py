@@ -99,6 +99,42 @@ def test_rows_without_a_finite_sum_keep_nothing_past_their_end(s):
         assert torch.equal(idx2[:idx.numel()], idx) and same_bits(val2[:idx.numel()], val)
 
 
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("where", ["q", "k", "v", "mask"])
+@pytest.mark.parametrize("kind", ["causal", "padded", "keys"])
+@pytest.mark.parametrize("h,kv,s,d", [(2, 2, 72, 64), (4, 2, 200, 128), (2, 1, 520, 64)])
+def test_values_that_are_not_finite_spread_as_over_a_dense_map(h, kv, s, d, kind, where, value):
+    """A masked key counts as well: its weight is 0, and 0 times an infinite value is NaN.  The dense map of the operators that go
+    through memory says which elements are NaN."""
+    from hyclora_amd.operators.compress_function import compress_attention_map
+    from hyclora_amd.operators.map_kernels import MapAttention
+    from hyclora_amd.operators.softmax_kernels import softmax_forward
+    b = 3
+    q, k, v, _ = (t.clone() for t in operands(b, h, kv, s, d, seed=s + h))
+    mask = masks(kind, b, s)
+    mask = mask.expand(mask.shape[0], 1, s, s).clone()
+    if where == "mask":
+        mask[-1, 0, s // 3, s - 2] = value
+    else:
+        {"q": q, "k": k, "v": v}[where][1, 0, s - 2, 5] = value
+    kr, vr = (t.repeat_interleave(h // kv, 1).float() for t in (k, v))
+    scores = (q.float() @ kr.transpose(-1, -2).contiguous()).to(BF16)
+    want = softmax_forward(scores, 1.0 / math.sqrt(d), mask)
+    o = want.float() @ vr.contiguous()
+    full = MapAttention(q, k, v, mask, want_map=True)
+    for got, ref in ((full.map, want), (full.o, o)):
+        assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+        finite = ref.isfinite()
+        assert rel(got[finite], ref[finite]) < 8 * 2 ** -9       # as in test_forward_and_kept_entries
+    threshold = torch.full((), 0.02, device="cuda")
+    part = MapAttention(q, k, v, mask, threshold=threshold)
+    assert same_bits(part.o, full.o)
+    idx, val, seg = compress_attention_map(full.map, threshold)
+    idx2, val2, seg2, count = part.bounded_entries(idx.numel() + 9)
+    assert count.value() == idx.numel() and torch.equal(seg2, seg)
+    assert torch.equal(idx2[:idx.numel()], idx) and same_bits(val2[:idx.numel()], val)
+
+
 @pytest.mark.parametrize("ratio", [0.0, 0.05, 1.0])
 @pytest.mark.parametrize("b,h,kv,s,d", [(1, 2, 2, 8, 64), (2, 4, 4, 32, 128), (2, 3, 1, 72, 64), (3, 8, 2, 136, 128), (1, 4, 2, 200, 128),
                                         (2, 2, 2, 256, 64), (1, 2, 1, 520, 128), (1, 1, 1, 4096, 64)])
