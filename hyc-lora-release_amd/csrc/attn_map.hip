@@ -456,21 +456,52 @@ struct MapBwdArgs {
     uint32_t* entries;                  // (row % 32 * 64 + key % 64) << 16 | value, grouped by 32-row x 64-key tile
     uint16_t* grads;                    // per entry: the map's gradient, then the score's
     uint32_t* tile_at;                  // [B * H * row blocks, tiles + 1]: where a tile's entries begin
+    uint32_t* wild;                     // [B * H * row blocks]: operands of the block that are not finite, kWildRows | kWildKeys
+    uint32_t* wild_sums;                // [B * H * row blocks]: rows whose d is not finite; of heads with such operands only
     uint16_t *grad_q, *grad_k, *grad_v;
     int B, S, H, KV;
     float scale;
 };
 
+// Work on tiles without a kept entry may only be left out where all operands of a head are finite: elsewhere 0 times an infinite
+// value, or an infinite gradient of the map times the 0 of an entry that is not kept, is NaN.
+constexpr uint32_t kWildRows = 1;       // q, grad_o or a kept entry of the rows
+constexpr uint32_t kWildKeys = 2;       // k or v of rows of these numbers (noted by the first query head of a group)
+
+// Whether a head has an operand that is not finite; the words of its row blocks are read by one wave (at most 128).
+__device__ __forceinline__ bool head_is_wild(const MapBwdArgs& A, int bh, int nrb, int lane) {
+    const int lead = bh - bh % A.H % (A.H / A.KV);
+    uint32_t w = 0;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int rb = min(lane + 64 * i, nrb - 1);
+        w |= (A.wild[(int64_t)bh * nrb + rb] & kWildRows) | (A.wild[(int64_t)lead * nrb + rb] & kWildKeys);
+    }
+    return __any(w != 0);
+}
+
 // Groups the entries of 32 rows by tile of 64 keys.  The entries of a tile come in no particular order (each has its own
-// place in the dense tile that the kernels below rebuild from them, so no result depends on it).
+// place in the dense tile that the kernels below rebuild from them, so no result depends on it).  Looks at the operands of
+// the 32 rows on the way, while it waits for its counts.
+template <int D>
 __global__ __launch_bounds__(256) void map_regroup_kernel(const MapBwdArgs A) {
-    __shared__ uint32_t place[kMapMax / kMapTile], below[2];
+    __shared__ uint32_t place[kMapMax / kMapTile], below[2], marks;
     const int nrb = (A.S + 31) / 32, nt = (A.S + kMapTile - 1) / kMapTile;
     const int bh = blockIdx.x / nrb, r0 = (int)(blockIdx.x % nrb) * 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = bh / A.H, head = bh % A.H, group = A.H / A.KV;
+    uint32_t mark = 0;
+    if (wave < 2) {
+        const int64_t at = ((int64_t)b * A.S * A.H + head) * D;
+        if (any_wild<D>(A.q + at, A.grad_o + at, A.H * D, r0 + wave * 16, A.S - 1, lane)) mark = kWildRows;
+    } else if (head % group == 0) {
+        const int64_t at = ((int64_t)b * A.S * A.KV + head / group) * D;
+        if (any_wild<D>(A.k + at, A.v + at, A.KV * D, r0 + wave % 2 * 16, A.S - 1, lane)) mark = kWildKeys;
+    }
     const int64_t elems = (int64_t)A.B * A.H * A.S * A.S;
     const int64_t e0 = ((int64_t)bh * A.S + r0) * A.S, e1 = e0 + (int64_t)min(32, A.S - r0) * A.S;
     if (threadIdx.x < (unsigned)nt) place[threadIdx.x] = 0;
     if (threadIdx.x < 2) below[threadIdx.x] = 0;
+    if (threadIdx.x == 2) marks = 0;
     __syncthreads();
     int64_t edge[2];
 #pragma unroll
@@ -510,14 +541,20 @@ __global__ __launch_bounds__(256) void map_regroup_kernel(const MapBwdArgs A) {
     for (int64_t i = first + threadIdx.x; i < last; i += 256) {
         uint32_t row, key;
         split((uint32_t)(A.indices[i] - e0), row, key);
-        const uint32_t slot = atomicAdd(&place[key / kMapTile], 1u);
-        A.entries[slot] = (row * kMapTile + key % kMapTile) << 16 | A.values[i];
+        const uint32_t slot = atomicAdd(&place[key / kMapTile], 1u), value = A.values[i];
+        A.entries[slot] = (row * kMapTile + key % kMapTile) << 16 | value;
+        if ((value & 0x7f80u) == 0x7f80u) mark |= kWildRows;
     }
+    if (mark) atomicOr(&marks, mark);
+    __syncthreads();
+    if (threadIdx.x == 0) A.wild[blockIdx.x] = marks;
 }
 
 // Entries of a tile that a wave holds in registers: 64 of each of kHeld loads.  With 5 % of a causal map kept, the tiles below
 // the diagonal hold 200 on average; the few fuller ones (a row's first keys) are worked through kHeld loads at a time.
 constexpr int kHeld = 4;
+
+constexpr uint32_t kNanPair = 0x7fc07fc0u;
 
 // Clears a wave's 32 x 64 patch
 __device__ __forceinline__ void clear_patch(char* patch, int lane) {
@@ -527,7 +564,9 @@ __device__ __forceinline__ void clear_patch(char* patch, int lane) {
 
 // grad_q of 128 rows.  First walk: g at the kept entries and the row sums d (the tile of a is rebuilt in LDS, the products of
 // one tile are 32 x 64 values of which a few percent are kept).  Second walk: ds from g, d and a per entry, its tile rebuilt in
-// LDS as the operand of ds k; ds stays in `grads` for the key / value kernel.  Tiles without an entry are left out.
+// LDS as the operand of ds k; ds stays in `grads` for the key / value kernel.  Tiles without an entry are left out, unless the
+// head has an operand that is not finite: then every tile is worked through, and in a row whose d is not finite the entries
+// that are not kept, (g - d) * 0, are NaN.
 template <int D>
 __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
     using Tile = AttnTile<D, kMapTile>;
@@ -549,7 +588,8 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
     uint64_t* wave_tiles = reinterpret_cast<uint64_t*>(lds + 2 * Tile::kBytes + 4 * MapPatch::kBytes + 4 * 128);
     const uint32_t* tile_at = A.tile_at + ((int64_t)bh * nrb + min(rb, nrb - 1)) * (nt + 1);
     const uint32_t t_beg = rb < nrb ? tile_at[min(lane, nt)] : 0u, t_end = rb < nrb ? tile_at[min(lane + 1, nt)] : 0u;     // of tile `lane`
-    const uint64_t own = __ballot(lane < nt && t_end > t_beg);
+    const bool wild = head_is_wild(A, bh, nrb, lane);
+    const uint64_t own = wild && rb < nrb ? tiles_of(A.S) : __ballot(lane < nt && t_end > t_beg);
     if (lane == 0) wave_tiles[wave] = own;
     __syncthreads();
     const uint64_t todo = uniform64(wave_tiles[0] | wave_tiles[1] | wave_tiles[2] | wave_tiles[3]);
@@ -572,7 +612,7 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
         const int t = __builtin_ctzll(tiles);
         beg = (uint32_t)__builtin_amdgcn_readlane((int)t_beg, t);
         n = (uint32_t)__builtin_amdgcn_readlane((int)t_end, t) - beg;
-        load(0, with_grads);
+        if (n) load(0, with_grads);
     };
     auto later = [&](int t) { return t < 63 ? own >> (t + 1) << (t + 1) : 0ull; };
     int buf = 0;
@@ -631,6 +671,11 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
     d = half_sum(d);
     if (lane < 32) row_sum[lane] = d;
     lds_order();
+    const bool wild_sum = !(__builtin_fabsf(d) < INFINITY);
+    if (wild && rb < nrb) {
+        const uint32_t rows = (uint32_t)__ballot(wild_sum && qrow < A.S);
+        if (lane == 0) A.wild_sums[(int64_t)bh * nrb + rb] = rows;
+    }
     f32x16 dq[D / 32];
 #pragma unroll
     for (int db = 0; db < D / 32; ++db) dq[db] = f32x16{};
@@ -638,7 +683,13 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
     walk_tiles(todo, buf, [&](int t, int bb) { Tile::request(kbase, t * kMapTile, A.S - 1, ldk, lds0 + bb * Tile::kBytes, wave, lane); },
                [&](int t, int bb) {
         if (!((own >> t) & 1)) return;
-        clear_patch(patch, lane);
+        if (wild) {
+            const uint32_t v = wild_sum ? kNanPair : 0u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(patch + (lane & 31) * 128 + (4 * h + i) * 16) = u32x4{v, v, v, v};
+        } else {
+            clear_patch(patch, lane);
+        }
         lds_order();
         auto put = [&](uint32_t i, uint32_t v, uint32_t g) {
             const uint16_t ds = f_to_bf(rbf((bf_to_f((uint16_t)g) - row_sum[v >> 22]) * bf_lo(v)) * A.scale);
@@ -687,6 +738,7 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
     const int ldq = A.H * D;
     const int key = blk * kMapRows + wave * 32 + (lane & 31);
     const int t0 = blk * 2, t1 = min(t0 + 1, nt), t2 = min(t0 + 2, nt);
+    const bool wild = head_is_wild(A, bh, nrb, lane);                    // then every step, with or without entries
     const uint32_t* tile_at = A.tile_at + (int64_t)bh * nrb * (nt + 1);
     // a step: 32 rows with entries, where those of the first tile begin, how many they and the second's are
     uint32_t* steps = reinterpret_cast<uint32_t*>(lds + 4 * Tile::kBytes + 8 * kPatch);
@@ -696,7 +748,7 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
     const uint16_t* qb = A.q + (int64_t)b * A.S * ldq + head * D;
     const uint16_t* gb = A.grad_o + (int64_t)b * A.S * ldq + head * D;
     // wave w rebuilds tile w % 2 of the two, of a (w < 2) or of ds
-    struct Pending { uint32_t beg, n, e[kHeld], v[kHeld]; };
+    struct Pending { uint32_t beg, n, nan_rows, e[kHeld], v[kHeld]; };
     auto load = [&](Pending& p, uint32_t from) {
 #pragma unroll
         for (int u = 0; u < kHeld; ++u) {
@@ -713,6 +765,7 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
         const uint32_t first = steps[3 * i + 1], both = steps[3 * i + 2];
         p.beg = __builtin_amdgcn_readfirstlane(wave & 1 ? first + (both & 0xffffu) : first);
         p.n = __builtin_amdgcn_readfirstlane(wave & 1 ? both >> 16 : both & 0xffffu);
+        p.nan_rows = wild && wave >> 1 ? A.wild_sums[(int64_t)bh * nrb + steps[3 * i]] : 0u;
         load(p, 0);
         return p;
     };
@@ -724,6 +777,8 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
             const uint32_t row = e >> 22, k = (e >> 16) & 63;
             *reinterpret_cast<uint16_t*>(patch + k * 64 + (((row >> 3) ^ ((k >> 2) & 3)) << 4) + (row & 7) * 2) = (uint16_t)v;
         };
+        for (uint32_t rows = p.nan_rows; rows; rows &= rows - 1) put((uint32_t)__builtin_ctz(rows) << 22 | (uint32_t)lane << 16, kNanPair);
+        lds_order();
         for (uint32_t from = 0;;) {
 #pragma unroll
             for (int u = 0; u < kHeld; ++u) if (from + (uint32_t)(lane + 64 * u) < p.n) put(p.e[u], wave >> 1 ? p.v[u] : p.e[u]);
@@ -749,11 +804,12 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
             const uint32_t* r = tile_at + (int64_t)s * (nt + 1);
             a0 = r[t0]; a1 = r[t1]; a2 = r[t2];
         }
-        const uint64_t m = __ballot(a2 > a0);
+        const bool step = a2 > a0 || (wild && s < nrb);
+        const uint64_t m = __ballot(step);
         if (lane == 0) wave_n[wave] = __popcll(m);
         __syncthreads();
         nsteps = wave_n[0] + wave_n[1];
-        if (a2 > a0) {
+        if (step) {
             const int place = (wave ? wave_n[0] : 0) + __popcll(m & ((1ull << lane) - 1));
             steps[3 * place] = s;
             steps[3 * place + 1] = a0;
@@ -818,14 +874,16 @@ __global__ __launch_bounds__(256) void group_sum_kernel(const uint16_t* __restri
     st16((blockIdx.y ? out1 : out0) + c * 8, pack8(acc));
 }
 
-struct MapBwdWorkspace { int64_t entries, grads, tile_at, heads, bytes; };
+struct MapBwdWorkspace { int64_t entries, grads, tile_at, wild, wild_sums, heads, bytes; };
 static MapBwdWorkspace map_bwd_workspace(int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D, int64_t capacity) {
     auto up = [](int64_t v) { return cdiv(v, 256) * 256; };
     MapBwdWorkspace w;
     w.entries = 0;
     w.grads = up(capacity * 4);
     w.tile_at = w.grads + up(capacity * 2);
-    w.heads = w.tile_at + up(B * H * cdiv(S, 32) * (cdiv(S, kMapTile) + 1) * 4);        // per query head: grad_k, then grad_v
+    w.wild = w.tile_at + up(B * H * cdiv(S, 32) * (cdiv(S, kMapTile) + 1) * 4);
+    w.wild_sums = w.wild + up(B * H * cdiv(S, 32) * 4);
+    w.heads = w.wild_sums + up(B * H * cdiv(S, 32) * 4);                                 // per query head: grad_k, then grad_v
     w.bytes = w.heads + (H == KV ? 0 : 2 * up(B * S * H * D * 2));
     return w;
 }
@@ -945,6 +1003,7 @@ extern "C" int hyc_map_bwd(const void* grad_o, const void* q, const void* k, con
     A.grad_o = (const uint16_t*)grad_o; A.q = (const uint16_t*)q; A.k = (const uint16_t*)k; A.v = (const uint16_t*)v;
     A.indices = indices; A.values = (const uint16_t*)values; A.seg_offsets = seg_offsets;
     A.entries = (uint32_t*)(ws + w.entries); A.grads = (uint16_t*)(ws + w.grads); A.tile_at = (uint32_t*)(ws + w.tile_at);
+    A.wild = (uint32_t*)(ws + w.wild); A.wild_sums = (uint32_t*)(ws + w.wild_sums);
     A.grad_q = (uint16_t*)grad_q; A.grad_k = (uint16_t*)grad_k; A.grad_v = (uint16_t*)grad_v;
     if (H != KV) {
         A.grad_k = (uint16_t*)(ws + w.heads);
@@ -953,11 +1012,12 @@ extern "C" int hyc_map_bwd(const void* grad_o, const void* q, const void* k, con
     A.B = (int)B; A.S = (int)S; A.H = (int)H; A.KV = (int)KV; A.scale = scale;
     hipStream_t st = (hipStream_t)stream;
     const dim3 rows((unsigned)(cdiv(S, 32) * B * H)), blocks((unsigned)(cdiv(S, kMapRows) * B * H));
-    map_regroup_kernel<<<rows, 256, 0, st>>>(A);
     if (D == 128) {
+        map_regroup_kernel<128><<<rows, 256, 0, st>>>(A);
         map_bwd_q_kernel<128><<<blocks, 256, 0, st>>>(A);
         map_bwd_kv_kernel<128><<<blocks, 256, 0, st>>>(A);
     } else {
+        map_regroup_kernel<64><<<rows, 256, 0, st>>>(A);
         map_bwd_q_kernel<64><<<blocks, 256, 0, st>>>(A);
         map_bwd_kv_kernel<64><<<blocks, 256, 0, st>>>(A);
     }

@@ -679,6 +679,8 @@ int hyc_flash_bwd(const void *grad_o, const void *q, const void *k, const void *
  *                hyc_sparse_write_bounded) and seg_offsets int64 [hyc_sparse_num_segments(B*H*S*S) + 1], whose last element is
  *                the number of kept entries; same q, k, mask, threshold and scale as the forward.
  * hyc_map_bwd    takes complete lists of `capacity` >= kept entries (< 2^31); workspace hyc_map_bwd_workspace(...) bytes.
+ *                NaN and infinities in its operands or lists make NaN wherever the dense formulas above do, at entries that are
+ *                not kept as well.
  * Fixed summation orders, no floating-point atomics: the same bits on every run.
  */
 int64_t hyc_map_workspace(int64_t B, int64_t S, int64_t H);

@@ -135,6 +135,17 @@ def test_values_that_are_not_finite_spread_as_over_a_dense_map(h, kv, s, d, kind
     assert torch.equal(idx2[:idx.numel()], idx) and same_bits(val2[:idx.numel()], val)
 
 
+def dense_backward(go, q, k, v, a):
+    """The gradients through the dense map `a`, from float64 products with the layers' roundings."""
+    kv, n_rep, d = k.shape[1], q.shape[1] // k.shape[1], q.shape[-1]
+    kr, vr = (t.repeat_interleave(n_rep, 1).double().contiguous() for t in (k, v))
+    g = (go.double() @ vr.transpose(-1, -2).contiguous()).to(BF16)
+    dsum = (a.float() * g.float()).to(BF16).double().sum(-1, keepdim=True)
+    ds = (((g.double() - dsum) * a.double()).to(BF16).float() / math.sqrt(d)).to(BF16).double()
+    group = lambda t: t.unflatten(1, (kv, n_rep)).sum(2)                              # noqa: E731
+    return ds @ kr, group(ds.transpose(-1, -2).contiguous() @ q.double()), group(a.double().transpose(-1, -2).contiguous() @ go.double())
+
+
 @pytest.mark.parametrize("ratio", [0.0, 0.05, 1.0])
 @pytest.mark.parametrize("b,h,kv,s,d", [(1, 2, 2, 8, 64), (2, 4, 4, 32, 128), (2, 3, 1, 72, 64), (3, 8, 2, 136, 128), (1, 4, 2, 200, 128),
                                         (2, 2, 2, 256, 64), (1, 2, 1, 520, 128), (1, 1, 1, 4096, 64)])
@@ -147,20 +158,55 @@ def test_backward_from_kept_entries(b, h, kv, s, d, ratio):
         get_statistics_softmax(full.map, ratio)
     idx, val, seg = compress_attention_map(full.map, thr)
     got = map_backward(go, q, k, v, idx, val, seg)
-    a = restore_attention_map(idx, val, seg, (b, h, s, s))
-    n_rep = h // kv
-    kr, vr = (t.repeat_interleave(n_rep, 1).double().contiguous() for t in (k, v))
-    g = (go.double() @ vr.transpose(-1, -2).contiguous()).to(BF16)
-    dsum = (a.float() * g.float()).to(BF16).double().sum(-1, keepdim=True)
-    ds = (((g.double() - dsum) * a.double()).to(BF16).float() / math.sqrt(d)).to(BF16).double()
-    group = lambda t: t.unflatten(1, (kv, n_rep)).sum(2)                              # noqa: E731
-    want = (ds @ kr, group(ds.transpose(-1, -2).contiguous() @ q.double()), group(a.double().transpose(-1, -2).contiguous() @ go.double()))
+    want = dense_backward(go, q, k, v, restore_attention_map(idx, val, seg, (b, h, s, s)))
     for x, w, name in zip(got, want, ("grad_q", "grad_k", "grad_v")):
         assert x.shape == w.shape
         # the same bf16 operands on both sides, up to last bits of g; fp32 sums and one rounding
         assert (rel(x, w) < 2 ** -8 if w.norm() > 0 else x.abs().max() == 0), (name, rel(x, w))
     again = map_backward(go, q, k, v, torch.cat([idx, idx.new_full((7,), -1)]), torch.cat([val, val.new_zeros(7)]), seg)
     assert all(torch.equal(x, y) for x, y in zip(got, again))          # room past the entries is not read
+
+
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("where", ["grad_o", "q", "k", "v", "map"])
+@pytest.mark.parametrize("threshold", [2.0, 0.1, 0.0])
+@pytest.mark.parametrize("h,kv,s,d", [(2, 2, 72, 64), (4, 2, 200, 128), (2, 1, 520, 64)])
+def test_gradients_that_are_not_finite_spread_as_over_a_dense_map(h, kv, s, d, threshold, where, value):
+    """Entries that are not kept count as well: their 0 times an infinite operand, or an infinite gradient of the map times their
+    0, is NaN.  At 2.0 nothing is kept, at 0.1 the later rows keep little or nothing."""
+    from hyclora_amd.operators.compress_function import compress_attention_map, restore_attention_map
+    from hyclora_amd.operators.map_kernels import MapAttention, map_backward
+    b = 3
+    q, k, v, go = (t.clone() for t in operands(b, h, kv, s, d, seed=s + h))
+    amap = MapAttention(q, k, v, masks("causal", b, s), want_map=True).map
+    if where == "map":
+        amap[1, 0, s - 3, s // 2] = value                      # kept by a threshold below infinity
+    else:
+        {"grad_o": go, "q": q, "k": k, "v": v}[where][1, 0, s - 3, 5] = value
+    idx, val, seg = compress_attention_map(amap, torch.full((), threshold, device="cuda"))
+    got = map_backward(go, q, k, v, idx, val, seg)
+    want = dense_backward(go, q, k, v, restore_attention_map(idx, val, seg, (b, h, s, s)))
+    for x, w, name in zip(got, want, ("grad_q", "grad_k", "grad_v")):
+        finite = w.isfinite()
+        assert torch.equal(x.isfinite(), finite), name
+        assert rel(x[finite], w[finite]) < 2 ** -8 if w[finite].norm() > 0 else x[finite].abs().max() == 0, name
+
+
+@pytest.mark.parametrize("s", [72, 96, 200])
+def test_gradients_of_rows_without_a_finite_sum(s):
+    """Lists of rows that are NaN throughout, at lengths with a partial last tile and a partial last block of rows."""
+    from hyclora_amd.operators.compress_function import restore_attention_map
+    from hyclora_amd.operators.map_kernels import MapAttention, map_backward
+    b, h, d = 2, 3, 64
+    q, k, v, go = operands(b, h, h, s, d, seed=s)
+    mask = masks("causal", b, s).expand(b, 1, s, s).clone()
+    mask[0, :, s - 1] = mask[1, :, 5] = float("-inf")
+    part = MapAttention(q, k, v, mask, threshold=torch.full((), 0.1, device="cuda"))
+    idx, val, seg = part.entries(int(part.entries(0)[2][-1]))
+    got = map_backward(go, q, k, v, idx, val, seg)
+    want = dense_backward(go, q, k, v, restore_attention_map(idx, val, seg, (b, h, s, s)))
+    for x, w in zip(got, want):
+        assert torch.equal(x.isfinite(), w.isfinite()) and rel(x[w.isfinite()], w[w.isfinite()]) < 2 ** -8
 
 
 @pytest.mark.parametrize("q_bit,b,s,fits", [(2, 1, 1016, False), (2, 1, 1024, True), (2, 2, 512, True), (2, 3, 64, False), (4, 1, 64, True), (8, 1, 8, True),
