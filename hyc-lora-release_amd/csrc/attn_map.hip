@@ -28,7 +28,7 @@ struct MapArgs {
     uint16_t *o, *map;                 // map: dense copy, or NULL
     const float* threshold;            // NULL: nothing is counted
     float *row_max, *row_inv;          // per row of the map
-    uint32_t* counts;
+    uint32_t *counts, *block_counts;   // kept entries of a row; of the 32 rows of a wave
     const uint64_t* classes;           // per mask batch and 32 rows: tiles with a live entry, tiles without a mask entry but 0
     const uint32_t* wild;              // per key / value head 64 words, a byte per 16 rows of a tile: not 0 if one is not finite
     uint32_t* walked_all;              // per workgroup of the forward: whether it walked every tile after all
@@ -118,6 +118,9 @@ __device__ __forceinline__ float keep_limit(float thr) {
     if (b & 0x80000000u) return (b & 0x7fffffffu) > 0x7f800000u ? INFINITY : __builtin_bit_cast(float, 0x8000u);
     return __builtin_bit_cast(float, b + ((b & 0x10000u) ? 0x7fffu : 0x8000u));
 }
+
+// blocks of 32 rows that the waves of a head's workgroups own (the last ones may lie past its rows)
+__host__ __device__ inline int64_t row_blocks(int64_t S) { return (S + kMapRows - 1) / kMapRows * (kMapRows / 32); }
 
 __device__ __forceinline__ uint64_t tiles_of(int S) {
     const int n = (S + kMapTile - 1) / kMapTile;
@@ -352,12 +355,50 @@ __global__ __launch_bounds__(256, 2) void map_fwd_kernel(const MapArgs A) {
     if (R.qrow < A.S) store_rows<D>(A.o + ((int64_t)R.b * A.S + R.qrow) * ldq + R.head * D, h, O, 1.0f);
     if (A.threshold) {
         const u32x2 both = __builtin_amdgcn_permlane32_swap(count, count, false, false);
+        const uint32_t kept = R.qrow < A.S ? both.x + both.y : 0u;
         if (R.qrow < A.S && h == 0) {
             A.row_max[R.flat] = row_max;
             A.row_inv[R.flat] = inv;
-            A.counts[R.flat] = both.x + both.y;
+            A.counts[R.flat] = kept;
         }
+        const uint32_t up_to = wave_inclusive_scan(kept);
+        if (lane == 31) A.block_counts[(int64_t)(R.b * A.H + R.head) * row_blocks(A.S) + R.q0 / 32] = up_to;
     }
+}
+
+// row_offsets[r] = kept entries of the rows before r, for every r up to B * H * S.  A workgroup scans the 1024 counts of its own rows
+// and adds up what lies before them by itself, from the counts of 32 rows: what grows with the square of the rows is a 1024th
+// of 32nds (from the counts of single rows, [512, 128, 16 heads, 64] took longer for this scan than for the attention).
+__global__ __launch_bounds__(1024) void map_row_scan_kernel(const uint32_t* counts, const uint32_t* block_counts, int64_t rows, int S, int64_t* offsets) {
+    __shared__ long long front_part[16];
+    __shared__ uint32_t wave_total[16];
+    const int t = threadIdx.x, lane = t & (kWave - 1), wave = t >> 6;
+    const int64_t base = (int64_t)blockIdx.x * 1024, blocks = base / S * row_blocks(S) + base % S / 32;
+    long long front = t < (int)(base % S % 32) ? counts[base - 1 - t] : 0;
+    for (int64_t f = t; f < blocks; f += 4 * 1024) {
+        uint32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = f + u * 1024 < blocks ? block_counts[f + u * 1024] : 0u;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) front += v[u];
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) front += __shfl_xor(front, o, kWave);
+    const int64_t row = base + t;
+    const uint32_t c = row < rows ? counts[row] : 0u, inc = wave_inclusive_scan(c);
+    if (lane == 0) front_part[wave] = front;
+    if (lane == kWave - 1) wave_total[wave] = inc;
+    __syncthreads();
+    long long at = 0;
+    uint32_t before = 0, total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        at += front_part[w];
+        before += w < wave ? wave_total[w] : 0u;
+        total += wave_total[w];
+    }
+    if (row < rows) offsets[row] = at + before + (inc - c);
+    if (t == 0 && base + 1024 >= rows) offsets[rows] = at + total;
 }
 
 // A 32-row x 64-key bf16 tile that one wave keeps in LDS: rows of 128 bytes, their 16-byte chunks permuted by the row.
@@ -889,7 +930,7 @@ static MapBwdWorkspace map_bwd_workspace(int64_t B, int64_t S, int64_t H, int64_
 }
 
 struct MapWorkspace {                   // offsets in bytes
-    int64_t row_max, row_inv, counts, row_offsets, classes, wild, walked_all, bytes;
+    int64_t row_max, row_inv, counts, block_counts, row_offsets, classes, wild, walked_all, bytes;
 };
 static MapWorkspace map_workspace(int64_t B, int64_t S, int64_t H) {
     const int64_t rows = B * H * S, nrb = cdiv(S, 32);
@@ -898,7 +939,8 @@ static MapWorkspace map_workspace(int64_t B, int64_t S, int64_t H) {
     w.row_max = 0;
     w.row_inv = up(rows * 4);
     w.counts = w.row_inv + up(rows * 4);
-    w.row_offsets = w.counts + up(rows * 4);
+    w.block_counts = w.counts + up(rows * 4);
+    w.row_offsets = w.block_counts + up(B * H * row_blocks(S) * 4);
     w.classes = w.row_offsets + up((rows + 1) * 8);
     w.wild = w.classes + up(B * nrb * 16);
     w.walked_all = w.wild + up(B * H * 64 * 4);
@@ -911,8 +953,6 @@ static int map_check(int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D) {
     if (S * H * D > (int64_t)1 << 30 || B > 65535 || cdiv(S, kMapRows) * B * H > (1 << 30)) return HYC_ERR_SHAPE;
     return HYC_OK;
 }
-
-int launch_row_scan(const uint32_t* counts, int64_t n, int64_t* offsets, hipStream_t st);      // softmax_map.hip
 
 }  // namespace hyc
 
@@ -928,6 +968,7 @@ static MapArgs map_args(const void* q, const void* k, const void* mask, int64_t 
     A.q = (const uint16_t*)q; A.k = (const uint16_t*)k; A.mask = (const uint16_t*)mask; A.mask_sb = msb; A.mask_sr = msr;
     A.threshold = threshold;
     A.row_max = (float*)(ws + w.row_max); A.row_inv = (float*)(ws + w.row_inv); A.counts = (uint32_t*)(ws + w.counts);
+    A.block_counts = (uint32_t*)(ws + w.block_counts);
     A.row_offsets = (const int64_t*)(ws + w.row_offsets); A.classes = (const uint64_t*)(ws + w.classes);
     A.wild = (const uint32_t*)(ws + w.wild); A.walked_all = (uint32_t*)(ws + w.walked_all);
     A.B = (int)B; A.S = (int)S; A.H = (int)H; A.KV = (int)KV; A.scale = scale;
@@ -957,7 +998,9 @@ extern "C" int hyc_map_fwd(const void* q, const void* k, const void* v, const vo
     const dim3 grid((unsigned)(cdiv(S, kMapRows) * B * H));
     if (D == 128) map_fwd_kernel<128><<<grid, 256, 0, st>>>(A);
     else map_fwd_kernel<64><<<grid, 256, 0, st>>>(A);
-    if (threshold) return launch_row_scan(A.counts, B * H * S, const_cast<int64_t*>(A.row_offsets), st);
+    if (threshold)
+        map_row_scan_kernel<<<dim3((unsigned)cdiv(B * H * S, 1024)), 1024, 0, st>>>(A.counts, A.block_counts, B * H * S, (int)S,
+                                                                                    const_cast<int64_t*>(A.row_offsets));
     return check_launch();
 }
 

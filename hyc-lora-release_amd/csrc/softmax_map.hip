@@ -739,13 +739,6 @@ extern "C" int hyc_hist_select(const uint32_t* hist, int64_t kth, float* thresho
     return check_launch();
 }
 
-namespace hyc {
-int launch_row_scan(const uint32_t* counts, int64_t n, int64_t* offsets, hipStream_t st) {
-    hipLaunchKernelGGL(seg_scan_kernel, dim3((unsigned)(n > 1024 ? cdiv(n, 1024) : 1)), dim3(1024), 0, st, counts, n, offsets);
-    return check_launch();
-}
-}  // namespace hyc
-
 extern "C" int64_t hyc_sparse_num_segments(int64_t n) { return n <= 0 ? 0 : cdiv(n, kSeg); }
 
 extern "C" int hyc_sparse_count(const void* a, int64_t n, const float* threshold, int compare_abs, uint32_t* seg_counts,

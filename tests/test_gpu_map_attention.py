@@ -72,6 +72,18 @@ def test_forward_and_kept_entries(b, h, kv, s, d, kind):
             assert torch.equal(idx2[:m], idx[:m]) and torch.equal(val2[:m], val[:m])
 
 
+@pytest.mark.parametrize("b,h,s", [(33, 16, 136), (5, 9, 1000), (260, 1, 8)])
+def test_entries_of_many_rows(b, h, s):
+    """More rows than a workgroup of the scan takes, starting inside a head and inside its blocks of 32 rows."""
+    from hyclora_amd.operators.compress_function import compress_attention_map
+    from hyclora_amd.operators.map_kernels import MapAttention
+    q, k, v, _ = operands(b, h, h, s, 64, seed=s)
+    threshold = torch.full((), 0.1, device="cuda")
+    idx, val, seg = compress_attention_map(MapAttention(q, k, v, want_map=True).map, threshold)
+    idx2, val2, seg2 = MapAttention(q, k, v, threshold=threshold).entries(idx.numel())
+    assert torch.equal(idx2, idx) and torch.equal(val2, val) and torch.equal(seg2, seg)
+
+
 def same_bits(a, b):
     return torch.equal(a.view(torch.int16), b.view(torch.int16))
 
