@@ -366,9 +366,9 @@ __global__ __launch_bounds__(256, 2) void map_fwd_kernel(const MapArgs A) {
     }
 }
 
-// row_offsets[r] = kept entries of the rows before r, for every r up to B * H * S.  A workgroup scans the 1024 counts of its own rows
-// and adds up what lies before them by itself, from the counts of 32 rows: what grows with the square of the rows is a 1024th
-// of 32nds (from the counts of single rows, [512, 128, 16 heads, 64] took longer for this scan than for the attention).
+// row_offsets[r] = kept entries of the rows before r, for every r up to B * H * S.  A workgroup scans the 1024 counts of its own
+// rows and adds up what lies before them by itself, from the counts of 32 rows: these reads grow with the square of the rows.
+// Forward with the count, [2048, 128, 16 heads, 64]: 675 us (573 without it); from the counts of single rows 1911.
 __global__ __launch_bounds__(1024) void map_row_scan_kernel(const uint32_t* counts, const uint32_t* block_counts, int64_t rows, int S, int64_t* offsets) {
     __shared__ long long front_part[16];
     __shared__ uint32_t wave_total[16];
