@@ -223,12 +223,21 @@ std::optional<std::tuple<OptT, OptT>> contract(const OptT& x, const OptT& q, con
 }
 
 // ---- products with a frozen weight --------------------------------------------------------------------------------
-// Columns to hand to the library first (0: all in one call); the rule and its figures stand at _whole_rounds in
-// models/compute_utils.py.
+// Columns of a [rows, cols] product to hand to the library first (0: all in one call).  Its bf16 kernels work on 256 x 256 tiles,
+// one per compute unit and round.  Where the tiles fill whole rounds and a remainder, one call spreads the remainder over all
+// units along the contraction, which costs up to half of the time again; the whole rounds in one call and the remaining columns in
+// another do not.  Measured with the frozen weight as it lies (forward) and transposed (backward), [rows, contraction] x cols,
+// us:  4096 x 4096 x 11008: 413 -> 271 and 347 -> 307;  2048 x 4096 x 11008: 160 -> 148, 280 -> 176;  8192 x 4096 x 11008: 645 ->
+// 506, 672 -> 579;  8192 x 5120 x 5120: 447 -> 302, 460 -> 339;  8192 x 5120 x 13824: 953 -> 786, 1008 -> 883;  4096 x 2048 x 5504: 90
+// -> 78, 99 -> 99;  4096 x 4096 x 14336: 333 -> 335, 384 -> 378.  Left in one call: a single whole round with more than half of
+// another behind it (2048 x 5120 x 13824: 207 -> 218, 232 -> 244), and row counts whose tiles do not divide a round (6144 x
+// 4096 x 14336: 547 -> 668).
 int64_t whole_rounds(int64_t rows, int64_t cols) {
     constexpr int64_t tile = 256, units = 256;
-    const int64_t down = (rows + tile - 1) / tile, across = (cols + tile - 1) / tile, rest = down * across % units;
-    if (units % down || down * across <= units || rest == 0 || (down * across < 2 * units && rest > units / 2)) return 0;
+    const int64_t down = (rows + tile - 1) / tile, across = (cols + tile - 1) / tile;
+    if (down <= 0 || units % down || down * across <= units) return 0;
+    const int64_t rest = down * across % units;
+    if (rest == 0 || (down * across < 2 * units && rest > units / 2)) return 0;
     return (across - rest / down) * tile;
 }
 // A few rows times a weight as it lies [K, N] (input gradients): this package's kernel where it is the faster one.  Measured
@@ -253,19 +262,27 @@ OptT few_rows(const Tensor& x, const Tensor& w) {                  // x [.., K],
     check("hyc_few_rows", hyc_few_rows(x.data_ptr(), w.data_ptr(), 0, out.data_ptr(), ws.data_ptr(), bytes, rows, n, k, stream_of(x)));
     return out;
 }
-Tensor frozen_product(const Tensor& x, const Tensor& w) {          // x [.., K] contiguous, w [K, N]
-    if (OptT done = few_rows(x, w)) return *done;
-    const int64_t k = w.size(0), n = w.size(1), rows = x.numel() / k;
+// x [.., K] times w [K, N], both bf16 and not to be differentiated, where one plain call of the library is not the way
+OptT frozen_matmul(const Tensor& x, const Tensor& w) {
+    if (at::GradMode::is_enabled() || !is_bf(x) || !is_bf(w) || x.dim() < 1 || w.dim() != 2 || x.numel() == 0 || x.size(-1) != w.size(0))
+        return std::nullopt;
+    if (OptT done = few_rows(x, w)) return done;
+    const int64_t k = w.size(0), n = w.size(1), rows = x.numel() / k, cut = whole_rounds(rows, n);
+    if (cut == 0) return std::nullopt;
     auto shape = x.sizes().vec();
     shape.back() = n;
-    const Tensor x2 = x.view({rows, k});
-    const int64_t cut = whole_rounds(rows, n);
-    if (cut == 0) return at::mm(x2, w).view(shape);
+    const Tensor x2 = x.reshape({rows, k});
     Tensor out = at::empty({rows, n}, x.options());
     Tensor a = out.narrow(1, 0, cut), b = out.narrow(1, cut, n - cut);
     at::mm_out(a, x2, w.narrow(1, 0, cut));
     at::mm_out(b, x2, w.narrow(1, cut, n - cut));
     return out.view(shape);
+}
+Tensor frozen_product(const Tensor& x, const Tensor& w) {          // x [.., K] contiguous, w [K, N]
+    if (OptT done = frozen_matmul(x, w)) return *done;
+    auto shape = x.sizes().vec();
+    shape.back() = w.size(1);
+    return at::mm(x.view({-1, w.size(0)}), w).view(shape);
 }
 bool weight_ok(const Tensor& w, int64_t in) { return is_bf(w) && w.dim() == 2 && w.size(1) == in && w.is_contiguous(); }
 
@@ -520,7 +537,8 @@ PYBIND11_MODULE(_native, m) {
     m.def("lora_add_quant_group", &lora_add_quant_group);
     m.def("lora_add_restore_group", &lora_add_restore_group);
     m.def("contract", &contract);
-    m.def("few_rows", &few_rows);
+    m.def("whole_rounds", &whole_rounds);
+    m.def("frozen_matmul", &frozen_matmul);
     m.def("lora_parts", &lora_parts);
     m.def("lora_forward", &lora_forward);
     m.def("lora_backward", &lora_backward);

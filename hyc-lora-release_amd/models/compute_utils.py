@@ -43,46 +43,14 @@ def heads_matmul(a: torch.Tensor, b: torch.Tensor, out_hidden: bool = False):
     return out
 
 
-_GEMM_TILE, _COMPUTE_UNITS = 256, 256
-
-
-def _whole_rounds(rows: int, cols: int) -> int:
-    """Columns of a [rows, cols] product to hand to the library first, 0 = all in one call.
-
-    Its bf16 kernels work on 256 x 256 tiles, one per compute unit and round.  Where the tiles fill whole rounds and a
-    remainder, one call spreads the remainder over all units along the contraction, which costs up to half of the time again;
-    the whole rounds in one call and the remaining columns in another do not.  Measured with the frozen weight as it lies
-    (forward) and transposed (backward), [rows, contraction] x cols:  4096 x 4096 x 11008: 413 -> 271 and 347 -> 307 us;
-    2048 x 4096 x 11008: 160 -> 148, 280 -> 176;  8192 x 4096 x 11008: 645 -> 506, 672 -> 579;  8192 x 5120 x 5120: 447 -> 302,
-    460 -> 339;  8192 x 5120 x 13824: 953 -> 786, 1008 -> 883;  4096 x 2048 x 5504: 90 -> 78, 99 -> 99;  4096 x 4096 x 14336: 333 ->
-    335, 384 -> 378.  Left in one call: a single whole round with more than half of another behind it (2048 x 5120 x 13824: 207 ->
-    218, 232 -> 244), and row counts whose tiles do not divide a round (6144 x 4096 x 14336: 547 -> 668)."""
-    down, across = -(-rows // _GEMM_TILE), -(-cols // _GEMM_TILE)
-    rest = down * across % _COMPUTE_UNITS
-    if _COMPUTE_UNITS % down or down * across <= _COMPUTE_UNITS or rest == 0:
-        return 0
-    if down * across < 2 * _COMPUTE_UNITS and rest > _COMPUTE_UNITS // 2:
-        return 0
-    return (across - rest // down) * _GEMM_TILE
-
-
 def frozen_matmul(x: torch.Tensor, w: torch.Tensor):
     """x @ w for a frozen weight (or its transposed view) w [K, N]: the kernel for a few rows (csrc/few_rows.hip) where that is the
-    faster one, else the library product, in the calls that suit its tiles."""
-    k, n = w.shape
+    faster one, else the library product, in the calls that suit its tiles (the rules stand in csrc/host/native.cpp)."""
     if x.is_cuda:
-        done = _lib.native().few_rows(x, w)
+        done = _lib.native().frozen_matmul(x, w)
         if done is not None:
             return done
-    rows = x.numel() // max(k, 1)
-    cut = _whole_rounds(rows, n) if x.is_cuda and x.dtype == w.dtype == torch.bfloat16 and not torch.is_grad_enabled() else 0
-    if cut == 0:
-        return x @ w
-    x2 = x.reshape(rows, k)
-    out = torch.empty(rows, n, device=x.device, dtype=x.dtype)
-    torch.mm(x2, w[:, :cut], out=out[:, :cut])
-    torch.mm(x2, w[:, cut:], out=out[:, cut:])
-    return out.view(*x.shape[:-1], n)
+    return x @ w
 
 
 def dense_weight(w: torch.Tensor, quant_state):

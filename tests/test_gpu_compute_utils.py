@@ -122,3 +122,29 @@ def test_frozen_matmul_in_whole_rounds(rows, n, k, transposed):
     assert got.shape == want.shape and got.is_contiguous()
     # one bf16 rounding (half a unit of 2^-8) and the order of up to 128 fp32 additions
     assert ((got.float() - want).abs() <= 2 ** -8 * want.abs() + 1e-4).all()
+
+
+@pytest.mark.parametrize("shape", [(0, 48), (2, 0)])
+def test_products_of_an_empty_batch(CU, dev, shape):
+    w, a_w, b_w, _, _, _ = lora_case(dev, 7)
+    x, gy = (torch.zeros(*shape, n, device=dev, dtype=BF16) for n in (w.shape[1], w.shape[0]))
+    with torch.no_grad():
+        assert CU.frozen_matmul(x, w.t()).shape == gy.shape
+        y, main, xa = CU.lora_forward(w, None, a_w.T, b_w.T, None, x)
+        assert y.shape == main.shape == gy.shape and xa.shape == (*shape, 16)
+        ga, gb, gx = CU.lora_backward(w, None, a_w.T, b_w.T, x, xa, gy)
+    assert gx.shape == x.shape and ga.shape[-2:] == a_w.T.shape and gb.shape[-2:] == b_w.T.shape
+
+
+@pytest.mark.parametrize("M,n_in,n_out", [(96, 256, 4096), (5, 256, 4096), (2048, 13824, 64), (2048, 64, 11008)])
+def test_backward_and_forward_of_a_projection_on_either_side_of_the_rules(CU, dev, M, n_in, n_out):
+    """One call of the native host side each: few rows against a long contraction, and products in whole rounds (forward of the
+    last shape, backward of the one before it)."""
+    w, a_w, b_w, _, x, gy = lora_case(dev, 9, B=1, M=M, n_in=n_in, n_out=n_out)
+    with torch.no_grad():
+        y, main, xa = CU.lora_forward(w, None, a_w.T, b_w.T, None, x)
+        gx = CU.lora_backward(w, None, a_w.T, b_w.T, x, xa, gy)[2]
+    X, Wd, G = x.double(), w.double(), gy.double()
+    assert_close_bf16(main, X @ Wd.T, what="frozen part")
+    assert_close_bf16(y, X @ Wd.T + (X @ a_w.double().T) @ b_w.double().T, what="projection output")
+    assert_close_bf16(gx, G @ Wd + (G @ b_w.double()) @ a_w.double(), what="grad x")

@@ -137,3 +137,11 @@ def test_bf16_vector_is_converted_once_per_tensor_and_again_after_a_change():
     import gc
     gc.collect()
     assert len(_lib._BF16_VECTORS) == n - 1
+
+
+def test_products_of_no_rows_are_not_split():
+    from hyclora_amd import _lib
+    rounds = _lib.native().whole_rounds
+    assert rounds(0, 11008) == rounds(0, 0) == rounds(4096, 0) == 0
+    # 16 x 43 tiles: two whole rounds of 256 and 176 more; a whole round and most of another; rows that do not divide a round
+    assert rounds(4096, 11008) == 32 * 256 and rounds(2048, 13824) == 0 and rounds(6144, 14336) == 0
