@@ -8,6 +8,7 @@
 // state is kept.
 #include <torch/extension.h>
 
+#include <ATen/autocast_mode.h>
 #include <c10/hip/HIPStream.h>
 
 #include <optional>
@@ -33,6 +34,11 @@ bool is_bf(const Tensor& t) { return t.defined() && t.is_cuda() && t.scalar_type
 bool plain(const Tensor& t) { return is_bf(t) && t.is_contiguous() && aligned(t); }
 bool plain_or_none(const OptT& t) { return !t || plain(*t); }
 bool vec(const Tensor& t, int64_t n) { return plain(t) && t.numel() == n; }            // per-channel vector
+// Whether the library's products of these operands may be called from here: not where a gradient is to be recorded, nor where
+// autocast makes them products of another type
+bool products_are_plain() {
+    return !at::GradMode::is_enabled() && !(at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16);
+}
 void* ptr(const OptT& t) { return t ? t->data_ptr() : nullptr; }
 bool bits_ok(int64_t b) { return b == 2 || b == 4 || b == 8; }
 bool packed(const Tensor& q, int64_t numel, int64_t bits) {
@@ -248,7 +254,7 @@ int64_t whole_rounds(int64_t rows, int64_t cols) {
 // gradient of a channel with x 90 times the rest by up to 6 %; and x W^T (4096 x 4096 18 / 22, 11008 x 4096 30 / 50), whose
 // last bits decide codes, so that a step in another order is a step with some other codes.
 OptT few_rows(const Tensor& x, const Tensor& w) {                  // x [.., K], w [K, N]
-    if (at::GradMode::is_enabled() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !is_bf(w) || w.dim() != 2 || w.device() != x.device())
+    if (!products_are_plain() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !is_bf(w) || w.dim() != 2 || w.device() != x.device())
         return std::nullopt;
     const int64_t k = w.size(0), n = w.size(1);
     if (x.size(-1) != k || !aligned(w)) return std::nullopt;
@@ -264,7 +270,7 @@ OptT few_rows(const Tensor& x, const Tensor& w) {                  // x [.., K],
 }
 // x [.., K] times w [K, N], both bf16 and not to be differentiated, where one plain call of the library is not the way
 OptT frozen_matmul(const Tensor& x, const Tensor& w) {
-    if (at::GradMode::is_enabled() || !is_bf(x) || !is_bf(w) || x.dim() < 1 || w.dim() != 2 || x.numel() == 0 || x.size(-1) != w.size(0))
+    if (!products_are_plain() || !is_bf(x) || !is_bf(w) || x.dim() < 1 || w.dim() != 2 || x.numel() == 0 || x.size(-1) != w.size(0))
         return std::nullopt;
     if (OptT done = few_rows(x, w)) return done;
     const int64_t k = w.size(0), n = w.size(1), rows = x.numel() / k, cut = whole_rounds(rows, n);
@@ -288,7 +294,7 @@ bool weight_ok(const Tensor& w, int64_t in) { return is_bf(w) && w.dim() == 2 &&
 
 // -> (x W^T, x A)
 std::optional<std::tuple<Tensor, Tensor>> lora_parts(const Tensor& w, const Tensor& la, const Tensor& x, const OptT& xa) {
-    if (at::GradMode::is_enabled() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !weight_ok(w, x.size(-1))) return std::nullopt;
+    if (!products_are_plain() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !weight_ok(w, x.size(-1))) return std::nullopt;
     if (!is_bf(la) || la.dim() != 2 || la.size(0) != x.size(-1) || (xa && !is_bf(*xa))) return std::nullopt;
     Tensor main = frozen_product(x, w.t());
     if (xa) return std::make_tuple(main, *xa);
@@ -322,7 +328,7 @@ pybind11::object lora_backward(const Tensor& w, const Tensor& la, const Tensor& 
                                const OptT& zero, int64_t bits, const Tensor& xa, const Tensor& grad_y, const OptT& accumulate, bool defer) {
     const pybind11::object none = pybind11::none();
     const Lora L(lb);
-    if (at::GradMode::is_enabled() || !plain(grad_y) || grad_y.numel() == 0 || !is_bf(w) || w.dim() != 2 || !w.is_contiguous() ||
+    if (!products_are_plain() || !plain(grad_y) || grad_y.numel() == 0 || !is_bf(w) || w.dim() != 2 || !w.is_contiguous() ||
         w.size(0) != grad_y.size(-1) || !L.fits(w.size(0)) || !plain(xa) || !is_bf(la) || la.dim() != 2 || la.size(0) != w.size(1) ||
         la.size(1) != L.r || w.size(1) % 32)
         return none;

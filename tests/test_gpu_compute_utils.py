@@ -148,3 +148,22 @@ def test_backward_and_forward_of_a_projection_on_either_side_of_the_rules(CU, de
     assert_close_bf16(main, X @ Wd.T, what="frozen part")
     assert_close_bf16(y, X @ Wd.T + (X @ a_w.double().T) @ b_w.double().T, what="projection output")
     assert_close_bf16(gx, G @ Wd + (G @ b_w.double()) @ a_w.double(), what="grad x")
+
+
+@pytest.mark.parametrize("M,n_in,n_out", [(48, 256, 384), (96, 256, 4096), (2048, 64, 11008), (2048, 11008, 64)])
+def test_products_under_autocast(CU, dev, M, n_in, n_out):
+    """Autocast to float16 makes the products float16, as torch's own; autocast to bfloat16 changes nothing."""
+    w, a_w, b_w, _, x, gy = lora_case(dev, 11, B=1, M=M, n_in=n_in, n_out=n_out)
+    with torch.no_grad():
+        plain = CU.lora_forward(w, None, a_w.T, b_w.T, None, x)
+        plain_back = CU.lora_backward(w, None, a_w.T, b_w.T, x, plain[2], gy)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert all(torch.equal(a, b) for a, b in zip(CU.lora_forward(w, None, a_w.T, b_w.T, None, x), plain))
+            assert all(torch.equal(a, b) for a, b in zip(CU.lora_backward(w, None, a_w.T, b_w.T, x, plain[2], gy), plain_back))
+        with torch.autocast("cuda", dtype=torch.float16):
+            y, main, _ = CU.lora_forward(w, None, a_w.T, b_w.T, None, x)
+            ga, gb, gx = CU.lora_backward(w, None, a_w.T, b_w.T, x, plain[2], gy)
+            assert CU.frozen_matmul(x, w.t()).dtype == CU.lora_parts(w, None, a_w.T, None, x)[0].dtype == torch.float16
+    assert y.dtype == main.dtype == gx.dtype == torch.float16
+    for a, b, what in zip((y, main, ga, gb, gx), (plain[0], plain[1], *plain_back), ("output", "frozen part", "grad A", "grad B", "grad x")):
+        assert_close_bf16(a, b, what=what)
