@@ -68,7 +68,7 @@ def lora_forward(w, w_quant_state, w_lora_a, w_lora_b, b, x, residual=None, x_lo
     take the torch expression.  `residual` (not in the reference's signature) is added to the first
     result in the same pass - the `x + o_final` that follows the projection in the layers.
     `x_lora_a`: x @ A where the producer of x has already formed it."""
-    if b is None:
+    if b is None and x.is_cuda:
         w, w_quant_state = dense_weight(w, w_quant_state), None
         done = _lib.native().lora_forward(w, w_lora_a, w_lora_b, x, residual, x_lora_a)
         if done is not None:
@@ -85,7 +85,7 @@ def lora_parts(w, w_quant_state, w_lora_a, b, x, x_lora_a=None):
     """-> (x @ W^T [+ b], x @ A): what lora_forward computes before the LoRA add.  x @ A is taken
     from `x_lora_a` when the caller has it already (the fused norm kernel forms it)."""
     w = dense_weight(w, w_quant_state)
-    if b is None:
+    if b is None and x.is_cuda:
         done = _lib.native().lora_parts(w, w_lora_a, x, x_lora_a)
         if done is not None:
             return done
@@ -114,13 +114,14 @@ def lora_backward(w, w_quant_state, w_lora_a, w_lora_b, x, x_lora_a, grad_y, x_c
     two terms and the operand that joins them, `(grad_y @ W, grad_y @ B^T, A^T)`, for lora_input_sum, which
     adds up the input gradients of projections that share their input in one pass."""
     wd = dense_weight(w, w_quant_state)          # [out, in]
-    q, scale, zero_point, q_bit = x_codes or (None, None, None, 0)
-    if zero_point is not None and zero_point.dtype != torch.bfloat16:
-        zero_point = _lib.bf16_vector(zero_point)
-    done = _lib.native().lora_backward(wd, w_lora_a, w_lora_b, None if x_codes else x, q, scale, zero_point, q_bit, x_lora_a, grad_y,
-                                       accumulate, defer_input)
-    if done is not None:
-        return done
+    if grad_y.is_cuda:
+        q, scale, zero_point, q_bit = x_codes or (None, None, None, 0)
+        if zero_point is not None and zero_point.dtype != torch.bfloat16:
+            zero_point = _lib.bf16_vector(zero_point)
+        done = _lib.native().lora_backward(wd, w_lora_a, w_lora_b, None if x_codes else x, q, scale, zero_point, q_bit, x_lora_a, grad_y,
+                                           accumulate, defer_input)
+        if done is not None:
+            return done
     dt = wd.dtype
     grad_y = grad_y.to(dt)
     w_lora_a, w_lora_b = w_lora_a.to(dt), w_lora_b.to(dt)

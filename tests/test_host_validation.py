@@ -145,3 +145,23 @@ def test_products_of_no_rows_are_not_split():
     assert rounds(0, 11008) == rounds(0, 0) == rounds(4096, 0) == 0
     # 16 x 43 tiles: two whole rounds of 256 and 176 more; a whole round and most of another; rows that do not divide a round
     assert rounds(4096, 11008) == 32 * 256 and rounds(2048, 13824) == 0 and rounds(6144, 14336) == 0
+
+
+@pytest.mark.parametrize("dtype", [BF, torch.float32])
+def test_projections_of_cpu_tensors_need_no_library(monkeypatch, tmp_path, dtype):
+    """lora_forward, lora_parts and lora_backward are torch expressions on the CPU, whether or not the kernels are built."""
+    from hyclora_amd import _lib
+    from hyclora_amd.models import compute_utils as CU
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libhyclora.so")
+    monkeypatch.setattr(_lib, "NATIVE_PATH", tmp_path / "_native.so")
+    g = torch.Generator().manual_seed(3)
+    rn = lambda *s: torch.randn(*s, generator=g).to(dtype)                            # noqa: E731
+    x, gy, w, a, b = rn(B, M, 64), rn(B, M, 96), rn(96, 64), rn(64, R), rn(R, 96)
+    y, main, xa = CU.lora_forward(w, None, a, b, None, x)
+    assert torch.equal(main, x @ w.t()) and torch.equal(xa, x @ a) and torch.equal(y, main + xa @ b)
+    assert torch.equal(CU.lora_parts(w, None, a, None, x)[0], main)
+    ga, gb, gx = CU.lora_backward(w, None, a, b, x, xa, gy)
+    assert torch.equal(gx, gy @ w + (gy @ b.mT) @ a.mT)
+    assert torch.equal(ga, x.mT @ (gy @ b.mT)) and torch.equal(gb, xa.mT @ gy)
