@@ -950,7 +950,7 @@ static MapWorkspace map_workspace(int64_t B, int64_t S, int64_t H) {
 
 static int map_check(int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D) {
     if (B < 0 || S < 0 || H <= 0 || KV <= 0 || H % KV || (D != 64 && D != 128) || S % 8 || S > kMapMax) return HYC_ERR_SHAPE;
-    if (S * H * D > (int64_t)1 << 30 || B > 65535 || cdiv(S, kMapRows) * B * H > (1 << 30)) return HYC_ERR_SHAPE;
+    if (S * H * D > (int64_t)1 << 30 || B * H > 1 << 22 || cdiv(S, 32) * B * H > 1 << 22) return HYC_ERR_SHAPE;     // fewer than 2^32 threads a launch
     return HYC_OK;
 }
 

@@ -340,8 +340,8 @@ __global__ __launch_bounds__(256, 2) void flash_bwd_kv_kernel(const FlashArgs A)
 
 int flash_check(int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D) {
     if (B < 0 || S < 0 || H <= 0 || KV <= 0 || H % KV || (D != 64 && D != 128)) return HYC_ERR_SHAPE;
-    if (S > (1 << 20) || S * H * D > (int64_t)1 << 30 || B * H > 1 << 20) return HYC_ERR_SHAPE;   // 32-bit offsets inside a batch element
-    if (cdiv(S, kFlashRows) * B * H > (1 << 30)) return HYC_ERR_SHAPE;
+    if (S > (1 << 20) || S * H * D > (int64_t)1 << 30) return HYC_ERR_SHAPE;                                        // 32-bit offsets inside a batch element
+    if (B * H > 1 << 23 || cdiv(S, kFlashRows) * B * H > 1 << 23) return HYC_ERR_SHAPE;                             // fewer than 2^32 threads a launch
     return HYC_OK;
 }
 

@@ -62,7 +62,7 @@ from ..operators.triton_fuse_lora_silu_hadamard_forward_kernels import triton_fu
 from ..operators import lora_kernels
 from ..operators._fuse import fuse_backward
 from ..operators.flash_kernels import flash_backward, flash_forward, flash_supported
-from ..operators.map_kernels import MapAttention, map_backward, map_supported
+from ..operators.map_kernels import MapAttention, map_backward, map_backward_supported, map_supported
 from .compute_utils import (frozen_matmul, head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum, lora_parts,
                             repeat_kv, repeat_kv_backward, rope_backward, rope_forward)
 
@@ -637,7 +637,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 return t
             q, k, v = rebuilt("q", H), rebuilt("k", KV), rebuilt("v", KV)
             del qkv
-        own_map = spec.attention == "map" and "a_raw" not in S and map_supported(q, k, v)
+        own_map = spec.attention == "map" and "a_raw" not in S and map_backward_supported(q, k, v, S["a_idx"])
         if not (own_map or (spec.attention == "sdpa" and ctx.own_flash)):
             k, v = repeat_kv(k, H // k.shape[1]), repeat_kv(v, H // v.shape[1])
 

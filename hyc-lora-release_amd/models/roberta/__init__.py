@@ -25,7 +25,7 @@ from ...operators.softmax_kernels import softmax_backward, softmax_backward_from
 from ...operators import lora_kernels
 from ..compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum,
                             lora_parts)
-from ...operators.map_kernels import MapAttention, map_backward, map_supported
+from ...operators.map_kernels import MapAttention, map_backward, map_backward_supported, map_supported
 from ..fused_decoder_layer import _note_map_entries, check_map_entries, keep_map_entries, lora_linear_parts
 
 MODES = ("baseline", "intra", "intra_inter")
@@ -277,7 +277,7 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
             q, k = deq("q", is_head=True, num_heads=H), deq("k", is_head=True, num_heads=H)
         else:
             q, k = hidden_to_head_shape(rebuilt("q"), H), hidden_to_head_shape(rebuilt("k"), H)
-        if "a_raw" not in S and map_supported(q, k, v):
+        if "a_raw" not in S and map_backward_supported(q, k, v, S["a_idx"]):
             grad_q, grad_k, grad_v = map_backward(grad_o, q, k, v, S["a_idx"], S["a_val"], S["a_seg"])
         else:
             grad_a = heads_matmul(grad_o, v.transpose(-2, -1))

@@ -17,7 +17,7 @@ def flash_supported(q, k, v):
     """Whether flash_forward / flash_backward take these operands."""
     return (q.is_cuda and q.dtype == k.dtype == v.dtype == BF16 and q.dim() == 4 and k.shape == v.shape and q.shape[0] == k.shape[0]
             and q.shape[2:] == k.shape[2:] and q.shape[3] in (64, 128) and q.shape[1] % k.shape[1] == 0 and q.numel() > 0
-            and q.shape[2] <= 1 << 20 and q[0].numel() <= 1 << 30)
+            and q.shape[2] <= 1 << 20 and q[0].numel() <= 1 << 30 and -(-q.shape[2] // 128) * q.shape[0] * q.shape[1] <= 1 << 23)
 
 
 def _hidden(t):

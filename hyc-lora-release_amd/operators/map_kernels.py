@@ -20,9 +20,16 @@ def map_supported(q, k, v, mask=None):
     """Whether map_forward takes these operands; mask: None or additive [B or 1, 1, S or 1, S]."""
     if not flash_supported(q, k, v) or q.shape[2] % 8 or q.shape[2] > MAX_ROW:
         return False
-    B, _, S, _ = q.shape
+    B, H, S, _ = q.shape
+    if -(-S // 32) * B * H > 1 << 22:
+        return False
     return mask is None or (mask.dim() == 4 and mask.is_cuda and mask.shape[0] in (1, B) and mask.shape[1] == 1 and
                             mask.shape[2] in (1, S) and mask.shape[3] == S)
+
+
+def map_backward_supported(q, k, v, idx):
+    """Whether map_backward takes these operands and a list `idx` of kept entries: the kernels count entries in 32 bits."""
+    return map_supported(q, k, v) and idx.numel() < 1 << 31
 
 
 class MapAttention:
@@ -75,8 +82,8 @@ class MapAttention:
 
 def map_backward(grad_o, q, k, v, idx, val, seg_offsets):
     """-> (grad_q, grad_k, grad_v), shaped like q, k, v, from the kept entries of the map."""
-    if not map_supported(q, k, v):
-        raise ValueError(f"map attention does not take {tuple(q.shape)}, {tuple(k.shape)}")
+    if not map_backward_supported(q, k, v, idx):
+        raise ValueError(f"map attention does not take {tuple(q.shape)}, {tuple(k.shape)} and a list of {idx.numel()} entries")
     B, H, S, D = q.shape
     if grad_o.shape != q.shape or grad_o.dtype != BF16:
         raise ValueError(f"grad_o must be bf16 {tuple(q.shape)}, got {tuple(grad_o.shape)} {grad_o.dtype}")

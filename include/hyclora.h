@@ -645,7 +645,7 @@ int hyc_lora_add_sum(const hyc_lora_sum_member *members, int count, void *y, int
  *   lse                   fp32 [B, H, S]: natural log of the row sums of exp(score * scale); output of the forward;
  *   delta                 fp32 [2, B, H, S] scratch of the backward (row sums of grad_o * o, and the log-sum-exps to base 2).
  *                         The backward's o may differ from the forward's: the layers pass the dequantised one.
- *   D 64 or 128, any S (up to 2^20, S*H*D <= 2^30), all pointers 16-byte aligned.  Scores, softmax and all sums are fp32, the
+ *   D 64 or 128, any S (up to 2^20, S*H*D <= 2^30, B*H*ceil(S/128) <= 2^23), all pointers 16-byte aligned.  Scores, softmax and all sums are fp32, the
  *   probabilities and score gradients are rounded to bf16 for the matrix cores.  Fixed summation order: the same bits on
  *   every run.
  */
@@ -667,7 +667,8 @@ int hyc_flash_bwd(const void *grad_o, const void *q, const void *k, const void *
  * attention products, softmax_backward and the repeat_kv copies (models/llama/fused_llama_layer_intra_inter_full_fuse.py:153-180,
  * :403-447; operators/compress_function.py:309-317; operators/softmax_kernels.py:7-38).
  *   q, o, grad_o, grad_q  bf16 [B, S, H, D] contiguous;  k, v, grad_k, grad_v  bf16 [B, S, KV, D] contiguous, H % KV == 0
- *                (grad_k, grad_v: each query head's rounded to bf16, a group's added in fp32 and rounded); D 64 or 128; S % 8 == 0, S <= 4096;
+ *                (grad_k, grad_v: each query head's rounded to bf16, a group's added in fp32 and rounded); D 64 or 128; S % 8 == 0,
+ *                S <= 4096, S*H*D <= 2^30, B*H*ceil(S/32) <= 2^22;
  *   mask         bf16 or NULL, added to every head: entry (b, i, j) at b * mask_stride_b + i * mask_stride_row + j (strides
  *                multiples of 8, 0 broadcasts).  Keys at or below -1e30 cost nothing where 32 rows x 64 keys are all so, all
  *                keys and values of the head are finite and no row of the 128 has a NaN sum or only such keys; otherwise they

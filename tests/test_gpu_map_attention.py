@@ -72,16 +72,32 @@ def test_forward_and_kept_entries(b, h, kv, s, d, kind):
             assert torch.equal(idx2[:m], idx[:m]) and torch.equal(val2[:m], val[:m])
 
 
-@pytest.mark.parametrize("b,h,s", [(33, 16, 136), (5, 9, 1000), (260, 1, 8)])
+@pytest.mark.parametrize("b,h,s", [(33, 16, 136), (5, 9, 1000), (260, 1, 8), (70000, 2, 8)])
 def test_entries_of_many_rows(b, h, s):
     """More rows than a workgroup of the scan takes, starting inside a head and inside its blocks of 32 rows."""
     from hyclora_amd.operators.compress_function import compress_attention_map
     from hyclora_amd.operators.map_kernels import MapAttention
     q, k, v, _ = operands(b, h, h, s, 64, seed=s)
+    mask = masks("keys", b, s)
     threshold = torch.full((), 0.1, device="cuda")
-    idx, val, seg = compress_attention_map(MapAttention(q, k, v, want_map=True).map, threshold)
-    idx2, val2, seg2 = MapAttention(q, k, v, threshold=threshold).entries(idx.numel())
+    idx, val, seg = compress_attention_map(MapAttention(q, k, v, mask, want_map=True).map, threshold)
+    idx2, val2, seg2 = MapAttention(q, k, v, mask, threshold=threshold).entries(idx.numel())
     assert torch.equal(idx2, idx) and torch.equal(val2, val) and torch.equal(seg2, seg)
+
+
+def test_very_many_rows_and_very_long_lists_go_through_memory():
+    from hyclora_amd.operators.flash_kernels import flash_supported
+    from hyclora_amd.operators.map_kernels import map_backward_supported, map_supported
+    like = lambda b, h, s: torch.empty(1, device="cuda", dtype=BF16).expand(b, h, s, 64)          # noqa: E731
+    q = like(2, 4, 512)
+    idx = torch.empty(1, device="cuda", dtype=torch.int64)
+    assert map_backward_supported(q, q, q, idx.expand((1 << 31) - 1)) and not map_backward_supported(q, q, q, idx.expand(1 << 31))
+    for b, s, fits in ((70000, 8, True), ((1 << 22) // 4, 8, True), ((1 << 22) // 4 + 1, 8, False), ((1 << 22) // 64, 512, True), ((1 << 22) // 64 + 1, 512, False)):
+        q = like(b, 4, s)
+        assert map_supported(q, q, q) is fits
+    for b, s, fits in (((1 << 23) // 4, 1, True), ((1 << 23) // 4 + 1, 1, False), ((1 << 23) // 16, 500, True), ((1 << 23) // 16 + 1, 500, False)):
+        q = like(b, 4, s)
+        assert flash_supported(q, q, q) is fits
 
 
 def same_bits(a, b):
