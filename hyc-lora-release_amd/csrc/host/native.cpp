@@ -32,7 +32,6 @@ void* stream_of(const Tensor& t) { return (void*)c10::hip::getCurrentHIPStream(t
 bool aligned(const Tensor& t, uintptr_t a = 16) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % a == 0; }
 bool is_bf(const Tensor& t) { return t.defined() && t.is_cuda() && t.scalar_type() == at::kBFloat16; }
 bool plain(const Tensor& t) { return is_bf(t) && t.is_contiguous() && aligned(t); }
-bool plain_or_none(const OptT& t) { return !t || plain(*t); }
 bool vec(const Tensor& t, int64_t n) { return plain(t) && t.numel() == n; }            // per-channel vector
 // Whether the library's products of these operands may be called from here: not where a gradient is to be recorded, nor where
 // autocast makes them products of another type
@@ -333,7 +332,9 @@ pybind11::object lora_backward(const Tensor& w, const Tensor& la, const Tensor& 
         la.size(1) != L.r || w.size(1) % 32)
         return none;
     const Tensor at_ = la.t();                                     // A^T [R, in]
-    if (!Lora(at_).fits(w.size(1)) || !plain_or_none(accumulate)) return none;
+    auto shape_x = grad_y.sizes().vec();
+    shape_x.back() = w.size(1);
+    if (!Lora(at_).fits(w.size(1)) || (accumulate && !(plain(*accumulate) && accumulate->sizes() == at::IntArrayRef(shape_x)))) return none;
     if (x ? !(plain(*x) && x->size(-1) == w.size(1)) : !(q && scale && vec(*scale, w.size(1)) && (!zero || vec(*zero, w.size(1))))) return none;
     auto both = contract(grad_y, std::nullopt, std::nullopt, std::nullopt, 0, xa, lb, w.size(0), true);
     if (!both) return none;
@@ -506,7 +507,7 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> gated_backward(const Tensor& x
                                                                  const Tensor& grad_o, int64_t bits, bool once) {
     const Gated G(grad_o, xa1, b1, s1, xa2, b2, s2);
     if (!G.ok || !bits_ok(bits) || !packed(q1, G.rows * G.n, bits) || !packed(q2, G.rows * G.n, bits) || !aligned(q1) || !aligned(q2) ||
-        q1.dim() != 3 || q2.dim() != 3 || q1.size(1) != grad_o.size(1) || q2.size(1) != grad_o.size(1))
+        q1.dim() != 3 || q1.size(0) != grad_o.size(0) || q1.size(1) != grad_o.size(1) || q2.sizes() != q1.sizes())
         return std::nullopt;
     Tensor o = at::empty_like(grad_o), gg = at::empty_like(grad_o), gu = at::empty_like(grad_o);
     auto* fn = once ? hyc_lora_silu_once_mul_bwd : hyc_lora_silu_mul_bwd;

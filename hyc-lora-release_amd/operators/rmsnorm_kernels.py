@@ -241,9 +241,10 @@ def rmsnorm_forward_compress(x, weight, eps, q_bit, scale_y=None, scale_x=None, 
     k = 0 if outlier_idx is None or scale_x is None else outlier_idx.numel()
     if k and table is None and outlier_idx.is_cuda:
         table = outlier_table(outlier_idx, x.shape[-1], cached=True)
-    done = _lib.native().norm_compress(x, weight, eps, q_bit, scale_y, scale_x, table, k, lora_a or [])
-    if done is not None:
-        return done if lora_a else done[:5]
+    if lora_a is None or lora_a:
+        done = _lib.native().norm_compress(x, weight, eps, q_bit, scale_y, scale_x, table, k, lora_a or [])
+        if done is not None:
+            return done if lora_a else done[:5]
     _lib.require_gpu(x, weight)
     if x.dtype != torch.bfloat16 or x.dim() != 3:
         raise NotImplementedError("rmsnorm_forward_compress takes bfloat16 [batch, seq, hidden] activations")

@@ -150,6 +150,14 @@ def test_backward_and_forward_of_a_projection_on_either_side_of_the_rules(CU, de
     assert_close_bf16(gx, G @ Wd + (G @ b_w.double()) @ a_w.double(), what="grad x")
 
 
+@pytest.mark.parametrize("shape", [(2, 48, 224), (1, 48, 256), (2, 47, 256)])
+def test_a_running_sum_of_another_shape_is_refused(CU, dev, shape):
+    w, a_w, b_w, _, x, gy = lora_case(dev, 13)
+    xa = x @ a_w.T
+    with torch.no_grad(), pytest.raises(ValueError, match="residual"):
+        CU.lora_backward(w, None, a_w.T, b_w.T, x, xa, gy, accumulate=torch.zeros(*shape, device=dev, dtype=BF16))
+
+
 @pytest.mark.parametrize("M,n_in,n_out", [(48, 256, 384), (96, 256, 4096), (2048, 64, 11008), (2048, 11008, 64)])
 def test_products_under_autocast(CU, dev, M, n_in, n_out):
     """Autocast to float16 makes the products float16, as torch's own; autocast to bfloat16 changes nothing."""

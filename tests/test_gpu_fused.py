@@ -26,6 +26,18 @@ def fz():
     return Fz
 
 
+def test_packed_codes_of_another_shape_are_refused(fz, dev):
+    z = lambda *s, dtype=BF16: torch.zeros(*s, device=dev, dtype=dtype)              # noqa: E731
+    xa, b, s = z(2, 8, 16), z(16, 64), z(1, 64)
+    codes = lambda *s: z(*s, dtype=torch.uint8)                                       # noqa: E731
+    fz.bwd(xa, b, codes(2, 8, 32), s, xa, b, codes(2, 8, 32), s, z(2, 8, 64), 4)
+    for shape in ((4, 8, 16), (1, 8, 64), (2, 4, 64)):
+        with pytest.raises(ValueError, match="packed codes"):
+            fz.bwd(xa, b, codes(*shape), s, xa, b, codes(*shape), s, z(2, 8, 64), 4)
+        with pytest.raises(ValueError, match="packed codes"):
+            fz.bwd(xa, b, codes(2, 8, 32), s, xa, b, codes(*shape), s, z(2, 8, 64), 4)
+
+
 def mlp_inputs(seed, B, M, H, I, R):
     """benchmark configuration 2 in the given size: x ~ N(0,1), frozen W ~ N(0,0.02), LoRA A
     kaiming-uniform(a=sqrt(5)) as PEFT initialises it, LoRA B ~ N(0,1e-3) (scaled up here so

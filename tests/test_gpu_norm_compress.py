@@ -214,6 +214,8 @@ def test_lora_a_contraction_limits(ops, dev):
     assert not ops.norm.lora_a_supported(z(2, 4, 1024), w, [z(512, 16)])           # adapter of another width
     with pytest.raises(NotImplementedError):
         ops.norm.rmsnorm_forward_compress(z(1, 3, 1024), w, 1e-5, 4, lora_a=ok)
+    with pytest.raises(NotImplementedError):
+        ops.norm.rmsnorm_forward_compress(z(2, 4, 1024), w, 1e-5, 4, lora_a=[])
 
 
 @pytest.mark.parametrize("shape", [(1, 8, 512), (2, 34, 4096)])
