@@ -364,11 +364,8 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 o, lse = flash_forward(q, k, v)
                 ctx.own_flash = True
                 if KEEP_ATTENTION_LSE:
-                    # beside the log-sum-exps, the rest of what torch's flash backward takes: a random state that is not
-                    # used without dropout, and no cumulative lengths
                     saved["sdpa_lse"] = lse
-                    saved["sdpa_rng"] = saved["sdpa_unused"] = torch.empty((), device=q.device, dtype=torch.int64)
-                    ctx.flash = (None, None, q.shape[2], q.shape[2])
+                del lse
             else:
                 k, v = repeat_kv(k, q.shape[1] // k.shape[1]), repeat_kv(v, q.shape[1] // v.shape[1])
             if not ctx.own_flash and KEEP_ATTENTION_LSE and attention_mask is None and q.is_cuda:
@@ -664,7 +661,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
         elif ctx.own_flash:
             # the attention output handed to the backward kernel is the dequantised one, as in the
             # reference (…intra_inter.py:450-461); grouped keys and values give grouped gradients
-            out, lse = (hidden_to_head_shape(deq("o"), H), S["sdpa_lse"]) if ctx.flash is not None else flash_forward(q, k, v)
+            out, lse = (hidden_to_head_shape(deq("o"), H), S["sdpa_lse"]) if "sdpa_lse" in S else flash_forward(q, k, v)
             grad_q, grad_k, grad_v = flash_backward(grad_o, q, k, v, out, lse)
             del q, k, v, out, grad_o
         elif ctx.flash is not None:

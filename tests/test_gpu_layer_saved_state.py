@@ -23,9 +23,9 @@ def oracle_backward_from_saved_state(t, out, layer_type, q_bit, attention, exact
     """Gradients in NAMES order.  exact=True: the same backward evaluated without intermediate bf16 rounding -
     float64 operands, the oracle's rounding dtype bound to float64; a dequantised activation is still rounded
     to bf16 once, which is part of the format.  library_attention=True (map-free layers): the attention backward
-    inside the oracle's walk is the library kernel the layer itself calls (torch's flash-attention backward, on
-    the oracle's own q, k, v, dequantised output and the saved log-sum-exps) instead of the dense fp32
-    restatement - everything that is not this repository's code is then the same on both sides."""
+    inside the oracle's walk is torch's flash-attention backward, on the oracle's own q, k, v, dequantised output
+    and the saved log-sum-exps, instead of the dense fp32 restatement: a flash backward that is not this
+    repository's (and, with heads other than 64 and 128 wide, the one that the layer itself calls)."""
     from oracle import hyc_oracle, layer_oracle
     S = layer_saved_state(out, t.heads)
     node = out.grad_fn
@@ -33,10 +33,15 @@ def oracle_backward_from_saved_state(t, out, layer_type, q_bit, attention, exact
     restated = layer_oracle._flash_backward
 
     def library_flash_backward(g_o, q, k, v, o, lse, scale):
-        cum_q, cum_k, max_q, max_k = node.flash
+        if node.own_flash:          # this package's kernels: the rest of the library's state is what a call without dropout has
+            cum_q, cum_k, max_q, max_k = None, None, q.shape[2], q.shape[2]
+            state = [torch.empty((), device=q.device, dtype=torch.int64)] * 2
+        else:
+            cum_q, cum_k, max_q, max_k = node.flash
+            state = [raw["sdpa_rng"], raw["sdpa_unused"]]
         assert abs(scale - q.shape[-1] ** -0.5) < 1e-12          # the library's default scale
         return torch.ops.aten._scaled_dot_product_flash_attention_backward(
-            g_o, q, k, v, o, lse, cum_q, cum_k, max_q, max_k, 0.0, True, raw["sdpa_rng"], raw["sdpa_unused"])
+            g_o, q, k, v, o, lse, cum_q, cum_k, max_q, max_k, 0.0, True, *state)
     up = (lambda v: v.double() if torch.is_tensor(v) and v.is_floating_point() else v) if exact else (lambda v: v)
     S = {k: up(v) for k, v in S.items()}
     weights = {n: tuple(up(m.weight.detach()) for m in t.P[n]) for n in t.P}
@@ -81,10 +86,10 @@ def compare(grads, expect, what, exact=None, rel_tol=1e-2, cos_tol=0.9999, names
     as close to the exact evaluation as the tolerance or twice the bf16 evaluation's own distance from it,
     whichever is larger - i.e. its error is rounding noise of the size the reference's own arithmetic has.
     Such cases are printed and counted.  `expect_library` (map-free layers): the bf16 evaluation again, with the
-    attention backward inside the oracle's walk done by the library kernel the layer calls (torch's
-    flash-attention backward, which rounds its probabilities to bf16 where the restatement keeps fp32 matrices):
-    a gradient that misses the restatement but meets THAT evaluation at the tolerance differs only by what the
-    library's kernel does, and counts as met."""
+    attention backward inside the oracle's walk done by torch's flash-attention backward, which rounds its
+    probabilities to bf16 where the restatement keeps fp32 matrices, as the layer's own kernels do: a gradient that
+    misses the restatement but meets THAT evaluation at the tolerance differs only by what a flash kernel does,
+    and counts as met."""
     report, bad, noise = [], [], []
     for i, (name, got, want) in enumerate(zip(names or NAMES, grads, expect)):
         if got is None:
@@ -150,6 +155,7 @@ def test_map_free_backward_from_the_layers_saved_state(dev, layer_type, q_bit, k
     layer.set_hyclora_config(config(layer_type, q_bit, thr=1))
     for step in ("calibrating", "frozen statistics"):
         out = run_fused(layer, t, use_mask=False)
+        assert out.grad_fn.own_flash and not {"sdpa_rng", "sdpa_unused"} & set(out.grad_fn.names)      # nothing kept but what backward reads
         expect = oracle_backward_from_saved_state(t, out, layer_type, q_bit, "flash")
         library = oracle_backward_from_saved_state(t, out, layer_type, q_bit, "flash", library_attention=True)
         exact = oracle_backward_from_saved_state(t, out, layer_type, q_bit, "flash", exact=True)
