@@ -1,7 +1,7 @@
 // Products of a few rows with a frozen weight, on the gfx950 matrix cores:
 //
-//   out[t, n] = sum_k x[t, k] w[n, k]      (w as it lies, [N, K]: forward)
-//   out[t, n] = sum_k x[t, k] w[k, n]      (w [K, N]: input gradients)
+//   out[t, n] = sum_k x[t, k] w[k, n]      (w [K, N]: input gradients; what the layers use, see few_rows in host/native.cpp)
+//   out[t, n] = sum_k x[t, k] w[n, k]      (w [N, K]: for callers of the C entry; the layers leave x W^T to the library)
 //
 // Bound by the one read of w: a short batch multiplies every weight once, 2 T flops a byte.  A library product of such a
 // shape gives its 256 x 256 tiles to a part of the chip.  Here the weight is cut into steps of 128 outputs x 64 of the

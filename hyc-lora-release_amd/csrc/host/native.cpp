@@ -248,10 +248,14 @@ int64_t whole_rounds(int64_t rows, int64_t cols) {
 // A few rows times a weight as it lies [K, N] (input gradients): this package's kernel where it is the faster one.  Measured
 // against the library at 96 rows, contraction x outputs, us: 4096 x 1024 15 / 20, 4096 x 4096 19 / 35, 4096 x 11008 32 / 35,
 // 5120 x 13824 47 / 48, 11008 x 4096 29 / 85, 13824 x 5120 46 / 114.  Left to the library: contractions under 4096 (2048 x 2048
-// 14 / 13, 2048 x 5504 20 / 18); 128 rows (4096 x 4096 21 / 39) and more, because the layers are compared there with an
-// oracle that makes the same library calls, and another order of the sums, no further from 64 bits, moves the norm-weight
-// gradient of a channel with x 90 times the rest by up to 6 %; and x W^T (4096 x 4096 18 / 22, 11008 x 4096 30 / 50), whose
-// last bits decide codes, so that a step in another order is a step with some other codes.
+// 14 / 13, 2048 x 5504 20 / 18).  Both are equally far from 64 bits: at 8 to 128 rows and these shapes 1 to 3 of 10000 results
+// of the kernel are not the correctly rounded value, 1 to 5 of the library's.  Two more limits are neither for speed nor for
+// accuracy, but because an order of the sums other than the library's moves results that are compared with it:
+//  - 128 rows and more (4096 x 4096 21 / 39).  Gradients of layers on 128 tokens are held to an oracle that makes the library's
+//    calls, and the norm-weight gradient of a channel with x 90 times the rest, a sum in which the terms nearly cancel, moves by
+//    up to 6 %, as it does at fewer rows;
+//  - x W^T (4096 x 4096 18 / 22, 11008 x 4096 30 / 50): its last bits decide codes, so a step in another order has some other
+//    codes.
 OptT few_rows(const Tensor& x, const Tensor& w) {                  // x [.., K], w [K, N]
     if (!products_are_plain() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !is_bf(w) || w.dim() != 2 || w.device() != x.device())
         return std::nullopt;
