@@ -8,8 +8,8 @@ pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
 
 
-def reference(q, k, v, g, causal):
-    """Output, log-sum-exps and gradients in float64, from the bf16 operands."""
+def reference(q, k, v, g, causal, given_o=None):
+    """Output, log-sum-exps and gradients in float64, from the bf16 operands; the gradients take `given_o` for the output."""
     n_rep = q.shape[1] // k.shape[1]
     q, k, v, g = (t.double() for t in (q, k, v, g))
     kr, vr = k.repeat_interleave(n_rep, 1), v.repeat_interleave(n_rep, 1)
@@ -21,7 +21,7 @@ def reference(q, k, v, g, causal):
     p = (s - lse[..., None]).exp()
     o = p @ vr
     dp = g @ vr.transpose(-1, -2).contiguous()
-    ds = p * (dp - (g * o).sum(-1, keepdim=True)) / math.sqrt(q.shape[-1])
+    ds = p * (dp - (g * (o if given_o is None else given_o.double())).sum(-1, keepdim=True)) / math.sqrt(q.shape[-1])
     group = lambda t: t.unflatten(1, (k.shape[1], n_rep)).sum(2)                      # noqa: E731
     return o, lse, ds @ kr, group(ds.transpose(-1, -2).contiguous() @ q), group(p.transpose(-1, -2).contiguous() @ g)
 
@@ -48,3 +48,60 @@ def test_flash_attention(b, h, kv, d, s, causal):
         assert err < 4 * 2 ** -8.5, (name, err.item())
     again = flash_backward(g, q, k, v, o, lse, causal)
     assert all(torch.equal(x, y) for x, y in zip(grads, again))
+
+
+def check(got, want):
+    for x, ref, name in zip(got, want, ("o", "grad_q", "grad_k", "grad_v")):
+        assert x.shape == ref.shape
+        err = (x.double() - ref).norm() / ref.norm()
+        assert err < 4 * 2 ** -8.5, (name, err.item())              # as above
+
+
+@pytest.mark.parametrize("s,h,kv", [(8192, 2, 1), (5001, 1, 1)])
+def test_long_sequences(s, h, kv):
+    from hyclora_amd.operators.flash_kernels import flash_backward, flash_forward
+    gen = torch.Generator(device="cuda").manual_seed(s)
+    hidden = lambda heads: torch.randn(1, s, heads, 128, generator=gen, device="cuda").to(BF16).transpose(1, 2)      # noqa: E731
+    q, k, v, g = hidden(h), hidden(kv), hidden(kv), hidden(h)
+    o, lse = flash_forward(q, k, v)
+    want = reference(q, k, v, g, True)
+    assert (lse.double() - want[1]).abs().max() < 1e-4
+    check((o,) + flash_backward(g, q, k, v, o, lse), (want[0],) + want[2:])
+
+
+@pytest.mark.parametrize("layout", ["heads", "odd", "wide"])
+def test_operands_in_any_layout(layout):
+    """[B, H, S, D] in memory, an address that is no multiple of 16 bytes, a slice of a wider tensor: copied first, same results."""
+    from hyclora_amd.operators.flash_kernels import flash_backward, flash_forward
+    b, h, kv, s, d = 2, 4, 2, 200, 128
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    hidden = lambda heads: torch.randn(b, s, heads, d, generator=gen, device="cuda").to(BF16).transpose(1, 2)      # noqa: E731
+    plain = hidden(h), hidden(kv), hidden(kv), hidden(h)
+
+    def lay(t):
+        if layout == "heads":
+            return t.contiguous()
+        if layout == "odd":
+            hidden_t = t.transpose(1, 2)
+            return torch.empty(t.numel() + 1, device="cuda", dtype=BF16)[1:].view(hidden_t.shape).copy_(hidden_t).transpose(1, 2)
+        return torch.empty(*t.shape[:-1], 2 * d, device="cuda", dtype=BF16)[..., d:].copy_(t)
+    q, k, v, g = (lay(t) for t in plain)
+    o, lse = flash_forward(q, k, v)
+    o2, lse2 = flash_forward(*plain[:3])
+    assert torch.equal(o, o2) and torch.equal(lse, lse2)
+    for x, y in zip(flash_backward(g, q, k, v, lay(o), lse), flash_backward(plain[3], *plain[:3], o2, lse2)):
+        assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+def test_backward_of_another_output(causal):
+    """The layers hand in the dequantised output, a few percent off the forward's."""
+    from hyclora_amd.operators.flash_kernels import flash_backward, flash_forward
+    b, h, kv, s, d = 2, 4, 2, 333, 128
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    hidden = lambda heads: torch.randn(b, s, heads, d, generator=gen, device="cuda").to(BF16).transpose(1, 2)      # noqa: E731
+    q, k, v, g = hidden(h), hidden(kv), hidden(kv), hidden(h)
+    o, lse = flash_forward(q, k, v, causal)
+    given = (o.float() + 0.05 * hidden(h).float()).to(BF16)
+    want = reference(q, k, v, g, causal, given)
+    check((o,) + flash_backward(g, q, k, v, given, lse, causal), (want[0],) + want[2:])

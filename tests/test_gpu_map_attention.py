@@ -27,7 +27,16 @@ def masks(kind, b, s):
         return torch.zeros(b, 1, s, s, device="cuda", dtype=BF16).masked_fill_((causal | left[:, None, :])[:, None], low)
     if kind == "keys":            # one mask row for all queries
         return torch.zeros(b, 1, 1, s, device="cuda", dtype=BF16).masked_fill_(left.flip(1)[:, None, None], low)
-    return torch.randn(1, 1, s, s, generator=torch.Generator(device="cuda").manual_seed(5), device="cuda").to(BF16)      # a bias
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    if kind == "low":             # values on both sides of -1e30, where keys begin to cost nothing; a third of the rows have only such
+        pick = lambda values, *shape: torch.tensor(values, device="cuda")[torch.randint(len(values), shape, generator=gen, device="cuda")]     # noqa: E731
+        m = pick([-0.9e30, -1.1e30, -3e30, -5e31, -1e38, low], b, 1, s, s)
+        m[:, :, :, s // 2:] = low
+        rows = torch.arange(s, device="cuda") // 40 % 3
+        m[:, :, rows == 1, : s // 4] = pick([0.0, -2.0, -0.4e30], b, 1, int((rows == 1).sum()), s // 4)
+        m[:, :, rows == 2] = pick([-2e30, -3e30, low], b, 1, int((rows == 2).sum()), s)
+        return m.to(BF16)
+    return torch.randn(1, 1, s, s, generator=gen, device="cuda").to(BF16)      # a bias
 
 
 def dense(q, k, mask):
@@ -45,7 +54,7 @@ def rel(got, want):
     return ((got.double() - want.double()).norm() / want.double().norm().clamp_min(1e-30)).item()
 
 
-@pytest.mark.parametrize("kind", ["none", "causal", "padded", "keys", "bias"])
+@pytest.mark.parametrize("kind", ["none", "causal", "padded", "keys", "bias", "low"])
 @pytest.mark.parametrize("b,h,kv,s,d", [(1, 2, 2, 8, 64), (2, 4, 4, 32, 128), (2, 3, 1, 72, 64), (3, 8, 2, 136, 128), (1, 4, 2, 200, 128),
                                         (2, 2, 2, 256, 64), (1, 2, 1, 520, 128), (1, 1, 1, 4096, 64)])
 def test_forward_and_kept_entries(b, h, kv, s, d, kind):
