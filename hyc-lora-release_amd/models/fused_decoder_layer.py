@@ -583,7 +583,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 G["down"] = (lora_kernels.lora_products(hadamard, u=grad_mid)[0].t(), grad_b_down)
             else:
                 G["down"] = (hadamard.to(wd.dtype).mT @ grad_mid, grad_b_down)
-            del hadamard, grad_down
+            del hadamard, grad_down, wd                   # a dequantised weight is let go before the next ones are made
         else:
             fn = None
             if spec.mode == "intra_inter":

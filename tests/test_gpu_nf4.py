@@ -89,6 +89,40 @@ def test_decoder_layer_on_nf4_weights(nf4, dev):
         assert (a is None and b is None) or torch.equal(a, b)
 
 
+@pytest.mark.parametrize("mode", ["intra", "intra_inter", "intra_inter_full_fuse"])
+def test_backward_holds_one_dequantised_weight_at_a_time(nf4, dev, monkeypatch, mode):
+    """A dequantised weight is as large as an activation of its width and thousands of tokens: the one of the down projection is
+    gone when the input gradients of gate and up are added up, and so are theirs."""
+    import weakref
+
+    import hyclora_amd  # noqa: F401
+    from hyclora_amd.models import compute_utils, fused_decoder_layer, llama
+    from test_gpu_layers import Lin, config, make_layer_inputs, run_fused
+    t = make_layer_inputs(dev, seed=72)
+    for n, (base, la, lb) in t.P.items():
+        packed, absmax, _ = O.nf4_quantize(base.weight.float().cpu(), blocksize=64)
+        wq = packed.reshape(-1, 1).to(dev)
+        wq.quant_state = nf4.make_quant_state(absmax.to(dev), tuple(base.weight.shape))
+        t.P[n] = (Lin(wq), la, lb)
+    layer = llama.make_fused_llama_layer(config(mode, 4))
+    out = run_fused(layer, t)
+    made, alive = [], []
+    dense, add_up = compute_utils.dense_weight, fused_decoder_layer.lora_input_sum
+
+    def dense_weight(w, qs):
+        w = dense(w, qs)
+        made.append(weakref.ref(w))
+        return w
+
+    def lora_input_sum(parts):
+        alive.append(sum(r() is not None for r in made))
+        return add_up(parts)
+    monkeypatch.setattr(compute_utils, "dense_weight", dense_weight)
+    monkeypatch.setattr(fused_decoder_layer, "lora_input_sum", lora_input_sum)
+    out.backward(t.grad)
+    assert len(made) == 7 and alive == [0, 0]
+
+
 def test_default_code_book_is_uploaded_once(nf4, dev):
     """Without a code book in the quant state the published table is used from a device tensor made once
     per device: a host tensor copied at every call would stall the stream (a pageable copy waits for it)."""
