@@ -8,8 +8,9 @@
 // formed transposed (a lane holds one row of the softmax), so the row sums need one exchange between the two halves of a wave
 // and the probabilities are the next product's operand as they stand.  The backward runs as two kernels, one per owned axis,
 // and forms scores twice instead of adding query gradients with atomics: the same bits on every run.
-// [1, 8192, 32 heads, 128], causal: forward 560 us (0.98 PFLOP/s), backward 1640 us (1.18 PFLOP/s of its seven products, 0.84
-// counting five); the library kernels behind torch's scaled_dot_product_attention took 1280 and 5330.  The first version of
+// [1, 8192, 32 heads, 128], causal, inside a layer step: forward 550 to 570 us (0.98 PFLOP/s), backward 700 + 920 to 740 + 980 us
+// (1.15 PFLOP/s of its seven products, 0.82 counting five); the library kernels behind torch's scaled_dot_product_attention took
+// 1280 and 5330.  The first version of
 // the tile (rows of whole 256 bytes, addresses formed per read, every product waiting for the operand read right before it)
 // took 615 and 2400 us.
 #include "hyc_attn_tile.hpp"
