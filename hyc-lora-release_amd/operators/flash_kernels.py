@@ -15,7 +15,7 @@ BF16 = torch.bfloat16
 
 def flash_supported(q, k, v):
     """Whether flash_forward / flash_backward take these operands."""
-    return (q.is_cuda and q.dtype == k.dtype == v.dtype == BF16 and q.dim() == 4 and k.shape == v.shape and q.shape[0] == k.shape[0]
+    return (q.is_cuda and q.device == k.device == v.device and q.dtype == k.dtype == v.dtype == BF16 and q.dim() == 4 and k.shape == v.shape and q.shape[0] == k.shape[0]
             and q.shape[2:] == k.shape[2:] and q.shape[3] in (64, 128) and q.shape[1] % k.shape[1] == 0 and q.numel() > 0
             and q.shape[2] <= 1 << 20 and q[0].numel() <= 1 << 30 and -(-q.shape[2] // 128) * q.shape[0] * q.shape[1] <= 1 << 23)
 
@@ -28,8 +28,8 @@ def _hidden(t):
 
 def _check(q, k, v):
     if not flash_supported(q, k, v):
-        raise ValueError(f"attention takes bf16 [B, H, S, D] queries and [B, KV, S, D] keys / values with D 64 or 128, got "
-                         f"{tuple(q.shape)} {q.dtype}, {tuple(k.shape)} {k.dtype}, {tuple(v.shape)} {v.dtype}")
+        raise ValueError(f"attention takes bf16 [B, H, S, D] queries and [B, KV, S, D] keys / values with D 64 or 128 on one GPU, got "
+                         f"{tuple(q.shape)} {q.dtype} {q.device}, {tuple(k.shape)} {k.dtype} {k.device}, {tuple(v.shape)} {v.dtype} {v.device}")
 
 
 def flash_forward(q, k, v, causal=True):

@@ -23,7 +23,7 @@ def map_supported(q, k, v, mask=None):
     B, H, S, _ = q.shape
     if -(-S // 32) * B * H > 1 << 22:
         return False
-    return mask is None or (mask.dim() == 4 and mask.is_cuda and mask.shape[0] in (1, B) and mask.shape[1] == 1 and
+    return mask is None or (mask.dim() == 4 and mask.device == q.device and mask.shape[0] in (1, B) and mask.shape[1] == 1 and
                             mask.shape[2] in (1, S) and mask.shape[3] == S)
 
 
@@ -67,8 +67,11 @@ class MapAttention:
         dev = self.q.device
         idx = torch.empty(capacity, device=dev, dtype=torch.int64)
         val = torch.empty(capacity, device=dev, dtype=BF16)
+        nseg = -(-B * H * S * S // 4096)
         if seg_offsets is None:
-            seg_offsets = torch.empty(-(-B * H * S * S // 4096) + 1, device=dev, dtype=torch.int64)
+            seg_offsets = torch.empty(nseg + 1, device=dev, dtype=torch.int64)
+        elif seg_offsets.device != dev or seg_offsets.dtype != torch.int64 or seg_offsets.numel() != nseg + 1 or not seg_offsets.is_contiguous():
+            raise ValueError(f"seg_offsets must be int64 [{nseg + 1}] on {dev}, got {seg_offsets.dtype} {tuple(seg_offsets.shape)} on {seg_offsets.device}")
         _lib.call("hyc_map_emit", self.q.data_ptr(), self.k.data_ptr(), _lib.ptr(self.mask), *self.mask_strides, self.threshold.data_ptr(),
                   self.workspace.data_ptr(), self.workspace.numel(), capacity, idx.data_ptr() if capacity else None,
                   val.data_ptr() if capacity else None, seg_offsets.data_ptr(), B, S, H, self.KV, D, self.scale, _lib.stream_of(idx))

@@ -93,6 +93,33 @@ def test_operands_in_any_layout(layout):
         assert torch.equal(x, y)
 
 
+def test_operands_that_are_not_on_the_gpu_are_refused():
+    """Before anything is launched: a host address would be read on the device."""
+    from hyclora_amd.operators.flash_kernels import flash_backward, flash_forward, flash_supported
+    from hyclora_amd.operators.map_kernels import MapAttention, map_backward, map_supported
+    q, k, v, g = (torch.zeros(1, 2, 64, 64, device="cuda", dtype=BF16) for _ in range(4))
+    lse = torch.zeros(1, 2, 64, device="cuda")
+    lists = torch.empty(0, device="cuda", dtype=torch.int64), torch.empty(0, device="cuda", dtype=BF16), torch.zeros(3, device="cuda", dtype=torch.int64)
+    mask = torch.zeros(1, 1, 64, 64, device="cuda", dtype=BF16)
+    assert flash_supported(q, k, v) and map_supported(q, k, v, mask) and not map_supported(q, k, v, mask.cpu())
+    for i in range(3):
+        ops = [t.cpu() if j == i else t for j, t in enumerate((q, k, v))]
+        assert not flash_supported(*ops) and not map_supported(*ops, mask)
+        for call in (lambda: flash_forward(*ops), lambda: flash_backward(g, *ops, q, lse), lambda: MapAttention(*ops, mask), lambda: map_backward(g, *ops, *lists)):
+            with pytest.raises(ValueError):
+                call()
+    with pytest.raises(ValueError):
+        MapAttention(q, k, v, mask.cpu())
+    att = MapAttention(q, k, v, threshold=torch.zeros(()))
+    for offsets in (torch.empty(3, dtype=torch.int64), torch.empty(2, device="cuda", dtype=torch.int64), torch.empty(3, device="cuda", dtype=torch.int32)):
+        with pytest.raises(ValueError):
+            att.entries(8, offsets)
+    for call in (lambda: flash_backward(g.cpu(), q, k, v, q, lse), lambda: flash_backward(g, q, k, v, q.cpu(), lse), lambda: flash_backward(g, q, k, v, q, lse.cpu()),
+                 lambda: map_backward(g.cpu(), q, k, v, *lists), *(lambda i=i: map_backward(g, q, k, v, *(t.cpu() if j == i else t for j, t in enumerate(lists))) for i in range(3))):
+        with pytest.raises(RuntimeError, match="GPU only"):
+            call()
+
+
 @pytest.mark.parametrize("causal", [True, False])
 def test_backward_of_another_output(causal):
     """The layers hand in the dequantised output, a few percent off the forward's."""
