@@ -369,6 +369,7 @@ def compress_attention_map(x: torch.Tensor, outlier, seg_offsets=None, compare_a
     if seg_offsets is not None:
         if seg_offsets.numel() != nseg + 1 or seg_offsets.dtype != torch.int64:
             raise ValueError("seg_offsets does not belong to a map of this size")
+        _lib.require_gpu(seg_offsets)
         offsets = seg_offsets
     else:
         counts = torch.empty(max(nseg, 1), device=x.device, dtype=torch.int32)
@@ -410,7 +411,7 @@ def restore_attention_map(idx, val, seg_offsets, shape):
     for d in shape:
         n *= int(d)
     check_map_lists(idx, val, seg_offsets, n)
-    _lib.require_gpu(idx, val)
+    _lib.require_gpu(idx, val, seg_offsets)
     idx = idx.reshape(-1).contiguous()
     val = val.to(BF16).reshape(-1).contiguous()
     st = _lib.stream_of(val)

@@ -6,6 +6,7 @@ of the reference's Triton kernels, carried only so that callers can hand them ba
 import torch
 
 from .. import _lib
+from .rmsnorm_kernels import _check_sizes
 
 HAS_APEX = False
 
@@ -29,6 +30,8 @@ def _check(x):
 
 def layernorm_forward(x, weight, bias, eps):
     """-> (y, mean fp32 [rows], rstd fp32 [rows], BLOCK_SIZE, num_warps).  Reference :125-147."""
+    _check_sizes(x, weight)
+    _check_sizes(x, bias)
     _lib.require_gpu(x, weight, bias)
     n = _check(x)
     x = x.contiguous()
@@ -49,6 +52,8 @@ def layernorm_backward(dy, x, w, b, m, v, needs_inputs_grad, eps, num_warps, BLO
     (which computes weight / bias gradient partials and discards them)."""
     if not needs_inputs_grad:
         return None, None, None
+    _check_sizes(x, w, dy, v)
+    _check_sizes(x, w, dy, m)
     _lib.require_gpu(dy, x, w, m, v)
     n = _check(x)
     if dy.dtype != torch.bfloat16:

@@ -156,6 +156,7 @@ ROPE_HEAD_DIM = 128          # the fused rotation needs heads as wide as a colum
 def _rope_tables(rope, seq_len):
     from .rope_kernels import _table
     cos, sin = rope
+    _lib.require_gpu(cos, sin)
     cos, sin = _table(cos, seq_len, ROPE_HEAD_DIM // 2), _table(sin, seq_len, ROPE_HEAD_DIM // 2)
     if cos.dtype != sin.dtype or cos.dtype not in (BF16, torch.float32):
         raise NotImplementedError("cos/sin tables must both be bfloat16 or both float32")

@@ -44,6 +44,7 @@ def dequantize_nf4(w, quant_state):
         raise NotImplementedError(f"only the nf4 code book is supported, got {qs.quant_type!r}")
     if getattr(qs, "dtype", torch.bfloat16) != torch.bfloat16:
         raise NotImplementedError("dequantize_nf4 produces bfloat16 weights")
+    _lib.require_gpu(qs.absmax)
     dev = w.device
     nested = bool(getattr(qs, "nested", False))
     if nested and len(qs.shape) == 2:                    # what a double-quantised checkpoint holds, statistics as they lie

@@ -21,7 +21,19 @@ def _weight(weight: torch.Tensor):
     return weight.to(torch.bfloat16).contiguous(), 0
 
 
+def _check_sizes(x, weight, dy=None, rstd=None):
+    """What the kernels take on trust: they read weight[0..N), dy like x, and rstd[row] for every row."""
+    n = x.shape[-1]
+    if weight.numel() != n:
+        raise ValueError(f"the weight must have {n} entries, got {weight.numel()}")
+    if dy is not None and (dy.numel() != x.numel() or dy.shape[-1] != n):
+        raise ValueError(f"dy {tuple(dy.shape)} is not of x's shape {tuple(x.shape)}")
+    if rstd is not None and rstd.numel() * n != x.numel():
+        raise ValueError(f"a row statistic must have one entry per row of {tuple(x.shape)}, got {rstd.numel()}")
+
+
 def rmsnorm_forward(x, weight, eps):
+    _check_sizes(x, weight)
     _lib.require_gpu(x, weight)
     if x.dtype != torch.bfloat16:
         raise NotImplementedError("rmsnorm_forward computes on bfloat16 activations")
@@ -46,6 +58,7 @@ def rmsnorm_forward(x, weight, eps):
 def _backward(dy, x, w, rstd, want_dw, residual=None):
     """-> (dx, dw or None).  With `residual` (bf16, dy's shape) dx is bf16(dx + residual): the
     gradient of the residual connection added in the same pass, same bits as adding it afterwards."""
+    _check_sizes(x, w, dy, rstd)
     _lib.require_gpu(dy, x, w, rstd, residual)
     if dy.dtype != torch.bfloat16 or x.dtype != torch.bfloat16:
         raise NotImplementedError("rmsnorm_backward computes on bfloat16 activations")
@@ -112,7 +125,7 @@ def rmsnorm_backward_from_codes(dy, q_x, scale_x, x_outlier, outlier_idx, q_bit,
     (q_x, scale_x, x_outlier, outlier_idx) - the same bits as
     outlier_addition_fuse_decompression_dequantization followed by rmsnorm_backward
     (fused_llama_layer_intra_inter_full_fuse.py:386-393), with `residual` added like there."""
-    _lib.require_gpu(dy, q_x, scale_x, w, rstd, residual)
+    _lib.require_gpu(dy, q_x, scale_x, w, rstd, residual, x_outlier, table)
     n = dy.shape[-1]
     k = 0 if outlier_idx is None else int(outlier_idx.numel())
     if k and table is None and outlier_idx.is_cuda:
@@ -238,6 +251,8 @@ def rmsnorm_forward_compress(x, weight, eps, q_bit, scale_y=None, scale_x=None, 
     [B, M, R] bf16 - lora_forward's `x @ w_lora_a` (models/utils/compute_utils.py:22) for each of them,
     formed while y is still on the chip instead of by one library GEMM each over y in memory
     (see lora_a_supported for the shapes this takes)."""
+    _check_sizes(x, weight)
+    _lib.require_gpu(x, weight, scale_y, scale_x, table, *(lora_a or []))
     k = 0 if outlier_idx is None or scale_x is None else outlier_idx.numel()
     if k and table is None and outlier_idx.is_cuda:
         table = outlier_table(outlier_idx, x.shape[-1], cached=True)
@@ -245,7 +260,6 @@ def rmsnorm_forward_compress(x, weight, eps, q_bit, scale_y=None, scale_x=None, 
         done = _lib.native().norm_compress(x, weight, eps, q_bit, scale_y, scale_x, table, k, lora_a or [])
         if done is not None:
             return done if lora_a else done[:5]
-    _lib.require_gpu(x, weight)
     if x.dtype != torch.bfloat16 or x.dim() != 3:
         raise NotImplementedError("rmsnorm_forward_compress takes bfloat16 [batch, seq, hidden] activations")
     if q_bit not in (2, 4, 8):

@@ -165,3 +165,24 @@ def test_projections_of_cpu_tensors_need_no_library(monkeypatch, tmp_path, dtype
     ga, gb, gx = CU.lora_backward(w, None, a, b, x, xa, gy)
     assert torch.equal(gx, gy @ w + (gy @ b.mT) @ a.mT)
     assert torch.equal(ga, x.mT @ (gy @ b.mT)) and torch.equal(gb, xa.mT @ gy)
+
+
+def test_norms_reject_weights_and_statistics_of_another_size():
+    from hyclora_amd.operators import layernorm_kernels as ln
+    from hyclora_amd.operators import rmsnorm_kernels as rms
+    from hyclora_amd.operators import rmsnorm_updatable_kernels as upd
+    x, w, stat = t(B, M, N), t(N), t(B * M, dtype=torch.float32)
+    for call in (lambda x, w, dy, s: rms.rmsnorm_forward(x, w, 1e-5), lambda x, w, dy, s: rms.rmsnorm_backward(dy, x, w, s, s, True, 1e-5, 4, 64),
+                 lambda x, w, dy, s: upd.rmsnorm_backward(dy, x, w, s, s, 1e-5, 4, 64), lambda x, w, dy, s: rms.rmsnorm_forward_compress(x, w, 1e-5, 4),
+                 lambda x, w, dy, s: ln.layernorm_forward(x, w, w, 1e-5), lambda x, w, dy, s: ln.layernorm_forward(x, t(N), w, 1e-5),
+                 lambda x, w, dy, s: ln.layernorm_backward(dy, x, w, w, stat, s, True, 1e-5, 4, 64),
+                 lambda x, w, dy, s: ln.layernorm_backward(dy, x, w, w, s, stat, True, 1e-5, 4, 64)):
+        with pytest.raises(RuntimeError, match="GPU only"):
+            call(x, w, x, stat)
+        with pytest.raises(ValueError):
+            call(x, t(N - 8), x, stat)
+    for call in (lambda dy, s: rms.rmsnorm_backward(dy, x, w, s, s, True, 1e-5, 4, 64), lambda dy, s: upd.rmsnorm_backward(dy, x, w, s, s, 1e-5, 4, 64),
+                 lambda dy, s: ln.layernorm_backward(dy, x, w, w, s, s, True, 1e-5, 4, 64)):
+        for dy, s in ((t(B, M - 1, N), stat), (t(B, M, N - 8), stat), (x, stat[:-1])):
+            with pytest.raises(ValueError):
+                call(dy, s)
