@@ -10,8 +10,8 @@
 // Bound by the vector units (roundings, two exponentials per score and walk) with the matrix cores beside them; the tiles and
 // the division of a workgroup are those of flash.hip.  Per element the dense route moved 2 bytes nine times (scores, map,
 // kept entries, restored map, both gradients); here only the entries move.  [4, 1024, 32 heads, 128], causal, 5 % kept:
-// forward 117 us and entries 80 us (library products, softmax with count, compaction: 357 us), backward 237 us (products,
-// restore + softmax backward: 537 us).  Of these, 6 and 12 us are the looks at the operands for NaN and infinities.
+// forward 106 us and entries 80 us (library products, softmax with count, compaction: 357 us), backward 237 us (products,
+// restore + softmax backward: 537 us).  Of these, 6 and 14 us are the looks at the operands for NaN and infinities.
 #include "hyc_attn_tile.hpp"
 
 namespace hyc {
@@ -42,7 +42,7 @@ struct MapArgs {
 
 // 16 rows of a tile of keys and of values, looked at by one wave: is an element infinite or NaN?
 template <int D>
-__device__ __forceinline__ bool any_wild(const uint16_t* k, const uint16_t* v, int ld, int row0, int row_last, int lane) {
+__device__ __forceinline__ bool tile_is_wild(const uint16_t* k, const uint16_t* v, int ld, int row0, int row_last, int lane) {
     typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
     constexpr int kLanes = D / 8, kRows = 64 / kLanes, kLoads = 16 / kRows;      // lanes of a row, rows of a load
     u32x4 e[2 * kLoads];
@@ -63,7 +63,7 @@ __device__ __forceinline__ bool any_wild(const uint16_t* k, const uint16_t* v, i
 // Which tiles matter.  Of the mask: bit t of classes[..][0] is set when some entry of the 32 rows x 64 keys is above kDead, of
 // classes[..][1] when all are zero.  A wave looks at 8 tiles (a byte of either word), a lane at 8 keys of the 32 rows; a
 // causal mask lets half of the tiles go.  Of the keys and values: tiles may only go where all of a head's are finite, since a
-// weight of 0 times an infinite value, or an infinite score under a mask of -inf, is NaN (one read of both, 6 us of 117 at
+// weight of 0 times an infinite value, or an infinite score under a mask of -inf, is NaN (one read of both, 6 us of 106 at
 // [4, 1024, 32 heads, 128]).
 template <int D>
 __global__ __launch_bounds__(256) void map_classes_kernel(const MapArgs A, int mask_wgs, int mask_batches) {
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void map_classes_kernel(const MapArgs A, int m
         const int i = (int)blockIdx.x - mask_wgs * mask_batches, nt = (S + kMapTile - 1) / kMapTile;
         const int kvh = i % A.KV, t = i / A.KV % nt, b = i / A.KV / nt;
         const int64_t at = ((int64_t)b * S * A.KV + kvh) * D;
-        const bool w = any_wild<D>(A.k + at, A.v + at, A.KV * D, t * kMapTile + wave * 16, S - 1, lane);
+        const bool w = tile_is_wild<D>(A.k + at, A.v + at, A.KV * D, t * kMapTile + wave * 16, S - 1, lane);
         if (lane == 0) reinterpret_cast<uint8_t*>(const_cast<uint32_t*>(A.wild))[((int64_t)(b * A.KV + kvh) * 64 + t) * 4 + wave] = w;
         return;
     }
@@ -497,52 +497,23 @@ struct MapBwdArgs {
     uint32_t* entries;                  // (row % 32 * 64 + key % 64) << 16 | value, grouped by 32-row x 64-key tile
     uint16_t* grads;                    // per entry: the map's gradient, then the score's
     uint32_t* tile_at;                  // [B * H * row blocks, tiles + 1]: where a tile's entries begin
-    uint32_t* wild;                     // [B * H * row blocks]: operands of the block that are not finite, kWildRows | kWildKeys
-    uint32_t* wild_sums;                // [B * H * row blocks]: rows whose d is not finite; of heads with such operands only
+    uint32_t* wild;                     // [B * H * row blocks]: what of the 32 rows is not finite, kWildQ | ...
+    uint32_t* wild_columns;             // [B * H * row blocks][3][4]: columns of q, k and grad_o that hold such an element, where wild says so
     uint16_t *grad_q, *grad_k, *grad_v;
     int B, S, H, KV;
     float scale;
 };
 
-// Work on tiles without a kept entry may only be left out where all operands of a head are finite: elsewhere 0 times an infinite
-// value, or an infinite gradient of the map times the 0 of an entry that is not kept, is NaN.
-constexpr uint32_t kWildRows = 1;       // q, grad_o or a kept entry of the rows
-constexpr uint32_t kWildKeys = 2;       // k or v of rows of these numbers (noted by the first query head of a group)
-
-// Whether a head has an operand that is not finite; the words of its row blocks are read by one wave (at most 128).
-__device__ __forceinline__ bool head_is_wild(const MapBwdArgs& A, int bh, int nrb, int lane) {
-    const int lead = bh - bh % A.H % (A.H / A.KV);
-    uint32_t w = 0;
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int rb = min(lane + 64 * i, nrb - 1);
-        w |= (A.wild[(int64_t)bh * nrb + rb] & kWildRows) | (A.wild[(int64_t)lead * nrb + rb] & kWildKeys);
-    }
-    return __any(w != 0);
-}
-
 // Groups the entries of 32 rows by tile of 64 keys.  The entries of a tile come in no particular order (each has its own
-// place in the dense tile that the kernels below rebuild from them, so no result depends on it).  Looks at the operands of
-// the 32 rows on the way, while it waits for its counts.
-template <int D>
+// place in the dense tile that the kernels below rebuild from them, so no result depends on it).
 __global__ __launch_bounds__(256) void map_regroup_kernel(const MapBwdArgs A) {
-    __shared__ uint32_t place[kMapMax / kMapTile], below[2], marks;
+    __shared__ uint32_t place[kMapMax / kMapTile], below[2];
     const int nrb = (A.S + 31) / 32, nt = (A.S + kMapTile - 1) / kMapTile;
     const int bh = blockIdx.x / nrb, r0 = (int)(blockIdx.x % nrb) * 32;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = bh / A.H, head = bh % A.H, group = A.H / A.KV;
-    uint32_t mark = 0;
-    if (wave < 2) {
-        const int64_t at = ((int64_t)b * A.S * A.H + head) * D;
-        if (any_wild<D>(A.q + at, A.grad_o + at, A.H * D, r0 + wave * 16, A.S - 1, lane)) mark = kWildRows;
-    } else if (head % group == 0) {
-        const int64_t at = ((int64_t)b * A.S * A.KV + head / group) * D;
-        if (any_wild<D>(A.k + at, A.v + at, A.KV * D, r0 + wave % 2 * 16, A.S - 1, lane)) mark = kWildKeys;
-    }
     const int64_t elems = (int64_t)A.B * A.H * A.S * A.S;
     const int64_t e0 = ((int64_t)bh * A.S + r0) * A.S, e1 = e0 + (int64_t)min(32, A.S - r0) * A.S;
     if (threadIdx.x < (unsigned)nt) place[threadIdx.x] = 0;
     if (threadIdx.x < 2) below[threadIdx.x] = 0;
-    if (threadIdx.x == 2) marks = 0;
     __syncthreads();
     int64_t edge[2];
 #pragma unroll
@@ -582,20 +553,63 @@ __global__ __launch_bounds__(256) void map_regroup_kernel(const MapBwdArgs A) {
     for (int64_t i = first + threadIdx.x; i < last; i += 256) {
         uint32_t row, key;
         split((uint32_t)(A.indices[i] - e0), row, key);
-        const uint32_t slot = atomicAdd(&place[key / kMapTile], 1u), value = A.values[i];
-        A.entries[slot] = (row * kMapTile + key % kMapTile) << 16 | value;
-        if ((value & 0x7f80u) == 0x7f80u) mark |= kWildRows;
+        const uint32_t slot = atomicAdd(&place[key / kMapTile], 1u);
+        A.entries[slot] = (row * kMapTile + key % kMapTile) << 16 | A.values[i];
     }
-    if (mark) atomicOr(&marks, mark);
-    __syncthreads();
-    if (threadIdx.x == 0) A.wild[blockIdx.x] = marks;
 }
 
 // Entries of a tile that a wave holds in registers: 64 of each of kHeld loads.  With 5 % of a causal map kept, the tiles below
 // the diagonal hold 200 on average; the few fuller ones (a row's first keys) are worked through kHeld loads at a time.
 constexpr int kHeld = 4;
 
-constexpr uint32_t kNanPair = 0x7fc07fc0u;
+// Entries that are not kept are never formed, but they are 0 only while everything is finite: 0 times an infinite value, or an
+// infinite gradient of the map times their 0, is NaN.  What follows, for one head of the formulas on top:
+//   grad_o[i, c] not finite:  d_i, so row i of grad_q and all of grad_k; column c of grad_v
+//   v not finite:             every d, so all of grad_q and grad_k
+//   d_i not finite (an entry that is NaN):  row i of grad_q, all of grad_k
+//   k[j, c] not finite:       column c of grad_q
+//   q[i, c] not finite:       column c of grad_k
+// The kernel of grad_q looks at the rows of its numbers in all four and sees to the rows; the kernel of grad_k and grad_v, which
+// runs after it, sees to the columns and to the rest.  The looks are one read of the operands: 14 us of 237 at [4, 1024, 32
+// heads, 128], 8 of 280 at [1, 2048, 32, 128] (14 and 17 in the kernel that groups the entries, where nothing else of theirs is read).
+enum : uint32_t { kWildQ = 1, kWildK = 2, kWildV = 4, kWildG = 8, kWildD = 16 };
+
+// Elements of 16 bytes that are infinite or NaN: is there one, and which (bit j: element j)?
+template <int N>
+__device__ __forceinline__ bool any_wild(const u32x4 (&e)[N]) {
+    typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+    u16x2 most = {0, 0};
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, e[i][j] & 0x7fff7fffu));
+    return most.x >= 0x7f80 || most.y >= 0x7f80;
+}
+__device__ __forceinline__ uint32_t wild_bits(u32x4 e) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) m |= ((e[j / 2] >> (16 * (j & 1))) & 0x7f80u) == 0x7f80u ? 1u << j : 0u;
+    return m;
+}
+// 32 rows of a tensor as a wave reads them fastest, whole rows side by side: lane l has chunk l % (D / 8) of every (512 / D)th row
+template <int D>
+struct WildRows {
+    static constexpr int kLanes = D / 8, kLoads = 32 * kLanes / 64;
+    u32x4 e[kLoads];
+    __device__ __forceinline__ void request(const uint16_t* base, int64_t ld, int row0, int row_last, int lane) {
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) e[i] = ld16(base + (int64_t)min(row0 + (i * 64 + lane) / kLanes, row_last) * ld + lane % kLanes * 8);
+    }
+    // the columns with such an element, a bit each, as D / 8 bytes
+    __device__ __forceinline__ void note_columns(uint8_t* out, int lane) const {
+        uint32_t m = 0;
+#pragma unroll
+        for (int i = 0; i < kLoads; ++i) m |= wild_bits(e[i]);
+#pragma unroll
+        for (int o = kLanes; o < 64; o *= 2) m |= (uint32_t)__shfl_xor((int)m, o, kWave);
+        if (lane < kLanes) out[lane] = (uint8_t)m;
+    }
+};
 
 // Clears a wave's 32 x 64 patch
 __device__ __forceinline__ void clear_patch(char* patch, int lane) {
@@ -605,9 +619,7 @@ __device__ __forceinline__ void clear_patch(char* patch, int lane) {
 
 // grad_q of 128 rows.  First walk: g at the kept entries and the row sums d (the tile of a is rebuilt in LDS, the products of
 // one tile are 32 x 64 values of which a few percent are kept).  Second walk: ds from g, d and a per entry, its tile rebuilt in
-// LDS as the operand of ds k; ds stays in `grads` for the key / value kernel.  Tiles without an entry are left out, unless the
-// head has an operand that is not finite: then every tile is worked through, and in a row whose d is not finite the entries
-// that are not kept, (g - d) * 0, are NaN.
+// LDS as the operand of ds k; ds stays in `grads` for the key / value kernel.  Tiles without an entry are left out.
 template <int D>
 __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
     using Tile = AttnTile<D, kMapTile>;
@@ -624,13 +636,19 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
     const int64_t row_off = ((int64_t)b * A.S + row_in) * ldq + head * D;
     bf16x8 G[D / 16];
     load_row_operands<D>(A.grad_o + row_off, h, G);
+    WildRows<D> q_rows, k_rows, v_rows;                                 // looked at below, while the first tile is on its way
+    const bool lead = head % (A.H / A.KV) == 0;                         // a group's keys and values: looked at by its first head
+    q_rows.request(A.q + ((int64_t)b * A.S * A.H + head) * D, ldq, rb * 32, A.S - 1, lane);
+    if (lead) {
+        k_rows.request(kbase, ldk, rb * 32, A.S - 1, lane);
+        v_rows.request(vbase, ldk, rb * 32, A.S - 1, lane);
+    }
     char* patch = lds + 2 * Tile::kBytes + wave * MapPatch::kBytes;
     float* row_sum = reinterpret_cast<float*>(lds + 2 * Tile::kBytes + 4 * MapPatch::kBytes + wave * 128);
     uint64_t* wave_tiles = reinterpret_cast<uint64_t*>(lds + 2 * Tile::kBytes + 4 * MapPatch::kBytes + 4 * 128);
     const uint32_t* tile_at = A.tile_at + ((int64_t)bh * nrb + min(rb, nrb - 1)) * (nt + 1);
     const uint32_t t_beg = rb < nrb ? tile_at[min(lane, nt)] : 0u, t_end = rb < nrb ? tile_at[min(lane + 1, nt)] : 0u;     // of tile `lane`
-    const bool wild = head_is_wild(A, bh, nrb, lane);
-    const uint64_t own = wild && rb < nrb ? tiles_of(A.S) : __ballot(lane < nt && t_end > t_beg);
+    const uint64_t own = __ballot(lane < nt && t_end > t_beg);
     if (lane == 0) wave_tiles[wave] = own;
     __syncthreads();
     const uint64_t todo = uniform64(wave_tiles[0] | wave_tiles[1] | wave_tiles[2] | wave_tiles[3]);
@@ -653,12 +671,42 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
         const int t = __builtin_ctzll(tiles);
         beg = (uint32_t)__builtin_amdgcn_readlane((int)t_beg, t);
         n = (uint32_t)__builtin_amdgcn_readlane((int)t_end, t) - beg;
-        if (n) load(0, with_grads);
+        load(0, with_grads);
     };
     auto later = [&](int t) { return t < 63 ? own >> (t + 1) << (t + 1) : 0ull; };
     int buf = 0;
     float d = 0.0f;
     fetch(own, false);
+    uint32_t marks = 0;                                                 // of the wave's rows
+    {
+        uint8_t* columns = reinterpret_cast<uint8_t*>(A.wild_columns + ((int64_t)bh * nrb + min(rb, nrb - 1)) * 12);
+        if (__any(any_wild(q_rows.e))) {
+            marks |= kWildQ;
+            if (rb < nrb) q_rows.note_columns(columns, lane);
+        }
+        if (lead) {
+            if (__any(any_wild(k_rows.e))) {
+                marks |= kWildK;
+                if (rb < nrb) k_rows.note_columns(columns + 16, lane);
+            }
+            if (__any(any_wild(v_rows.e))) marks |= kWildV;
+        }
+    }
+    u32x4 g_rows[D / 16];
+#pragma unroll
+    for (int t = 0; t < D / 16; ++t) g_rows[t] = __builtin_bit_cast(u32x4, G[t]);
+    const bool wild_g = any_wild(g_rows);
+    if (__any(wild_g)) {
+        marks |= kWildG;
+        uint8_t* columns = reinterpret_cast<uint8_t*>(A.wild_columns + ((int64_t)bh * nrb + min(rb, nrb - 1)) * 12 + 8);
+#pragma unroll
+        for (int t = 0; t < D / 16; ++t) {                              // lane l: columns 16t + 8h .. of row l % 32
+            uint32_t m = wild_bits(g_rows[t]);
+#pragma unroll
+            for (int o = 1; o < 32; o *= 2) m |= (uint32_t)__shfl_xor((int)m, o, kWave);
+            if (rb < nrb && (lane & 31) == 0) columns[2 * t + h] = (uint8_t)m;
+        }
+    }
     walk_tiles(todo, buf, [&](int t, int bb) { Tile::request(vbase, t * kMapTile, A.S - 1, ldk, lds0 + bb * Tile::kBytes, wave, lane); },
                [&](int t, int bb) {
         if (!((own >> t) & 1)) return;
@@ -709,13 +757,14 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
         lds_order();
         fetch(later(t), false);
     });
+    if (wild_g) d = NAN;
     d = half_sum(d);
     if (lane < 32) row_sum[lane] = d;
     lds_order();
-    const bool wild_sum = !(__builtin_fabsf(d) < INFINITY);
-    if (wild && rb < nrb) {
-        const uint32_t rows = (uint32_t)__ballot(wild_sum && qrow < A.S);
-        if (lane == 0) A.wild_sums[(int64_t)bh * nrb + rb] = rows;
+    const bool wild_row = !(__builtin_fabsf(d) < INFINITY);
+    if (rb < nrb) {
+        if (__any(wild_row)) marks |= kWildD;
+        if (lane == 0) A.wild[(int64_t)bh * nrb + rb] = marks;
     }
     f32x16 dq[D / 32];
 #pragma unroll
@@ -724,13 +773,7 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
     walk_tiles(todo, buf, [&](int t, int bb) { Tile::request(kbase, t * kMapTile, A.S - 1, ldk, lds0 + bb * Tile::kBytes, wave, lane); },
                [&](int t, int bb) {
         if (!((own >> t) & 1)) return;
-        if (wild) {
-            const uint32_t v = wild_sum ? kNanPair : 0u;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4*>(patch + (lane & 31) * 128 + (4 * h + i) * 16) = u32x4{v, v, v, v};
-        } else {
-            clear_patch(patch, lane);
-        }
+        clear_patch(patch, lane);
         lds_order();
         auto put = [&](uint32_t i, uint32_t v, uint32_t g) {
             const uint16_t ds = f_to_bf(rbf((bf_to_f((uint16_t)g) - row_sum[v >> 22]) * bf_lo(v)) * A.scale);
@@ -758,7 +801,35 @@ __global__ __launch_bounds__(256, 2) void map_bwd_q_kernel(const MapBwdArgs A) {
         order_products<D / 8, 2, 4>();
         lds_order();
     });
-    if (qrow < A.S) store_rows<D>(A.grad_q + row_off, h, dq, 1.0f);
+    if (qrow < A.S) store_rows<D>(A.grad_q + row_off, h, dq, wild_row ? NAN : 1.0f);
+}
+
+// Rows row0 .. row0 + 31 of the three gradients of a head with something that is not finite: NaN over what has been stored
+// there, in the columns that have it.  A lane overwrites what it stored itself (grad_k, grad_v) or what the kernel before left.
+template <int D>
+__device__ __forceinline__ void map_spread(const MapBwdArgs& A, int bh, int nrb, int row0, int lane, uint32_t marks) {
+    const int h = lane >> 5, b = bh / A.H, head = bh % A.H, lead = bh - head % (A.H / A.KV), row = row0 + (lane & 31);
+    const bool all_k = __any(marks & (kWildV | kWildD)), all_q = __any(marks & kWildV);
+    const int64_t off = (((int64_t)b * A.S + row) * A.H + head) * D;
+#pragma unroll 1
+    for (int i = 0; i < D / 32; ++i) {
+        uint32_t q = 0, k = 0, g = 0;
+#pragma unroll 1
+        for (int rb = 0; rb < nrb; ++rb) {
+            const uint32_t own = A.wild[(int64_t)bh * nrb + rb], keys = A.wild[(int64_t)lead * nrb + rb];
+            if (own & kWildQ) q |= A.wild_columns[((int64_t)bh * nrb + rb) * 12 + i];
+            if (keys & kWildK) k |= A.wild_columns[((int64_t)lead * nrb + rb) * 12 + 4 + i];
+            if (own & kWildG) g |= A.wild_columns[((int64_t)bh * nrb + rb) * 12 + 8 + i];
+        }
+        if (row >= A.S) continue;
+#pragma unroll 1
+        for (int c = 0; c < 32; ++c) {
+            if (((c >> 2) & 1) != h) continue;
+            if (all_k || (q >> c & 1)) A.grad_k[off + 32 * i + c] = 0x7fc0;
+            if (g >> c & 1) A.grad_v[off + 32 * i + c] = 0x7fc0;
+            if (all_q || (k >> c & 1)) A.grad_q[off + 32 * i + c] = 0x7fc0;
+        }
+    }
 }
 
 // grad_k and grad_v of 128 keys of one query head, over the rows that keep an entry there, 32 rows at a time: the transposed
@@ -779,7 +850,14 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
     const int ldq = A.H * D;
     const int key = blk * kMapRows + wave * 32 + (lane & 31);
     const int t0 = blk * 2, t1 = min(t0 + 1, nt), t2 = min(t0 + 2, nt);
-    const bool wild = head_is_wild(A, bh, nrb, lane);                    // then every step, with or without entries
+    uint32_t marks = 0;                                                 // of the head; row blocks are at most 128
+    {
+        const int lead = bh - head % (A.H / A.KV);
+        for (int i = 0; i < 2; ++i) {
+            const int64_t rb = min(lane + 64 * i, nrb - 1);
+            marks |= (A.wild[(int64_t)bh * nrb + rb] & ~(uint32_t)(kWildK | kWildV)) | (A.wild[(int64_t)lead * nrb + rb] & (kWildK | kWildV));
+        }
+    }
     const uint32_t* tile_at = A.tile_at + (int64_t)bh * nrb * (nt + 1);
     // a step: 32 rows with entries, where those of the first tile begin, how many they and the second's are
     uint32_t* steps = reinterpret_cast<uint32_t*>(lds + 4 * Tile::kBytes + 8 * kPatch);
@@ -789,7 +867,7 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
     const uint16_t* qb = A.q + (int64_t)b * A.S * ldq + head * D;
     const uint16_t* gb = A.grad_o + (int64_t)b * A.S * ldq + head * D;
     // wave w rebuilds tile w % 2 of the two, of a (w < 2) or of ds
-    struct Pending { uint32_t beg, n, nan_rows, e[kHeld], v[kHeld]; };
+    struct Pending { uint32_t beg, n, e[kHeld], v[kHeld]; };
     auto load = [&](Pending& p, uint32_t from) {
 #pragma unroll
         for (int u = 0; u < kHeld; ++u) {
@@ -806,7 +884,6 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
         const uint32_t first = steps[3 * i + 1], both = steps[3 * i + 2];
         p.beg = __builtin_amdgcn_readfirstlane(wave & 1 ? first + (both & 0xffffu) : first);
         p.n = __builtin_amdgcn_readfirstlane(wave & 1 ? both >> 16 : both & 0xffffu);
-        p.nan_rows = wild && wave >> 1 ? A.wild_sums[(int64_t)bh * nrb + steps[3 * i]] : 0u;
         load(p, 0);
         return p;
     };
@@ -818,8 +895,6 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
             const uint32_t row = e >> 22, k = (e >> 16) & 63;
             *reinterpret_cast<uint16_t*>(patch + k * 64 + (((row >> 3) ^ ((k >> 2) & 3)) << 4) + (row & 7) * 2) = (uint16_t)v;
         };
-        for (uint32_t rows = p.nan_rows; rows; rows &= rows - 1) put((uint32_t)__builtin_ctz(rows) << 22 | (uint32_t)lane << 16, kNanPair);
-        lds_order();
         for (uint32_t from = 0;;) {
 #pragma unroll
             for (int u = 0; u < kHeld; ++u) if (from + (uint32_t)(lane + 64 * u) < p.n) put(p.e[u], wave >> 1 ? p.v[u] : p.e[u]);
@@ -845,12 +920,11 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
             const uint32_t* r = tile_at + (int64_t)s * (nt + 1);
             a0 = r[t0]; a1 = r[t1]; a2 = r[t2];
         }
-        const bool step = a2 > a0 || (wild && s < nrb);
-        const uint64_t m = __ballot(step);
+        const uint64_t m = __ballot(a2 > a0);
         if (lane == 0) wave_n[wave] = __popcll(m);
         __syncthreads();
         nsteps = wave_n[0] + wave_n[1];
-        if (step) {
+        if (a2 > a0) {
             const int place = (wave ? wave_n[0] : 0) + __popcll(m & ((1ull << lane) - 1));
             steps[3 * place] = s;
             steps[3 * place + 1] = a0;
@@ -897,6 +971,7 @@ __global__ __launch_bounds__(256, 2) void map_bwd_kv_kernel(const MapBwdArgs A) 
         store_rows<D>(A.grad_k + off, h, dk, 1.0f);
         store_rows<D>(A.grad_v + off, h, dv, 1.0f);
     }
+    if (__any(marks != 0)) map_spread<D>(A, bh, nrb, blk * kMapRows + wave * 32, lane, marks);
 }
 
 // out[t, kv, :] = sum of in[t, kv * group + 0 .. group - 1, :], fp32 sums in that order, one rounding; D / 8 chunks a row
@@ -915,7 +990,7 @@ __global__ __launch_bounds__(256) void group_sum_kernel(const uint16_t* __restri
     st16((blockIdx.y ? out1 : out0) + c * 8, pack8(acc));
 }
 
-struct MapBwdWorkspace { int64_t entries, grads, tile_at, wild, wild_sums, heads, bytes; };
+struct MapBwdWorkspace { int64_t entries, grads, tile_at, wild, wild_columns, heads, bytes; };
 static MapBwdWorkspace map_bwd_workspace(int64_t B, int64_t S, int64_t H, int64_t KV, int64_t D, int64_t capacity) {
     auto up = [](int64_t v) { return cdiv(v, 256) * 256; };
     MapBwdWorkspace w;
@@ -923,8 +998,8 @@ static MapBwdWorkspace map_bwd_workspace(int64_t B, int64_t S, int64_t H, int64_
     w.grads = up(capacity * 4);
     w.tile_at = w.grads + up(capacity * 2);
     w.wild = w.tile_at + up(B * H * cdiv(S, 32) * (cdiv(S, kMapTile) + 1) * 4);
-    w.wild_sums = w.wild + up(B * H * cdiv(S, 32) * 4);
-    w.heads = w.wild_sums + up(B * H * cdiv(S, 32) * 4);                                 // per query head: grad_k, then grad_v
+    w.wild_columns = w.wild + up(B * H * cdiv(S, 32) * 4);
+    w.heads = w.wild_columns + up(B * H * cdiv(S, 32) * 48);                             // per query head: grad_k, then grad_v
     w.bytes = w.heads + (H == KV ? 0 : 2 * up(B * S * H * D * 2));
     return w;
 }
@@ -1046,7 +1121,7 @@ extern "C" int hyc_map_bwd(const void* grad_o, const void* q, const void* k, con
     A.grad_o = (const uint16_t*)grad_o; A.q = (const uint16_t*)q; A.k = (const uint16_t*)k; A.v = (const uint16_t*)v;
     A.indices = indices; A.values = (const uint16_t*)values; A.seg_offsets = seg_offsets;
     A.entries = (uint32_t*)(ws + w.entries); A.grads = (uint16_t*)(ws + w.grads); A.tile_at = (uint32_t*)(ws + w.tile_at);
-    A.wild = (uint32_t*)(ws + w.wild); A.wild_sums = (uint32_t*)(ws + w.wild_sums);
+    A.wild = (uint32_t*)(ws + w.wild); A.wild_columns = (uint32_t*)(ws + w.wild_columns);
     A.grad_q = (uint16_t*)grad_q; A.grad_k = (uint16_t*)grad_k; A.grad_v = (uint16_t*)grad_v;
     if (H != KV) {
         A.grad_k = (uint16_t*)(ws + w.heads);
@@ -1055,12 +1130,11 @@ extern "C" int hyc_map_bwd(const void* grad_o, const void* q, const void* k, con
     A.B = (int)B; A.S = (int)S; A.H = (int)H; A.KV = (int)KV; A.scale = scale;
     hipStream_t st = (hipStream_t)stream;
     const dim3 rows((unsigned)(cdiv(S, 32) * B * H)), blocks((unsigned)(cdiv(S, kMapRows) * B * H));
+    map_regroup_kernel<<<rows, 256, 0, st>>>(A);
     if (D == 128) {
-        map_regroup_kernel<128><<<rows, 256, 0, st>>>(A);
         map_bwd_q_kernel<128><<<blocks, 256, 0, st>>>(A);
         map_bwd_kv_kernel<128><<<blocks, 256, 0, st>>>(A);
     } else {
-        map_regroup_kernel<64><<<rows, 256, 0, st>>>(A);
         map_bwd_q_kernel<64><<<blocks, 256, 0, st>>>(A);
         map_bwd_kv_kernel<64><<<blocks, 256, 0, st>>>(A);
     }
