@@ -227,6 +227,51 @@ std::optional<std::tuple<OptT, OptT>> contract(const OptT& x, const OptT& q, con
     return std::make_tuple(p1, p2);
 }
 
+// The rank-R products of projections that share their input x (dense, or codes): member (A, B, x A, grad_y) -> (grad A, grad B,
+// grad_y B^T), each the bits of its own contract() calls, in one launch for all grad_y and one that reads x once
+using Adapter = std::tuple<Tensor, Tensor, Tensor, Tensor>;
+std::optional<std::vector<std::tuple<Tensor, Tensor, Tensor>>> lora_products_shared(const std::vector<Adapter>& members, const OptT& x, const OptT& q,
+                                                                                    const OptT& scale, const OptT& zero, int64_t bits) {
+    if (!products_are_plain() || members.size() < 2 || members.size() > 3) return std::nullopt;
+    const size_t count = members.size();
+    int64_t T = 0, r = 0, k = 0, ws_g = 0, ws_x = 0;
+    hyc_contract_job g[3] = {}, s[3] = {};
+    for (size_t i = 0; i < count; ++i) {
+        const auto& [la, lb, xa, grad] = members[i];
+        const Lora L(lb);
+        if (!plain(grad) || grad.dim() < 2 || grad.numel() == 0 || !L.fits(grad.size(-1)) || L.r > 16 || (i && L.r != r)) return std::nullopt;
+        const int64_t rows = grad.numel() / L.n;
+        if ((i && rows != T) || !plain(xa) || xa.size(-1) != L.r || xa.numel() != rows * L.r) return std::nullopt;
+        if (!is_bf(la) || la.dim() != 2 || la.size(1) != L.r || (i && la.size(0) != k)) return std::nullopt;
+        T = rows; r = L.r; k = la.size(0);
+        if (!Lora(la.t()).fits(k)) return std::nullopt;
+        g[i].x = grad.data_ptr(); g[i].u = xa.data_ptr(); g[i].v = L.p; g[i].v_transposed = L.transposed; g[i].N = L.n; g[i].p1_transposed = 1;
+        ws_g += hyc_lora_contract_workspace(T, L.n, r, 1, 1);
+        ws_x += hyc_lora_contract_workspace(T, k, r, 1, 0);
+    }
+    if (x ? !(plain(*x) && x->size(-1) == k && x->numel() == T * k)
+          : !(q && scale && bits_ok(bits) && packed(*q, T * k, bits) && aligned(*q) && vec(*scale, k) && (!zero || vec(*zero, k))))
+        return std::nullopt;
+    const Tensor& like = std::get<3>(members[0]);
+    std::vector<std::tuple<Tensor, Tensor, Tensor>> out;
+    for (size_t i = 0; i < count; ++i) {
+        auto shape = like.sizes().vec();
+        shape.back() = r;
+        Tensor ga = at::empty({r, k}, like.options()), gb = at::empty({g[i].N, r}, like.options()), mid = at::empty(shape, like.options());
+        g[i].p1 = gb.data_ptr();
+        g[i].p2 = mid.data_ptr();
+        s[i].u = mid.data_ptr(); s[i].p1 = ga.data_ptr(); s[i].N = k;
+        out.emplace_back(ga.t(), gb.t(), mid);
+    }
+    if (x) s[0].x = x->data_ptr();
+    else { s[0].q = q->data_ptr(); s[0].scale = scale->data_ptr(); s[0].zero_point = ptr(zero); }
+    const int64_t bytes = std::max<int64_t>(std::max(ws_g, ws_x), 16);
+    Tensor ws = at::empty({bytes}, like.options().dtype(at::kByte));
+    check("hyc_lora_contract_group", hyc_lora_contract_group(g, (int)count, 0, 0, ws.data_ptr(), bytes, T, r, stream_of(like)));
+    check("hyc_lora_contract_group", hyc_lora_contract_group(s, (int)count, 1, x ? 0 : (int)bits, ws.data_ptr(), bytes, T, r, stream_of(like)));
+    return out;
+}
+
 // ---- products with a frozen weight --------------------------------------------------------------------------------
 // Columns of a [rows, cols] product to hand to the library first (0: all in one call).  Its bf16 kernels work on 256 x 256 tiles,
 // one per compute unit and round.  Where the tiles fill whole rounds and a remainder, one call spreads the remainder over all
@@ -293,6 +338,13 @@ Tensor frozen_product(const Tensor& x, const Tensor& w) {          // x [.., K] 
     auto shape = x.sizes().vec();
     shape.back() = w.size(1);
     return at::mm(x.view({-1, w.size(0)}), w).view(shape);
+}
+// The input gradient grad_y W of a frozen weight [out, in]
+OptT frozen_input_grad(const Tensor& grad_y, const Tensor& w) {
+    if (!products_are_plain() || !plain(grad_y) || grad_y.dim() < 2 || grad_y.numel() == 0 || !is_bf(w) || w.dim() != 2 || !w.is_contiguous() ||
+        w.size(0) != grad_y.size(-1))
+        return std::nullopt;
+    return frozen_product(grad_y, w);
 }
 bool weight_ok(const Tensor& w, int64_t in) { return is_bf(w) && w.dim() == 2 && w.size(1) == in && w.is_contiguous(); }
 
@@ -549,6 +601,8 @@ PYBIND11_MODULE(_native, m) {
     m.def("lora_add_quant_group", &lora_add_quant_group);
     m.def("lora_add_restore_group", &lora_add_restore_group);
     m.def("contract", &contract);
+    m.def("lora_products_shared", &lora_products_shared);
+    m.def("frozen_input_grad", &frozen_input_grad);
     m.def("whole_rounds", &whole_rounds);
     m.def("frozen_matmul", &frozen_matmul);
     m.def("lora_parts", &lora_parts);

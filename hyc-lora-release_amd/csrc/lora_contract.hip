@@ -12,48 +12,68 @@
 //                              compressed (the reference dequantises first,
 //                              fused_llama_layer_intra_inter_full_fuse.py:375-383, :469-481).
 // A library GEMM runs each of them at a fraction of the memory rate (output tiles 16 wide) and
-// reads X once per product.
+// reads X once per product.  One launch takes the products of several projections: up to three X of
+// one row count, or up to three rank-R products of one X (the codes of x are then read and decoded once).
 //
-// Layout.  A workgroup of 4 waves owns a strip of 256 rows and a group of column tiles (128
-// columns each); wave w walks rows 64w .. 64w+63 of the strip, 16 at a time.  X is held twice:
+// What bounds it: the read of X and, for small tensors, the two launches.  A wave has 16 KB of X on the
+// way at any time and nothing else to wait for.
+//
+// Layout.  A workgroup of 4 waves owns a strip of rows and 512 columns; wave w keeps to the 128 columns
+// 128w .. of them and walks down the strip, 16 rows a step, 4 steps of loads ahead.  So the sums of P1 stay
+// in the wave's registers to the end of the strip, V is read once, and only P2 is added up across the
+// four waves (through LDS, every 64 rows).  (Waves side by side along the rows, 64 rows each, had all their
+// loads in one burst per tile and met at a barrier per tile for P1.)  X is held twice:
 //   "chunk" form  lane (j = l%16, g = l/16): rows 4g .. 4g+3, columns 8j .. 8j+7  (16-byte loads)
-//   "row"   form  lane (i = l%16, g = l/16): row i, columns 16s + 4g .. +3, s = 0..7
+//   "row"   form  lane (i = l%16, g = l/16): row i, columns 32s + 8g .. +7, s = 0..3
 // P1 uses the chunk form as the B operand of v_mfma_f32_16x16x16_bf16 with permuted column slots
 // (MFMA u takes column 8j + u of every lane), so a lane ends up with 8 consecutive columns of 4
-// LoRA rows; P2 uses the row form as the A operand, K running over the columns.  Only the chunk
-// form is loaded from memory (256 contiguous bytes per row and instruction); the row form is the
-// same tile turned through LDS, wave by wave.
-// Sums across waves (P1: the four waves of a workgroup through LDS, then across strips; P2: across
-// column groups) go through fp32 partial buffers in a fixed order - no atomics, so results do not
-// depend on scheduling - and a small second kernel adds the partials and rounds to bf16.
+// LoRA rows; P2 uses the row form as the A operand of v_mfma_f32_16x16x32_bf16, K running over the
+// columns.  Only the chunk form is loaded from memory (256 contiguous bytes per row and instruction);
+// the row form is the same tile turned through LDS, wave by wave.  U lies transposed in LDS, one 8-byte
+// read an operand.
+// Sums across strips (P1) and across column blocks (P2) go through fp32 partial planes that a small second
+// kernel adds in order - no atomics, so results do not depend on scheduling - and rounds to bf16; where
+// there is only one plane the results are written at once, and if that is so for all of them there is no
+// second kernel (P1 of up to 256 rows).
+#include <algorithm>
+
 #include "hyc_pack.hpp"
 
 namespace hyc {
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
 constexpr int kCtThreads = 256;
 constexpr int kCtWaves = kCtThreads / kWave;
-#ifndef HYC_CT_STEPS
-#define HYC_CT_STEPS 4
-#endif
-constexpr int kCtSteps = HYC_CT_STEPS;                    // 16-row steps per wave
-constexpr int kCtStrip = kCtWaves * kCtSteps * 16;        // 256 rows per workgroup
-constexpr int kCtTile = 128;                              // columns per tile
+constexpr int kCtTile = 128;                              // columns per wave
+constexpr int kCtBlock = kCtWaves * kCtTile;              // columns per workgroup
+constexpr int kCtSub = 64;                                // rows between two sums of P2 across the waves; the shortest strip
+constexpr int kCtSteps = kCtSub / 16;                     // steps of loads in flight
+constexpr int kCtMaxStrip = 256;
 constexpr int kCtPitch = kCtTile + 8;                     // LDS row pitch of a transposed tile (bf16 elements)
-static Knob g_ct_max_groups{32};                          // column groups (bounds the P2 partials); see hyc_set_tuning
+constexpr int kCtUPitch = kCtMaxStrip + 4;                // LDS pitch of a rank's column of U
+constexpr int kCtMembers = 3;                             // X's in a launch, or rank-R products of one X
+static Knob g_ct_strip{0};                                // rows of a strip, 0: by size; see hyc_set_tuning
+static Knob g_ct_max_groups{32};                          // no longer read; kept for callers that set it
 
-struct ContractArgs {
+struct ContractMember {
     const uint16_t* x;                   // dense X [T, N]
     const uint8_t* q;                    // or packed codes [T, N*q_bit/8] with
     const uint16_t* s; const uint16_t* zp;   //   steps / zero points bf16 [N]
-    const uint16_t* u;                   // [T, R]
-    const uint16_t* v;                   // [R, N], or [N, R] with v_transposed
-    float* part1;                        // [strips][16*NB][N]
-    float* part2;                        // [groups][T][16*NB]
+    const uint16_t* u[4];                // per rank block of 16: [T, R], at the block's first rank
+    const uint16_t* v[4];                // [R, N], or [N, R] with v_transposed, likewise
+    uint16_t* p1[4]; uint16_t* p2[4];    // results, where there is one plane only
+    float* part1;                        // [strips][16*blocks][N], or null
+    float* part2;                        // [col_blocks][T][16*blocks], or null
+    int N, C, v_transposed, p1_transposed, strip_rows;
+    uint32_t col_blocks;
+    uint32_t first_wg;
+};
+struct ContractArgs {
+    ContractMember m[kCtMembers];
+    int members, R, blocks;
+    int live[4];                         // ranks of a block
     int64_t T;
-    int N, C, R;
-    int tiles_per_group, groups, v_transposed;
-    int passes;                          // the rank is covered 16*NB at a time; see the kernel
-    int64_t n_blocks;                    // strips * groups
 };
 
 __device__ __forceinline__ s16x4 pick_column(const u32x4 (&xv)[4], int u8) {
@@ -65,167 +85,142 @@ __device__ __forceinline__ s16x4 pick_column(const u32x4 (&xv)[4], int u8) {
     return __builtin_bit_cast(s16x4, pk);
 }
 
-template <int QBIT, bool ZP, bool P1, bool P2, int NB, bool MULTI = false>
+// blockIdx.x: member, strip, column block; blockIdx.y: which NB rank blocks of 16 (ranks past 32 are covered by several
+// workgroups, each reading X again, through the cache: every accumulator and operand scales with the blocks held at once)
+template <int QBIT, bool ZP, bool P1, bool P2, int NB>
 __global__ __launch_bounds__(kCtThreads) void lora_contract_kernel(const ContractArgs a) {
     static_assert(QBIT == 0 || !P2, "the column contraction reads dense X only");
-    __shared__ float red[P1 ? kCtWaves * 16 * kCtTile : 1];
-    __shared__ __attribute__((aligned(16))) uint16_t tr[P2 ? kCtWaves : 1][P2 ? 16 * kCtPitch : 8];
+    __shared__ __attribute__((aligned(16))) uint16_t ul[P1 ? NB * 16 * kCtUPitch : 8];
+    __shared__ __attribute__((aligned(16))) uint16_t tr[P2 ? kCtWaves : 1][P2 ? 2 * 16 * kCtPitch : 8];
+    __shared__ __attribute__((aligned(16))) float sum2[2][P2 ? kCtWaves * kCtSub * 16 * NB : 4];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, g = lane >> 4;
-    // Workgroups go round-robin over the 8 XCDs, each with its own L2.  A 128-column tile of packed
-    // codes is 16*q bytes per row, so 8/q neighbouring tiles share every 128-byte line: the block
-    // index is permuted so that those tiles run on one XCD and the line is fetched from HBM once
-    // (measured before: 2.1x the algorithmic bytes at q = 4).
-    constexpr int kShare = QBIT ? 8 / QBIT : 1;
-    int64_t logical = blockIdx.x;
-    if constexpr (kShare > 1) {
-        const int64_t super = logical / (8 * kShare);
-        const int local = (int)(logical % (8 * kShare));
-        logical = super * (8 * kShare) + (local % 8) * kShare + local / 8;
-    }
-    if (logical >= a.n_blocks) return;                          // padding of the permuted grid (uniform)
-    const int group = (int)(logical % a.groups);
-    const int64_t strip = logical / a.groups;
-    const int64_t row_base = strip * kCtStrip + (int64_t)wave * (kCtSteps * 16);
+    const uint32_t wg = blockIdx.x;
+    const int mi = (a.members > 1 && wg >= a.m[1].first_wg ? 1 : 0) + (a.members > 2 && wg >= a.m[2].first_wg ? 1 : 0);
+    const ContractMember& m = a.m[mi];
+    const uint32_t local = wg - m.first_wg, in_strip = local / m.col_blocks;
+    const int64_t strip = in_strip;
+    const int cb = (int)(local - in_strip * m.col_blocks);
+    const int b0 = blockIdx.y * NB;                             // first rank block
+    const int N = m.N, R = a.R;
+    const int64_t row0 = strip * m.strip_rows;
+    const int rows = (int)(a.T - row0 < m.strip_rows ? a.T - row0 : m.strip_rows);
+    const int c0 = cb * kCtBlock + wave * kCtTile;
+    const int chunk = c0 / 8 + j;
+    const bool active = chunk < m.C, full = c0 + kCtTile <= N;
     constexpr int QB = QBIT ? QBIT : 8;
     constexpr float kHalf = (float)(1 << (QB - 1));
-    const int row_bytes = a.N * QB / 8;
 
-    // Ranks beyond 16*NB are covered in passes over the workgroup's tiles, 16*NB LoRA rows at a time:
-    // every accumulator and operand of the contraction scales with the number of rank blocks held at
-    // once (about 100 registers per block), and with more than one block the kernel is down to one wave
-    // per SIMD with nothing to hide its loads behind.  A later pass finds the tiles in the cache the
-    // first one pulled them through.
-    // (MULTI is a template parameter: with the loop bound read from the arguments the one-pass kernel
-    // of the usual ranks ran 42 instead of 31 us.)
-    const int passes = MULTI ? a.passes : 1;
-    const int rows_all = 16 * NB * passes;                    // LoRA rows of a partial plane
-    for (int pass = 0; pass < passes; ++pass) {
-    const int rb = pass * 16 * NB;
-    f32x4 acc2[P2 ? kCtSteps : 1][NB];
+    // Every load is issued whatever the lane (rows, columns and ranks past the end read the last one and are zeroed afterwards): a
+    // load under a condition makes the compiler wait for all that is in flight at its next use.
+    // U: thread (row t/8, rank pair t%8) of 32 rows an iteration; first in the queue, so that waiting for it leaves X in flight
+    uint32_t uw[P1 ? NB : 1][P1 ? kCtMaxStrip / 32 : 1];
+    const int up = threadIdx.x & 7, ur = threadIdx.x >> 3;
+    if constexpr (P1) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int k = 0; k < kCtMaxStrip / 32; ++k) {
+                const int r = 32 * k + ur < rows ? 32 * k + ur : rows - 1, rank = 2 * up < a.live[b0 + nb] ? 2 * up : 0;
+                uw[nb][k] = *reinterpret_cast<const uint32_t*>(m.u[b0 + nb] + (row0 + r) * R + rank);
+            }
+    }
+    // V operand of the column contraction: lane (rank j, g), columns c0 + 32s + 8g .. +7; [N, R]: the eight columns are R elements apart
+    // (whole dwords, the wanted half picked afterwards: 16-bit loads into register halves would each wait for the one before)
+    uint32_t e[P2 ? NB : 1][4][8];
     if constexpr (P2) {
 #pragma unroll
-        for (int st = 0; st < kCtSteps; ++st)
+        for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) acc2[st][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int s = 0; s < 4; ++s) {
+                const int col = c0 + 32 * s + 8 * g < N ? c0 + 32 * s + 8 * g : 0;
+                const int rank = j < a.live[b0 + nb] ? j : 0;
+                if (m.v_transposed) {
+                    const uint16_t* p = m.v[b0 + nb] + (int64_t)col * R + (rank & ~1);
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) e[nb][s][k] = *reinterpret_cast<const uint32_t*>(p + k * R);
+                } else {
+                    const uint16_t* p = m.v[b0 + nb] + (int64_t)rank * N + col;
+                    const u32x2 lo = ld8(p), hi = ld8(p + 4);
+                    e[nb][s][0] = lo.x; e[nb][s][1] = lo.y; e[nb][s][2] = hi.x; e[nb][s][3] = hi.y;
+                }
+            }
+    }
+    // per-column constants of the dequantiser
+    float sc[8], zz[8];
+    const int ld_chunk = active ? chunk : m.C - 1;
+    PackedSlot<QB> slot(ld_chunk);
+    if constexpr (QBIT != 0) {
+        unpack8(ld16(m.s + ld_chunk * 8), sc);
+        if constexpr (ZP) unpack8(ld16(m.zp + ld_chunk * 8), zz);
+    }
+    // X of one step in chunk form
+    u32x4 xv[kCtSteps][4];
+    const int64_t x_pitch = QBIT == 0 ? 2 * (int64_t)N : (int64_t)N * QB / 8;
+    const char* x_base = (QBIT == 0 ? (const char*)m.x + 16 * (int64_t)ld_chunk : (const char*)m.q + slot.offset) + row0 * x_pitch;
+    auto load = [&](u32x4 (&dst)[4], int r0) {
+#pragma unroll
+        for (int vv = 0; vv < 4; ++vv) {
+            const int r = r0 + 4 * g + vv < rows ? r0 + 4 * g + vv : rows - 1;
+            const char* p = x_base + r * x_pitch;
+            if constexpr (QBIT == 0) {
+                dst[vv] = ld16(p);
+            } else {
+                const u32x2 w = ld8(p);
+                dst[vv].x = w.x;
+                dst[vv].y = w.y;
+            }
+        }
+    };
+#pragma unroll
+    for (int st = 0; st < kCtSteps; ++st) load(xv[st], 16 * st);
+
+    if constexpr (P1) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int k = 0; k < kCtMaxStrip / 32; ++k) {
+                uint16_t* p = ul + (nb * 16 + 2 * up) * kCtUPitch + 32 * k + ur;
+                const uint32_t w = 32 * k + ur < rows && 2 * up < a.live[b0 + nb] ? uw[nb][k] : 0u;
+                p[0] = (uint16_t)w;
+                p[kCtUPitch] = (uint16_t)(w >> 16);
+            }
+        __syncthreads();
+    }
+    u32x4 vop[P2 ? NB : 1][4];
+    if constexpr (P2) {
+        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;         // high or low halves of two dwords
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const auto& d = e[nb][s];
+                vop[nb][s] = m.v_transposed ? u32x4{__builtin_amdgcn_perm(d[1], d[0], sel), __builtin_amdgcn_perm(d[3], d[2], sel),
+                                                    __builtin_amdgcn_perm(d[5], d[4], sel), __builtin_amdgcn_perm(d[7], d[6], sel)}
+                                            : u32x4{d[0], d[1], d[2], d[3]};
+                if (!(j < a.live[b0 + nb] && c0 + 32 * s + 8 * g < N)) vop[nb][s] = u32x4{0, 0, 0, 0};
+            }
     }
 
-    for (int ct = 0; ct < a.tiles_per_group; ++ct) {
-        const int col_tile = group * a.tiles_per_group + ct;
-        const int c0 = col_tile * kCtTile;
-        if (c0 >= a.N) break;                                   // uniform over the workgroup
-        const int chunk = col_tile * (kCtTile / 8) + j;
-        const bool active = chunk < a.C;
-
-        // V operand of the column contraction: lane (r = 16nb + j, g), columns c0 + 16s + 4g .. +3
-        s16x4 vop[P2 ? NB : 1][8];
-        if constexpr (P2) {
-            if (a.v_transposed) {
-                // [N, R] layout: the four columns of an operand are R elements apart; all loads
-                // first, packing afterwards, so that they overlap
-                // (whole dwords, the wanted half picked afterwards: 16-bit loads into register halves
-                // would each wait for the one before)
-                uint32_t e[NB][8][4];
+    f32x4 acc1[P1 ? NB : 1][8];
+    if constexpr (P1) {
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    const int r = rb + 16 * nb + j;
+        for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-                    for (int s8 = 0; s8 < 8; ++s8) {
-                        const int col = c0 + 16 * s8 + 4 * g;
-                        const bool ok = r < a.R && col < a.N;
-                        const uint16_t* p = a.v + (ok ? (int64_t)col * a.R + (r & ~1) : 0);
+            for (int u8 = 0; u8 < 8; ++u8) acc1[nb][u8] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    int half = 0;                                               // of sum2: one barrier per 64 rows is enough with two
+    for (int base = 0; base < rows; base += kCtSub, half ^= 1) {
+        // two steps at a time, so that their chains through LDS and the matrix cores run side by side
 #pragma unroll
-                        for (int kk = 0; kk < 4; ++kk)
-                            e[nb][s8][kk] = ok ? *reinterpret_cast<const uint32_t*>(p + kk * a.R) : 0u;
-                    }
-                }
-                const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;     // high or low halves of two dwords
+        for (int s2 = 0; s2 < kCtSteps; s2 += 2) {
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                    for (int s8 = 0; s8 < 8; ++s8) {
-                        const u32x2 w = {__builtin_amdgcn_perm(e[nb][s8][1], e[nb][s8][0], sel),
-                                         __builtin_amdgcn_perm(e[nb][s8][3], e[nb][s8][2], sel)};
-                        vop[nb][s8] = __builtin_bit_cast(s16x4, w);
-                    }
-            } else {
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    const int r = rb + 16 * nb + j;
-#pragma unroll
-                    for (int s8 = 0; s8 < 8; ++s8) {
-                        const int col = c0 + 16 * s8 + 4 * g;
-                        u32x2 w = {0, 0};
-                        if (r < a.R && col < a.N) w = ld8(a.v + (int64_t)r * a.N + col);
-                        vop[nb][s8] = __builtin_bit_cast(s16x4, w);
-                    }
-                }
-            }
-        }
-        // per-column constants of the dequantiser
-        float sc[8], zz[8];
-        PackedSlot<QB> slot(chunk);
-        if constexpr (QBIT != 0) {
-            u32x4 sv = {0, 0, 0, 0}, zv = {0, 0, 0, 0};
-            if (active) sv = ld16(a.s + chunk * 8);
-            unpack8(sv, sc);
-            if constexpr (ZP) {
-                if (active) zv = ld16(a.zp + chunk * 8);
-            }
-            unpack8(zv, zz);
-        }
-
-        f32x4 acc1[P1 ? NB : 1][8];
-        if constexpr (P1) {
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                for (int u8 = 0; u8 < 8; ++u8) acc1[nb][u8] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        }
-
-        // every load of the tile is issued before the first MFMA: a wave sees the memory latency once
-        u32x4 xv[kCtSteps][4];
-        uint32_t uw[P1 ? kCtSteps : 1][NB][4];
-        {
-#pragma unroll
-            for (int st = 0; st < kCtSteps; ++st) {
-                const int64_t t0 = row_base + 16 * st;
-                // chunk form of the tile
-#pragma unroll
-                for (int vv = 0; vv < 4; ++vv) {
-                    const int64_t t = t0 + 4 * g + vv;
-                    xv[st][vv] = u32x4{0, 0, 0, 0};
-                    if (active && t < a.T) {
-                        if constexpr (QBIT == 0) {
-                            xv[st][vv] = ld16(a.x + t * a.N + chunk * 8);
-                        } else {
-                            const u32x2 w = ld8(a.q + t * row_bytes + slot.offset);
-                            xv[st][vv].x = w.x;
-                            xv[st][vv].y = w.y;
-                        }
-                    }
-                }
-                // U operand: lane (r = 16nb + j, g), rows t0 + 4g .. +3 (whole dwords, see above)
-#pragma unroll
-                for (int nb = 0; nb < (P1 ? NB : 0); ++nb) {
-                    const int r = rb + 16 * nb + j;
-#pragma unroll
-                    for (int kk = 0; kk < 4; ++kk) {
-                        const int64_t t = t0 + 4 * g + kk;
-                        const bool ok = r < a.R && t < a.T;
-                        uw[st][nb][kk] = ok ? *reinterpret_cast<const uint32_t*>(a.u + t * a.R + (r & ~1)) : 0u;
-                    }
-                }
-            }
-        }
-#pragma unroll
-        for (int st = 0; st < kCtSteps; ++st) {
-            if constexpr (P1) {
+            for (int st = s2; st < s2 + 2; ++st) {
+                const int r0 = base + 16 * st;
                 if constexpr (QBIT != 0) {
 #pragma unroll
                     for (int vv = 0; vv < 4; ++vv) {
-                        const bool live = active && row_base + 16 * st + 4 * g + vv < a.T;
                         float c[8], f[8];
                         slot.decode(u32x2{xv[st][vv].x, xv[st][vv].y}, c);
 #pragma unroll
@@ -233,181 +228,210 @@ __global__ __launch_bounds__(kCtThreads) void lora_contract_kernel(const Contrac
                             if constexpr (ZP) f[e] = rbf((c[e] - kHalf) - zz[e]) * sc[e];
                             else f[e] = (c[e] - kHalf) * sc[e];
                         }
-                        xv[st][vv] = live ? pack8(f) : u32x4{0, 0, 0, 0};
+                        xv[st][vv] = pack8(f);
                     }
                 }
-                s16x4 uop[NB];
-                const uint32_t usel = (j & 1) ? 0x07060302u : 0x05040100u;
+                if (!full || r0 + 16 > rows) {                  // uniform: rows and columns past the end count as zeros
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb) {
-                    const u32x2 pk = {__builtin_amdgcn_perm(uw[st][nb][1], uw[st][nb][0], usel),
-                                      __builtin_amdgcn_perm(uw[st][nb][3], uw[st][nb][2], usel)};
-                    uop[nb] = __builtin_bit_cast(s16x4, pk);
+                    for (int vv = 0; vv < 4; ++vv)
+                        if (!(active && r0 + 4 * g + vv < rows)) xv[st][vv] = u32x4{0, 0, 0, 0};
                 }
+                if constexpr (P2) {
+                    // to the row form through this wave's corner of LDS: read straight from memory it would be 16 rows x 64
+                    // bytes per load instruction
+                    uint16_t* tw = tr[wave] + (st - s2) * 16 * kCtPitch;
 #pragma unroll
-                for (int u8 = 0; u8 < 8; ++u8) {
-                    const s16x4 xop = pick_column(xv[st], u8);
-#pragma unroll
-                    for (int nb = 0; nb < NB; ++nb)
-                        acc1[nb][u8] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(uop[nb], xop, acc1[nb][u8], 0, 0, 0);
+                    for (int vv = 0; vv < 4; ++vv) *reinterpret_cast<u32x4*>(tw + (4 * g + vv) * kCtPitch + 8 * j) = xv[st][vv];
                 }
             }
             if constexpr (P2) {
-                // row form of the tile (lane (i = j, g): row i, columns 16s + 4g .. +3) through this
-                // wave's corner of LDS: read straight from memory it would be 16 rows x 32 bytes per
-                // load instruction
-                uint16_t* tw = tr[wave];
-#pragma unroll
-                for (int vv = 0; vv < 4; ++vv) *reinterpret_cast<u32x4*>(tw + (4 * g + vv) * kCtPitch + 8 * j) = xv[st][vv];
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
+            }
+            if constexpr (P1) {
 #pragma unroll
-                for (int s8 = 0; s8 < 8; ++s8) {
-                    const u32x2 w = *reinterpret_cast<const u32x2*>(tw + j * kCtPitch + 16 * s8 + 4 * g);
-                    const s16x4 xop = __builtin_bit_cast(s16x4, w);
+                for (int st = s2; st < s2 + 2; ++st) {
+                    s16x4 uop[NB];
 #pragma unroll
                     for (int nb = 0; nb < NB; ++nb)
-                        acc2[st][nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(xop, vop[nb][s8], acc2[st][nb], 0, 0, 0);
+                        uop[nb] = __builtin_bit_cast(s16x4, *reinterpret_cast<const u32x2*>(ul + (nb * 16 + j) * kCtUPitch + base + 16 * st + 4 * g));
+#pragma unroll
+                    for (int u8 = 0; u8 < 8; ++u8) {
+                        const s16x4 xop = pick_column(xv[st], u8);
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc1[nb][u8] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(uop[nb], xop, acc1[nb][u8], 0, 0, 0);
+                    }
                 }
+            }
+#pragma unroll
+            for (int st = s2; st < s2 + 2; ++st) load(xv[st], base + 16 * st + kCtSub);
+            if constexpr (P2) {
+                f32x4 acc2[2][NB];
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb) acc2[h][nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int s = 0; s < 4; ++s)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const bf16x8 xop = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(tr[wave] + (16 * h + j) * kCtPitch + 32 * s + 8 * g));
+#pragma unroll
+                        for (int nb = 0; nb < NB; ++nb)
+                            acc2[h][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xop, __builtin_bit_cast(bf16x8, vop[nb][s]), acc2[h][nb], 0, 0, 0);
+                    }
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+#pragma unroll
+                    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+                        for (int vv = 0; vv < 4; ++vv)
+                            sum2[half][((wave * kCtSub + 16 * (s2 + h) + 4 * g + vv) * NB + nb) * 16 + j] = acc2[h][nb][vv];
             }
         }
-
-        if constexpr (P1) {
-            // add the four waves' tiles in wave order and hand the strip's partial to memory
+        if constexpr (P2) {
+            // the waves' parts of 64 rows, added in wave order (zeros from a wave past the last column): thread t owns 4 ranks of
+            // NB (row, block) pairs
+            __syncthreads();
 #pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                __syncthreads();
+            for (int k = 0; k < NB; ++k) {
+                const int i = k * kCtThreads + threadIdx.x;
+                const int row = i / (4 * NB), nb = (i >> 2) % NB, r4 = (i & 3) * 4;
+                f32x4 s = *reinterpret_cast<const f32x4*>(sum2[half] + (row * NB + nb) * 16 + r4);
 #pragma unroll
-                for (int u8 = 0; u8 < 8; ++u8) {
-                    const f32x4 v4 = acc1[nb][u8];
-                    const float e[4] = {v4.x, v4.y, v4.z, v4.w};
-#pragma unroll
-                    for (int vv = 0; vv < 4; ++vv) red[(wave * 16 + 4 * g + vv) * kCtTile + 8 * j + u8] = e[vv];
-                }
-                __syncthreads();
-                // thread tid owns 8 consecutive columns of one LoRA row
-                const int tid = threadIdx.x;
-                const int r = tid >> 4, cc = (tid & 15) * 8;
-                if (c0 + cc < a.N) {
-                    float sum[8];
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) sum[e] = red[r * kCtTile + cc + e];
-#pragma unroll
-                    for (int w = 1; w < kCtWaves; ++w)
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) sum[e] += red[(w * 16 + r) * kCtTile + cc + e];
-                    float* dst = a.part1 + ((strip * rows_all + rb + 16 * nb + r) * (int64_t)a.N + c0 + cc);
-                    *reinterpret_cast<f32x4*>(dst) = f32x4{sum[0], sum[1], sum[2], sum[3]};
-                    *reinterpret_cast<f32x4*>(dst + 4) = f32x4{sum[4], sum[5], sum[6], sum[7]};
+                for (int w = 1; w < kCtWaves; ++w) s += *reinterpret_cast<const f32x4*>(sum2[half] + ((w * kCtSub + row) * NB + nb) * 16 + r4);
+                if (base + row < rows) {
+                    const int64_t t = row0 + base + row;
+                    if (m.part2) {
+                        *reinterpret_cast<f32x4*>(m.part2 + ((int64_t)cb * a.T + t) * (16 * a.blocks) + 16 * (b0 + nb) + r4) = s;
+                    } else {
+                        uint32_t* p = reinterpret_cast<uint32_t*>(m.p2[b0 + nb] + t * R + r4);
+                        if (r4 < a.live[b0 + nb]) p[0] = pk_bf16(s.x, s.y);
+                        if (r4 + 2 < a.live[b0 + nb]) p[1] = pk_bf16(s.z, s.w);
+                    }
                 }
             }
         }
     }
 
-    if constexpr (P2) {
+    if constexpr (P1) {
+        if (!active) return;
 #pragma unroll
-        for (int st = 0; st < kCtSteps; ++st)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb) {
-                const f32x4 v4 = acc2[st][nb];
-                const float e[4] = {v4.x, v4.y, v4.z, v4.w};
+        for (int nb = 0; nb < NB; ++nb) {
+            if (m.part1) {
 #pragma unroll
                 for (int vv = 0; vv < 4; ++vv) {
-                    const int64_t t = row_base + 16 * st + 4 * g + vv;
-                    if (t < a.T) a.part2[((int64_t)group * a.T + t) * rows_all + rb + 16 * nb + j] = e[vv];
+                    float* dst = m.part1 + (strip * (16 * a.blocks) + 16 * (b0 + nb) + 4 * g + vv) * (int64_t)N + chunk * 8;
+                    float e[8];
+#pragma unroll
+                    for (int u8 = 0; u8 < 8; ++u8) e[u8] = acc1[nb][u8][vv];
+                    *reinterpret_cast<f32x4*>(dst) = f32x4{e[0], e[1], e[2], e[3]};
+                    *reinterpret_cast<f32x4*>(dst + 4) = f32x4{e[4], e[5], e[6], e[7]};
+                }
+            } else if (m.p1_transposed) {
+#pragma unroll
+                for (int u8 = 0; u8 < 8; ++u8) {
+                    uint32_t* p = reinterpret_cast<uint32_t*>(m.p1[b0 + nb] + (int64_t)(chunk * 8 + u8) * R + 4 * g);
+                    const f32x4 s = acc1[nb][u8];
+                    if (4 * g < a.live[b0 + nb]) p[0] = pk_bf16(s.x, s.y);
+                    if (4 * g + 2 < a.live[b0 + nb]) p[1] = pk_bf16(s.z, s.w);
+                }
+            } else {
+#pragma unroll
+                for (int vv = 0; vv < 4; ++vv) {
+                    float e[8];
+#pragma unroll
+                    for (int u8 = 0; u8 < 8; ++u8) e[u8] = acc1[nb][u8][vv];
+                    uint32_t* p = reinterpret_cast<uint32_t*>(m.p1[b0 + nb] + (int64_t)(4 * g + vv) * N + chunk * 8);
+                    if (4 * g + vv < a.live[b0 + nb]) {
+#pragma unroll
+                        for (int h = 0; h < 4; ++h) p[h] = pk_bf16(e[2 * h], e[2 * h + 1]);
+                    }
                 }
             }
+        }
     }
-    }   // pass
 }
 
 // out[i][c] = bf16( sum_k part[k][i][c] ), i < rows_out, c < cols_out, partial planes of
-// [rows_part][cols_part] floats; two such reductions per launch (either may be empty).
+// [rows_part][cols_part] floats; up to six such reductions per launch.  Bound by latency: a block takes 64 vectors of W
+// floats and each of its waves a quarter of the planes, up to 8 loads in flight, and the quarters meet in LDS in
+// plane order (one thread for all planes of a vector: 6 us for 32 planes of [16, 4096], of which 4 waiting).
 struct ReduceJob {
     const float* part; uint16_t* out;
-    int64_t rows_out, rows_part;
+    int64_t rows_out, plane;                  // plane: floats from one plane to the next
     int cols_out, cols_part, planes;
-    int64_t blocks;
     int transposed;          // out is [cols_out][rows_out]: rows_out <= 64 and even, cols_out % 4 == 0
+    int64_t first_block;
 };
-constexpr int kReduceTCols = 64;     // columns a block of the transposed form owns (all rows of them)
-
-// out[c][i] = bf16( sum_k part[k][i][c] ): the sums of kReduceTCols columns x all rows meet in LDS and leave as
-// one contiguous run of the transposed output.  Planes are added in index order, as in the plain form, so
-// the values are the plain form's.
-__device__ __forceinline__ void reduce_transposed(const ReduceJob& jb, int64_t blk) {
-    __shared__ uint16_t tile[kReduceTCols * 64];
-    const int c4 = threadIdx.x & 15, r0 = threadIdx.x >> 4;
-    const int64_t c0 = blk * kReduceTCols;
-    const int64_t c = c0 + 4 * c4;
-    const int rows = (int)jb.rows_out;
-    const int64_t plane = jb.rows_part * (int64_t)jb.cols_part;
-    if (c < jb.cols_out) {
-        for (int r = r0; r < rows; r += 16) {
-            const float* p = jb.part + (int64_t)r * jb.cols_part + c;
-            f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
-            int k = 0;
-            for (; k + 4 <= jb.planes; k += 4) {
-                f32x4 v[4];
-#pragma unroll
-                for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const f32x4*>(p + (k + u) * plane);
-#pragma unroll
-                for (int u = 0; u < 4; ++u) sum += v[u];
-            }
-            for (; k < jb.planes; ++k) sum += *reinterpret_cast<const f32x4*>(p + k * plane);
-            const uint32_t lo = pk_bf16(sum.x, sum.y), hi = pk_bf16(sum.z, sum.w);
-            tile[(4 * c4 + 0) * rows + r] = (uint16_t)lo;
-            tile[(4 * c4 + 1) * rows + r] = (uint16_t)(lo >> 16);
-            tile[(4 * c4 + 2) * rows + r] = (uint16_t)hi;
-            tile[(4 * c4 + 3) * rows + r] = (uint16_t)(hi >> 16);
-        }
-    }
-    __syncthreads();
-    const int64_t cols_here = jb.cols_out - c0 < kReduceTCols ? jb.cols_out - c0 : kReduceTCols;
-    const int n_pairs = (int)(cols_here * rows / 2);
-    uint32_t* out = reinterpret_cast<uint32_t*>(jb.out + c0 * rows);
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(tile);
-    for (int i = threadIdx.x; i < n_pairs; i += 256) out[i] = src[i];
-}
-
-// A thread owns W neighbouring outputs of one row (cols_out % W == 0) and reads one W-wide vector
-// per plane; planes are added in index order.
+constexpr int kReduceJobs = 2 * kCtMembers;
+struct ReduceArgs { ReduceJob j[kReduceJobs]; int jobs; };
+constexpr int kReduceWaves = 4;
 template <int W>
-__global__ __launch_bounds__(256) void contract_reduce_kernel(const ReduceJob j0, const ReduceJob j1) {
+__global__ __launch_bounds__(256) void contract_reduce_kernel(const ReduceArgs a) {
     typedef float fvec __attribute__((ext_vector_type(W)));
-    const bool second = (int64_t)blockIdx.x >= j0.blocks;
-    const ReduceJob& jb = second ? j1 : j0;
-    const int64_t blk = second ? blockIdx.x - j0.blocks : blockIdx.x;
-    if (jb.transposed) {                  // the same for every thread of the block
-        reduce_transposed(jb, blk);
-        return;
-    }
-    const int64_t n_out = jb.rows_out * jb.cols_out;
-    const int64_t idx = (blk * 256 + threadIdx.x) * W;
-    if (idx >= n_out) return;
-    const int64_t plane = jb.rows_part * (int64_t)jb.cols_part;
-    const int64_t i = idx / jb.cols_out;
-    const float* p = jb.part + i * jb.cols_part + (idx - i * jb.cols_out);
+    __shared__ __attribute__((aligned(16))) float quarter[kReduceWaves][kWave * W];
+    int ji = 0;
+    for (int k = 1; k < a.jobs; ++k) ji += (int64_t)blockIdx.x >= a.j[k].first_block ? 1 : 0;
+    const ReduceJob& jb = a.j[ji];
+    const int64_t blk = blockIdx.x - jb.first_block;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    // a block's vectors: 64 in a row, or (transposed) W columns x 16 lanes of 4 rows
+    const uint32_t col_groups = (uint32_t)(jb.cols_out + 16 * W - 1) / (16 * W);
+    const uint32_t tr4 = (uint32_t)blk / col_groups;
+    const int64_t tr0 = (int64_t)tr4 * 4, tc0 = (int64_t)((uint32_t)blk - tr4 * col_groups) * (16 * W);
+    const int64_t idx = (blk * kWave + lane) * W;             // cols_out % W == 0: a vector lies in one row
+    // (a 64-bit division takes longer than the loads)
+    const bool small = jb.rows_out * jb.cols_out <= UINT32_MAX;
+    const int64_t row = jb.transposed ? tr0 + (lane >> 4) : small ? (int64_t)((uint32_t)idx / (uint32_t)jb.cols_out) : idx / jb.cols_out;
+    const int64_t col = jb.transposed ? tc0 + (lane & 15) * W : idx - row * jb.cols_out;
+    const bool valid = row < jb.rows_out && col < jb.cols_out;
+    // a wave's share is a run of planes, eight of them in flight
+    const float* p = jb.part + row * jb.cols_part + col;
+    const int share = (jb.planes + kReduceWaves - 1) / kReduceWaves;
+    const int k0 = wave * share, k1 = k0 + share < jb.planes ? k0 + share : jb.planes;
     float sum[W];
 #pragma unroll
     for (int e = 0; e < W; ++e) sum[e] = 0.0f;
-    int k = 0;
-    for (; k + 4 <= jb.planes; k += 4) {                    // four planes in flight
-        fvec v[4];
+    if (valid)
+        for (int k = k0; k < k1; k += 8) {
+            fvec v[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const fvec*>(p + (k + u) * plane);
+            for (int u = 0; u < 8; ++u) v[u] = *reinterpret_cast<const fvec*>(p + (k + u < k1 ? k + u : k1 - 1) * jb.plane);
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < 8; ++u)
 #pragma unroll
-            for (int e = 0; e < W; ++e) sum[e] += v[u][e];
+                for (int e = 0; e < W; ++e) sum[e] += k + u < k1 ? v[u][e] : 0.0f;
+        }
+#pragma unroll
+    for (int e = 0; e < W; ++e) quarter[wave][lane * W + e] = sum[e];
+    __syncthreads();
+    if (wave != 0) return;
+    if (jb.transposed) {
+        // lane = a column, whose 4 ranks leave together
+        for (int c = lane; c < 16 * W; c += kWave) {
+            if (tc0 + c >= jb.cols_out) continue;
+            float t[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                t[r] = quarter[0][r * 16 * W + c];
+#pragma unroll
+                for (int w = 1; w < kReduceWaves; ++w) t[r] += quarter[w][r * 16 * W + c];
+            }
+            uint32_t* out = reinterpret_cast<uint32_t*>(jb.out + (tc0 + c) * jb.rows_out + tr0);
+            out[0] = pk_bf16(t[0], t[1]);
+            if (tr0 + 2 < jb.rows_out) out[1] = pk_bf16(t[2], t[3]);
+        }
+        return;
     }
-    for (; k < jb.planes; ++k) {
-        const fvec v = *reinterpret_cast<const fvec*>(p + k * plane);
+    if (!valid) return;
 #pragma unroll
-        for (int e = 0; e < W; ++e) sum[e] += v[e];
-    }
+    for (int w = 1; w < kReduceWaves; ++w)
+#pragma unroll
+        for (int e = 0; e < W; ++e) sum[e] += quarter[w][lane * W + e];
     uint32_t* out = reinterpret_cast<uint32_t*>(jb.out + idx);
 #pragma unroll
     for (int e = 0; e < W; e += 2) out[e / 2] = pk_bf16(sum[e], sum[e + 1]);
@@ -415,26 +439,28 @@ __global__ __launch_bounds__(256) void contract_reduce_kernel(const ReduceJob j0
 
 // ------------------------------------------------------------------------------------
 template <int QBIT, bool ZP, bool P1, bool P2>
-static void contract_launch_nb(ContractArgs a, dim3 grid, int nb, hipStream_t st) {
-    // nb = rank blocks of 16.  One or two are held at once; three run as three passes of one, four as
-    // two passes of two (measured on [4096, 11008], both products: 101 and 109 us against 120 and 279 us
-    // for kernels that held three or four blocks at once and spilled).
+static void contract_launch(const ContractArgs& a, int64_t wgs, hipStream_t st) {
+    // rank blocks held at once: all of up to three, two of four; both products of three take one at a time
     const dim3 block(kCtThreads);
-    a.passes = nb <= 2 ? 1 : (nb == 3 ? 3 : 2);
+    const int nb = a.blocks == 4 ? 2 : (P1 && P2 && a.blocks == 3 ? 1 : a.blocks);
+    const dim3 grid((unsigned)wgs, (unsigned)(a.blocks / nb));
     if (nb == 1) hipLaunchKernelGGL((lora_contract_kernel<QBIT, ZP, P1, P2, 1>), grid, block, 0, st, a);
     else if (nb == 2) hipLaunchKernelGGL((lora_contract_kernel<QBIT, ZP, P1, P2, 2>), grid, block, 0, st, a);
-    else if (nb == 3) hipLaunchKernelGGL((lora_contract_kernel<QBIT, ZP, P1, P2, 1, true>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((lora_contract_kernel<QBIT, ZP, P1, P2, 2, true>), grid, block, 0, st, a);
+    else if constexpr (!(P1 && P2)) hipLaunchKernelGGL((lora_contract_kernel<QBIT, ZP, P1, P2, 3>), grid, block, 0, st, a);
 }
 
-static int64_t contract_geometry(int64_t T, int64_t N, int64_t R, int* tiles_per_group, int* groups, int64_t* strips,
-                                 int* nb) {
-    const int64_t tiles = cdiv(N, kCtTile);
-    *tiles_per_group = (int)cdiv(tiles, g_ct_max_groups.get());
-    *groups = (int)cdiv(tiles, *tiles_per_group);
-    *strips = cdiv(T, kCtStrip);
-    *nb = (int)cdiv(R, 16);
-    return 0;
+// Rows of a strip: 256 where that leaves 160 workgroups and more or is all there is, else 128.  Fewer strips are fewer planes of P1 (2 x
+// 16 N x 4 bytes each), more strips more units at work: both products at 128 and 256 rows [T, N], us: [4096, 11008] 32.1 / 30.2 (352
+// workgroups at 256), [2040, 13824] 22.5 / 20.3 (216), [2048, 11008] 21.0 / 18.2 (176), [4096, 4096] 16.6 / 17.2 (128), [2040, 5120] 15.5 /
+// 16.3 (80), [2048, 4096] 14.9 / 16.0 (64).  It depends on T and N alone, so that the sums are in one order whatever else is in the
+// launch and whatever X is read from.
+// Without P1 a strip leaves nothing behind, and 64 rows are the fastest at every shape measured ([4096, 11008] 24.5 against 26.5 at 256,
+// [512, 4096] 7.6 against 11.4).
+static int strip_rows(int64_t T, int64_t N, bool want1) {
+    const int fixed = g_ct_strip.get();
+    if (fixed) return fixed;
+    if (!want1) return kCtSub;
+    return T <= kCtMaxStrip || cdiv(T, kCtMaxStrip) * cdiv(N, kCtBlock) >= 160 ? kCtMaxStrip : 128;
 }
 
 int tune_contract(const char* key, int value) {
@@ -443,7 +469,114 @@ int tune_contract(const char* key, int value) {
         g_ct_max_groups.set(value);
         return HYC_OK;
     }
+    if (strcmp(key, "contract_strip_rows") == 0) {
+        if (value < 0 || value > kCtMaxStrip || value % kCtSub) return HYC_ERR_ARG;
+        g_ct_strip.set(value);
+        return HYC_OK;
+    }
     return 1;
+}
+
+// `count` products of X's of their own, or (`shared`) of the X of the first; one rank R for all, up to 16 where there are several
+static int contract_jobs(const hyc_contract_job* jobs, int count, bool shared, int q_bit, void* workspace, int64_t workspace_bytes,
+                         int64_t T, int64_t R, hipStream_t st) {
+    const hyc_contract_job& h = jobs[0];
+    const bool codes = h.q != nullptr, want1 = h.p1 != nullptr, want2 = h.p2 != nullptr;
+    if (codes && q_bit != 2 && q_bit != 4 && q_bit != 8) return HYC_ERR_QBIT;
+    if (T < 0 || T > ((int64_t)1 << 40)) return HYC_ERR_SHAPE;
+    if (R < 2 || R > 64 || R % 2 != 0 || (count > 1 && R > 16)) return HYC_ERR_RANK;
+    if (!want1 && !want2) return HYC_ERR_NULL;
+    for (int i = 0; i < count; ++i) {
+        const hyc_contract_job& jb = jobs[i];
+        if (jb.N < 0 || jb.N % 32 != 0 || jb.N > (1 << 28)) return HYC_ERR_SHAPE;
+        if ((jb.p1 != nullptr) != want1 || (jb.p2 != nullptr) != want2 || (want1 && !jb.u) || (want2 && !jb.v)) return HYC_ERR_NULL;
+        if (i && shared && (jb.N != h.N || jb.v_transposed != h.v_transposed || jb.p1_transposed != h.p1_transposed)) return HYC_ERR_ARG;
+        if (i == 0 || !shared) {
+            if (codes ? (jb.x != nullptr || !jb.q || !jb.scale || want2 || (jb.zero_point != nullptr) != (h.zero_point != nullptr))
+                      : (jb.x == nullptr || jb.q != nullptr))
+                return HYC_ERR_ARG;
+        }
+    }
+    if (!workspace) return HYC_ERR_NULL;
+    for (int i = 0; i < count; ++i)
+        if (T * jobs[i].N == 0) {
+            if (count == 1) return HYC_OK;
+            return HYC_ERR_SHAPE;
+        }
+    auto off = [](const void* p, uintptr_t by) { return p && (reinterpret_cast<uintptr_t>(p) & (by - 1)) != 0; };
+    for (int i = 0; i < count; ++i) {
+        const hyc_contract_job& jb = jobs[i];
+        if (off(jb.x, 16) || off(jb.scale, 16) || off(jb.zero_point, 16) || off(jb.q, 8) || off(jb.v, 8) || off(jb.u, 4) || off(jb.p1, 4) ||
+            off(jb.p2, 4))
+            return HYC_ERR_ALIGN;
+    }
+    if (!aligned16(workspace)) return HYC_ERR_ALIGN;
+
+    ContractArgs a{};
+    ReduceArgs ra{};
+    a.T = T; a.R = (int)R; a.members = shared ? 1 : count;
+    a.blocks = shared ? count : (int)cdiv(R, 16);
+    for (int b = 0; b < 4; ++b) a.live[b] = shared ? (int)R : (int)std::min<int64_t>(16, std::max<int64_t>(0, R - 16 * b));
+    const int64_t rows16 = 16 * a.blocks;
+    char* ws = (char*)workspace;
+    int64_t used = 0, wgs = 0, rblocks = 0;
+    const int w = (want2 && R % 4 != 0) ? 2 : 4;             // N % 32 == 0; R is even
+    auto reduce = [&](const float* part, uint16_t* out, int64_t rows_out, int64_t plane, int64_t cols_out, int64_t cols_part, int64_t planes, int transposed) {
+        ReduceJob& jb = ra.j[ra.jobs++];
+        jb.part = part; jb.out = out; jb.rows_out = rows_out; jb.plane = plane; jb.cols_out = (int)cols_out; jb.cols_part = (int)cols_part;
+        jb.planes = (int)planes; jb.transposed = transposed; jb.first_block = rblocks;
+        rblocks += transposed ? cdiv(rows_out, 4) * cdiv(cols_out, 16 * w) : cdiv(rows_out * cols_out, kWave * w);
+    };
+    for (int i = 0; i < a.members; ++i) {
+        const hyc_contract_job& jb = jobs[i];
+        ContractMember& m = a.m[i];
+        m.x = (const uint16_t*)jb.x; m.q = (const uint8_t*)jb.q; m.s = (const uint16_t*)jb.scale; m.zp = (const uint16_t*)jb.zero_point;
+        m.N = (int)jb.N; m.C = (int)(jb.N / 8); m.v_transposed = jb.v_transposed; m.p1_transposed = jb.p1_transposed;
+        m.col_blocks = (int)cdiv(jb.N, kCtBlock);
+        m.strip_rows = strip_rows(T, jb.N, want1);
+        const int64_t strips = cdiv(T, m.strip_rows);
+        m.first_wg = (uint32_t)wgs;
+        wgs += strips * m.col_blocks;
+        if (want1 && strips > 1) { m.part1 = (float*)(ws + used); used += strips * rows16 * jb.N * 4; }
+        if (want2 && m.col_blocks > 1) { m.part2 = (float*)(ws + used); used += (int64_t)m.col_blocks * T * rows16 * 4; }
+        for (int b = 0; b < a.blocks; ++b) {
+            const hyc_contract_job& from = shared ? jobs[b] : jb;
+            const int64_t r = shared ? 0 : 16 * b;           // first rank of the block in its operands
+            if (from.u) m.u[b] = (const uint16_t*)from.u + r;
+            if (from.v) m.v[b] = (const uint16_t*)from.v + (from.v_transposed ? r : r * jb.N);
+            if (from.p1) m.p1[b] = (uint16_t*)from.p1 + (from.p1_transposed ? r : r * jb.N);
+            if (from.p2) m.p2[b] = (uint16_t*)from.p2 + r;
+        }
+        for (int b = 0; b < (shared ? count : 1); ++b) {     // the ranks of one result lie together, whatever blocks they were formed in
+            if (m.part1) reduce(m.part1 + 16 * b * jb.N, (uint16_t*)jobs[shared ? b : i].p1, R, rows16 * jb.N, jb.N, jb.N, strips, jb.p1_transposed);
+            if (m.part2) reduce(m.part2 + 16 * b, (uint16_t*)jobs[shared ? b : i].p2, T, T * rows16, R, rows16, m.col_blocks, 0);
+        }
+    }
+    if (workspace_bytes < used) return HYC_ERR_ARG;
+    if (wgs > INT32_MAX || rblocks > INT32_MAX) return HYC_ERR_SHAPE;
+    if (codes) {
+        const bool zp = h.zero_point != nullptr;
+#define HYC_CT_CODES(QB)                                                        \
+        do {                                                                    \
+            if (zp) contract_launch<QB, true, true, false>(a, wgs, st);         \
+            else contract_launch<QB, false, true, false>(a, wgs, st);           \
+        } while (0)
+        if (q_bit == 8) HYC_CT_CODES(8);
+        else if (q_bit == 4) HYC_CT_CODES(4);
+        else HYC_CT_CODES(2);
+#undef HYC_CT_CODES
+    } else if (want1 && want2) {
+        contract_launch<0, false, true, true>(a, wgs, st);
+    } else if (want1) {
+        contract_launch<0, false, true, false>(a, wgs, st);
+    } else {
+        contract_launch<0, false, false, true>(a, wgs, st);
+    }
+    if (ra.jobs == 0) return check_launch();
+    if (hipGetLastError() != hipSuccess) return HYC_ERR_LAUNCH;
+    if (w == 4) hipLaunchKernelGGL(contract_reduce_kernel<4>, dim3((unsigned)rblocks), dim3(256), 0, st, ra);
+    else hipLaunchKernelGGL(contract_reduce_kernel<2>, dim3((unsigned)rblocks), dim3(256), 0, st, ra);
+    return check_launch();
 }
 
 }  // namespace hyc
@@ -452,12 +585,10 @@ using namespace hyc;
 
 extern "C" int64_t hyc_lora_contract_workspace(int64_t T, int64_t N, int64_t R, int want_p1, int want_p2) {
     if (T <= 0 || N <= 0 || R < 2 || R > 64) return 0;
-    int tpg, groups, nb;
-    int64_t strips;
-    contract_geometry(T, N, R, &tpg, &groups, &strips, &nb);
+    const int64_t strips = cdiv(T, strip_rows(T, N, want_p1 != 0)), cols = cdiv(N, kCtBlock), rows16 = 16 * cdiv(R, 16);
     int64_t bytes = 0;
-    if (want_p1) bytes += strips * 16 * nb * N * 4;
-    if (want_p2) bytes += (int64_t)groups * T * 16 * nb * 4;
+    if (want_p1 && strips > 1) bytes += strips * rows16 * N * 4;
+    if (want_p2 && cols > 1) bytes += cols * T * rows16 * 4;
     return bytes;
 }
 
@@ -465,76 +596,13 @@ extern "C" int hyc_lora_contract(const void* x, const void* q, const void* scale
                                  const void* u, const void* v, int v_transposed, void* p1, int p1_transposed, void* p2,
                                  void* workspace, int64_t workspace_bytes, int64_t T, int64_t N, int64_t R,
                                  void* stream) {
-    const bool codes = q != nullptr;
-    const bool want1 = p1 != nullptr, want2 = p2 != nullptr;
-    if (codes && q_bit != 2 && q_bit != 4 && q_bit != 8) return HYC_ERR_QBIT;
-    if (T < 0 || N < 0 || N % 32 != 0 || N > (1 << 28) || T > ((int64_t)1 << 40)) return HYC_ERR_SHAPE;
-    if (R < 2 || R > 64 || R % 2 != 0) return HYC_ERR_RANK;
-    if (!want1 && !want2) return HYC_ERR_NULL;
-    if (codes ? (x != nullptr || !scale || want2) : (x == nullptr)) return HYC_ERR_ARG;
-    if ((want1 && !u) || (want2 && !v) || !workspace) return HYC_ERR_NULL;
-    if (T * N == 0) return HYC_OK;
-    if ((x && !aligned16(x)) || (scale && !aligned16(scale)) || (zero_point && !aligned16(zero_point)) ||
-        (q && (reinterpret_cast<uintptr_t>(q) & 7u)) || (v && (reinterpret_cast<uintptr_t>(v) & 7u)) ||
-        (reinterpret_cast<uintptr_t>(u) & 3u) || !aligned16(workspace) ||
-        (p1 && (reinterpret_cast<uintptr_t>(p1) & 3u)) || (p2 && (reinterpret_cast<uintptr_t>(p2) & 3u)))
-        return HYC_ERR_ALIGN;
-    if (v && !v_transposed && ((N * 2) % 8 != 0)) return HYC_ERR_ALIGN;
-    ContractArgs a{};
-    a.x = (const uint16_t*)x; a.q = (const uint8_t*)q; a.s = (const uint16_t*)scale; a.zp = (const uint16_t*)zero_point;
-    a.u = (const uint16_t*)u; a.v = (const uint16_t*)v; a.v_transposed = v_transposed;
-    a.T = T; a.N = (int)N; a.C = (int)(N / 8); a.R = (int)R;
-    int nb;
-    int64_t strips;
-    contract_geometry(T, N, R, &a.tiles_per_group, &a.groups, &strips, &nb);
-    const int64_t bytes1 = want1 ? strips * 16 * nb * N * 4 : 0;
-    const int64_t bytes2 = want2 ? (int64_t)a.groups * T * 16 * nb * 4 : 0;
-    if (workspace_bytes < bytes1 + bytes2) return HYC_ERR_ARG;
-    a.part1 = (float*)workspace;
-    a.part2 = (float*)((char*)workspace + bytes1);
-    a.n_blocks = strips * a.groups;
-    const int64_t pad = codes ? 8 * (8 / q_bit) : 1;            // see the block-index permutation in the kernel
-    if (cdiv(a.n_blocks, pad) * pad > INT32_MAX) return HYC_ERR_SHAPE;
-    const dim3 grid((unsigned)(cdiv(a.n_blocks, pad) * pad));
-    hipStream_t st = (hipStream_t)stream;
-    if (codes) {
-        const bool zp = zero_point != nullptr;
-#define HYC_CT_CODES(QB)                                                                   \
-        do {                                                                               \
-            if (zp) contract_launch_nb<QB, true, true, false>(a, grid, nb, st);            \
-            else contract_launch_nb<QB, false, true, false>(a, grid, nb, st);              \
-        } while (0)
-        if (q_bit == 8) HYC_CT_CODES(8);
-        else if (q_bit == 4) HYC_CT_CODES(4);
-        else HYC_CT_CODES(2);
-#undef HYC_CT_CODES
-    } else if (want1 && want2) {
-        contract_launch_nb<0, false, true, true>(a, grid, nb, st);
-    } else if (want1) {
-        contract_launch_nb<0, false, true, false>(a, grid, nb, st);
-    } else {
-        contract_launch_nb<0, false, false, true>(a, grid, nb, st);
-    }
-    if (hipGetLastError() != hipSuccess) return HYC_ERR_LAUNCH;
-    ReduceJob j1{}, j2{};
-    const int w = (want2 && R % 4 != 0) ? 2 : 4;             // N % 32 == 0; R is even
-    if (want1) {
-        j1.part = a.part1; j1.out = (uint16_t*)p1; j1.rows_out = R; j1.rows_part = 16 * nb;
-        j1.cols_out = (int)N; j1.cols_part = (int)N; j1.planes = (int)strips;
-        j1.blocks = cdiv(R * N, 256 * w);
-        if (p1_transposed) {
-            j1.transposed = 1;
-            j1.blocks = cdiv(N, kReduceTCols);
-        }
-    }
-    if (want2) {
-        j2.part = a.part2; j2.out = (uint16_t*)p2; j2.rows_out = T; j2.rows_part = T;
-        j2.cols_out = (int)R; j2.cols_part = 16 * nb; j2.planes = a.groups;
-        j2.blocks = cdiv(T * R, 256 * w);
-    }
-    if (j1.blocks + j2.blocks > INT32_MAX) return HYC_ERR_SHAPE;
-    const dim3 rgrid((unsigned)(j1.blocks + j2.blocks));
-    if (w == 4) hipLaunchKernelGGL(contract_reduce_kernel<4>, rgrid, dim3(256), 0, st, j1, j2);
-    else hipLaunchKernelGGL(contract_reduce_kernel<2>, rgrid, dim3(256), 0, st, j1, j2);
-    return check_launch();
+    const hyc_contract_job job = {x, q, scale, zero_point, u, v, p1, p2, N, v_transposed, p1_transposed};
+    return contract_jobs(&job, 1, false, q_bit, workspace, workspace_bytes, T, R, (hipStream_t)stream);
+}
+
+extern "C" int hyc_lora_contract_group(const hyc_contract_job* jobs, int count, int shared, int q_bit, void* workspace,
+                                       int64_t workspace_bytes, int64_t T, int64_t R, void* stream) {
+    if (!jobs) return HYC_ERR_NULL;
+    if (count < 1 || count > kCtMembers) return HYC_ERR_ARG;
+    return contract_jobs(jobs, count, shared != 0 && count > 1, q_bit, workspace, workspace_bytes, T, R, (hipStream_t)stream);
 }

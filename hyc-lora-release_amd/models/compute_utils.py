@@ -160,6 +160,28 @@ def lora_backward(w, w_quant_state, w_lora_a, w_lora_b, x, x_lora_a, grad_y, x_c
     return grad_a, grad_b, grad_x
 
 
+def lora_backward_shared(members, x, x_codes=None):
+    """lora_backward(..., defer_input=True) of two or three projections that share their input x, given like there:
+    members [(w, w_quant_state, w_lora_a, w_lora_b, x_lora_a, grad_y), ...] -> the list of its results, the same bits.
+    The rank-R products of all members take two launches and their reductions, and x (or its codes) is read once; the
+    weights are dequantised one at a time."""
+    out = None
+    if x_codes is None or x_codes[2] is None or x_codes[2].dtype == torch.bfloat16:
+        q, scale, zero_point, q_bit = x_codes or (None, None, None, 0)
+        if all(gy.is_cuda and (w.dtype if qs is None else getattr(qs, "dtype", torch.bfloat16)) == torch.bfloat16 for w, qs, _, _, _, gy in members):
+            out = _lib.native().lora_products_shared([(la, lb, xa, gy) for _, _, la, lb, xa, gy in members], None if x_codes else x, q, scale,
+                                                     zero_point, q_bit)
+    if out is None:
+        return [lora_backward(w, qs, la, lb, x, xa, gy, x_codes=x_codes, defer_input=True) for w, qs, la, lb, xa, gy in members]
+    results = []
+    for (w, qs, la, _, _, gy), (grad_a, grad_b, grad_mid) in zip(members, out):
+        wd = dense_weight(w, qs)
+        grad_x = _lib.native().frozen_input_grad(gy, wd)
+        results.append((grad_a, grad_b, (frozen_matmul(gy, wd) if grad_x is None else grad_x, grad_mid, la.mT)))
+        del wd
+    return results
+
+
 def lora_input_sum(parts):
     """Sum of the input gradients of projections that share their input, from the deferred terms lora_backward
     returns: acc = t_0; acc += t_1; ... with t_i = (grad_y @ W)_i + (grad_y @ B^T)_i @ A_i^T, every operation

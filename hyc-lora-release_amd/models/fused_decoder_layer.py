@@ -63,8 +63,8 @@ from ..operators import lora_kernels
 from ..operators._fuse import fuse_backward
 from ..operators.flash_kernels import flash_backward, flash_forward, flash_supported
 from ..operators.map_kernels import MapAttention, map_backward, map_backward_supported, map_supported
-from .compute_utils import (frozen_matmul, head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum, lora_parts,
-                            repeat_kv, repeat_kv_backward, rope_backward, rope_forward)
+from .compute_utils import (frozen_matmul, head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_backward_shared, lora_forward,
+                            lora_input_sum, lora_parts, repeat_kv, repeat_kv_backward, rope_backward, rope_forward)
 
 MODES = ("baseline", "intra", "intra_inter", "intra_inter_full_fuse")
 # Map-free attention keeps the flash kernel's row log-sum-exps for backward, whose kernel is then
@@ -490,21 +490,34 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                                                                     q_bit, **kw)
             return decompression_dequantization(S[name + "_q"], S[name + "_s"], q_bit, **kw)
 
-        def back(name, inp, inp_lora_a, grad_y, accumulate=None, defer_input=False):
-            """Backward of projection `name`.  `inp` is its input, or the name under which the layer
-            saved that input: a compressed one is then read from its codes, not dequantised.  With
-            `defer_input` the input gradient comes back as its terms, for lora_input_sum."""
+        def stored_input(inp):
+            """(x, codes) of an input given as a tensor or by the name under which the layer saved it: a compressed one is
+            then read from its codes, not dequantised."""
+            if not isinstance(inp, str):
+                return inp, None
+            if inp + "_raw" in S:
+                return S[inp + "_raw"], None
+            return None, (S[inp + "_q"], S[inp + "_s"], S.get(inp + "_z"), q_bit)
+
+        def back(name, inp, inp_lora_a, grad_y):
+            """Backward of projection `name`."""
             w, _, qs, la, lb = W[name]
-            codes = None
-            if isinstance(inp, str):
-                if inp + "_raw" in S:
-                    inp = S[inp + "_raw"]
-                else:
-                    codes, inp = (S[inp + "_q"], S[inp + "_s"], S.get(inp + "_z"), q_bit), None
-            ga, gb, gx = lora_backward(w, qs, la, lb, inp, inp_lora_a, grad_y, x_codes=codes, accumulate=accumulate,
-                                       defer_input=defer_input)
+            x, codes = stored_input(inp)
+            ga, gb, gx = lora_backward(w, qs, la, lb, x, inp_lora_a, grad_y, x_codes=codes)
             G[name] = (ga, gb)
             return gx
+
+        def back_shared(grads, inp):
+            """Backward of projections that share the input `inp`: {name: gradient of its output} -> the sum of their
+            input gradients (`grad_x += grad_x_temp`), added up in one pass."""
+            x, codes = stored_input(inp)
+            members = [(W[n][0], W[n][2], W[n][3], W[n][4], S[n + "_lora_a"], g) for n, g in grads.items()]
+            terms = []
+            for n, (ga, gb, term) in zip(grads, lora_backward_shared(members, x, codes)):
+                G[n] = (ga, gb)
+                terms.append(term)
+            del members
+            return lora_input_sum(terms)
 
         def rebuilt_hidden_group(names, rotate=()):
             """Outputs of projections `names` as forward produced them, from the codes of their frozen parts
@@ -609,9 +622,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 grad_fn = silu_backward(gate, grad_h1)
                 del grad_h1
             del grad_down, up, fn, gate
-        # gate and up share their input: their input gradients are added up in one pass (`grad_x += grad_x_temp`)
-        grad_x2 = lora_input_sum([back("gate", "x_norm_2", S["gate_lora_a"], grad_fn, defer_input=True),
-                                  back("up", "x_norm_2", S["up_lora_a"], grad_h2, defer_input=True)])
+        grad_x2 = back_shared({"gate": grad_fn, "up": grad_h2}, "x_norm_2")
         del grad_fn, grad_h2
         grad_medium, grad_nw2 = norm_backward(grad_x2, "x_medium", norm_weight_2, S["rstd_2"], ctx.norm_grads[1], grad_output)
         del grad_x2
@@ -690,9 +701,7 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
         grad_k = rope_backward(grad_k.transpose(1, 2), cos, sin).transpose(1, 2)
         grad_q, grad_k, grad_v = (head_to_hidden_shape(t) for t in (grad_q, grad_k, grad_v))
 
-        grad_x = lora_input_sum([back("q", "x_norm_1", S["q_lora_a"], grad_q, defer_input=True),
-                                 back("k", "x_norm_1", S["k_lora_a"], grad_k, defer_input=True),
-                                 back("v", "x_norm_1", S["v_lora_a"], grad_v, defer_input=True)])
+        grad_x = back_shared({"q": grad_q, "k": grad_k, "v": grad_v}, "x_norm_1")
         del grad_q, grad_k, grad_v
         as_reference = spec.reference_outlier_list and spec.mode in ("intra_inter", "intra_inter_full_fuse")
         grad_input, grad_nw1 = norm_backward(grad_x, "x", norm_weight_1, S["rstd_1"], ctx.norm_grads[0], grad_medium,

@@ -23,7 +23,7 @@ from ...operators.gelu_kernels import gelu_backward
 from ...operators.layernorm_kernels import layernorm_backward, layernorm_forward
 from ...operators.softmax_kernels import softmax_backward, softmax_backward_from_compressed, softmax_forward
 from ...operators import lora_kernels
-from ..compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_forward, lora_input_sum,
+from ..compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_backward_shared, lora_forward, lora_input_sum,
                             lora_parts)
 from ...operators.map_kernels import MapAttention, map_backward, map_backward_supported, map_supported
 from ..fused_decoder_layer import _note_map_entries, check_map_entries, keep_map_entries, lora_linear_parts
@@ -224,18 +224,20 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
             return outlier_addition_fuse_decompression_dequantization(S[name + "_q"], S[name + "_s"], S[name + "_o"],
                                                                       S[name + "_idx"], q_bit)
 
-        def back(name, inp, inp_lora_a, grad_y, accumulate=None, defer_input=False):
-            """Backward of projection `name`; `inp` is its input or the name the layer saved it under
-            (a compressed input is then read from its codes, not dequantised)."""
+        def stored_input(inp):
+            """(x, codes) of an input given as a tensor or by the name under which the layer saved it (a compressed input is
+            then read from its codes, not dequantised)."""
+            if not isinstance(inp, str):
+                return inp, None
+            if inp + "_raw" in S:
+                return S[inp + "_raw"], None
+            return None, (S[inp + "_q"], S[inp + "_s"], None, q_bit)
+
+        def back(name, inp, inp_lora_a, grad_y):
+            """Backward of projection `name`."""
             w, qs, la, lb = W[name]
-            codes = None
-            if isinstance(inp, str):
-                if inp + "_raw" in S:
-                    inp = S[inp + "_raw"]
-                else:
-                    codes, inp = (S[inp + "_q"], S[inp + "_s"], None, q_bit), None
-            G[name + "_a"], G[name + "_b"], gx = lora_backward(w, qs, la, lb, inp, inp_lora_a, grad_y, x_codes=codes,
-                                                                 accumulate=accumulate, defer_input=defer_input)
+            x, codes = stored_input(inp)
+            G[name + "_a"], G[name + "_b"], gx = lora_backward(w, qs, la, lb, x, inp_lora_a, grad_y, x_codes=codes)
             return gx
 
         def rebuilt(name):
@@ -295,10 +297,14 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
         del q, k, v, grad_o
         grad_q, grad_k, grad_v = (head_to_hidden_shape(t) for t in (grad_q, grad_k, grad_v))
 
-        # q, k and v share their input: their input gradients are added up in one pass
-        grad_x = lora_input_sum([back("q", "x", S["q_lora_a"], grad_q, defer_input=True),
-                                 back("k", "x", S["k_lora_a"], grad_k, defer_input=True),
-                                 back("v", "x", S["v_lora_a"], grad_v, defer_input=True)])
+        # q, k and v share their input: their rank-R products go together and their input gradients are added up in one pass
+        members = [(*W[n], S[n + "_lora_a"], g) for n, g in (("q", grad_q), ("k", grad_k), ("v", grad_v))]
+        terms = []
+        for n, (ga, gb, term) in zip(("q", "k", "v"), lora_backward_shared(members, *stored_input("x"))):
+            G[n + "_a"], G[n + "_b"] = ga, gb
+            terms.append(term)
+        del members
+        grad_x = lora_input_sum(terms)
         grad_input = grad_x + grad_ln1
 
         def five(n):

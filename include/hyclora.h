@@ -43,7 +43,7 @@ int hyc_abi_version(void);
 
 /* Launch-shape knobs, FOR BENCHMARKING ONLY: process-wide state in a library whose entry points are otherwise
  * stateless.  Results never depend on them except where said ("stats_waves": the last bits of the sums of
- * squares).  Each knob is an atomic integer that an entry point reads once per launch, so a launch on another
+ * squares; "contract_strip_rows").  Each knob is an atomic integer that an entry point reads once per launch, so a launch on another
  * thread runs with the old or the new value of each knob, never a torn one; a pair of calls that must agree
  * (hyc_channel_stats_strips, then hyc_channel_stats) must not straddle a change.  Keys: "quant_rows_per_wave" (rows each wave walks in hyc_quant_pack,
  * default 8), "dequant_rows_per_wave" (same for hyc_unpack_dequant, default 2),
@@ -56,8 +56,9 @@ int hyc_abi_version(void);
  * "fuse_rows_per_wave" (same for both fused LoRA-SiLU kernels, multiple of 16; default 0 = by code width
  * and size: backward 32; forward 96 for tensors of 2^24 elements and more, else 32; at 8 bits 32 in both
  * directions for tensors of 2^24 elements and more, else 16; "fuse_fwd_rows_per_wave" / "fuse_bwd_rows_per_wave" set one of them),
- * "contract_max_groups" (column groups hyc_lora_contract cuts a row strip into, default 32; changes the
- * workspace hyc_lora_contract_workspace asks for), "stats_waves" (waves hyc_channel_stats aims to launch,
+ * "contract_strip_rows" (rows of a strip of hyc_lora_contract, 64, 128, 192 or 256; default 0 = by size; changes the
+ * workspace hyc_lora_contract_workspace asks for and the order of the sums), "contract_max_groups" (accepted, without
+ * effect: a strip's column blocks are of one width), "stats_waves" (waves hyc_channel_stats aims to launch,
  * default 4096; sets the number of row strips hyc_channel_stats_strips returns and so the order in which the
  * sums of squares are added).  Unknown key or bad value: HYC_ERR_ARG.  No
  * counterpart in the reference (its launch shapes come from triton.autotune). */
@@ -600,15 +601,38 @@ int hyc_lora_add_restore_group(const hyc_lora_add_member *members, int count, in
  * accumulation rounded once.
  *   R even, 2..64; N % 32 == 0; any T.
  *   workspace: device scratch of hyc_lora_contract_workspace(T, N, R, p1 != NULL, p2 != NULL) bytes,
- *   16-byte aligned, contents undefined on entry and exit; partial sums are combined in a fixed
- *   order (no atomics), so results are reproducible.  Tuning key "contract_max_groups" (default 32):
- *   upper bound on the column groups a row strip is split into (each adds a plane of p2 partials).
+ *   16-byte aligned, not NULL, contents undefined on entry and exit; partial sums are combined in a fixed
+ *   order (no atomics), so results are reproducible.
  */
 int64_t hyc_lora_contract_workspace(int64_t T, int64_t N, int64_t R, int want_p1, int want_p2);
 int hyc_lora_contract(const void *x, const void *q, const void *scale, const void *zero_point, int q_bit,
                       const void *u, const void *v, int v_transposed, void *p1, int p1_transposed, void *p2,
                       void *workspace, int64_t workspace_bytes, int64_t T, int64_t N, int64_t R,
                       void *stream);
+
+/* The same products of several projections in one launch: `count` (1 to 3) jobs with T rows and rank R each, R <= 16
+ * where there are several.  shared 0: every job has an X of its own, of its own width (all dense, or all codes of one
+ * q_bit, with or without a zero point); shared 1: every job reads the X (and q, scale, zero_point) of the first, which is
+ * then read and decoded once - the gradients of the adapters that share an input.  All jobs want the same of p1 and p2.
+ * Each result is the bits of its own hyc_lora_contract call.  The jobs are in host memory (copied at the call).
+ * workspace: the sum of hyc_lora_contract_workspace over the jobs; empty operands: HYC_ERR_SHAPE where count > 1.
+ * Replaces the rank-R products of the q, k, v and of the gate, up projections' lora_backward calls
+ * (models/llama/fused_llama_layer_intra_inter_full_fuse.py:375-383, :454-481 with models/utils/compute_utils.py:28-36). */
+typedef struct hyc_contract_job {
+    const void *x;              /* bf16 [T, N], or NULL with */
+    const void *q;              /*   packed codes [T, N*q_bit/8], */
+    const void *scale;          /*   steps bf16 [N] */
+    const void *zero_point;     /*   and zero points bf16 [N] or NULL */
+    const void *u;              /* bf16 [T, R], or NULL without p1 */
+    const void *v;              /* bf16 [R, N] or, with v_transposed, [N, R], or NULL without p2 */
+    void *p1;                   /* bf16 [R, N] or, with p1_transposed, [N, R], or NULL */
+    void *p2;                   /* bf16 [T, R] or NULL */
+    int64_t N;
+    int v_transposed;
+    int p1_transposed;
+} hyc_contract_job;
+int hyc_lora_contract_group(const hyc_contract_job *jobs, int count, int shared, int q_bit, void *workspace,
+                            int64_t workspace_bytes, int64_t T, int64_t R, void *stream);
 
 /* ---------------------------------------------------------------------------------------
  * Sum of two or three LoRA adds in one pass:  y = t_0 (+) t_1 [(+) t_2],  t_i = bf16(x_i + bf16(xa_i . b_i)),

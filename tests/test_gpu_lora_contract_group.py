@@ -1,0 +1,91 @@
+"""The rank-R products of several projections in one launch (hyc_lora_contract_group behind lora_backward_shared) against the
+calls of the single projections, bit for bit, and the single calls at the edges of their row strips, planes and column
+blocks against float64."""
+import pytest
+import torch
+
+from helpers import BF16, assert_close_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def M():
+    import hyclora_amd  # noqa: F401
+    from hyclora_amd.models import compute_utils
+    from hyclora_amd.operators import compress_function, lora_kernels
+
+    class Ns:
+        cu, cf, lk = compute_utils, compress_function, lora_kernels
+    return Ns
+
+
+def randn(g, *shape, scale=1.0):
+    return (torch.randn(*shape, generator=g) * scale).to(BF16).cuda()
+
+
+# rows: one, around a step of 16, around the 64 rows of a sum of the second product, around strips of 128 and 256 and one plane
+@pytest.mark.parametrize("T", [1, 15, 17, 63, 64, 65, 127, 129, 255, 256, 257, 385, 513])
+@pytest.mark.parametrize("N,R", [(32, 2), (128, 16), (480, 6), (512, 16), (544, 20), (1056, 64)])
+def test_edges_against_float64(M, T, N, R):
+    g = torch.Generator().manual_seed(T * 1000 + N + R)
+    x, u, v = randn(g, T, N), randn(g, T, R), randn(g, R, N, scale=0.1)
+    p1, p2 = M.lk.lora_products(x, u, v)
+    d = lambda t: t.double().cpu()
+    assert_close_bf16(p1.cpu(), (d(u).t() @ d(x)).to(BF16), what="u^T x")
+    assert_close_bf16(p2.cpu(), (d(x) @ d(v).t()).to(BF16), what="x v^T")
+    t1, t2 = M.lk.lora_products(x, u, v.t().contiguous().t(), p1_transposed=True)
+    assert torch.equal(t1.t(), p1) and torch.equal(t2, p2)
+
+
+def test_rows_past_the_end_do_not_count(M):
+    """What lies behind the last row (and right of the last column of a wave's tile) in memory may be anything."""
+    g = torch.Generator().manual_seed(1)
+    T, N, R = 37, 160, 16
+    big = torch.full((T + 200, N), float("nan"), dtype=BF16, device="cuda")
+    u_big = torch.full((T + 200, R), float("inf"), dtype=BF16, device="cuda")
+    x, u, v = randn(g, T, N), randn(g, T, R), randn(g, R, N, scale=0.1)
+    big[:T], u_big[:T] = x, u
+    for got, want in zip(M.lk.lora_products(big[:T], u_big[:T], v), M.lk.lora_products(x, u, v)):
+        assert torch.equal(got, want) and bool(torch.isfinite(got.float()).all())
+
+
+@pytest.mark.parametrize("T", [1, 96, 257, 1030])
+@pytest.mark.parametrize("widths", [(512, 512), (4096, 1024, 1024), (96, 544, 32)])
+@pytest.mark.parametrize("R", [4, 16])
+@pytest.mark.parametrize("q_bit", [None, 2, 4, 8])
+def test_shared_input_matches_single_calls(M, T, widths, R, q_bit):
+    g = torch.Generator().manual_seed(T + sum(widths) + R)
+    K = 544
+    x = randn(g, 1, T, K)
+    codes = None
+    if q_bit is not None:
+        s = M.cf.get_statistics_only_quant(x, q_bit, "per-channel")
+        codes = (M.cf.compression_pack_quant_base(x, q_bit, "per-channel", 1, 1, {"scale": s})[0], s, None, q_bit)
+    members = [(randn(g, n, K, scale=0.05), None, randn(g, R, K, scale=0.1).t(), randn(g, n, R, scale=0.1).t(), randn(g, 1, T, R), randn(g, 1, T, n))
+               for n in widths]
+    with torch.no_grad():
+        together = M.cu.lora_backward_shared(members, None if codes else x, codes)
+        native = M.cu._lib.native().lora_products_shared([(m[2], m[3], m[4], m[5]) for m in members], None if codes else x,
+                                                         *(codes or (None, None, None, 0)))
+        assert native is not None                               # the launch that this test is about
+        for (w, qs, la, lb, xa, gy), (ga, gb, (gx, mid, at)) in zip(members, together):
+            ga1, gb1, (gx1, mid1, at1) = M.cu.lora_backward(w, qs, la, lb, None if codes else x, xa, gy, x_codes=codes, defer_input=True)
+            assert torch.equal(ga, ga1) and torch.equal(gb, gb1) and torch.equal(mid, mid1) and torch.equal(gx, gx1) and torch.equal(at, at1)
+            assert ga.t().is_contiguous() and gb.t().is_contiguous()
+
+
+def test_group_refusals(M):
+    """What the group does not take goes the way of the single calls: ranks past 16, ranks that differ, one member, host tensors."""
+    g = torch.Generator().manual_seed(2)
+    native = M.cu._lib.native()
+    x = randn(g, 1, 20, 64)
+    member = lambda r, n=96, t=20: (randn(g, r, 64).t(), randn(g, n, r).t(), randn(g, 1, t, r), randn(g, 1, t, n))   # noqa: E731
+    with torch.no_grad():
+        call = lambda ms: native.lora_products_shared(ms, x, None, None, None, 0)   # noqa: E731
+        assert call([member(16), member(16)]) is not None
+        assert call([member(20), member(20)]) is None and call([member(16), member(8)]) is None and call([member(16)]) is None
+        assert call([member(16)] * 4) is None and call([member(16), member(16, t=10)]) is None and call([member(16), member(16, n=80)]) is None
+        host = tuple(t.cpu() for t in member(16))
+        assert call([member(16), host]) is None
+    assert call([member(16), member(16)]) is None                # gradients are to be recorded
