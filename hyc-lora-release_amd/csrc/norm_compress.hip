@@ -202,10 +202,11 @@ static int compute_units() {
 // operands, and the adapter rows are loaded in the same column order, 16 bytes a lane, so that two
 // consecutive steps consume whole 128-byte lines), and leaves a [rows x 16] fp32 partial per block;
 // the slabs' partials are added in column order through LDS and rounded once.
-template <int QBIT, bool W32, int MAXW, bool XA>
-__global__ __launch_bounds__(MAXW * kWave) __attribute__((amdgpu_waves_per_eu(XA && MAXW <= 8 ? 2 : 4)))
+template <int QBIT, bool W32, int MAXW, int NB>
+__global__ __launch_bounds__(MAXW * kWave) __attribute__((amdgpu_waves_per_eu(NB > 0 && MAXW <= 8 ? 2 : 4)))
 void rmsnorm_fwd_compress_slab_kernel(const NormCompressArgs a, const XaArgs xa, int rows_per_group) {
     constexpr int G = kSlabRows;
+    constexpr bool XA = NB > 0;
     constexpr int kXaRows = kXaRowsFor<MAXW>;
     extern __shared__ float slab_part[];                // [2][G][waves][64], then (XA) [waves][kXaRows][kXaPitch] bf16
     const int lane = threadIdx.x & (kWave - 1);
@@ -240,6 +241,31 @@ void rmsnorm_fwd_compress_slab_kernel(const NormCompressArgs a, const XaArgs xa,
     const bool has_outlier = (tv.x | tv.y | tv.z | tv.w) != 0u;
     const bool fast = __ballot(!(qy.fast && qx.fast)) == 0ull;          // uniform across the wave
     const float zero8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+
+    // The adapter rows of the first kAhead steps of the contraction are on their way during the row loop (kEarly).  Four neighbouring
+    // lanes read the 64 bytes that a step takes of one row (lane l: row l/4, 16 bytes at columns 32m + 8(l%4) of the slab), and the
+    // operand, lane (i, g) = row i, columns 32m + 8g .. +7, comes of it by a permutation: read in the operand's own order, neighbouring
+    // lanes are in 16 rows, and the cache takes a cycle for each (3.5 us an adapter and workgroup against 1.3).  A row past a
+    // block's last is the last one again: column i of the products, which is not stored.
+    constexpr int kSteps = kWave * 8 / 32, kAhead = NB <= 3 ? 8 : 6;
+    constexpr bool kEarly = MAXW <= 8;                  // 16 waves have no registers for it while the row loop runs
+    u32x4 bw[XA ? kAhead : 1][XA ? NB : 1];
+    const uint16_t* wp[XA ? NB : 1];
+    auto fetch = [&](int m) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) bw[m % kAhead][b] = ld16(wp[b] + 32 * m);
+    };
+    auto fetch_first = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < kAhead; ++m) fetch(m);
+    };
+    if constexpr (XA) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int i = (lane >> 2) < xa.valid[b] ? (lane >> 2) : xa.valid[b] - 1;
+            wp[b] = xa.w[b] + (int64_t)i * N + wave * (kWave * 8) + 8 * (lane & 3);
+        }
+    }
 
     u32x4 xv[G];
     auto request = [&](int64_t r) __attribute__((always_inline)) {
@@ -312,44 +338,28 @@ void rmsnorm_fwd_compress_slab_kernel(const NormCompressArgs a, const XaArgs xa,
     // The LoRA-A contraction of the tile rows [t0, t0 + nrows) that the steps above left in LDS.
     auto contract = [&](int64_t t0, int nrows) __attribute__((always_inline)) {
         const int i = lane & 15, g = lane >> 4;
-        f32x4 acc[kXaBlocks];
-        const uint16_t* wp[kXaBlocks];
+        f32x4 acc[XA ? NB : 1];
 #pragma unroll
-        for (int b = 0; b < kXaBlocks; ++b) {
-            acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            const bool have = b < xa.nb && i < xa.valid[b];
-            wp[b] = have ? xa.w[b] + (int64_t)i * N + wave * (kWave * 8) + 8 * g : nullptr;
-        }
-        const uint16_t* yrow = ytile + i * kXaPitch + 8 * g;
+        for (int b = 0; b < NB; ++b) acc[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        const uint16_t* yrow = ytile + (i < kXaRows ? i : 0) * kXaPitch + 8 * g;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");          // the tile rows written by this wave's other lanes
         __builtin_amdgcn_wave_barrier();
-        u32x4 bw[2][kXaBlocks];
-        auto fetch = [&](int m, u32x4 (&dst)[kXaBlocks]) __attribute__((always_inline)) {
+        if constexpr (!kEarly) fetch_first();
 #pragma unroll
-            for (int b = 0; b < kXaBlocks; ++b) {
-                dst[b] = u32x4{0, 0, 0, 0};
-                if (b < xa.nb && wp[b]) dst[b] = ld16(wp[b] + 32 * m);
+        for (int m = 0; m < kSteps; ++m) {
+            __builtin_amdgcn_sched_barrier(0);                          // or the loads move down to their uses
+            const u32x4 av = *reinterpret_cast<const u32x4*>(yrow + 32 * m);
+            const s16x4 a0 = __builtin_bit_cast(s16x4, u32x2{av.x, av.y});
+            const s16x4 a1 = __builtin_bit_cast(s16x4, u32x2{av.z, av.w});
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                u32x4 w4 = bw[m % kAhead][b];
+#pragma unroll
+                for (int d = 0; d < 4; ++d) w4[d] = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (4 * i + g), (int)w4[d]);
+                acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, __builtin_bit_cast(s16x4, u32x2{w4.x, w4.y}), acc[b], 0, 0, 0);
+                acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, __builtin_bit_cast(s16x4, u32x2{w4.z, w4.w}), acc[b], 0, 0, 0);
             }
-        };
-        fetch(0, bw[0]);
-#pragma unroll 2
-        for (int m = 0; m < kWave * 8 / 32; m += 2) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                if (m + h + 1 < kWave * 8 / 32) fetch(m + h + 1, bw[(h + 1) & 1]);
-                u32x4 av = {0, 0, 0, 0};
-                if (i < kXaRows) av = *reinterpret_cast<const u32x4*>(yrow + 32 * (m + h));
-                const s16x4 a0 = __builtin_bit_cast(s16x4, u32x2{av.x, av.y});
-                const s16x4 a1 = __builtin_bit_cast(s16x4, u32x2{av.z, av.w});
-#pragma unroll
-                for (int b = 0; b < kXaBlocks; ++b) {
-                    if (b < xa.nb) {
-                        const u32x4 w4 = bw[h & 1][b];
-                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a0, __builtin_bit_cast(s16x4, u32x2{w4.x, w4.y}), acc[b], 0, 0, 0);
-                        acc[b] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a1, __builtin_bit_cast(s16x4, u32x2{w4.z, w4.w}), acc[b], 0, 0, 0);
-                    }
-                }
-            }
+            if (m + kAhead < kSteps) fetch(m + kAhead);
         }
         // the slab's partial, rows x (16 per block), into this wave's own tile region (its reads of it
         // are done: a wave's LDS operations complete in order)
@@ -358,22 +368,18 @@ void rmsnorm_fwd_compress_slab_kernel(const NormCompressArgs a, const XaArgs xa,
         __builtin_amdgcn_wave_barrier();
         if (g < kXaRows / 4) {
 #pragma unroll
-            for (int b = 0; b < kXaBlocks; ++b) {
-                if (b < xa.nb) {
-                    const float e[4] = {acc[b].x, acc[b].y, acc[b].z, acc[b].w};
+            for (int b = 0; b < NB; ++b)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) part[(4 * g + v) * (16 * kXaBlocks) + 16 * b + i] = e[v];
-                }
-            }
+                for (int v = 0; v < 4; ++v) part[(4 * g + v) * (16 * NB) + 16 * b + i] = acc[b][v];
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
         const float* all = reinterpret_cast<const float*>(reinterpret_cast<const uint16_t*>(slab_part + 2 * G * nw * kWave));
         constexpr int kWaveFloats = kXaRows * kXaPitch / 2;             // a wave's tile region in floats
-        for (int o = threadIdx.x; o < kXaRows * 16 * kXaBlocks; o += blockDim.x) {
-            const int row = o / (16 * kXaBlocks), c = o % (16 * kXaBlocks), b = c >> 4, j = c & 15;
-            if (row < nrows && b < xa.nb && j < xa.valid[b]) {
+        for (int o = threadIdx.x; o < nrows * 16 * NB; o += blockDim.x) {
+            const int row = o / (16 * NB), c = o % (16 * NB), b = c >> 4, j = c & 15;
+            if (j < xa.valid[b]) {
                 float sum = 0.0f;
                 for (int w = 0; w < nw; ++w) sum += all[w * kWaveFloats + o];          // slabs in column order
                 xa.out[b][(t0 + row) * xa.stride[b] + j] = f_to_bf(sum);
@@ -390,6 +396,7 @@ void rmsnorm_fwd_compress_slab_kernel(const NormCompressArgs a, const XaArgs xa,
         }
         step(r, buf, (int)(r - r0), std::false_type{}, fast_tag);
     };
+    if constexpr (XA && kEarly) fetch_first();
     // every wave of the workgroup makes the same number of steps whichever branch it takes
     if (fast) run(std::true_type{});
     else run(std::false_type{});
@@ -633,7 +640,13 @@ static int launch_nc(const NormCompressArgs& a, const XaArgs& xa, hipStream_t st
             const int64_t resident = (int64_t)compute_units() * (16 / (waves <= 8 ? waves : 16));
             rows_per_group = (int)(cdiv(cdiv(a.rows, resident), (int64_t)kSlabRows) * kSlabRows);
         }
-        if (xa.nb > 0) rows_per_group = waves <= 8 ? kXaRowsFor<8> : kXaRowsFor<16>;      // one matrix-core tile per workgroup
+        if (xa.nb > 0) {
+            // a strip is one matrix-core tile at most; fewer rows where that still leaves every compute unit one workgroup only: a
+            // strip's rows are a serial chain
+            const int64_t even = cdiv(cdiv(a.rows, (int64_t)compute_units()), (int64_t)kSlabRows) * kSlabRows;
+            const int tile = waves <= 8 ? kXaRowsFor<8> : kXaRowsFor<16>;
+            rows_per_group = even < tile ? (int)even : tile;
+        }
         const int64_t groups = cdiv(a.rows, (int64_t)rows_per_group);
         if (groups > INT32_MAX) return HYC_ERR_SHAPE;
         size_t lds = 2 * kSlabRows * waves * kWave * sizeof(float);
@@ -642,14 +655,24 @@ static int launch_nc(const NormCompressArgs& a, const XaArgs& xa, hipStream_t st
             if constexpr (W32) {
                 return HYC_ERR_ARG;                             // the contraction is built for bf16 norm weights only
             } else {
-                lds += (size_t)waves * rows_per_group * kXaPitch * sizeof(uint16_t);
-                if (waves <= 8) launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, false, 8, true>, grid, block, lds, st, a, xa, rows_per_group);
-                else launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, false, 16, true>, grid, block, lds, st, a, xa, rows_per_group);
+                lds += (size_t)waves * (waves <= 8 ? kXaRowsFor<8> : kXaRowsFor<16>) * kXaPitch * sizeof(uint16_t);
+#define HYC_NC_XA(NB)                                                                                                             \
+    case NB:                                                                                                                      \
+        if (waves <= 8) launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, false, 8, NB>, grid, block, lds, st, a, xa, rows_per_group); \
+        else launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, false, 16, NB>, grid, block, lds, st, a, xa, rows_per_group);     \
+        break;
+                switch (xa.nb) {
+                    HYC_NC_XA(1)
+                    HYC_NC_XA(2)
+                    HYC_NC_XA(3)
+                    HYC_NC_XA(4)
+                }
+#undef HYC_NC_XA
             }
         } else if (waves <= 8) {
-            launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, W32, 8, false>, grid, block, lds, st, a, xa, rows_per_group);
+            launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, W32, 8, 0>, grid, block, lds, st, a, xa, rows_per_group);
         } else {
-            launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, W32, 16, false>, grid, block, lds, st, a, xa, rows_per_group);
+            launch_slab(rmsnorm_fwd_compress_slab_kernel<QBIT, W32, 16, 0>, grid, block, lds, st, a, xa, rows_per_group);
         }
         return check_launch();
     }
