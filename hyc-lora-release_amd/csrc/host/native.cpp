@@ -348,15 +348,52 @@ OptT frozen_input_grad(const Tensor& grad_y, const Tensor& w) {
 }
 bool weight_ok(const Tensor& w, int64_t in) { return is_bf(w) && w.dim() == 2 && w.size(1) == in && w.is_contiguous(); }
 
+// x A for one to three adapters [K, R] of one x, from one read of x, where that is the way.  This package's kernel against the library's
+// product, us (16 ranks): [96, 4096] 4.8 / 7.6, [96, 11008] 7.6 / 24, [2048, 4096] 8.9 / 14.3, [2048, 11008] 14.7 / 34, [4096, 768] 4.2 / 5.2, [4096, 4096]
+// 10.4 / 14.7, [4096, 11008] 23.2 / 36.6;  the other way round at [2048, 5120] 11.6 / 10.1, and to the library: [4096, 13824] 26.9 / 23.0, [8192, 4096]
+// 17.4 / 15.2, [8192, 11008] 42.6 / 40.8.  A call of the library costs the host 20 us more.
+std::vector<Tensor> adapter_products(const Tensor& x, const std::vector<Tensor>& adapters) {
+    TORCH_CHECK(plain(x) && x.dim() >= 2 && x.numel() > 0, "x must be a contiguous bfloat16 tensor on the GPU");
+    const int64_t k = x.size(-1), rows = x.numel() / k;
+    for (const Tensor& a : adapters) TORCH_CHECK(is_bf(a) && a.dim() == 2 && a.size(0) == k, "an adapter must be [", k, ", R] bfloat16, got ", a.sizes());
+    const bool ours = k % 32 == 0 && (k <= 4096 ? rows * k < int64_t{1} << 25 : rows <= (k <= 12288 ? 4096 : 3072));
+    hyc_contract_job jobs[3] = {};
+    int64_t r = 0;
+    bool group = ours && !adapters.empty() && adapters.size() <= 3;
+    for (size_t i = 0; group && i < adapters.size(); ++i) {
+        const Tensor v = adapters[i].t();                          // [R, K]
+        const Lora V(v);
+        group = V.ok && V.n == k && V.r % 2 == 0 && V.r >= 2 && V.r <= (adapters.size() > 1 ? 16 : 64) && (i == 0 || V.r == r) &&
+                v.device() == x.device() && (i == 0 || V.transposed == jobs[0].v_transposed);
+        r = V.r;
+        jobs[i].x = x.data_ptr(); jobs[i].v = V.p; jobs[i].v_transposed = V.transposed; jobs[i].N = k;
+    }
+    std::vector<Tensor> out;
+    auto shape = x.sizes().vec();
+    if (!group) {
+        for (const Tensor& a : adapters) {
+            shape.back() = a.size(1);
+            out.push_back(at::mm(x.view({-1, k}), a).view(shape));
+        }
+        return out;
+    }
+    shape.back() = r;
+    for (size_t i = 0; i < adapters.size(); ++i) {
+        out.push_back(at::empty(shape, x.options()));
+        jobs[i].p2 = out.back().data_ptr();
+    }
+    const int64_t bytes = std::max<int64_t>((int64_t)adapters.size() * hyc_lora_contract_workspace(rows, k, r, 0, 1), 16);
+    Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
+    check("hyc_lora_contract_group", hyc_lora_contract_group(jobs, (int)adapters.size(), 1, 0, ws.data_ptr(), bytes, rows, r, stream_of(x)));
+    return out;
+}
+
 // -> (x W^T, x A)
 std::optional<std::tuple<Tensor, Tensor>> lora_parts(const Tensor& w, const Tensor& la, const Tensor& x, const OptT& xa) {
     if (!products_are_plain() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !weight_ok(w, x.size(-1))) return std::nullopt;
     if (!is_bf(la) || la.dim() != 2 || la.size(0) != x.size(-1) || (xa && !is_bf(*xa))) return std::nullopt;
     Tensor main = frozen_product(x, w.t());
-    if (xa) return std::make_tuple(main, *xa);
-    auto shape = x.sizes().vec();
-    shape.back() = la.size(1);
-    return std::make_tuple(main, at::mm(x.view({-1, la.size(0)}), la).view(shape));
+    return std::make_tuple(main, xa ? *xa : adapter_products(x, {la})[0]);
 }
 
 // -> (x W^T + (x A) B [+ residual], x W^T, x A)
@@ -602,6 +639,7 @@ PYBIND11_MODULE(_native, m) {
     m.def("lora_add_restore_group", &lora_add_restore_group);
     m.def("contract", &contract);
     m.def("lora_products_shared", &lora_products_shared);
+    m.def("adapter_products", &adapter_products);
     m.def("frozen_input_grad", &frozen_input_grad);
     m.def("whole_rounds", &whole_rounds);
     m.def("frozen_matmul", &frozen_matmul);

@@ -36,6 +36,7 @@
 // there is only one plane the results are written at once, and if that is so for all of them there is no
 // second kernel (P1 of up to 256 rows).
 #include <algorithm>
+#include <type_traits>
 
 #include "hyc_pack.hpp"
 
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(kCtThreads) void lora_contract_kernel(const Contrac
     static_assert(QBIT == 0 || !P2, "the column contraction reads dense X only");
     __shared__ __attribute__((aligned(16))) uint16_t ul[P1 ? NB * 16 * kCtUPitch : 8];
     __shared__ __attribute__((aligned(16))) uint16_t tr[P2 ? kCtWaves : 1][P2 ? 2 * 16 * kCtPitch : 8];
-    __shared__ __attribute__((aligned(16))) float sum2[2][P2 ? kCtWaves * kCtSub * 16 * NB : 4];
+    __shared__ __attribute__((aligned(16))) float sum2[P1 ? 2 : 1][P2 ? kCtWaves * kCtSub * 16 * NB : 4];
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane & 15, g = lane >> 4;
@@ -210,8 +211,8 @@ __global__ __launch_bounds__(kCtThreads) void lora_contract_kernel(const Contrac
 #pragma unroll
             for (int u8 = 0; u8 < 8; ++u8) acc1[nb][u8] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-    int half = 0;                                               // of sum2: one barrier per 64 rows is enough with two
-    for (int base = 0; base < rows; base += kCtSub, half ^= 1) {
+    auto sub = [&](int base, int half, auto ahead_tag) __attribute__((always_inline)) {
+        constexpr bool AHEAD = decltype(ahead_tag)::value;          // 64 more rows follow
         // two steps at a time, so that their chains through LDS and the matrix cores run side by side
 #pragma unroll
         for (int s2 = 0; s2 < kCtSteps; s2 += 2) {
@@ -264,8 +265,10 @@ __global__ __launch_bounds__(kCtThreads) void lora_contract_kernel(const Contrac
                     }
                 }
             }
+            if constexpr (AHEAD) {
 #pragma unroll
-            for (int st = s2; st < s2 + 2; ++st) load(xv[st], base + 16 * st + kCtSub);
+                for (int st = s2; st < s2 + 2; ++st) load(xv[st], base + 16 * st + kCtSub);
+            }
             if constexpr (P2) {
                 f32x4 acc2[2][NB];
 #pragma unroll
@@ -315,7 +318,11 @@ __global__ __launch_bounds__(kCtThreads) void lora_contract_kernel(const Contrac
                 }
             }
         }
-    }
+    };
+    int base = 0, half = 0;                                     // half of sum2: with two, one barrier per 64 rows is enough
+    if constexpr (P1)                                           // without P1 a strip is 64 rows
+        for (; base + kCtSub < rows; base += kCtSub, half ^= 1) sub(base, half, std::true_type{});
+    sub(base, half, std::false_type{});
 
     if constexpr (P1) {
         if (!active) return;
@@ -353,6 +360,83 @@ __global__ __launch_bounds__(kCtThreads) void lora_contract_kernel(const Contrac
                 }
             }
         }
+    }
+}
+
+// P2 alone, for X of many rows or few columns: a workgroup of 8 waves owns 16 rows and the whole contraction, so there are no
+// partial planes and no second kernel.  A wave takes 128 of every 1024 columns, 32 (64 bytes of a row) an operand.  X and V are
+// read four neighbouring lanes to a row's 64 bytes, and the operands (lane (i, g): row i, columns 8g .. +7 of the 32) come of that by a
+// lane permutation: in the operands' own order neighbouring lanes are in 16 rows, and the cache takes a cycle for each.  Two
+// turns of loads are on their way.
+constexpr int kRowsThreads = 512, kRowsWaves = kRowsThreads / kWave, kRowsCols = kRowsWaves * kCtTile;
+template <int NB>
+__global__ __launch_bounds__(kRowsThreads, 2) void lora_rows_kernel(const ContractArgs a) {
+    constexpr int kAhead = 2;
+    __shared__ float part[kRowsWaves][NB * 256];
+    const ContractMember& m = a.m[0];
+    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int i = lane & 15, g = lane >> 4, N = m.N, R = a.R, b0 = blockIdx.y * NB;
+    const int64_t row0 = (int64_t)blockIdx.x * 16;
+    const int rows = a.T - row0 < 16 ? (int)(a.T - row0) : 16;
+    const int lr = lane >> 2, lc = 8 * (lane & 3);
+    const uint16_t* xp = m.x + (row0 + (lr < rows ? lr : rows - 1)) * N + lc;       // rows past the end: not stored
+    const uint16_t* vp[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) vp[nb] = m.v[b0 + nb] + (int64_t)(lr < a.live[b0 + nb] ? lr : 0) * N + lc;
+    u32x4 x[kAhead][4], v[kAhead][NB][4];
+    auto load = [&](int d, int c0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const int c = c0 + 32 * s < N ? c0 + 32 * s : 0;                        // uniform; columns past the end: not multiplied
+            x[d][s] = ld16(xp + c);
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) v[d][nb][s] = ld16(vp[nb] + c);
+        }
+    };
+    auto operand = [&](u32x4 w) __attribute__((always_inline)) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) w[d] = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * (4 * i + g), (int)w[d]);
+        return __builtin_bit_cast(bf16x8, w);
+    };
+    f32x4 acc[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[nb] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int w0 = wave * kCtTile;
+#pragma unroll
+    for (int d = 0; d < kAhead; ++d) load(d, w0 + d * kRowsCols);
+    for (int c0 = w0; c0 < N; c0 += kAhead * kRowsCols) {
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) {
+            const int c = c0 + d * kRowsCols;
+            bf16x8 xo[4], vo[NB][4];
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                xo[s] = operand(c + 32 * s < N ? x[d][s] : u32x4{0, 0, 0, 0});
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) vo[nb][s] = operand(c + 32 * s < N ? v[d][nb][s] : u32x4{0, 0, 0, 0});
+            }
+            load(d, c + kAhead * kRowsCols);
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) acc[nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xo[s], vo[nb][s], acc[nb], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[wave][nb * 256 + (4 * g + e) * 16 + i] = acc[nb][e];
+    __syncthreads();
+    // the waves' parts in wave order; a thread owns two ranks of a row
+    for (int o = threadIdx.x; o < NB * 128; o += kRowsThreads) {
+        const int nb = o >> 7, row = (o >> 3) & 15, r = (o & 7) * 2;
+        float s0 = part[0][nb * 256 + row * 16 + r], s1 = part[0][nb * 256 + row * 16 + r + 1];
+#pragma unroll
+        for (int w = 1; w < kRowsWaves; ++w) {
+            s0 += part[w][nb * 256 + row * 16 + r];
+            s1 += part[w][nb * 256 + row * 16 + r + 1];
+        }
+        if (row < rows && r < a.live[b0 + nb]) *reinterpret_cast<uint32_t*>(m.p2[b0 + nb] + (row0 + row) * R + r) = pk_bf16(s0, s1);
     }
 }
 
@@ -457,10 +541,20 @@ static void contract_launch(const ContractArgs& a, int64_t wgs, hipStream_t st) 
 // Without P1 a strip leaves nothing behind, and 64 rows are the fastest at every shape measured ([4096, 11008] 24.5 against 26.5 at 256,
 // [512, 4096] 7.6 against 11.4).
 static int strip_rows(int64_t T, int64_t N, bool want1) {
+    if (!want1) return kCtSub;
     const int fixed = g_ct_strip.get();
     if (fixed) return fixed;
-    if (!want1) return kCtSub;
     return T <= kCtMaxStrip || cdiv(T, kCtMaxStrip) * cdiv(N, kCtBlock) >= 160 ? kCtMaxStrip : 128;
+}
+
+// Whether x V^T alone goes to the kernel that keeps whole rows to a workgroup: up to 4096 columns, V as it lies.  That kernel against
+// the planes and their sum, us (16 ranks): [4096, 768] 4.2 / 7.8, [96, 4096] 4.8 / 6.2, [512, 4096] 6.0 / 7.7, [4096, 4096] 10.4 / 13.2, [8192, 4096]
+// 17.4 / 19.5;  from 5120 columns on the rows' serial chain is the longer: [2048, 5120] 12.5 / 11.6, [96, 11008] 12.4 / 7.6, [2048, 11008]
+// 21.3 / 14.7, [4096, 11008] 25.4 / 23.2.
+static bool whole_rows(const hyc_contract_job* jobs, int count, int64_t T) {
+    for (int i = 0; i < count; ++i)
+        if (jobs[i].v_transposed || !aligned16(jobs[i].v)) return false;
+    return jobs[0].N <= 4096 && cdiv(T, 16) <= INT32_MAX;
 }
 
 int tune_contract(const char* key, int value) {
@@ -517,6 +611,20 @@ static int contract_jobs(const hyc_contract_job* jobs, int count, bool shared, i
     a.T = T; a.R = (int)R; a.members = shared ? 1 : count;
     a.blocks = shared ? count : (int)cdiv(R, 16);
     for (int b = 0; b < 4; ++b) a.live[b] = shared ? (int)R : (int)std::min<int64_t>(16, std::max<int64_t>(0, R - 16 * b));
+    if (want2 && !want1 && a.members == 1 && whole_rows(jobs, shared ? count : 1, T)) {
+        ContractMember& m = a.m[0];
+        m.x = (const uint16_t*)h.x; m.N = (int)h.N;
+        for (int b = 0; b < a.blocks; ++b) {
+            m.v[b] = (const uint16_t*)(shared ? jobs[b].v : h.v) + (shared ? 0 : 16 * b * h.N);
+            m.p2[b] = (uint16_t*)(shared ? jobs[b].p2 : h.p2) + (shared ? 0 : 16 * b);
+        }
+        const int nb = a.blocks == 4 ? 2 : a.blocks;
+        const dim3 grid((unsigned)cdiv(T, 16), (unsigned)(a.blocks / nb)), block(kRowsThreads);
+        if (nb == 1) hipLaunchKernelGGL(lora_rows_kernel<1>, grid, block, 0, st, a);
+        else if (nb == 2) hipLaunchKernelGGL(lora_rows_kernel<2>, grid, block, 0, st, a);
+        else hipLaunchKernelGGL(lora_rows_kernel<3>, grid, block, 0, st, a);
+        return check_launch();
+    }
     const int64_t rows16 = 16 * a.blocks;
     char* ws = (char*)workspace;
     int64_t used = 0, wgs = 0, rblocks = 0;

@@ -56,7 +56,7 @@ int hyc_abi_version(void);
  * "fuse_rows_per_wave" (same for both fused LoRA-SiLU kernels, multiple of 16; default 0 = by code width
  * and size: backward 32; forward 96 for tensors of 2^24 elements and more, else 32; at 8 bits 32 in both
  * directions for tensors of 2^24 elements and more, else 16; "fuse_fwd_rows_per_wave" / "fuse_bwd_rows_per_wave" set one of them),
- * "contract_strip_rows" (rows of a strip of hyc_lora_contract, 64, 128, 192 or 256; default 0 = by size; changes the
+ * "contract_strip_rows" (rows of a strip of hyc_lora_contract with p1, 64, 128, 192 or 256; default 0 = by size; changes the
  * workspace hyc_lora_contract_workspace asks for and the order of the sums), "contract_max_groups" (accepted, without
  * effect: a strip's column blocks are of one width), "stats_waves" (waves hyc_channel_stats aims to launch,
  * default 4096; sets the number of row strips hyc_channel_stats_strips returns and so the order in which the

@@ -38,6 +38,21 @@ def test_edges_against_float64(M, T, N, R):
     assert torch.equal(t1.t(), p1) and torch.equal(t2, p2)
 
 
+# x A alone: whole rows in a workgroup of 16 rows and turns of 1024 columns, two ahead, up to 4096 columns; planes beyond
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 64, 200])
+@pytest.mark.parametrize("N", [32, 96, 992, 1024, 1056, 2048, 3104, 4096, 4128])
+@pytest.mark.parametrize("ranks", [(2,), (16,), (40,), (64,), (16, 16), (8, 8, 8)])
+def test_adapter_products_against_float64(M, T, N, ranks):
+    g = torch.Generator().manual_seed(T * 1000 + N + sum(ranks))
+    x, adapters = randn(g, 1, T, N), [randn(g, r, N, scale=0.1) for r in ranks]
+    with torch.no_grad():
+        got = M.cu._lib.native().adapter_products(x, [a.t() for a in adapters])
+        again = M.cu._lib.native().adapter_products(x, [a.t() for a in adapters])
+    for p2, p2_again, a in zip(got, again, adapters):
+        assert p2.shape == (1, T, a.shape[0]) and torch.equal(p2, p2_again)
+        assert_close_bf16(p2.cpu(), (x.double().cpu() @ a.double().cpu().t()).to(BF16), what="x A")
+
+
 def test_rows_past_the_end_do_not_count(M):
     """What lies behind the last row (and right of the last column of a wave's tile) in memory may be anything."""
     g = torch.Generator().manual_seed(1)
