@@ -92,6 +92,7 @@ _SIGNATURES = {
     "hyc_lora_contract_workspace": (_L, [_L, _L, _L, _I, _I]),
     "hyc_lora_contract": (_I, [_P, _P, _P, _P, _I, _P, _P, _I, _P, _I, _P, _P, _L, _L, _L, _L, _P]),
     "hyc_lora_contract_group": (_I, [_P, _I, _I, _I, _P, _L, _L, _L, _P]),
+    "hyc_lora_gemm": (_I, [_P] + [_I] * 5 + [_L, _L, _P]),
     "hyc_lora_add": (_I, [_P, _P, _I, _P, _P, _P, _L, _L, _L, _P]),
     "hyc_lora_add_quant": (_I, [_P, _P, _I] + [_P] * 5 + [_L, _L, _L, _I, _P]),
     "hyc_lora_add_restore": (_I, [_P, _P, _I] + [_P] * 4 + [_L, _L, _L, _I, _P]),

@@ -32,11 +32,6 @@ struct FewArgs {
     int steps_k, total, groups;        // steps of a block of outputs, of all, workgroups
 };
 
-template <int N>
-__device__ __forceinline__ void wait_older_copies_and_barrier() {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
-}
-
 // first step of a workgroup, and the workgroup that has a step
 __device__ __forceinline__ int few_first(const FewArgs& A, int group) { return (int)((int64_t)group * A.total / A.groups); }
 __device__ __forceinline__ int few_group(const FewArgs& A, int step) { return (int)(((int64_t)(step + 1) * A.groups + A.total - 1) / A.total) - 1; }

@@ -416,6 +416,95 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> lora_forward(const Tensor& w, 
     return std::make_tuple(*y, main, a);
 }
 
+// ---- projections in one pass, product included ----------------------------------------------------------------------
+// Whether hyc_lora_gemm takes the operands of one projection of `rows` rows: W [n, k] (or, as an input gradient, [k, n]), B and x A
+bool gemm_member(const Tensor& w, const Tensor& lb, const Tensor& xa, int64_t rows, int64_t n, int64_t k, const OptT& bias, hyc_gemm_member& m) {
+    const Lora L(lb);
+    if (!is_bf(w) || w.dim() != 2 || !w.is_contiguous() || !aligned(w) || n % 128 || k % 64 || rows * k >= int64_t{1} << 31 || n * k >= int64_t{1} << 31)
+        return false;
+    if (!L.fits(n) || L.r > 16 || !plain(xa) || xa.size(-1) != L.r || xa.numel() != rows * L.r || (bias && !vec(*bias, n))) return false;
+    m = {};
+    m.w = w.data_ptr(); m.xa = xa.data_ptr(); m.b = L.p; m.b_transposed = L.transposed; m.bias = ptr(bias); m.N = n; m.K = k;
+    return true;
+}
+// Where that kernel is the way: weights of up to 2^22 elements, an encoder's.  us, against the library's product and the passes it
+// replaces: [4096, 1024] x 4096 53 / 63, [4096, 4096] x 1024 52 / 51, [1024, 1024] x 4096 21 / 29, [8192, 768] x 3072 64 / 90, [2048, 2048] x 2048 31 / 35;
+// [2048, 4096] x 4096 81 / 79, [512, 4096] x 4096 50 / 39.  It is the longer with few rows ([256, 3072] x 768 as an input gradient 32 / 17),
+// where a call of the library costs the host 20 us, which is what such a step is bound by.
+bool gemm_is_faster(int64_t n, int64_t k) { return n * k <= int64_t{1} << 22; }
+
+// (W, A, B, bias, steps) of projections of one x -> (y, x A, codes of the frozen part) each: bf16(main + (x A) B), main = bf16(x W^T [+
+// bias]); gelu: of that; residual: added to it; steps (all members or none): the codes of main.  main_only: y = main, for a caller that
+// needs it before its steps are known
+using Projection = std::tuple<Tensor, Tensor, Tensor, OptT, OptT>;
+std::optional<std::vector<std::tuple<Tensor, Tensor, OptT>>> lora_project(const Tensor& x, const std::vector<Projection>& members, int64_t bits, bool gelu,
+                                                                          const OptT& residual, bool main_only) {
+    if (!products_are_plain() || !plain(x) || x.dim() != 3 || x.numel() == 0 || members.empty() || members.size() > 3) return std::nullopt;
+    const int64_t k = x.size(-1), rows = x.numel() / k;
+    const bool codes = std::get<4>(members[0]).has_value();
+    if ((codes && !bits_ok(bits)) || (main_only && (codes || gelu || residual))) return std::nullopt;
+    std::vector<Tensor> adapters;
+    for (const auto& [w, la, lb, bias, scale] : members) {
+        if (!is_bf(w) || w.dim() != 2 || w.size(1) != k || !gemm_is_faster(w.size(0), k) || scale.has_value() != codes ||
+            (scale && !vec(*scale, w.size(0))))
+            return std::nullopt;
+        if (!is_bf(la) || la.dim() != 2 || la.size(0) != k || la.size(1) != lb.size(0) || lb.size(0) != std::get<2>(members[0]).size(0)) return std::nullopt;
+        if (w.size(0) % 128 || k % 64 || lb.size(0) > 16 || !Lora(lb).fits(w.size(0)) || (bias && !vec(*bias, w.size(0)))) return std::nullopt;
+        adapters.push_back(la);
+    }
+    auto shape = x.sizes().vec();
+    if (residual) {
+        shape.back() = std::get<0>(members[0]).size(0);
+        if (members.size() != 1 || !plain(*residual) || residual->sizes() != at::IntArrayRef(shape)) return std::nullopt;
+    }
+    const std::vector<Tensor> xa = adapter_products(x, adapters);
+    hyc_gemm_member m[3];
+    std::vector<std::tuple<Tensor, Tensor, OptT>> out;
+    for (size_t i = 0; i < members.size(); ++i) {
+        const auto& [w, la, lb, bias, scale] = members[i];
+        if (!gemm_member(w, lb, xa[i], rows, w.size(0), k, bias, m[i])) return std::nullopt;
+        shape.back() = w.size(0);
+        Tensor y = at::empty(shape, x.options());
+        OptT q;
+        if (scale) {
+            q = bytes_like(y, w.size(0), bits);
+            m[i].q = q->data_ptr();
+            m[i].scale = scale->data_ptr();
+        }
+        m[i].x = x.data_ptr(); m[i].residual = ptr(residual); m[i].y = y.data_ptr();
+        if (main_only) m[i].xa = nullptr;
+        out.emplace_back(y, xa[i], q);
+    }
+    check("hyc_lora_gemm", hyc_lora_gemm(m, (int)members.size(), 0, 0, codes ? (int)bits : 0, gelu, rows, std::get<2>(members[0]).size(0), stream_of(x)));
+    return out;
+}
+
+// (grad_y, W, grad_y B^T, A^T) of projections that share their input -> the sum of their input gradients, each bf16(grad_y W + (grad_y
+// B^T) A^T), in that order [+ residual]
+using InputGrad = std::tuple<Tensor, Tensor, Tensor, Tensor>;
+OptT lora_input_grad(const std::vector<InputGrad>& members, const OptT& residual) {
+    if (!products_are_plain() || members.empty() || members.size() > 3) return std::nullopt;
+    const Tensor& first = std::get<0>(members[0]);
+    if (!plain(first) || first.dim() < 2 || first.numel() == 0) return std::nullopt;
+    const int64_t rows = first.numel() / first.size(-1), n = std::get<1>(members[0]).size(1), r = std::get<3>(members[0]).size(0);
+    hyc_gemm_member m[3];
+    for (size_t i = 0; i < members.size(); ++i) {
+        const auto& [g, w, mid, at_] = members[i];
+        if (!plain(g) || g.numel() != rows * g.size(-1) || w.dim() != 2 || w.size(0) != g.size(-1) || w.size(1) != n || at_.size(0) != r ||
+            !gemm_is_faster(n, w.size(0)) || !gemm_member(w, at_, mid, rows, n, w.size(0), std::nullopt, m[i]))
+            return std::nullopt;
+        m[i].x = g.data_ptr();
+    }
+    auto shape = first.sizes().vec();
+    shape.back() = n;
+    if (residual && !(plain(*residual) && residual->sizes() == at::IntArrayRef(shape))) return std::nullopt;
+    Tensor y = at::empty(shape, first.options());
+    m[0].y = y.data_ptr();
+    m[0].residual = ptr(residual);
+    check("hyc_lora_gemm", hyc_lora_gemm(m, (int)members.size(), 1, members.size() > 1, 0, 0, rows, r, stream_of(first)));
+    return y;
+}
+
 // lora_backward of models/compute_utils.py: -> (grad A, grad B, grad x) or, deferred, (grad A, grad B, (grad_y W, grad_y B^T, A^T))
 pybind11::object lora_backward(const Tensor& w, const Tensor& la, const Tensor& lb, const OptT& x, const OptT& q, const OptT& scale,
                                const OptT& zero, int64_t bits, const Tensor& xa, const Tensor& grad_y, const OptT& accumulate, bool defer) {
@@ -437,6 +526,8 @@ pybind11::object lora_backward(const Tensor& w, const Tensor& la, const Tensor& 
                 : contract(std::nullopt, q, scale, zero, bits, grad_mid, std::nullopt, w.size(1), false);
     if (!ga) return none;
     const Tensor grad_a = std::get<0>(*ga)->t();
+    if (!defer)
+        if (OptT done = lora_input_grad({{grad_y, w, grad_mid, at_}}, accumulate)) return pybind11::make_tuple(grad_a, grad_b, *done);
     Tensor grad_x = frozen_product(grad_y, w);
     if (defer) return pybind11::make_tuple(grad_a, grad_b, pybind11::make_tuple(grad_x, grad_mid, at_));
     OptT sum = lora_add(grad_x, grad_mid, at_, accumulate, true);
@@ -640,6 +731,9 @@ PYBIND11_MODULE(_native, m) {
     m.def("contract", &contract);
     m.def("lora_products_shared", &lora_products_shared);
     m.def("adapter_products", &adapter_products);
+    m.def("lora_project", &lora_project, pybind11::arg("x"), pybind11::arg("members"), pybind11::arg("bits"), pybind11::arg("gelu"),
+          pybind11::arg("residual"), pybind11::arg("main_only") = false);
+    m.def("lora_input_grad", &lora_input_grad);
     m.def("frozen_input_grad", &frozen_input_grad);
     m.def("whole_rounds", &whole_rounds);
     m.def("frozen_matmul", &frozen_matmul);

@@ -46,6 +46,12 @@ __device__ __forceinline__ void wait_copies_and_barrier() {
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
 }
 
+// The same while the N youngest copies of the wave stay under way
+template <int N>
+__device__ __forceinline__ void wait_older_copies_and_barrier() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+}
+
 // A tile of ROWS rows of D bf16 in LDS, as 1 KB blocks of 16 rows x 4 chunks (of 16 bytes): block (row / 16, chunk / 4),
 // inside it the 64 bytes of a row together, its chunks in the order chunk ^ (row / 4).  A wave's copy fills one block, four
 // neighbouring lanes 64 contiguous bytes of memory: with the lanes of a row 16 apart (chunk-major blocks) the copies found 64

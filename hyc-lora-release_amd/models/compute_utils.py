@@ -182,6 +182,24 @@ def lora_backward_shared(members, x, x_codes=None):
     return results
 
 
+def lora_backward_sum(members, x, x_codes=None, residual=None):
+    """lora_backward_shared with the input gradients added up: -> ([(grad lora_A, grad lora_B), ...], their sum [+ residual]), the
+    additions in bf16 and in order.  Where the products are small enough for this package's kernel they, their LoRA adds
+    and the sum are one launch."""
+    if all(qs is None and gy.is_cuda and w.dtype == torch.bfloat16 for w, qs, _, _, _, gy in members) and x_codes is not None and x_codes[2] is None:
+        out = _lib.native().lora_products_shared([(la, lb, xa, gy) for _, _, la, lb, xa, gy in members], None, x_codes[0], x_codes[1], None, x_codes[3])
+        if out is not None:
+            grads = [(ga, gb) for ga, gb, _ in out]
+            grad_x = _lib.native().lora_input_grad([(gy, w, mid, la.mT) for (w, _, la, _, _, gy), (_, _, mid) in zip(members, out)], residual)
+            if grad_x is None:
+                grad_x = lora_input_sum([(frozen_matmul(gy, w), mid, la.mT) for (w, _, la, _, _, gy), (_, _, mid) in zip(members, out)])
+                grad_x = grad_x if residual is None else grad_x + residual
+            return grads, grad_x
+    terms = lora_backward_shared(members, x, x_codes)
+    grad_x = lora_input_sum([t for _, _, t in terms])
+    return [(ga, gb) for ga, gb, _ in terms], grad_x if residual is None else grad_x + residual
+
+
 def lora_input_sum(parts):
     """Sum of the input gradients of projections that share their input, from the deferred terms lora_backward
     returns: acc = t_0; acc += t_1; ... with t_i = (grad_y @ W)_i + (grad_y @ B^T)_i @ A_i^T, every operation

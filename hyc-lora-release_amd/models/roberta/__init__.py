@@ -22,9 +22,9 @@ from ...operators.compress_function import (compress_attention_map, compression_
 from ...operators.gelu_kernels import gelu_backward
 from ...operators.layernorm_kernels import layernorm_backward, layernorm_forward
 from ...operators.softmax_kernels import softmax_backward, softmax_backward_from_compressed, softmax_forward
+from ... import _lib
 from ...operators import lora_kernels
-from ..compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_backward_shared, lora_forward, lora_input_sum,
-                            lora_parts)
+from ..compute_utils import (head_to_hidden_shape, heads_matmul, hidden_to_head_shape, lora_backward, lora_backward_sum, lora_forward, lora_parts)
 from ...operators.map_kernels import MapAttention, map_backward, map_backward_supported, map_supported
 from ..fused_decoder_layer import _note_map_entries, check_map_entries, keep_map_entries, lora_linear_parts
 
@@ -72,15 +72,38 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
         raw = mode == "baseline"
         whole = mode in ("baseline", "intra")
 
+        def project(names, inp, codes=False, gelu=False, residual=None, main_only=False):
+            """Projections `names` of inp, product and all that follows in one kernel: {name: (output, x @ A)} or None where that
+            kernel is not the way.  With `codes` (frozen steps) the frozen parts are quantised as well; with `main_only` the
+            output is the frozen part."""
+            if not inp.is_cuda or (codes and (calib or raw)) or any(W[n][2] is not None for n in names):
+                return None
+            done = _lib.native().lora_project(inp, [(W[n][0], W[n][3], W[n][4], W[n][1], sv[n]['scale'] if codes else None) for n in names], q_bit or 0,
+                                              gelu, residual, main_only)
+            if done is None:
+                return None
+            out = {}
+            for n, (y, xa, q) in zip(names, done):
+                if codes:
+                    stats[(n, "scale")] = saved[n + "_main_s"] = sv[n]['scale']
+                    saved[n + "_main_q"] = q
+                out[n] = (y, xa)
+            return out
+
         def proj(name, inp, residual=None):
             w, b, qs, la, lb = W[name]
+            done = project((name,), inp, residual=residual)
+            if done is not None:
+                return done[name][0], None, done[name][1]
             return lora_forward(w, qs, la, lb, b, inp, residual=residual)
 
         def proj_quant(name, inp):
             """Projection with the frozen part quantised on the way, one kernel for codes + LoRA add
             (the reference: separate passes, …intra_inter.py:90-121) -> (output, x @ A)."""
             w, b, qs, la, lb = W[name]
-            main, xa = lora_parts(w, qs, la, b, inp)
+            # while calibrating, the same sums as afterwards
+            done = project((name,), inp, main_only=True)
+            main, xa = done[name] if done else lora_parts(w, qs, la, b, inp)
             lb = lb.to(main.dtype)
             if not (lora_kernels.supported(main, xa, lb) and main.dim() == 3):
                 quant(name + "_main", main, name)
@@ -113,9 +136,9 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
             k, _, saved["k_lora_a"] = proj("k", x)
             v, _, saved["v_lora_a"] = proj("v", x)
         else:
-            q, saved["q_lora_a"] = proj_quant("q", x)
-            k, saved["k_lora_a"] = proj_quant("k", x)
-            v, saved["v_lora_a"] = proj_quant("v", x)
+            qkv = project(("q", "k", "v"), x, codes=True) or {n: proj_quant(n, x) for n in ("q", "k", "v")}
+            (q, saved["q_lora_a"]), (k, saved["k_lora_a"]), (v, saved["v_lora_a"]) = qkv["q"], qkv["k"], qkv["v"]
+            del qkv
         quant("x", x)
         q, k, v = (hidden_to_head_shape(t, num_heads) for t in (q, k, v))
         if whole:
@@ -177,9 +200,11 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
         if whole:
             up, _, saved["up_lora_a"] = proj("up", x_medium)
         else:
-            up, saved["up_lora_a"] = proj_quant("up", x_medium)
+            done = project(("up",), x_medium, codes=True, gelu=True)
+            up, saved["up_lora_a"] = (None, done["up"][1]) if done else proj_quant("up", x_medium)
         quant("x_medium", x_medium)
-        fn = torch.nn.functional.gelu(up)
+        fn = torch.nn.functional.gelu(up) if up is not None else done["up"][0]
+        done = None
         if whole:
             quant("up", up)
         del up
@@ -233,11 +258,11 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
                 return S[inp + "_raw"], None
             return None, (S[inp + "_q"], S[inp + "_s"], None, q_bit)
 
-        def back(name, inp, inp_lora_a, grad_y):
+        def back(name, inp, inp_lora_a, grad_y, accumulate=None):
             """Backward of projection `name`."""
             w, qs, la, lb = W[name]
             x, codes = stored_input(inp)
-            G[name + "_a"], G[name + "_b"], gx = lora_backward(w, qs, la, lb, x, inp_lora_a, grad_y, x_codes=codes)
+            G[name + "_a"], G[name + "_b"], gx = lora_backward(w, qs, la, lb, x, inp_lora_a, grad_y, x_codes=codes, accumulate=accumulate)
             return gx
 
         def rebuilt(name):
@@ -263,9 +288,8 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
         del fn
         grad_fn = gelu_backward(up, grad_down)
         del up, grad_down
-        grad_up = back("up", "x_medium", S["up_lora_a"], grad_fn)
-        grad_medium = grad_ln2 + grad_up
-        del grad_ln2, grad_up, grad_fn
+        grad_medium = back("up", "x_medium", S["up_lora_a"], grad_fn, accumulate=grad_ln2)       # grad_ln2 + the gradient of the MLP's input
+        del grad_ln2, grad_fn
         grad_ln1, _, _ = layernorm_backward(grad_medium, deq_cb("o_final"), nw1, nb1, S["mean_1"], S["rstd_1"], True, _EPS,
                                             ctx.num_warps, ctx.block_size)
         del grad_medium
@@ -297,15 +321,12 @@ class FusedRobertaLayerFunc(torch.autograd.Function):
         del q, k, v, grad_o
         grad_q, grad_k, grad_v = (head_to_hidden_shape(t) for t in (grad_q, grad_k, grad_v))
 
-        # q, k and v share their input: their rank-R products go together and their input gradients are added up in one pass
+        # q, k and v share their input: their products go together, and their input gradients and the residual connection's are added up
         members = [(*W[n], S[n + "_lora_a"], g) for n, g in (("q", grad_q), ("k", grad_k), ("v", grad_v))]
-        terms = []
-        for n, (ga, gb, term) in zip(("q", "k", "v"), lora_backward_shared(members, *stored_input("x"))):
+        grads, grad_input = lora_backward_sum(members, *stored_input("x"), residual=grad_ln1)
+        for n, (ga, gb) in zip(("q", "k", "v"), grads):
             G[n + "_a"], G[n + "_b"] = ga, gb
-            terms.append(term)
         del members
-        grad_x = lora_input_sum(terms)
-        grad_input = grad_x + grad_ln1
 
         def five(n):
             return (None, None, None, G[n + "_a"], G[n + "_b"])

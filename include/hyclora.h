@@ -635,6 +635,33 @@ int hyc_lora_contract_group(const hyc_contract_job *jobs, int count, int shared,
                             int64_t workspace_bytes, int64_t T, int64_t R, void *stream);
 
 /* ---------------------------------------------------------------------------------------
+ * One to three projections with a frozen weight and a LoRA adapter in one launch, product included, at sizes where a library product
+ * is bound by its launch:   main = bf16(x W^T) [then bf16(main + bias)]   or, with w_is_kn,   main = bf16(x W),
+ *   y = bf16(main + bf16(xa . b));  gelu: y = bf16(gelu(y)), the erf form;  residual: y = bf16(residual + y);
+ *   q_bit: q = the packed codes of main with steps `scale`, as hyc_lora_add_quant forms them (w_is_kn 0 only);
+ *   sum (w_is_kn only): one y, that of the first member: y = t_0 (+) t_1 (+) t_2 [(+) residual of the first], t_i the y of
+ *   member i, every (+) a bf16 addition in that order, as hyc_lora_add_sum adds.
+ * Sums along the contraction are fp32 in one order that depends on nothing else.
+ * Replaces lora_forward / lora_backward's input gradient (models/utils/compute_utils.py:18-36) and the passes around them in the
+ * layers (models/roberta/fused_roberta_layer_intra_inter.py:90-121).
+ *   N % 128 == 0, K % 64 == 0, T >= 1, T*K and N*K below 2^31; R a multiple of 4 up to 16.  No workspace. */
+typedef struct hyc_gemm_member {
+    const void *x;              /* bf16 [T, K] */
+    const void *w;              /* bf16 [N, K] or, with w_is_kn, [K, N] */
+    const void *xa;             /* bf16 [T, R], or NULL without codes, gelu and sum: y = main */
+    const void *b;              /* bf16 [R, N] or, with b_transposed, [N, R] */
+    const void *bias;           /* bf16 [N] or NULL; w_is_kn or not, not with sum */
+    const void *residual;       /* bf16 [T, N] or NULL */
+    const void *scale;          /* bf16 [N], with q_bit */
+    void *q;                    /* uint8 [T, N*q_bit/8], with q_bit */
+    void *y;                    /* bf16 [T, N] */
+    int64_t N, K;
+    int b_transposed;
+} hyc_gemm_member;
+int hyc_lora_gemm(const hyc_gemm_member *members, int count, int w_is_kn, int sum, int q_bit, int gelu, int64_t T, int64_t R,
+                  void *stream);
+
+/* ---------------------------------------------------------------------------------------
  * Sum of two or three LoRA adds in one pass:  y = t_0 (+) t_1 [(+) t_2],  t_i = bf16(x_i + bf16(xa_i . b_i)),
  * every (+) a bf16 addition in that order - the bits of hyc_lora_add(x_0), then hyc_lora_add(x_1, residual = y),
  * then hyc_lora_add(x_2, residual = y).
