@@ -544,7 +544,8 @@ std::optional<std::tuple<OptT, Tensor>> quantize(const Tensor& x, const Tensor& 
     const int64_t k = channel ? channel->numel() : 0;
     Tensor q = bytes_like(x, N, bits);
     OptT kept;
-    if (channel) kept = at::zeros({B, M, k}, x.options());         // a list position without a column reads as zeros
+    // a list position without a column reads as zeros: the kernel's work for lists of a usual length
+    if (channel) kept = k <= HYC_OUTLIER_ZERO_MAX ? at::empty({B, M, k}, x.options()) : at::zeros({B, M, k}, x.options());
     check("hyc_quant_pack", hyc_quant_pack(x.data_ptr(), s.data_ptr(), ptr(z), q.data_ptr(), k ? (const int64_t*)channel->data_ptr() : nullptr, k,
                                            k ? kept->data_ptr() : nullptr, 0, B, M, N, M * N, N, N, 0, (int)bits, stream_of(x)));
     return std::make_tuple(kept, q);

@@ -30,6 +30,21 @@ struct QuantCols {
             fast = fast && hyc_scale_is_fast(s[j]);
         }
     }
+    // Whether the whole wave may use hyc_code_zp_word's rule for its zero points; if so the constants become that rule's:
+    // s = s16, rn = y, z = z16.
+    __device__ __forceinline__ bool scale_for_zero_point(float (&z)[8]) {
+        bool ok = fast;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ok = ok && fabsf(z[j]) <= HYC_ZP_MAX;
+        if (__ballot(!ok) != 0ull) return false;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            rn[j] = HYC_ZP_SCALE / s[j];
+            s[j] *= 1.0f / HYC_ZP_SCALE;
+            z[j] *= HYC_ZP_SCALE;
+        }
+        return true;
+    }
 };
 
 // Device form of hyc_code_word_fast: the same fused multiply-add, with the clamp done by one
@@ -45,10 +60,24 @@ __device__ __forceinline__ uint32_t code_word_fast_dev(float x, float rn) {
     return __float_as_uint(mc);
 }
 
-// low bytes of four dwords -> one dword (byte j from w_j)
+// Device form of hyc_code_zp_word: the clamps are one instruction each, the second with a NaN's way to the lower bound as above
+template <int QBIT>
+__device__ __forceinline__ uint32_t code_zp_word_dev(float x, float y, float s16, float z16) {
+    float q = __builtin_amdgcn_fmed3f(x * y, -HYC_ZP_QUOTIENT_MAX, HYC_ZP_QUOTIENT_MAX);
+    q = fmaf(fmaf(-q, s16, x), y, q);
+    float t = q + z16, tc;
+    asm("v_med3_f32 %0, %1, %2, %3"
+        : "=v"(tc) : "v"(t), "v"(HYC_ZP_SCALE * ((float)(1 << (QBIT - 1)) - 1.0f)), "v"(-HYC_ZP_SCALE * (float)(1 << (QBIT - 1))));
+    const int i = (int)tc;
+    return (uint32_t)(i + (i >> 31) + 32768 + (1 << (QBIT + 15)));
+}
+
+// bytes BYTE of four dwords -> one dword (byte j from w_j)
+template <int BYTE = 0>
 __device__ __forceinline__ uint32_t low_bytes(uint32_t w0, uint32_t w1, uint32_t w2, uint32_t w3) {
-    const uint32_t w01 = __builtin_amdgcn_perm(w1, w0, 0x0c0c0400u);   // selector 0-3: bytes of 2nd operand, 4-7: of 1st
-    const uint32_t w23 = __builtin_amdgcn_perm(w3, w2, 0x0c0c0400u);
+    constexpr uint32_t kSel = 0x0c0c0400u + 0x0101u * BYTE;             // selector 0-3: bytes of 2nd operand, 4-7: of 1st
+    const uint32_t w01 = __builtin_amdgcn_perm(w1, w0, kSel);
+    const uint32_t w23 = __builtin_amdgcn_perm(w3, w2, kSel);
     return __builtin_amdgcn_perm(w23, w01, 0x05040100u);
 }
 
@@ -62,6 +91,12 @@ __device__ __forceinline__ void codes_to_words(const float (&f)[8], const QuantC
         for (int j = 0; j < 8; ++j) w[j] = code_word_fast_dev<QBIT>(f[j], q.rn[j]);
         lo = low_bytes(w[0], w[1], w[2], w[3]);
         hi = low_bytes(w[4], w[5], w[6], w[7]);
+    } else if constexpr (FAST) {                         // q, z after scale_for_zero_point
+        uint32_t w[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) w[j] = code_zp_word_dev<QBIT>(f[j], q.rn[j], q.s[j], z[j]);
+        lo = low_bytes<2>(w[0], w[1], w[2], w[3]);
+        hi = low_bytes<2>(w[4], w[5], w[6], w[7]);
     } else {
         int c[8];
 #pragma unroll

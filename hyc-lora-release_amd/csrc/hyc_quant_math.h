@@ -113,4 +113,26 @@ HYC_HD int hyc_code_from_t_exact(float t, int q_bit) {
     return (int)r + (1 << (q_bit - 1));
 }
 
+// The zero-point rule without a division, for steps that take the reciprocal path and zero points up to 2^64.  Everything is kept
+// times 2^16: y = 65536 / s (rounded once), s16 = s / 65536, z16 = z * 65536.  x * y is the quotient to within an ulp; its remainder
+// x - q s is exact (8-bit significands of x and s), so the second multiply-add gives the correctly rounded quotient (Markstein's
+// theorem), the scaling by a power of two changes no rounding, and t is 65536 (x/s + z) as the IEEE operations round it.  Quotients
+// past 2^100 are held there before the remainder is taken, so that an infinite x leaves an infinite t and not a NaN.  Rounded
+// half away from zero in integers: the clamped t truncated to 2^-16 lies on the same side of every tie, and adding half a unit
+// (one less for negative values) and dropping 16 bits is roundf.  The biased code is byte 2 of hyc_code_zp_word.
+#define HYC_ZP_MAX 1.8446744073709552e19f       /* 2^64 */
+#define HYC_ZP_QUOTIENT_MAX 1.2676506002282294e30f   /* 2^100 */
+#define HYC_ZP_SCALE 65536.0f
+HYC_HD int hyc_code_zp_word(float x, float y, float s16, float z16, int q_bit) {
+    const float lo = -HYC_ZP_SCALE * (float)(1 << (q_bit - 1)), hi = HYC_ZP_SCALE * ((float)(1 << (q_bit - 1)) - 1.0f);
+    float q = x * y;
+    q = q > HYC_ZP_QUOTIENT_MAX ? HYC_ZP_QUOTIENT_MAX : (q < -HYC_ZP_QUOTIENT_MAX ? -HYC_ZP_QUOTIENT_MAX : q);
+    q = fmaf(fmaf(-q, s16, x), y, q);
+    float t = q + z16;
+    t = (t > lo) ? t : lo;
+    t = fminf(t, hi);
+    const int i = (int)t;
+    return i + (i >> 31) + 32768 + (1 << (q_bit + 15));
+}
+
 #endif  // HYC_QUANT_MATH_H

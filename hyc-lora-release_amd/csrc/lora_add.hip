@@ -188,6 +188,7 @@ __device__ __forceinline__ void lora_add_block(const LoraAddArgs& a, int block) 
     if (row_begin >= row_end) return;
     bool fast = false;
     if constexpr (MODE == kAddQuant && !ZP) fast = __ballot(!qc.fast) == 0ull;
+    if constexpr (MODE == kAddQuant && ZP) fast = qc.scale_for_zero_point(z);
     if constexpr (MODE != kAddPlain) {
         if (a.cos_t) {                                          // uniform over the grid
             auto run = [&](auto fast_tag) {
@@ -195,14 +196,14 @@ __device__ __forceinline__ void lora_add_block(const LoraAddArgs& a, int block) 
                 if (a.rope_f32) lora_add_rows<QBIT, KSTEPS, MODE, ZP, F, false, 2>(a, row_begin, row_end, lane, chunk, active, qc, z, B);
                 else lora_add_rows<QBIT, KSTEPS, MODE, ZP, F, false, 1>(a, row_begin, row_end, lane, chunk, active, qc, z, B);
             };
-            if constexpr (MODE == kAddQuant && !ZP) {
+            if constexpr (MODE == kAddQuant) {
                 if (fast) { run(std::true_type{}); return; }
             }
             run(std::false_type{});
             return;
         }
     }
-    if constexpr (MODE == kAddQuant && !ZP) {
+    if constexpr (MODE == kAddQuant) {
         if (fast) {
             lora_add_rows<QBIT, KSTEPS, MODE, ZP, true>(a, row_begin, row_end, lane, chunk, active, qc, z, B);
             return;

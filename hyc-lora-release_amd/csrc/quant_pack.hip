@@ -47,10 +47,10 @@ constexpr int kQuantThreads = kQuantWaves * kWave;
 constexpr int kRowUnroll = HYC_Q_UNROLL;       // quantiser: independent 128-bit loads in flight per lane
 constexpr int kDeqUnroll = HYC_D_UNROLL;       // dequantiser: rows per group
 
-static Knob g_quant_rows_per_wave{8};     // strip heights; see hyc_set_tuning
+static Knob g_quant_rows_per_wave{0};     // strip heights, 0: by size (see quant_rows_by_size); see hyc_set_tuning
 static Knob g_dequant_rows_per_wave{2};
-static Knob g_quant_outlier_rows_per_wave{8};     // the same two with an outlier list
-static Knob g_dequant_outlier_rows_per_wave{8};
+static Knob g_quant_outlier_rows_per_wave{0};     // the same two with an outlier list
+static Knob g_dequant_outlier_rows_per_wave{0};
 
 struct QuantArgs {
     uint16_t* x;            // bf16 activations (input of quantise / output of dequantise)
@@ -82,11 +82,17 @@ struct OutlierLane {
     }
 };
 
-__device__ __forceinline__ OutlierLane find_outliers(const int64_t* oidx, int k, int wave_col0, int col0, int lane) {
+// The lane's entry of the first 64, requested before the wave's rows (waiting for it then leaves those in flight)
+__device__ __forceinline__ int first_entries(const int64_t* oidx, int k, int lane) {
+    const int ch = (int)oidx[lane < k ? lane : 0];
+    return lane < k ? ch : -1;
+}
+
+__device__ __forceinline__ OutlierLane find_outliers(const int64_t* oidx, int k, int wave_col0, int col0, int lane, int first) {
     OutlierLane o;
     for (int base = 0; base < k; base += kWave) {
         const int e = base + lane;
-        const int ch = (e < k) ? (int)oidx[e] : -1;
+        const int ch = base == 0 ? first : (e < k) ? (int)oidx[e] : -1;
         const bool hit = (unsigned)(ch - wave_col0) < (unsigned)(kWave * 8);
         unsigned long long hits = __ballot(hit);
         while (hits) {
@@ -156,6 +162,26 @@ __device__ __forceinline__ void extract_rest(const OutlierLane& o, uint32_t bits
     }
 }
 
+// A list position without a column of its own - a channel outside the tensor, the earlier copies of a repeated one - reads as zero.
+// Written by the waves of the first column tile for their rows, for lists of up to kOutlierZeroMax entries (every entry is compared
+// with all behind it); callers clear x_outlier beforehand for longer ones.
+constexpr int kOutlierZeroMax = HYC_OUTLIER_ZERO_MAX;
+__device__ __forceinline__ void clear_unused(const QuantArgs& a, int64_t row0, int64_t row1, int lane, int first) {
+    for (int base = 0; base < a.k; base += kWave) {
+        const int e = base + lane;
+        const int ch = base == 0 ? first : e < a.k ? (int)a.oidx[e] : -1;
+        bool unused = (unsigned)ch >= (unsigned)a.N;
+        for (int b2 = base; b2 < a.k; b2 += kWave) {
+            const int c2 = b2 == base ? ch : b2 + lane < a.k ? (int)a.oidx[b2 + lane] : -1;
+            const int n = a.k - b2 < kWave ? a.k - b2 : kWave;
+            for (int i = 0; i < n; ++i)
+                unused = unused || (e < b2 + i && ch == __builtin_amdgcn_readlane(c2, i));
+        }
+        if (unused && e < a.k)
+            for (int64_t t = row0; t < row1; ++t) a.xo[t * a.k + e] = 0;
+    }
+}
+
 // Walks the rows t = b*M + m of a [B, M, .] tensor with independent batch and row strides
 // without a division per row.
 struct RowCursor {
@@ -222,10 +248,15 @@ __device__ __forceinline__ void quant_rows(const QuantArgs& a, int64_t row0, int
     RowCursor cur(row0, a.M, a.stride_b, a.stride_m);
     u32x4 v[kRowUnroll];
     int64_t roff[kRowUnroll];
+    int entry = -1;
+    if constexpr (OUTL) entry = first_entries(a.oidx, a.k, chunk & (kWave - 1));
     load_rows<FULL>(a, cur, row0, row1, active, coff, v, roff);
     // the first rows are already on their way while the wave looks up its outlier columns
     OutlierLane ol;
-    if constexpr (OUTL) ol = find_outliers(a.oidx, a.k, (chunk & ~(kWave - 1)) * 8, chunk * 8, chunk & (kWave - 1));
+    if constexpr (OUTL) {
+        ol = find_outliers(a.oidx, a.k, (chunk & ~(kWave - 1)) * 8, chunk * 8, chunk & (kWave - 1), entry);
+        if (a.k <= kOutlierZeroMax && chunk < kWave) clear_unused(a, row0, row1, chunk, entry);     // uniform: the wave of the first columns
+    }
     const OutlierFirst of(ol);
     const bool in_place = OUTL && a.zero_input != 0;
     const uint32_t loop_bits = in_place ? ol.mask : of.rest;     // what extract_rest handles, per lane
@@ -304,7 +335,8 @@ void quant_pack_kernel(const QuantArgs a) {
     const bool full = (col_tile + 1) * kWave <= a.C && row1 - row0 == a.rows_per_wave &&
                       a.rows_per_wave % kRowUnroll == 0;      // uniform across the wave
     // one slow column anywhere in the wave sends the whole wave down the IEEE-division path
-    if (ZP || __ballot(!qc.fast) != 0ull)
+    const bool fast = ZP ? qc.scale_for_zero_point(z) : __ballot(!qc.fast) == 0ull;
+    if (!fast)
         quant_rows<QBIT, ZP, OUTL, false, false>(a, row0, row1, active, chunk, coff, qc, z);
     else if (full)
         quant_rows<QBIT, ZP, OUTL, true, true>(a, row0, row1, active, chunk, coff, qc, z);
@@ -429,10 +461,12 @@ __global__ __launch_bounds__(kQuantThreads) void unpack_dequant_kernel(const Qua
                 if (FULL || (active && t0 + u < row1)) st16_nt(xrow[u], o[u]);
         };
         // next group's loads go out before this group's stores (see quant_rows)
+        int entry = -1;
+        if constexpr (OUTL) entry = first_entries(a.oidx, a.k, lane);
         load_codes(row0);
         // the first codes are already on their way while the wave looks up its outlier columns
         if constexpr (OUTL) {
-            ol = find_outliers(a.oidx, a.k, col_tile * kWave * 8, col0, lane);
+            ol = find_outliers(a.oidx, a.k, col_tile * kWave * 8, col0, lane, entry);
             of = OutlierFirst(ol);
         }
         load_outliers(row0);
@@ -500,6 +534,17 @@ static QuantArgs make_args(const void* x, const void* scale, const void* zp, con
     return a;
 }
 
+// Strip heights by size: a small tensor is one short generation of waves, whose strips are serial chains; long strips spread the columns'
+// constants over more rows.  us at 2, 4, 8, 16 rows, quantiser: [1024, 4096] 4.8 4.1 4.6 5.9, with outliers 8.8 7.1 7.5 9.4; [256, 2048] 3.2 3.0
+// 3.7 5.1; [2331, 5120] 2 bits 10.1 6.9 7.1 7.8, with zero points (whose constants take a division each) 15.7 10.0 8.4 10.1; [4096, 4096] 12.7 9.4
+// 8.6 8.5, with outliers 28 18.5 12.6 13.2; [8192, 4096] with zero points 37.7 21.7 19.6 17.3; [4096, 11008] 30.3 21.9 20.4 23.0.  Dequantiser with
+// outliers: [256, 4096] 3.4 4.0 4.8 6.3, [1024, 4096] 5.0 5.2 5.9 8.0, [4096, 4096] 11.6 9.5 9.4 9.9 (without: 2 at every size).
+static int quant_rows_by_size(int64_t elements, bool zero_point) {
+    if (zero_point) return elements > (1 << 24) ? 16 : 8;
+    return elements <= 3 * (1 << 21) ? 4 : 8;
+}
+static int dequant_rows_by_size(int64_t elements) { return elements <= 3 * (1 << 21) ? 2 : 8; }
+
 #define HYC_LAUNCH_QBIT(KERNEL, QB)                                                                 \
     do {                                                                                            \
         if (zp && k)       hipLaunchKernelGGL((KERNEL<QB, true, true>), grid, block, 0, st, a);    \
@@ -530,6 +575,7 @@ extern "C" int hyc_quant_pack(const void* x, const void* scale, const void* zero
     const void* zp = zero_point;
     QuantArgs a = make_args(x, scale, zp, q, outlier_idx, k, x_outlier, zero_input, B, M, N, stride_b, stride_m,
                             head_dim, stride_h, (outlier_idx && k) ? g_quant_outlier_rows_per_wave.get() : g_quant_rows_per_wave.get());
+    if (a.rows_per_wave == 0) a.rows_per_wave = quant_rows_by_size(a.T * N, zp != nullptr);
     const int64_t row_tiles = cdiv(a.T, (int64_t)kQuantWaves * a.rows_per_wave);
     if (row_tiles * a.col_tiles > INT32_MAX) return HYC_ERR_SHAPE;
     const dim3 grid((unsigned)(row_tiles * a.col_tiles)), block(kQuantThreads);
@@ -550,6 +596,7 @@ extern "C" int hyc_unpack_dequant(const void* q, const void* scale, const void* 
     const void* zp = zero_point;
     QuantArgs a = make_args(x, scale, zp, q, outlier_idx, k, x_outlier, 0, B, M, N, stride_b, stride_m, head_dim,
                             stride_h, (outlier_idx && k) ? g_dequant_outlier_rows_per_wave.get() : g_dequant_rows_per_wave.get());
+    if (a.rows_per_wave == 0) a.rows_per_wave = dequant_rows_by_size(a.T * N);
     const int64_t row_tiles = cdiv(a.T, (int64_t)kQuantWaves * a.rows_per_wave);
     if (row_tiles * a.col_tiles > INT32_MAX) return HYC_ERR_SHAPE;
     const dim3 grid((unsigned)(row_tiles * a.col_tiles)), block(kQuantThreads);

@@ -46,9 +46,9 @@ int hyc_abi_version(void);
  * squares; "contract_strip_rows").  Each knob is an atomic integer that an entry point reads once per launch, so a launch on another
  * thread runs with the old or the new value of each knob, never a torn one; a pair of calls that must agree
  * (hyc_channel_stats_strips, then hyc_channel_stats) must not straddle a change.  Keys: "quant_rows_per_wave" (rows each wave walks in hyc_quant_pack,
- * default 8), "dequant_rows_per_wave" (same for hyc_unpack_dequant, default 2),
+ * by size until set), "dequant_rows_per_wave" (same for hyc_unpack_dequant, default 2),
  * "quant_outlier_rows_per_wave" / "dequant_outlier_rows_per_wave" (the same two when called with
- * an outlier list; default 8 each: a wave first has to find its outlier columns in the list),
+ * an outlier list; by size until set),
  * "norm_compress_slab" (0 / 1: whether hyc_rmsnorm_fwd_compress and, for rows wider than 4096 channels,
  * hyc_rmsnorm_bwd without a weight gradient may use the column-slab kernels, default 1)
  * and "norm_compress_rows_per_group" (rows a workgroup of that kernel walks, even; 0 = chosen from the
@@ -86,10 +86,13 @@ int hyc_set_tuning(const char *key, int value);
  *   outlier_idx int64 [k] channel numbers or NULL (k = 0).  Those columns are copied to
  *              x_outlier (bf16 [B, M, k], column order = order of outlier_idx) and are
  *              quantised as if they were zero.  If zero_input != 0 the columns are also
- *              zeroed in x itself, as the reference does.
+ *              zeroed in x itself, as the reference does.  A list position without a column of its
+ *              own (a channel outside the tensor, the earlier copies of a repeated one) is
+ *              written as zeros for k <= HYC_OUTLIER_ZERO_MAX, else left as it is.
  *   code rule  t = fp32(x)/fp32(scale) (+ zero_point); r = roundf(t) (ties away from zero);
  *              code = clamp(r, -2^(q-1), 2^(q-1)-1) + 2^(q-1); NaN -> 0.
  */
+#define HYC_OUTLIER_ZERO_MAX 256
 int hyc_quant_pack(const void *x, const void *scale, const void *zero_point, void *q,
                    const int64_t *outlier_idx, int64_t k, void *x_outlier, int zero_input,
                    int64_t B, int64_t M, int64_t N,
