@@ -370,25 +370,33 @@ def compress_attention_map(x: torch.Tensor, outlier, seg_offsets=None, compare_a
         if seg_offsets.numel() != nseg + 1 or seg_offsets.dtype != torch.int64:
             raise ValueError("seg_offsets does not belong to a map of this size")
         _lib.require_gpu(seg_offsets)
-        offsets = seg_offsets
+        offsets, kept = seg_offsets, None
     else:
+        # the count leaves the kept entries in scratch memory, a quarter of the map, for the write
+        kept = torch.empty(_lib.lib().hyc_sparse_kept_bytes(n), device=x.device, dtype=torch.uint8)
         counts = torch.empty(max(nseg, 1), device=x.device, dtype=torch.int32)
         offsets = torch.empty(nseg + 1, device=x.device, dtype=torch.int64)
-        _lib.call("hyc_sparse_count", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), counts.data_ptr(),
-                  offsets.data_ptr(), st)
+        _lib.call("hyc_sparse_count_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), counts.data_ptr(), offsets.data_ptr(),
+                  kept.data_ptr(), st)
+
+    def write(idx, val):
+        if kept is None:
+            _lib.call("hyc_sparse_write_bounded", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), idx.numel(),
+                      idx.data_ptr(), val.data_ptr(), st)
+        else:
+            _lib.call("hyc_sparse_write_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), kept.data_ptr(), idx.numel(),
+                      idx.data_ptr(), val.data_ptr(), st)
     if capacity is not None:
         capacity = int(capacity)
         idx = torch.empty(capacity, device=x.device, dtype=torch.int64)
         val = torch.empty(capacity, device=x.device, dtype=BF16)
-        _lib.call("hyc_sparse_write_bounded", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(),
-                  capacity, idx.data_ptr(), val.data_ptr(), st)
+        write(idx, val)
         return idx, val, offsets, PendingCount(offsets[-1:])
     nnz = int(offsets[-1].item())      # the one host sync; to_sparse() has the same one
     idx = torch.empty(nnz, device=x.device, dtype=torch.int64)
     val = torch.empty(nnz, device=x.device, dtype=BF16)
     if nnz:
-        _lib.call("hyc_sparse_write", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(),
-                  idx.data_ptr(), val.data_ptr(), st)
+        write(idx, val)
     return idx, val, offsets
 
 

@@ -205,6 +205,10 @@ int hyc_hist_select(const uint32_t *hist, int64_t kth, float *threshold, void *s
  *                      output positions >= capacity are not written.  The list is complete exactly
  *                      when seg_offsets[nseg] <= capacity, which the caller checks when it suits it;
  *                      a truncated list must not be handed to hyc_sparse_restore / hyc_softmax_bwd_restore.
+ *   hyc_sparse_count_staged / hyc_sparse_write_staged    the count and the bounded write of one map with the kept entries handed
+ *                      from one to the other in `kept`, device scratch of hyc_sparse_kept_bytes(n) (a quarter of the map's)
+ *                      bytes, 4-byte aligned: the map is then read once, but for segments that keep more than an eighth
+ *                      of their elements.  Same lists.
  *   hyc_sparse_segment_offsets  rebuilds seg_offsets from an ascending index list (for sparse
  *                      tensors that did not come from hyc_sparse_count).
  *   hyc_sparse_restore out bf16 [n] (16-byte aligned): zeros, with values[i] at indices[i].
@@ -217,6 +221,11 @@ int hyc_sparse_write(const void *a, int64_t n, const float *threshold, int compa
 int hyc_sparse_write_bounded(const void *a, int64_t n, const float *threshold, int compare_abs,
                              const int64_t *seg_offsets, int64_t capacity, int64_t *indices, void *values,
                              void *stream);
+int64_t hyc_sparse_kept_bytes(int64_t n);
+int hyc_sparse_count_staged(const void *a, int64_t n, const float *threshold, int compare_abs, uint32_t *seg_counts,
+                            int64_t *seg_offsets, void *kept, void *stream);
+int hyc_sparse_write_staged(const void *a, int64_t n, const float *threshold, int compare_abs, const int64_t *seg_offsets,
+                            const void *kept, int64_t capacity, int64_t *indices, void *values, void *stream);
 int hyc_sparse_segment_offsets(const int64_t *indices, int64_t nnz, int64_t n, int64_t *seg_offsets,
                                void *stream);
 int hyc_sparse_restore(const int64_t *indices, const void *values, const int64_t *seg_offsets,
