@@ -388,10 +388,11 @@ def compress_attention_map(x: torch.Tensor, outlier, seg_offsets=None, compare_a
                       idx.data_ptr(), val.data_ptr(), st)
     if capacity is not None:
         capacity = int(capacity)
+        pending = PendingCount(offsets[-1:])            # known before the lists are written: who waits for it does not wait for those
         idx = torch.empty(capacity, device=x.device, dtype=torch.int64)
         val = torch.empty(capacity, device=x.device, dtype=BF16)
         write(idx, val)
-        return idx, val, offsets, PendingCount(offsets[-1:])
+        return idx, val, offsets, pending
     nnz = int(offsets[-1].item())      # the one host sync; to_sparse() has the same one
     idx = torch.empty(nnz, device=x.device, dtype=torch.int64)
     val = torch.empty(nnz, device=x.device, dtype=BF16)
