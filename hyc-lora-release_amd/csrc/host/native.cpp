@@ -703,6 +703,43 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> gated_backward(const Tensor& x
     return std::make_tuple(o, gg, gu);
 }
 
+// The gated product of layers that keep every activation as codes; `steps` of gate, up, fn and the product, in that order
+std::optional<std::vector<Tensor>> silu_mul_codes(const Tensor& gate, const Tensor& up, const std::vector<Tensor>& steps, int64_t bits) {
+    if (!plain(gate) || !plain(up) || gate.dim() < 2 || gate.sizes() != up.sizes() || !bits_ok(bits) || steps.size() != 4 || gate.numel() == 0)
+        return std::nullopt;
+    const int64_t n = gate.size(-1);
+    if (n % 32) return std::nullopt;
+    const void* s[4];
+    void* q[4];
+    std::vector<Tensor> out;
+    for (int k = 0; k < 4; ++k) {
+        if (!vec(steps[k], n)) return std::nullopt;
+        out.push_back(bytes_like(gate, n, bits));
+        s[k] = steps[k].data_ptr();
+        q[k] = out[k].data_ptr();
+    }
+    out.push_back(at::empty_like(gate));
+    check("hyc_silu_mul_codes", hyc_silu_mul_codes(gate.data_ptr(), up.data_ptr(), s, q, out[4].data_ptr(), gate.numel() / n, n, (int)bits,
+                                                   stream_of(gate)));
+    return out;
+}
+std::optional<std::tuple<Tensor, Tensor>> silu_mul_bwd_codes(const std::vector<Tensor>& codes, const std::vector<Tensor>& steps, const Tensor& grad,
+                                                             int64_t bits) {
+    if (!plain(grad) || grad.dim() < 2 || grad.numel() == 0 || !bits_ok(bits) || codes.size() != 3 || steps.size() != 3) return std::nullopt;
+    const int64_t n = grad.size(-1);
+    if (n % 32) return std::nullopt;
+    const void *s[3], *q[3];
+    for (int k = 0; k < 3; ++k) {
+        if (!vec(steps[k], n) || !packed(codes[k], grad.numel(), bits) || !aligned(codes[k])) return std::nullopt;
+        s[k] = steps[k].data_ptr();
+        q[k] = codes[k].data_ptr();
+    }
+    Tensor gg = at::empty_like(grad), gu = at::empty_like(grad);
+    check("hyc_silu_mul_bwd_codes", hyc_silu_mul_bwd_codes(q, s, grad.data_ptr(), gg.data_ptr(), gu.data_ptr(), grad.numel() / n, n, (int)bits,
+                                                           stream_of(grad)));
+    return std::make_tuple(gg, gu);
+}
+
 // ---- NF4 weights --------------------------------------------------------------------------------------------------
 OptT nf4_dequant(const Tensor& packed_w, const Tensor& absmax, const Tensor& code2, const Tensor& absmax2, const OptT& offset, const Tensor& table,
                  int64_t rows, int64_t cols, int64_t blocksize, int64_t blocksize2) {
@@ -749,5 +786,7 @@ PYBIND11_MODULE(_native, m) {
     m.def("rope", &rope);
     m.def("gated_forward", &gated_forward);
     m.def("gated_backward", &gated_backward);
+    m.def("silu_mul_codes", &silu_mul_codes);
+    m.def("silu_mul_bwd_codes", &silu_mul_bwd_codes);
     m.def("nf4_dequant", &nf4_dequant);
 }

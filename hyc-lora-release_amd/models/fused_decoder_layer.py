@@ -55,7 +55,8 @@ from ..operators.compress_function import (compress_attention_map, compression_p
 from ..operators.rmsnorm_kernels import _backward as _rmsnorm_backward
 from ..operators.rmsnorm_kernels import (backward_from_codes_supported, lora_a_supported, rmsnorm_backward_from_codes, rmsnorm_forward,
                                          rmsnorm_forward_compress)
-from ..operators.silu_kernels import silu_backward, silu_hadamard, silu_hadamard_backward, silu_once_hadamard
+from ..operators.silu_kernels import (silu_backward, silu_hadamard, silu_hadamard_backward, silu_hadamard_backward_codes,
+                                      silu_hadamard_codes, silu_once_hadamard)
 from ..operators.softmax_kernels import softmax_backward, softmax_backward_from_compressed, softmax_forward
 from ..operators.triton_fuse_lora_silu_hadamard_backward_kernels import triton_fuse_silu_backward
 from ..operators.triton_fuse_lora_silu_hadamard_forward_kernels import triton_fuse_silu_forward
@@ -437,19 +438,32 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             else:                                           # 'intra' and 'baseline'
                 gate, _, gate_lora_a = proj("gate", x_norm_2)
                 up, _, up_lora_a = proj("up", x_norm_2)
-                fn = F.silu(gate)
-                quant("gate", gate)
-                hadamard = up * fn
-                quant("up", up)
-                quant("fn", fn)
-                del fn
+                # both products, silu and the four quantisers in one pass where the steps are known: [2040, 13824], 8 bits,
+                # 110 -> 60 us
+                kept = ("gate", "up", "fn", "hadamard")
+                done = None
+                if not raw and not calib and gate.is_cuda:
+                    done = silu_hadamard_codes(gate, up, [sv[n]["scale"] for n in kept], q_bit)
+                if done is not None:
+                    for n, codes in zip(kept, done):
+                        stats[(n, "scale")] = saved[n + "_s"] = sv[n]["scale"]
+                        saved[n + "_q"] = codes
+                    hadamard = done[4]
+                    del done, codes
+                else:
+                    fn = F.silu(gate)
+                    quant("gate", gate)
+                    hadamard = up * fn
+                    quant("up", up)
+                    quant("fn", fn)
+                    del fn
             del gate, up
         saved["gate_lora_a"], saved["up_lora_a"] = gate_lora_a, up_lora_a
         if not norm_2_done:
             quant("x_norm_2", x_norm_2)
         del x_norm_2
         x_out, _, saved["down_lora_a"] = proj("down", hadamard, residual=x_medium)
-        if whole:
+        if whole and "hadamard_q" not in saved:
             quant("hadamard", hadamard)
         del hadamard
 
@@ -599,7 +613,8 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
             del hadamard, grad_down, wd                   # a dequantised weight is let go before the next ones are made
         else:
             fn = None
-            if spec.mode == "intra_inter":
+            whole = spec.mode != "intra_inter"
+            if not whole:
                 gu = rebuilt_hidden_group(("gate", "up"))
                 gate, up = gu["gate"][0], gu["up"][0]
                 del gu
@@ -608,20 +623,28 @@ class FusedDecoderLayerFunc(torch.autograd.Function):
                 else:
                     hadamard = up * F.silu(gate)
             else:
-                hadamard, up, fn, gate = deq("hadamard"), deq("up"), deq("fn"), deq("gate")
+                hadamard = "hadamard"                         # by its saved name: read from its codes
             grad_down = back("down", hadamard, S["down_lora_a"], grad_output)
             del hadamard
-            if fn is None and grad_down.dtype == gate.dtype == torch.bfloat16:
+            if whole:
+                kept, done = ("gate", "up", "fn"), None
+                if "fn_q" in S and grad_down.is_cuda:
+                    done = silu_hadamard_backward_codes([S[n + "_q"] for n in kept], [S[n + "_s"] for n in kept], grad_down, q_bit)
+                if done is not None:
+                    grad_fn, grad_h2 = done
+                    up = gate = None
+                else:
+                    up, fn, gate = deq("up"), deq("fn"), deq("gate")
+                    grad_fn, grad_h2 = silu_backward(gate, grad_down * up), grad_down * fn
+                del done
+            elif grad_down.dtype == gate.dtype == torch.bfloat16:
                 # grad_down * up, silu_backward of it, and grad_down * silu(gate): one pass
                 grad_fn, grad_h2 = silu_hadamard_backward(gate, up, grad_down)
             else:
-                if fn is None:
-                    fn = F.silu(gate)
-                grad_h1 = grad_down * up
-                grad_h2 = grad_down * fn
-                grad_fn = silu_backward(gate, grad_h1)
-                del grad_h1
-            del grad_down, up, fn, gate
+                fn = F.silu(gate)
+                grad_fn, grad_h2 = silu_backward(gate, grad_down * up), grad_down * fn
+            del grad_down, up, gate
+            fn = None
         grad_x2 = back_shared({"gate": grad_fn, "up": grad_h2}, "x_norm_2")
         del grad_fn, grad_h2
         grad_medium, grad_nw2 = norm_backward(grad_x2, "x_medium", norm_weight_2, S["rstd_2"], ctx.norm_grads[1], grad_output)

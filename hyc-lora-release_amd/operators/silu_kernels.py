@@ -36,3 +36,16 @@ def silu_hadamard_backward(x, u, g):
     _lib.call("hyc_silu_mul_bwd", x.data_ptr(), u.data_ptr(), g.data_ptr(), gx.data_ptr(), gu.data_ptr(), x.numel(),
               _lib.stream_of(x))
     return gx, gu
+
+
+def silu_hadamard_codes(gate, up, scales, quantize_bit):
+    """(gate_q, up_q, fn_q, hadamard_q, hadamard) of fn = F.silu(gate), hadamard = up * fn in one pass, the codes by the
+    four step vectors `scales`: the values of F.silu, the product and four quantisers, as the reference's layer composes
+    them (models/llama/fused_llama_layer_intra.py:234-255).  None where the kernel does not take the operands."""
+    return _lib.native().silu_mul_codes(gate, up, list(scales), quantize_bit)
+
+
+def silu_hadamard_backward_codes(codes, scales, grad, quantize_bit):
+    """(silu_backward(gate, grad * up), grad * fn) from the codes of gate, up and fn, or None where the kernel does not
+    take the operands (models/llama/fused_llama_layer_intra.py:330-362)."""
+    return _lib.native().silu_mul_bwd_codes(list(codes), list(scales), grad, quantize_bit)

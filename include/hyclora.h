@@ -473,6 +473,14 @@ int hyc_silu_once_mul(const void *x1, const void *x2, void *out, int64_t n, void
  * that do not use the fused LoRA kernels (models/llama/fused_llama_layer_intra_inter.py:362-381). */
 int hyc_silu_mul_bwd(const void *x, const void *u, const void *g, void *grad_x, void *grad_u, int64_t n,
                      void *stream);
+/* The gated product of layers that keep every activation as codes: fn = bf16(silu(gate)), out = bf16(up * fn), and the codes of
+ * gate, up, fn and out by steps[0..3] into codes[0..3]; gate, up and out [T, N], N a multiple of 32
+ * (models/llama/fused_llama_layer_intra.py:234-255). */
+int hyc_silu_mul_codes(const void *gate, const void *up, const void *const *steps, void *const *codes, void *out,
+                       int64_t T, int64_t N, int q_bit, void *stream);
+/* Its backward from the codes of gate, up and fn: grad_up = grad * fn, grad_gate = hyc_silu_bwd(gate, bf16(grad * up)) (:330-362). */
+int hyc_silu_mul_bwd_codes(const void *const *codes, const void *const *steps, const void *grad, void *grad_gate,
+                           void *grad_up, int64_t T, int64_t N, int q_bit, void *stream);
 int hyc_gelu_bwd(const void *x, const void *g, void *out, int64_t n, void *stream);
 
 /* ---------------------------------------------------------------------------------------
