@@ -75,6 +75,7 @@ struct QuantArgs {
 struct OutlierLane {
     uint32_t mask = 0;        // bit j: column col0 + j is an outlier
     uint32_t pos[4] = {0, 0, 0, 0};  // 16-bit list positions, two per dword
+    bool unused = false;      // an entry the wave sees has no column of its own (see clear_unused)
     // dword p of the lane's chunk with its outlier columns cleared: d & keep(p)
     __device__ __forceinline__ uint32_t keep(int p) const {
         const uint32_t two = mask >> (2 * p);
@@ -88,12 +89,13 @@ __device__ __forceinline__ int first_entries(const int64_t* oidx, int k, int lan
     return lane < k ? ch : -1;
 }
 
-__device__ __forceinline__ OutlierLane find_outliers(const int64_t* oidx, int k, int wave_col0, int col0, int lane, int first) {
+__device__ __forceinline__ OutlierLane find_outliers(const int64_t* oidx, int k, int N, int wave_col0, int col0, int lane, int first) {
     OutlierLane o;
     for (int base = 0; base < k; base += kWave) {
         const int e = base + lane;
         const int ch = base == 0 ? first : (e < k) ? (int)oidx[e] : -1;
         const bool hit = (unsigned)(ch - wave_col0) < (unsigned)(kWave * 8);
+        if (wave_col0 == 0) o.unused = o.unused || (e < k && (unsigned)ch >= (unsigned)N);
         unsigned long long hits = __ballot(hit);
         while (hits) {
             const int src = __ffsll((long long)hits) - 1;
@@ -101,6 +103,7 @@ __device__ __forceinline__ OutlierLane find_outliers(const int64_t* oidx, int k,
             const int c = __builtin_amdgcn_readlane(ch, src);
             const int d = c - col0;
             if ((unsigned)d < 8u) {
+                o.unused = o.unused || (o.mask >> d & 1u);
                 o.mask |= 1u << d;
                 const uint32_t p = (uint32_t)(base + src) << (16 * (d & 1));
                 const uint32_t keep = 0xffff0000u >> (16 * (d & 1));
@@ -163,16 +166,19 @@ __device__ __forceinline__ void extract_rest(const OutlierLane& o, uint32_t bits
 }
 
 // A list position without a column of its own - a channel outside the tensor, the earlier copies of a repeated one - reads as zero.
-// Written by the waves of the first column tile for their rows, for lists of up to kOutlierZeroMax entries (every entry is compared
-// with all behind it); callers clear x_outlier beforehand for longer ones.
+// find_outliers notes where there is one: the wave whose window holds a channel sees its copies, the waves of the first window see the
+// channels outside.  Only these waves look for the positions (every entry against all behind it) and clear them for their rows, for
+// lists of up to kOutlierZeroMax entries; callers clear x_outlier beforehand for longer ones.  (Done by the waves of the first window
+// whatever the list, it cost them 2 us each, on one compute die where the windows of a row are a multiple of 8: 34 -> 48 us for
+// [8192, 8192] at 2 bits, 52 -> 55 for [6904, 13664].)
 constexpr int kOutlierZeroMax = HYC_OUTLIER_ZERO_MAX;
-__device__ __forceinline__ void clear_unused(const QuantArgs& a, int64_t row0, int64_t row1, int lane, int first) {
+__device__ __forceinline__ void clear_unused(const QuantArgs& a, int64_t row0, int64_t row1, int lane) {
     for (int base = 0; base < a.k; base += kWave) {
         const int e = base + lane;
-        const int ch = base == 0 ? first : e < a.k ? (int)a.oidx[e] : -1;
+        const int ch = e < a.k ? (int)a.oidx[e] : -1;
         bool unused = (unsigned)ch >= (unsigned)a.N;
         for (int b2 = base; b2 < a.k; b2 += kWave) {
-            const int c2 = b2 == base ? ch : b2 + lane < a.k ? (int)a.oidx[b2 + lane] : -1;
+            const int c2 = b2 + lane < a.k ? (int)a.oidx[b2 + lane] : -1;
             const int n = a.k - b2 < kWave ? a.k - b2 : kWave;
             for (int i = 0; i < n; ++i)
                 unused = unused || (e < b2 + i && ch == __builtin_amdgcn_readlane(c2, i));
@@ -240,11 +246,12 @@ __device__ __forceinline__ void load_rows(const QuantArgs& a, RowCursor& cur, in
 // whole number of row groups).  That variant has no predicates or branches around its memory
 // operations, which is what lets the compiler count outstanding operations exactly and emit
 // s_waitcnt vmcnt(<stores in flight>) instead of vmcnt(0) at the top of the loop.
+// -> whether clear_unused is the wave's to run
 template <int QBIT, bool ZP, bool OUTL, bool FAST, bool FULL>
-__device__ __forceinline__ void quant_rows(const QuantArgs& a, int64_t row0, int64_t row1, bool active, int chunk,
+__device__ __forceinline__ bool quant_rows(const QuantArgs& a, int64_t row0, int64_t row1, bool active, int chunk,
                                            int64_t coff, const QuantCols<QBIT>& qc, const float (&z)[8]) {
     const int row_bytes = a.N * QBIT / 8;
-    if (row0 >= row1) return;
+    if (row0 >= row1) return false;
     RowCursor cur(row0, a.M, a.stride_b, a.stride_m);
     u32x4 v[kRowUnroll];
     int64_t roff[kRowUnroll];
@@ -254,8 +261,7 @@ __device__ __forceinline__ void quant_rows(const QuantArgs& a, int64_t row0, int
     // the first rows are already on their way while the wave looks up its outlier columns
     OutlierLane ol;
     if constexpr (OUTL) {
-        ol = find_outliers(a.oidx, a.k, (chunk & ~(kWave - 1)) * 8, chunk * 8, chunk & (kWave - 1), entry);
-        if (a.k <= kOutlierZeroMax && chunk < kWave) clear_unused(a, row0, row1, chunk, entry);     // uniform: the wave of the first columns
+        ol = find_outliers(a.oidx, a.k, a.N, (chunk & ~(kWave - 1)) * 8, chunk * 8, chunk & (kWave - 1), entry);
     }
     const OutlierFirst of(ol);
     const bool in_place = OUTL && a.zero_input != 0;
@@ -306,6 +312,7 @@ __device__ __forceinline__ void quant_rows(const QuantArgs& a, int64_t row0, int
         compute(v, t0, lo, hi);                                // last group: nothing left to load
     }
     store(t0, lo, hi);
+    return OUTL && __any(ol.unused);
 }
 
 template <int QBIT, bool ZP, bool OUTL>
@@ -336,12 +343,16 @@ void quant_pack_kernel(const QuantArgs a) {
                       a.rows_per_wave % kRowUnroll == 0;      // uniform across the wave
     // one slow column anywhere in the wave sends the whole wave down the IEEE-division path
     const bool fast = ZP ? qc.scale_for_zero_point(z) : __ballot(!qc.fast) == 0ull;
+    bool unused;
     if (!fast)
-        quant_rows<QBIT, ZP, OUTL, false, false>(a, row0, row1, active, chunk, coff, qc, z);
+        unused = quant_rows<QBIT, ZP, OUTL, false, false>(a, row0, row1, active, chunk, coff, qc, z);
     else if (full)
-        quant_rows<QBIT, ZP, OUTL, true, true>(a, row0, row1, active, chunk, coff, qc, z);
+        unused = quant_rows<QBIT, ZP, OUTL, true, true>(a, row0, row1, active, chunk, coff, qc, z);
     else
-        quant_rows<QBIT, ZP, OUTL, true, false>(a, row0, row1, active, chunk, coff, qc, z);
+        unused = quant_rows<QBIT, ZP, OUTL, true, false>(a, row0, row1, active, chunk, coff, qc, z);
+    if constexpr (OUTL) {
+        if (unused && a.k <= kOutlierZeroMax) clear_unused(a, row0, row1, lane);
+    }
 }
 
 // ------------------------------------------------------------------------------------
@@ -466,7 +477,7 @@ __global__ __launch_bounds__(kQuantThreads) void unpack_dequant_kernel(const Qua
         load_codes(row0);
         // the first codes are already on their way while the wave looks up its outlier columns
         if constexpr (OUTL) {
-            ol = find_outliers(a.oidx, a.k, col_tile * kWave * 8, col0, lane, entry);
+            ol = find_outliers(a.oidx, a.k, a.N, col_tile * kWave * 8, col0, lane, entry);
             of = OutlierFirst(ol);
         }
         load_outliers(row0);
@@ -535,9 +546,9 @@ static QuantArgs make_args(const void* x, const void* scale, const void* zp, con
 }
 
 // Strip heights by size: a small tensor is one short generation of waves, whose strips are serial chains; long strips spread the columns'
-// constants over more rows.  us at 2, 4, 8, 16 rows, quantiser: [1024, 4096] 4.8 4.1 4.6 5.9, with outliers 8.8 7.1 7.5 9.4; [256, 2048] 3.2 3.0
+// constants over more rows.  us at 2, 4, 8, 16 rows, quantiser: [1024, 4096] 4.8 4.1 4.6 5.9, with outliers 7.1 6.0 7.1 10.1; [256, 2048] 3.2 3.0
 // 3.7 5.1; [2331, 5120] 2 bits 10.1 6.9 7.1 7.8, with zero points (whose constants take a division each) 15.7 10.0 8.4 10.1; [4096, 4096] 12.7 9.4
-// 8.6 8.5, with outliers 28 18.5 12.6 13.2; [8192, 4096] with zero points 37.7 21.7 19.6 17.3; [4096, 11008] 30.3 21.9 20.4 23.0.  Dequantiser with
+// 8.6 8.5, with outliers 20.1 12.2 9.7 11.3; [8192, 4096] with zero points 37.7 21.7 19.6 17.3; [4096, 11008] 30.3 21.9 20.4 23.0.  Dequantiser with
 // outliers: [256, 4096] 3.4 4.0 4.8 6.3, [1024, 4096] 5.0 5.2 5.9 8.0, [4096, 4096] 11.6 9.5 9.4 9.9 (without: 2 at every size).
 static int quant_rows_by_size(int64_t elements, bool zero_point) {
     if (zero_point) return elements > (1 << 24) ? 16 : 8;
