@@ -39,6 +39,12 @@ bool products_are_plain() {
     return !at::GradMode::is_enabled() && !(at::autocast::is_autocast_enabled(at::kCUDA) && at::autocast::get_autocast_dtype(at::kCUDA) != at::kBFloat16);
 }
 void* ptr(const OptT& t) { return t ? t->data_ptr() : nullptr; }
+// Whether operands lie on the GPU of `like`.  Asked wherever a kernel of this package stands in for library calls, which refuse
+// operands of several devices: a kernel would take an address of another GPU's memory for one of its own
+bool there(const Tensor& t, const Tensor& like) { return t.defined() && t.device() == like.device(); }
+bool there(const OptT& t, const Tensor& like) { return !t || there(*t, like); }
+template <class... T>
+bool together(const Tensor& like, const T&... others) { return (there(others, like) && ...); }
 bool bits_ok(int64_t b) { return b == 2 || b == 4 || b == 8; }
 bool packed(const Tensor& q, int64_t numel, int64_t bits) {
     return q.defined() && q.is_cuda() && q.scalar_type() == at::kByte && q.is_contiguous() && q.numel() * 8 == numel * bits;
@@ -238,6 +244,7 @@ std::optional<std::vector<std::tuple<Tensor, Tensor, Tensor>>> lora_products_sha
     hyc_contract_job g[3] = {}, s[3] = {};
     for (size_t i = 0; i < count; ++i) {
         const auto& [la, lb, xa, grad] = members[i];
+        if (!together(std::get<3>(members[0]), la, lb, xa, grad, x, q, scale, zero)) return std::nullopt;
         const Lora L(lb);
         if (!plain(grad) || grad.dim() < 2 || grad.numel() == 0 || !L.fits(grad.size(-1)) || L.r > 16 || (i && L.r != r)) return std::nullopt;
         const int64_t rows = grad.numel() / L.n;
@@ -417,8 +424,10 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> lora_forward(const Tensor& w, 
 }
 
 // ---- projections in one pass, product included ----------------------------------------------------------------------
-// Whether hyc_lora_gemm takes the operands of one projection of `rows` rows: W [n, k] (or, as an input gradient, [k, n]), B and x A
-bool gemm_member(const Tensor& w, const Tensor& lb, const Tensor& xa, int64_t rows, int64_t n, int64_t k, const OptT& bias, hyc_gemm_member& m) {
+// Whether hyc_lora_gemm takes the operands of one projection of the rows of x: W [n, k] (or, as an input gradient, [k, n]), B and x A
+bool gemm_member(const Tensor& x, const Tensor& w, const Tensor& lb, const Tensor& xa, int64_t rows, int64_t n, int64_t k, const OptT& bias,
+                 hyc_gemm_member& m) {
+    if (!together(x, w, lb, xa, bias)) return false;
     const Lora L(lb);
     if (!is_bf(w) || w.dim() != 2 || !w.is_contiguous() || !aligned(w) || n % 128 || k % 64 || rows * k >= int64_t{1} << 31 || n * k >= int64_t{1} << 31)
         return false;
@@ -445,6 +454,7 @@ std::optional<std::vector<std::tuple<Tensor, Tensor, OptT>>> lora_project(const 
     if ((codes && !bits_ok(bits)) || (main_only && (codes || gelu || residual))) return std::nullopt;
     std::vector<Tensor> adapters;
     for (const auto& [w, la, lb, bias, scale] : members) {
+        if (!together(x, w, la, lb, bias, scale, residual)) return std::nullopt;
         if (!is_bf(w) || w.dim() != 2 || w.size(1) != k || !gemm_is_faster(w.size(0), k) || scale.has_value() != codes ||
             (scale && !vec(*scale, w.size(0))))
             return std::nullopt;
@@ -462,7 +472,7 @@ std::optional<std::vector<std::tuple<Tensor, Tensor, OptT>>> lora_project(const 
     std::vector<std::tuple<Tensor, Tensor, OptT>> out;
     for (size_t i = 0; i < members.size(); ++i) {
         const auto& [w, la, lb, bias, scale] = members[i];
-        if (!gemm_member(w, lb, xa[i], rows, w.size(0), k, bias, m[i])) return std::nullopt;
+        if (!gemm_member(x, w, lb, xa[i], rows, w.size(0), k, bias, m[i])) return std::nullopt;
         shape.back() = w.size(0);
         Tensor y = at::empty(shape, x.options());
         OptT q;
@@ -490,8 +500,9 @@ OptT lora_input_grad(const std::vector<InputGrad>& members, const OptT& residual
     hyc_gemm_member m[3];
     for (size_t i = 0; i < members.size(); ++i) {
         const auto& [g, w, mid, at_] = members[i];
+        if (!together(first, g, residual)) return std::nullopt;
         if (!plain(g) || g.numel() != rows * g.size(-1) || w.dim() != 2 || w.size(0) != g.size(-1) || w.size(1) != n || at_.size(0) != r ||
-            !gemm_is_faster(n, w.size(0)) || !gemm_member(w, at_, mid, rows, n, w.size(0), std::nullopt, m[i]))
+            !gemm_is_faster(n, w.size(0)) || !gemm_member(g, w, at_, mid, rows, n, w.size(0), std::nullopt, m[i]))
             return std::nullopt;
         m[i].x = g.data_ptr();
     }
@@ -705,15 +716,17 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> gated_backward(const Tensor& x
 
 // The gated product of layers that keep every activation as codes; `steps` of gate, up, fn and the product, in that order
 std::optional<std::vector<Tensor>> silu_mul_codes(const Tensor& gate, const Tensor& up, const std::vector<Tensor>& steps, int64_t bits) {
-    if (!plain(gate) || !plain(up) || gate.dim() < 2 || gate.sizes() != up.sizes() || !bits_ok(bits) || steps.size() != 4 || gate.numel() == 0)
+    if (!plain(gate) || !plain(up) || !together(gate, up) || gate.dim() < 2 || gate.sizes() != up.sizes() || !bits_ok(bits) || steps.size() != 4 ||
+        gate.numel() == 0)
         return std::nullopt;
     const int64_t n = gate.size(-1);
     if (n % 32) return std::nullopt;
     const void* s[4];
     void* q[4];
     std::vector<Tensor> out;
+    for (const Tensor& step : steps)
+        if (!together(gate, step) || !vec(step, n)) return std::nullopt;
     for (int k = 0; k < 4; ++k) {
-        if (!vec(steps[k], n)) return std::nullopt;
         out.push_back(bytes_like(gate, n, bits));
         s[k] = steps[k].data_ptr();
         q[k] = out[k].data_ptr();
@@ -730,7 +743,7 @@ std::optional<std::tuple<Tensor, Tensor>> silu_mul_bwd_codes(const std::vector<T
     if (n % 32) return std::nullopt;
     const void *s[3], *q[3];
     for (int k = 0; k < 3; ++k) {
-        if (!vec(steps[k], n) || !packed(codes[k], grad.numel(), bits) || !aligned(codes[k])) return std::nullopt;
+        if (!together(grad, steps[k], codes[k]) || !vec(steps[k], n) || !packed(codes[k], grad.numel(), bits) || !aligned(codes[k])) return std::nullopt;
         s[k] = steps[k].data_ptr();
         q[k] = codes[k].data_ptr();
     }
