@@ -54,7 +54,7 @@ __global__ __launch_bounds__(kGcThreads) void gated_codes_fwd_kernel(const Gated
         qc[k].load(a.s[k], p.chunk * 8, p.active);
         fast = fast && qc[k].fast;
     }
-    const int row_bytes = a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;               // (the product first would pass 2^31 at 2^28 channels)
     auto run = [&](auto fast_tag) __attribute__((always_inline)) {
         constexpr bool FAST = decltype(fast_tag)::value;
         const float zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kGcThreads) void gated_codes_bwd_kernel(const Gated
     float s[3][8];
 #pragma unroll
     for (int k = 0; k < 3; ++k) unpack8(ld16(a.s[k] + p.ld_chunk * 8), s[k]);
-    const int64_t row_bytes = (int64_t)a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;
     u32x2 w[3];
     u32x4 gv;
     auto request = [&](int64_t t) __attribute__((always_inline)) {

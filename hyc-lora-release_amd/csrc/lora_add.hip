@@ -83,7 +83,7 @@ __device__ __forceinline__ void lora_add_rows(const LoraAddArgs& a, int64_t row_
                                               const BOperand<KSTEPS>& B) {
     const int g = lane >> 4;
     const int col0 = chunk * 8;
-    const int row_bytes = a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;               // (the product first would pass 2^31 at 2^28 channels)
     constexpr float kHalf = (float)(1 << (QBIT - 1));
     const PackedSlot<QBIT> slot(chunk);
     for (int64_t row0 = row_begin; row0 < row_end; row0 += kTileRows) {

@@ -94,7 +94,7 @@ __device__ __forceinline__ void fuse_fwd_rows(const FuseArgs& a, int64_t row_beg
                                               bool active, const QuantCols<QBIT>& c1, const QuantCols<QBIT>& c2,
                                               const BOperand<KSTEPS>& B1, const BOperand<KSTEPS>& B2) {
     const int g = lane >> 4;
-    const int row_bytes = a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;               // (the product first would pass 2^31 at 2^28 channels)
     const float zero8[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     auto load_x = [&](int64_t row0, u32x4 (&xv1)[4], u32x4 (&xv2)[4]) {
 #pragma unroll
@@ -157,7 +157,7 @@ __device__ __forceinline__ void fuse_fwd_rows_full(const FuseArgs& a, int64_t ro
                                                    const BOperand<KSTEPS>& B1, const BOperand<KSTEPS>& B2,
                                                    int wave = 0, uint8_t* stage = nullptr) {
     const int g = lane >> 4, i = lane & 15;
-    const int row_bytes = a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;               // (the product first would pass 2^31 at 2^28 channels)
     // MERGE: the waves of a workgroup that share the 128-byte lines of a row's codes (CT neighbouring column
     // tiles) hand their pieces over through LDS, and every line is written to memory whole, by one wave
     constexpr int CT = kFuseColTiles<QBIT>, RS = kFuseWaves / CT;
@@ -339,7 +339,7 @@ HYC_FUSE_KERNEL(HYC_BWD_DEEP) void lora_silu_bwd_kernel(const FuseArgs a) {
     B1.load(a.b1, a.N, a.R, col0, active, g, a.b_transposed != 0);
     B2.load(a.b2, a.N, a.R, col0, active, g, a.b_transposed != 0);
     const PackedSlot<QBIT> slot(chunk);
-    const int row_bytes = a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;               // (the product first would pass 2^31 at 2^28 channels)
 
     const int64_t row_begin = (row_tile * RS + wave / CT) * (int64_t)a.rows_per_wave;
     int64_t row_end = row_begin + a.rows_per_wave;

@@ -250,7 +250,7 @@ __device__ __forceinline__ void load_rows(const QuantArgs& a, RowCursor& cur, in
 template <int QBIT, bool ZP, bool OUTL, bool FAST, bool FULL>
 __device__ __forceinline__ bool quant_rows(const QuantArgs& a, int64_t row0, int64_t row1, bool active, int chunk,
                                            int64_t coff, const QuantCols<QBIT>& qc, const float (&z)[8]) {
-    const int row_bytes = a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;               // (the product first would pass 2^31 at 2^28 channels)
     if (row0 >= row1) return false;
     RowCursor cur(row0, a.M, a.stride_b, a.stride_m);
     u32x4 v[kRowUnroll];
@@ -387,7 +387,7 @@ __global__ __launch_bounds__(kQuantThreads) void unpack_dequant_kernel(const Qua
     const int64_t row0 = (row_tile * kQuantWaves + wave) * (int64_t)a.rows_per_wave;
     int64_t row1 = row0 + a.rows_per_wave;
     if (row1 > a.T) row1 = a.T;
-    const int row_bytes = a.N * QBIT / 8;
+    const int row_bytes = a.N / 8 * QBIT;               // (the product first would pass 2^31 at 2^28 channels)
 
     const PackedSlot<QBIT> slot(chunk);
 
