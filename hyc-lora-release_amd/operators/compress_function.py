@@ -372,33 +372,44 @@ def compress_attention_map(x: torch.Tensor, outlier, seg_offsets=None, compare_a
         _lib.require_gpu(seg_offsets)
         offsets, kept = seg_offsets, None
     else:
-        # the count leaves the kept entries in scratch memory, a quarter of the map, for the write
-        kept = torch.empty(_lib.lib().hyc_sparse_kept_bytes(n), device=x.device, dtype=torch.uint8)
+        # the count leaves the kept entries in scratch memory, a quarter of the map, for the write; where that does not fit beside
+        # the lists the map is read twice
         counts = torch.empty(max(nseg, 1), device=x.device, dtype=torch.int32)
         offsets = torch.empty(nseg + 1, device=x.device, dtype=torch.int64)
-        _lib.call("hyc_sparse_count_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), counts.data_ptr(), offsets.data_ptr(),
-                  kept.data_ptr(), st)
-
-    def write(idx, val):
+        try:
+            kept = torch.empty(_lib.lib().hyc_sparse_kept_bytes(n), device=x.device, dtype=torch.uint8)
+        except torch.OutOfMemoryError:
+            kept = None
         if kept is None:
-            _lib.call("hyc_sparse_write_bounded", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), idx.numel(),
-                      idx.data_ptr(), val.data_ptr(), st)
+            _lib.call("hyc_sparse_count", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), counts.data_ptr(), offsets.data_ptr(), st)
         else:
-            _lib.call("hyc_sparse_write_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), kept.data_ptr(), idx.numel(),
+            _lib.call("hyc_sparse_count_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), counts.data_ptr(), offsets.data_ptr(),
+                      kept.data_ptr(), st)
+
+    def lists(room):
+        return torch.empty(room, device=x.device, dtype=torch.int64), torch.empty(room, device=x.device, dtype=BF16)
+
+    def written(room):
+        nonlocal kept
+        try:
+            idx, val = lists(room)
+        except torch.OutOfMemoryError:
+            if kept is None:
+                raise
+            kept = None
+            idx, val = lists(room)
+        if kept is None:
+            _lib.call("hyc_sparse_write_bounded", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), room, idx.data_ptr(),
+                      val.data_ptr(), st)
+        else:
+            _lib.call("hyc_sparse_write_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), kept.data_ptr(), room,
                       idx.data_ptr(), val.data_ptr(), st)
+        return idx, val
     if capacity is not None:
-        capacity = int(capacity)
         pending = PendingCount(offsets[-1:])            # known before the lists are written: who waits for it does not wait for those
-        idx = torch.empty(capacity, device=x.device, dtype=torch.int64)
-        val = torch.empty(capacity, device=x.device, dtype=BF16)
-        write(idx, val)
-        return idx, val, offsets, pending
+        return *written(int(capacity)), offsets, pending
     nnz = int(offsets[-1].item())      # the one host sync; to_sparse() has the same one
-    idx = torch.empty(nnz, device=x.device, dtype=torch.int64)
-    val = torch.empty(nnz, device=x.device, dtype=BF16)
-    if nnz:
-        write(idx, val)
-    return idx, val, offsets
+    return *(written(nnz) if nnz else lists(0)), offsets
 
 
 def check_map_lists(idx, val, seg_offsets, numel: int) -> None:

@@ -36,3 +36,26 @@ def test_segments_of_every_density(n, compare_abs):
         # the lists again, exact, from the offsets alone
         again = cf.compress_attention_map(x.cuda(), thr.cuda(), out[2], compare_abs=compare_abs)
         assert torch.equal(again[0].cpu(), want) and torch.equal(again[1].cpu().view(torch.int16), x[want].view(torch.int16))
+
+
+@pytest.mark.parametrize("kept,room_mb", [(0.01, 28), (0.05, 68)])
+def test_scratch_that_does_not_fit(kept, room_mb):
+    """Where memory is left for the lists but not for a quarter of the map (32 of 128 MB) as well, the map is read twice: first the scratch
+    itself does not fit, then the lists do not fit beside it."""
+    import hyclora_amd  # noqa: F401
+    from hyclora_amd.operators import compress_function as cf
+    x = torch.rand(1 << 26, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3)).to(BF16)
+    thr = torch.tensor(1 - kept, device="cuda")
+    want = [t.cpu() for t in cf.compress_attention_map(x, thr)]
+    nnz = want[0].numel()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (room_mb << 20)) / total)
+        for capacity in (None, nnz):
+            got = cf.compress_attention_map(x, thr, capacity=capacity)
+            assert all(torch.equal(a.cpu(), b) for a, b in zip(got[:3], want))
+            del got
+            torch.cuda.empty_cache()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
