@@ -370,40 +370,45 @@ def compress_attention_map(x: torch.Tensor, outlier, seg_offsets=None, compare_a
         if seg_offsets.numel() != nseg + 1 or seg_offsets.dtype != torch.int64:
             raise ValueError("seg_offsets does not belong to a map of this size")
         _lib.require_gpu(seg_offsets)
-        offsets, kept = seg_offsets, None
+        offsets, scratch, kept = seg_offsets, None, None
     else:
-        # the count leaves the kept entries in scratch memory, a quarter of the map, for the write; where that does not fit beside
-        # the lists the map is read twice
-        counts = torch.empty(max(nseg, 1), device=x.device, dtype=torch.int32)
+        # The count leaves the kept entries in scratch memory, a quarter of the map, for the write; where that does not fit beside
+        # the lists the map is read twice.  So it is for lists of exact size up to 2^24 elements: the host waits for the count, which
+        # takes longer when it leaves entries behind (a call, us, read twice / once: 2^20 elements 33 / 37, 2^24 38 / 44, 2^25 53 / 52; with a capacity
+        # 38 / 35, 43 / 39, 58 / 46).
         offsets = torch.empty(nseg + 1, device=x.device, dtype=torch.int64)
-        try:
-            kept = torch.empty(_lib.lib().hyc_sparse_kept_bytes(n), device=x.device, dtype=torch.uint8)
-        except torch.OutOfMemoryError:
-            kept = None
+        count_bytes = -(-nseg // 4) * 16 + 16
+        kept = None
+        if capacity is not None or n > 1 << 24:
+            try:
+                scratch = torch.empty(count_bytes + _lib.lib().hyc_sparse_kept_bytes(n), device=x.device, dtype=torch.uint8)
+                kept = scratch.data_ptr() + count_bytes
+            except torch.OutOfMemoryError:
+                pass
         if kept is None:
-            _lib.call("hyc_sparse_count", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), counts.data_ptr(), offsets.data_ptr(), st)
+            scratch = torch.empty(count_bytes, device=x.device, dtype=torch.uint8)
+            _lib.call("hyc_sparse_count", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), scratch.data_ptr(), offsets.data_ptr(), st)
         else:
-            _lib.call("hyc_sparse_count_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), counts.data_ptr(), offsets.data_ptr(),
-                      kept.data_ptr(), st)
+            _lib.call("hyc_sparse_count_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), scratch.data_ptr(), offsets.data_ptr(), kept, st)
 
     def lists(room):
         return torch.empty(room, device=x.device, dtype=torch.int64), torch.empty(room, device=x.device, dtype=BF16)
 
     def written(room):
-        nonlocal kept
+        nonlocal scratch, kept
         try:
             idx, val = lists(room)
         except torch.OutOfMemoryError:
             if kept is None:
                 raise
-            kept = None
+            scratch = kept = None
             idx, val = lists(room)
         if kept is None:
             _lib.call("hyc_sparse_write_bounded", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), room, idx.data_ptr(),
                       val.data_ptr(), st)
         else:
-            _lib.call("hyc_sparse_write_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), kept.data_ptr(), room,
-                      idx.data_ptr(), val.data_ptr(), st)
+            _lib.call("hyc_sparse_write_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), kept, room, idx.data_ptr(),
+                      val.data_ptr(), st)
         return idx, val
     if capacity is not None:
         pending = PendingCount(offsets[-1:])            # known before the lists are written: who waits for it does not wait for those
