@@ -55,7 +55,6 @@ constexpr int kCtPitch = kCtTile + 8;                     // LDS row pitch of a 
 constexpr int kCtUPitch = kCtMaxStrip + 4;                // LDS pitch of a rank's column of U
 constexpr int kCtMembers = 3;                             // X's in a launch, or rank-R products of one X
 static Knob g_ct_strip{0};                                // rows of a strip, 0: by size; see hyc_set_tuning
-static Knob g_ct_max_groups{32};                          // no longer read; kept for callers that set it
 
 struct ContractMember {
     const uint16_t* x;                   // dense X [T, N]
@@ -558,11 +557,8 @@ static bool whole_rows(const hyc_contract_job* jobs, int count, int64_t T) {
 }
 
 int tune_contract(const char* key, int value) {
-    if (strcmp(key, "contract_max_groups") == 0) {
-        if (value < 1 || value > 65536) return HYC_ERR_ARG;
-        g_ct_max_groups.set(value);
-        return HYC_OK;
-    }
+    if (strcmp(key, "contract_max_groups") == 0)              // without effect; accepted from callers that set it
+        return value < 1 || value > 65536 ? HYC_ERR_ARG : HYC_OK;
     if (strcmp(key, "contract_strip_rows") == 0) {
         if (value < 0 || value > kCtMaxStrip || value % kCtSub) return HYC_ERR_ARG;
         g_ct_strip.set(value);

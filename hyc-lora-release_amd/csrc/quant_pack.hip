@@ -47,10 +47,12 @@ constexpr int kQuantThreads = kQuantWaves * kWave;
 constexpr int kRowUnroll = HYC_Q_UNROLL;       // quantiser: independent 128-bit loads in flight per lane
 constexpr int kDeqUnroll = HYC_D_UNROLL;       // dequantiser: rows per group
 
-static Knob g_quant_rows_per_wave{0};     // strip heights, 0: by size (see quant_rows_by_size); see hyc_set_tuning
-static Knob g_dequant_rows_per_wave{2};
-static Knob g_quant_outlier_rows_per_wave{0};     // the same two with an outlier list
-static Knob g_dequant_outlier_rows_per_wave{0};
+constexpr int kByRule = 0;                // strip heights by size (see quant_rows_by_size) until hyc_set_tuning sets one
+constexpr int kDequantRows = 2;
+static Knob g_quant_rows_per_wave{kByRule};
+static Knob g_dequant_rows_per_wave{kDequantRows};
+static Knob g_quant_outlier_rows_per_wave{kByRule};     // the same two with an outlier list
+static Knob g_dequant_outlier_rows_per_wave{kByRule};
 
 struct QuantArgs {
     uint16_t* x;            // bf16 activations (input of quantise / output of dequantise)
@@ -586,7 +588,7 @@ extern "C" int hyc_quant_pack(const void* x, const void* scale, const void* zero
     const void* zp = zero_point;
     QuantArgs a = make_args(x, scale, zp, q, outlier_idx, k, x_outlier, zero_input, B, M, N, stride_b, stride_m,
                             head_dim, stride_h, (outlier_idx && k) ? g_quant_outlier_rows_per_wave.get() : g_quant_rows_per_wave.get());
-    if (a.rows_per_wave == 0) a.rows_per_wave = quant_rows_by_size(a.T * N, zp != nullptr);
+    if (a.rows_per_wave == kByRule) a.rows_per_wave = quant_rows_by_size(a.T * N, zp != nullptr);
     const int64_t row_tiles = cdiv(a.T, (int64_t)kQuantWaves * a.rows_per_wave);
     if (row_tiles * a.col_tiles > INT32_MAX) return HYC_ERR_SHAPE;
     const dim3 grid((unsigned)(row_tiles * a.col_tiles)), block(kQuantThreads);
@@ -607,7 +609,7 @@ extern "C" int hyc_unpack_dequant(const void* q, const void* scale, const void* 
     const void* zp = zero_point;
     QuantArgs a = make_args(x, scale, zp, q, outlier_idx, k, x_outlier, 0, B, M, N, stride_b, stride_m, head_dim,
                             stride_h, (outlier_idx && k) ? g_dequant_outlier_rows_per_wave.get() : g_dequant_rows_per_wave.get());
-    if (a.rows_per_wave == 0) a.rows_per_wave = dequant_rows_by_size(a.T * N);
+    if (a.rows_per_wave == kByRule) a.rows_per_wave = dequant_rows_by_size(a.T * N);
     const int64_t row_tiles = cdiv(a.T, (int64_t)kQuantWaves * a.rows_per_wave);
     if (row_tiles * a.col_tiles > INT32_MAX) return HYC_ERR_SHAPE;
     const dim3 grid((unsigned)(row_tiles * a.col_tiles)), block(kQuantThreads);
@@ -621,10 +623,11 @@ int hyc::tune_quant(const char* key, int value) {
                            &g_dequant_outlier_rows_per_wave};
     const char* const names[4] = {"quant_rows_per_wave", "dequant_rows_per_wave", "quant_outlier_rows_per_wave",
                                   "dequant_outlier_rows_per_wave"};
+    const int defaults[4] = {kByRule, kDequantRows, kByRule, kByRule};
     for (int i = 0; i < 4; ++i) {
         if (strcmp(key, names[i]) != 0) continue;
-        if (value < 1 || value > 4096) return HYC_ERR_ARG;
-        knobs[i]->set(value);
+        if (value != -1 && (value < 1 || value > 4096)) return HYC_ERR_ARG;
+        knobs[i]->set(value == -1 ? defaults[i] : value);
         return HYC_OK;
     }
     return 1;  // not one of this file's keys

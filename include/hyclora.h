@@ -45,10 +45,11 @@ int hyc_abi_version(void);
  * stateless.  Results never depend on them except where said ("stats_waves": the last bits of the sums of
  * squares; "contract_strip_rows").  Each knob is an atomic integer that an entry point reads once per launch, so a launch on another
  * thread runs with the old or the new value of each knob, never a torn one; a pair of calls that must agree
- * (hyc_channel_stats_strips, then hyc_channel_stats) must not straddle a change.  Keys: "quant_rows_per_wave" (rows each wave walks in hyc_quant_pack,
- * by size until set), "dequant_rows_per_wave" (same for hyc_unpack_dequant, default 2),
+ * (hyc_channel_stats_strips, then hyc_channel_stats; hyc_lora_contract_workspace, then hyc_lora_contract or _group, which refuse a
+ * workspace that has become too small) must not straddle a change.  Keys: "quant_rows_per_wave" (rows each wave walks in
+ * hyc_quant_pack, by size until set), "dequant_rows_per_wave" (same for hyc_unpack_dequant, default 2),
  * "quant_outlier_rows_per_wave" / "dequant_outlier_rows_per_wave" (the same two when called with
- * an outlier list; by size until set),
+ * an outlier list; by size until set; -1 puts the default of any of these four back),
  * "norm_compress_slab" (0 / 1: whether hyc_rmsnorm_fwd_compress and, for rows wider than 4096 channels,
  * hyc_rmsnorm_bwd without a weight gradient may use the column-slab kernels, default 1)
  * and "norm_compress_rows_per_group" (rows a workgroup of that kernel walks, even; 0 = chosen from the

@@ -63,7 +63,18 @@ def test_argument_validation_without_launch(L):
     try:
         assert h.hyc_set_tuning(b"quant_rows_per_wave", 16) == 0
     finally:
-        assert h.hyc_set_tuning(b"quant_rows_per_wave", 8) == 0
+        assert h.hyc_set_tuning(b"quant_rows_per_wave", -1) == 0
+
+
+@pytest.mark.parametrize("key", [b"quant_rows_per_wave", b"dequant_rows_per_wave", b"quant_outlier_rows_per_wave", b"dequant_outlier_rows_per_wave"])
+def test_strip_heights_can_be_set_back(L, key):
+    """-1: the height by size (or the fixed default) that the process started with."""
+    h = L.lib()
+    try:
+        assert h.hyc_set_tuning(key, 16) == 0
+        assert h.hyc_set_tuning(key, -2) == -8 and h.hyc_set_tuning(key, 4097) == -8
+    finally:
+        assert h.hyc_set_tuning(key, -1) == 0
 
 
 def test_argument_validation_of_the_newer_entry_points(L):

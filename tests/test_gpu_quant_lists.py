@@ -56,3 +56,28 @@ def test_codes_with_zero_points(N, q_bit, B, M, n, slow):
         s[::97], z[9::131] = 1e-20, 1e25
     _, q = N.quantize(x.cuda(), s.cuda(), z.cuda(), None, q_bit)
     assert torch.equal(q.cpu(), O.compress(x, s, q_bit, z))
+
+
+@pytest.mark.parametrize("B,M,n", [(1, 5, 32), (2, 37, 512), (1, 130, 1056)])
+def test_strip_heights(N, B, M, n):
+    """Results do not depend on the rows that a wave walks, with and without a list, with and without zero points."""
+    from hyclora_amd import _lib
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(B, M, n, generator=g).to(BF16).cuda()
+    s, z = (0.05 + torch.rand(n, generator=g)).to(BF16).cuda(), torch.randint(-8, 8, (n,), generator=g).to(BF16).cuda()
+    idx = torch.randperm(n, generator=g)[:min(n, 70)].cuda()
+    keys = ("quant_rows_per_wave", "dequant_rows_per_wave", "quant_outlier_rows_per_wave", "dequant_outlier_rows_per_wave")
+
+    def call():
+        kept, q = N.quantize(x, s, None, idx, 4)
+        qz, qp = N.quantize(x, s, z, None, 4)[1], N.quantize(x, s, None, None, 4)[1]
+        return kept, q, qz, qp, N.dequantize(q, s, None, kept, idx, 4), N.dequantize(qz, s, z, None, None, 4), N.dequantize(qp, s, None, None, None, 4)
+    want = call()
+    try:
+        for rows in (1, 2, 3, 4, 8, 16):
+            for key in keys:
+                _lib.set_tuning(key, rows)
+            assert all(torch.equal(a, b) for a, b in zip(call(), want)), rows
+    finally:
+        for key in keys:
+            _lib.set_tuning(key, -1)
