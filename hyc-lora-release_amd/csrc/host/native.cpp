@@ -424,23 +424,32 @@ std::optional<std::tuple<Tensor, Tensor, Tensor>> lora_forward(const Tensor& w, 
 }
 
 // ---- projections in one pass, product included ----------------------------------------------------------------------
-// Whether hyc_lora_gemm takes the operands of one projection of the rows of x: W [n, k] (or, as an input gradient, [k, n]), B and x A
+// Whether hyc_lora_gemm takes a weight W [n, k] (or, as an input gradient, [k, n]) for `rows` rows
+bool gemm_weight(const Tensor& w, int64_t rows, int64_t n, int64_t k) {
+    return is_bf(w) && w.dim() == 2 && w.is_contiguous() && aligned(w) && n % 128 == 0 && k % 64 == 0 && rows * k < int64_t{1} << 31 &&
+           n * k < int64_t{1} << 31;
+}
+// The operands of one projection of the rows of x: W, B and x A
 bool gemm_member(const Tensor& x, const Tensor& w, const Tensor& lb, const Tensor& xa, int64_t rows, int64_t n, int64_t k, const OptT& bias,
                  hyc_gemm_member& m) {
     if (!together(x, w, lb, xa, bias)) return false;
     const Lora L(lb);
-    if (!is_bf(w) || w.dim() != 2 || !w.is_contiguous() || !aligned(w) || n % 128 || k % 64 || rows * k >= int64_t{1} << 31 || n * k >= int64_t{1} << 31)
-        return false;
+    if (!gemm_weight(w, rows, n, k)) return false;
     if (!L.fits(n) || L.r > 16 || !plain(xa) || xa.size(-1) != L.r || xa.numel() != rows * L.r || (bias && !vec(*bias, n))) return false;
     m = {};
     m.w = w.data_ptr(); m.xa = xa.data_ptr(); m.b = L.p; m.b_transposed = L.transposed; m.bias = ptr(bias); m.N = n; m.K = k;
     return true;
 }
-// Where that kernel is the way: weights of up to 2^22 elements, an encoder's.  us, against the library's product and the passes it
-// replaces: [4096, 1024] x 4096 53 / 63, [4096, 4096] x 1024 52 / 51, [1024, 1024] x 4096 21 / 29, [8192, 768] x 3072 64 / 90, [2048, 2048] x 2048 31 / 35;
-// [2048, 4096] x 4096 81 / 79, [512, 4096] x 4096 50 / 39.  It is the longer with few rows ([256, 3072] x 768 as an input gradient 32 / 17),
-// where a call of the library costs the host 20 us, which is what such a step is bound by.
-bool gemm_is_faster(int64_t n, int64_t k) { return n * k <= int64_t{1} << 22; }
+// Where that kernel is the way: weights of up to 2^22 elements, an encoder's, and contractions of up to 4096.  On the device, us, this
+// kernel / the library with the passes it replaces: input gradients [rows, k] x n  [4096, 768] x 768 15 / 22, [4096, 768] x 3072 38 / 41, [4096, 3072] x 768
+// 40 / 44, [4096, 4096] x 1024 50 / 49, [2048, 2048] x 2048 31 / 33; projections with bias and codes  [4096, 768] x 3072 40 / 59, [4096, 3072] x 768 49 / 49,
+// [4096, 2048] x 2048 50 / 62.  A workgroup walks the whole contraction, 0.65 us for 64 of it, which the library splits where tiles are few: under 192
+// tiles of 128 x 128 a long one takes longer here (gradients [256, 768] x 768 14 / 12, [64, 2048] x 2048 27 / 18, [256, 3072] x 768 36 / 18,
+// [256, 4096] x 1024 46 / 23; projections [256, 3072] x 768 45 / 25, [256, 4096] x 1024 55 / 32).  It is this kernel's all the same: steps of
+// that size wait for the host, and the library's way costs a step 20 to 50 us for a gradient and 100 for a projection (whole steps, both ways
+// in turn: encoder of 768 at 32 tokens 897 / 948, of 1024 at 512 tokens 939 / 1105, decoder of 2048 at 64 tokens 1211 / 1228).  Past 4096 it
+// is more than that makes up for: [64, 8192] x 512 85 / 18.
+bool gemm_is_faster(int64_t n, int64_t k) { return n * k <= int64_t{1} << 22 && k <= 4096; }
 
 // (W, A, B, bias, steps) of projections of one x -> (y, x A, codes of the frozen part) each: bf16(main + (x A) B), main = bf16(x W^T [+
 // bias]); gelu: of that; residual: added to it; steps (all members or none): the codes of main.  main_only: y = main, for a caller that
@@ -455,11 +464,11 @@ std::optional<std::vector<std::tuple<Tensor, Tensor, OptT>>> lora_project(const 
     std::vector<Tensor> adapters;
     for (const auto& [w, la, lb, bias, scale] : members) {
         if (!together(x, w, la, lb, bias, scale, residual)) return std::nullopt;
-        if (!is_bf(w) || w.dim() != 2 || w.size(1) != k || !gemm_is_faster(w.size(0), k) || scale.has_value() != codes ||
-            (scale && !vec(*scale, w.size(0))))
+        if (w.dim() != 2 || w.size(1) != k || !gemm_weight(w, rows, w.size(0), k) || !gemm_is_faster(w.size(0), k) ||
+            scale.has_value() != codes || (scale && !vec(*scale, w.size(0))))
             return std::nullopt;
         if (!is_bf(la) || la.dim() != 2 || la.size(0) != k || la.size(1) != lb.size(0) || lb.size(0) != std::get<2>(members[0]).size(0)) return std::nullopt;
-        if (w.size(0) % 128 || k % 64 || lb.size(0) > 16 || !Lora(lb).fits(w.size(0)) || (bias && !vec(*bias, w.size(0)))) return std::nullopt;
+        if (lb.size(0) > 16 || !Lora(lb).fits(w.size(0)) || (bias && !vec(*bias, w.size(0)))) return std::nullopt;
         adapters.push_back(la);
     }
     auto shape = x.sizes().vec();

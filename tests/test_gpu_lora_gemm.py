@@ -130,3 +130,25 @@ def test_what_the_kernel_does_not_take(M):
         assert call(x, w, la, lb, bias, res, residual=res[:, :10]) is None and call(x[:, :, ::2], w, la, lb, bias, res) is None
         assert M.native.lora_input_grad([(res, w, randn(g, 1, 20, 8), la.t()[:4])], None) is None
     assert call(*ok()) is None                                 # gradients are to be recorded
+
+
+@pytest.mark.parametrize("rows,n,k", [(64, 2048, 2048), (64, 512, 8192), (200, 768, 3072), (1, 1024, 4096), (300, 1024, 4096), (130, 896, 4160)])
+@pytest.mark.parametrize("gradient", [True, False])
+def test_contractions_past_the_rule_are_the_librarys(M, rows, n, k, gradient):
+    """Both sides of the rule, and that what follows it gives the projection's input gradient either way."""
+    ours = k <= 4096
+    g = torch.Generator().manual_seed(rows + k)
+    with torch.no_grad():
+        if gradient:
+            gy, w, mid, at = randn(g, 1, rows, k), randn(g, k, n, scale=k ** -0.5), randn(g, 1, rows, 16), randn(g, 16, n, scale=0.1)
+            done = M.native.lora_input_grad([(gy, w, mid, at)], None)
+            lb, x, xa = randn(g, k, 16, scale=0.1).t(), randn(g, 1, rows, n), randn(g, 1, rows, 16)
+            _, _, gx = M.cu.lora_backward(w, None, at.t().contiguous(), lb, x, xa, gy)
+            _, _, (_, own_mid, _) = M.cu.lora_backward(w, None, at.t().contiguous(), lb, x, xa, gy, defer_input=True)    # gy B^T, rounded
+            low = own_mid.double() @ at.double()
+            main = gy.double() @ w.double()
+            close_to(gx, main + low, [main, low], "input gradient")
+        else:
+            x, w, la, lb, bias, _ = project_operands(g, rows, n, k, 16)
+            done = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, False, None)
+    assert (done is not None) == ours
