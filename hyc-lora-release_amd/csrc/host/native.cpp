@@ -355,18 +355,34 @@ OptT frozen_input_grad(const Tensor& grad_y, const Tensor& w) {
 }
 bool weight_ok(const Tensor& w, int64_t in) { return is_bf(w) && w.dim() == 2 && w.size(1) == in && w.is_contiguous(); }
 
-// x A for one to three adapters [K, R] of one x, from one read of x, where that is the way.  This package's kernel against the library's
-// product, us (16 ranks): [96, 4096] 4.8 / 7.6, [96, 11008] 7.6 / 24, [2048, 4096] 8.9 / 14.3, [2048, 11008] 14.7 / 34, [4096, 768] 4.2 / 5.2, [4096, 4096]
-// 10.4 / 14.7, [4096, 11008] 23.2 / 36.6;  the other way round at [2048, 5120] 11.6 / 10.1, and to the library: [4096, 13824] 26.9 / 23.0, [8192, 4096]
-// 17.4 / 15.2, [8192, 11008] 42.6 / 40.8.  A call of the library costs the host 20 us more.
+// Whether x A of `members` adapters [k, r] is for this package's kernels.  Several adapters: always, x is read once ([2048, 4096] 10 / 16 and 12 / 24 us for
+// two and three, [8192, 4096] 19 / 26 and 24 / 39).  One, this package / the library, us at 16 ranks:
+//  - up to 4096 columns a workgroup has 16 rows to itself: one generation of workgroups, 4096 rows, is the shorter at every width ([4096, 768] 4.3 / 4.8,
+//    [2048, 2048] 4.4 / 6.0, [4096, 4096] 7.4 / 12.6), a second is not ([8192, 768] 5.7 / 5.2, [6000, 2048] 7.0 / 6.8, [8192, 4096] 14.1 / 13.7).  Ranks
+//    past 16 fill it with half the rows: 64 ranks, [2048, 1024] 5.9 / 6.8, [2048, 4096] 10 / 16, [4096, 2048] 11 / 8, [16384, 1024] 24 / 10;
+//  - past that its partial planes cost a second pass, and the library is the shorter where it has its own splits of the contraction, which are
+//    those of multiples of 512: [1536, 5120] 7.4 / 7.0, [1536, 8192] 8.7 / 8.8, [1536, 13824] 13.4 / 14.4, but [2048, 5120] 8.7 / 7.1, [2048, 13824] 16.0 /
+//    14.8, [4096, 8192] 17 / 14.  Other widths: [4096, 5504] 14 / 21, [2048, 11008] 14 / 26, [4096, 11008] 21 / 28, [4096, 13056] 23 / 31 (6912: 15.7 / 18.9, and
+//    16.0 / 13.8 at 4000 rows); 64 ranks [2048, 11008] 25 / 36, [4096, 11008] 40 / 40.
+//  - an adapter that lies as [k, r] goes through the planes at any width: [1024, 768] 7.3 / 5.1, [1024, 2048] 7.0 / 6.9, [2048, 4096] 7.7 / 8.4, [2048, 8192] 10 / 14,
+//    [2048, 13824] 16 / 18, [4096, 2048] 8.3 / 6.9, [4096, 13824] 24 / 21.
+// A call of the library costs the host 10 us more.
+bool adapters_are_ours(int64_t rows, int64_t k, int64_t r, bool lies_kr, size_t members) {
+    if (k % 32) return false;
+    if (members > 1) return true;
+    if (lies_kr) return k >= 2048 && rows <= 2048;
+    return rows <= (k > 4096 && k % 512 == 0 ? 1536 : r <= 16 ? 4096 : 2048);
+}
+
+// x A for one to three adapters [K, R] of one x, from one read of x, where that is the way
 std::vector<Tensor> adapter_products(const Tensor& x, const std::vector<Tensor>& adapters) {
     TORCH_CHECK(plain(x) && x.dim() >= 2 && x.numel() > 0, "x must be a contiguous bfloat16 tensor on the GPU");
     const int64_t k = x.size(-1), rows = x.numel() / k;
     for (const Tensor& a : adapters) TORCH_CHECK(is_bf(a) && a.dim() == 2 && a.size(0) == k, "an adapter must be [", k, ", R] bfloat16, got ", a.sizes());
-    const bool ours = k % 32 == 0 && (k <= 4096 ? rows * k < int64_t{1} << 25 : rows <= (k <= 12288 ? 4096 : 3072));
     hyc_contract_job jobs[3] = {};
     int64_t r = 0;
-    bool group = ours && !adapters.empty() && adapters.size() <= 3;
+    bool group = !adapters.empty() && adapters.size() <= 3 &&
+                 adapters_are_ours(rows, k, adapters[0].size(1), adapters[0].stride(1) == 1, adapters.size());
     for (size_t i = 0; group && i < adapters.size(); ++i) {
         const Tensor v = adapters[i].t();                          // [R, K]
         const Lora V(v);

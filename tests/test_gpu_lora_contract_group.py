@@ -53,6 +53,21 @@ def test_adapter_products_against_float64(M, T, N, ranks):
         assert_close_bf16(p2.cpu(), (x.double().cpu() @ a.double().cpu().t()).to(BF16), what="x A")
 
 
+@pytest.mark.parametrize("T,N,r,lies_kr,library", [
+    (1536, 4608, 16, False, False), (1537, 4608, 16, False, True), (2040, 5120, 16, False, True), (4096, 96, 16, False, False), (4097, 96, 16, False, True),
+    (2048, 1024, 64, False, False), (2049, 1024, 64, False, True), (1600, 5504, 16, False, False), (300, 768, 16, True, True), (300, 2048, 16, True, False)])
+def test_sides_of_the_adapter_rule(M, T, N, r, lies_kr, library):
+    """Past the rows, widths and layouts where this package's kernels are the shorter, one adapter is the library's product, bit for bit."""
+    g = torch.Generator().manual_seed(T + N)
+    x, a = randn(g, 1, T, N), randn(g, r, N, scale=0.1).t()
+    a = a.contiguous() if lies_kr else a
+    with torch.no_grad():
+        got, = M.cu._lib.native().adapter_products(x, [a])
+        assert_close_bf16(got.cpu(), (x.double() @ a.double()).to(BF16).cpu(), what="x A")
+        if library:
+            assert torch.equal(got[0], torch.mm(x[0], a))
+
+
 def test_rows_past_the_end_do_not_count(M):
     """What lies behind the last row (and right of the last column of a wave's tile) in memory may be anything."""
     g = torch.Generator().manual_seed(1)
