@@ -532,18 +532,22 @@ static void contract_launch(const ContractArgs& a, int64_t wgs, hipStream_t st) 
     else if constexpr (!(P1 && P2)) hipLaunchKernelGGL((lora_contract_kernel<QBIT, ZP, P1, P2, 3>), grid, block, 0, st, a);
 }
 
-// Rows of a strip: 256 where that leaves 160 workgroups and more or is all there is, else 128.  Fewer strips are fewer planes of P1 (2 x
-// 16 N x 4 bytes each), more strips more units at work: both products at 128 and 256 rows [T, N], us: [4096, 11008] 32.1 / 30.2 (352
-// workgroups at 256), [2040, 13824] 22.5 / 20.3 (216), [2048, 11008] 21.0 / 18.2 (176), [4096, 4096] 16.6 / 17.2 (128), [2040, 5120] 15.5 /
-// 16.3 (80), [2048, 4096] 14.9 / 16.0 (64).  It depends on T and N alone, so that the sums are in one order whatever else is in the
-// launch and whatever X is read from.
+// Rows of a strip: 256 where that leaves 160 workgroups and more or is all there is, 64 where even those are 64 workgroups and less, else 128.
+// Fewer strips are fewer planes of P1 (2 x 16 N x 4 bytes each), more strips more units at work: both products at 128 and 256 rows [T, N],
+// us: [4096, 11008] 32.1 / 30.2 (352 workgroups at 256), [2040, 13824] 22.5 / 20.3 (216), [2048, 11008] 21.0 / 18.2 (176), [4096, 4096] 16.6 / 17.2
+// (128), [2040, 5120] 15.5 / 16.3 (80), [2048, 4096] 14.9 / 16.0 (64);  at 64 and 128 rows, both products and P1 from codes: [300, 768] 8.5 / 9.9 and 8.4 /
+// 9.6 (10 workgroups at 64), [1000, 2048] 9.4 / 10.4 and 9.2 / 10.2 (64), [4096, 96] 9.1 / 10.1 and 9.2 / 10.8 (64), [680, 4096] 10.0 / 10.7 and 10.1 / 10.3 (88),
+// but three projections in a launch 32 / 29 there, 24 / 25 at [300, 4096] (40), 20.8 / 23.2 at [1000, 768] (32).  It depends on T and N alone, so
+// that the sums are in one order whatever else is in the launch and whatever X is read from.
 // Without P1 a strip leaves nothing behind, and 64 rows are the fastest at every shape measured ([4096, 11008] 24.5 against 26.5 at 256,
 // [512, 4096] 7.6 against 11.4).
 static int strip_rows(int64_t T, int64_t N, bool want1) {
     if (!want1) return kCtSub;
     const int fixed = g_ct_strip.get();
     if (fixed) return fixed;
-    return T <= kCtMaxStrip || cdiv(T, kCtMaxStrip) * cdiv(N, kCtBlock) >= 160 ? kCtMaxStrip : 128;
+    const int64_t col_blocks = cdiv(N, kCtBlock);
+    if (T <= kCtMaxStrip || cdiv(T, kCtMaxStrip) * col_blocks >= 160) return kCtMaxStrip;
+    return cdiv(T, kCtSub) * col_blocks <= 64 ? kCtSub : 128;
 }
 
 // Whether x V^T alone goes to the kernel that keeps whole rows to a workgroup: up to 4096 columns, V as it lies.  That kernel against

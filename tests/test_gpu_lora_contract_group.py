@@ -38,6 +38,34 @@ def test_edges_against_float64(M, T, N, R):
     assert torch.equal(t1.t(), p1) and torch.equal(t2, p2)
 
 
+# every height of a strip at rows that leave a short last one, one and several planes; and by size (0) at 64, 128 and 256 rows
+@pytest.mark.parametrize("T,N,R,strip", [(T, N, R, s) for T in (65, 257, 513, 777) for N, R in ((544, 20), (1056, 16)) for s in (64, 128, 192, 256)]
+                         + [(321, 1056, 16, 0), (1030, 4128, 16, 0), (2041, 10272, 16, 0)])
+def test_strip_heights(M, T, N, R, strip):
+    from hyclora_amd import _lib
+    g = torch.Generator().manual_seed(T + N + strip)
+    x, u, v = randn(g, T, N), randn(g, T, R), randn(g, R, N, scale=0.1)
+    s = M.cf.get_statistics_only_quant(x[None], 4, "per-channel")
+    q = M.cf.compression_pack_quant_base(x[None], 4, "per-channel", 1, 1, {"scale": s})[0]
+    dense = M.cf.decompression_dequantization(q, s, 4)[0]
+    d = lambda t: t.double()   # noqa: E731
+    try:
+        _lib.set_tuning("contract_strip_rows", strip)
+        p1, p2 = M.lk.lora_products(x, u, v)
+        coded = M.lk.lora_product_from_codes(q, s, u[None], None, 4)
+        with torch.no_grad():
+            members = [(randn(g, R, N, scale=0.1).t(), v, u[None], x[None])] * 2 if R <= 16 else None
+            group = members and M.cu._lib.native().lora_products_shared(members, None, q, s, None, 4)
+            single = M.lk.lora_product_from_codes(q, s, group[0][2], None, 4) if group else None
+    finally:
+        _lib.set_tuning("contract_strip_rows", 0)
+    assert_close_bf16(p1.cpu(), (d(u).t() @ d(x)).to(BF16).cpu(), what="u^T x")
+    assert_close_bf16(p2.cpu(), (d(x) @ d(v).t()).to(BF16).cpu(), what="x v^T")
+    assert_close_bf16(coded.cpu(), (d(u).t() @ d(dense)).to(BF16).cpu(), what="u^T x from codes")
+    for ga, gb, mid in group or ():
+        assert torch.equal(mid[0], p2) and torch.equal(gb, p1) and torch.equal(ga.t(), single)
+
+
 # x A alone: whole rows in a workgroup of 16 rows and turns of 1024 columns, two ahead, up to 4096 columns; planes beyond
 @pytest.mark.parametrize("T", [1, 15, 16, 17, 64, 200])
 @pytest.mark.parametrize("N", [32, 96, 992, 1024, 1056, 2048, 3104, 4096, 4128])
