@@ -635,7 +635,8 @@ static int launch_nc(const NormCompressArgs& a, const XaArgs& xa, hipStream_t st
         const int waves = a.N / (kWave * 8);
         // Strip height: all workgroups resident at once (16 waves per compute unit), each walking as
         // long a strip as that allows - the per-column constants are set up once per strip.
-        int rows_per_group = g_slab_rows_per_group.get();
+        const int fixed = g_slab_rows_per_group.get();
+        int rows_per_group = fixed;
         if (rows_per_group == 0) {
             const int64_t resident = (int64_t)compute_units() * (16 / (waves <= 8 ? waves : 16));
             rows_per_group = (int)(cdiv(cdiv(a.rows, resident), (int64_t)kSlabRows) * kSlabRows);
@@ -645,7 +646,8 @@ static int launch_nc(const NormCompressArgs& a, const XaArgs& xa, hipStream_t st
             // strip's rows are a serial chain
             const int64_t even = cdiv(cdiv(a.rows, (int64_t)compute_units()), (int64_t)kSlabRows) * kSlabRows;
             const int tile = waves <= 8 ? kXaRowsFor<8> : kXaRowsFor<16>;
-            rows_per_group = even < tile ? (int)even : tile;
+            const int64_t want = fixed ? fixed : even;
+            rows_per_group = want < tile ? (int)want : tile;
         }
         const int64_t groups = cdiv(a.rows, (int64_t)rows_per_group);
         if (groups > INT32_MAX) return HYC_ERR_SHAPE;

@@ -52,8 +52,8 @@ int hyc_abi_version(void);
  * an outlier list; by size until set; -1 puts the default of any of these four back),
  * "norm_compress_slab" (0 / 1: whether hyc_rmsnorm_fwd_compress and, for rows wider than 4096 channels,
  * hyc_rmsnorm_bwd without a weight gradient may use the column-slab kernels, default 1)
- * and "norm_compress_rows_per_group" (rows a workgroup of that kernel walks, even; 0 = chosen from the
- * row count, the default),
+ * and "norm_compress_rows_per_group" (rows a workgroup of that kernel walks, even, with adapters no more than a
+ * matrix-core tile: 16, or 8 past 4096 channels; 0 = chosen from the row count, the default),
  * "fuse_rows_per_wave" (same for both fused LoRA-SiLU kernels, multiple of 16; default 0 = by code width
  * and size: backward 32; forward 96 for tensors of 2^24 elements and more, else 32; at 8 bits 32 in both
  * directions for tensors of 2^24 elements and more, else 16; "fuse_fwd_rows_per_wave" / "fuse_bwd_rows_per_wave" set one of them),

@@ -166,8 +166,8 @@ def test_lora_a_contraction_in_the_norm_pass(ops, dev, shape, ranks):
     """y @ lora_A^T for every adapter fed by the norm's output, formed inside the norm kernel
     (compute_utils.py:22 via ...full_fuse.py:111-117, :218-226): against the float64 product of the
     kernel's own y rounded once (the oracle's lora_products: >= 99 % of the values the same bits, all
-    within tolerance), with every other output of the call unchanged bit for bit; row counts that do
-    not fill the last 8-row tile, ranks that do not fill a 16-row block, 1 to 16 waves per workgroup."""
+    within tolerance), with every other output of the call unchanged bit for bit; strips of 2 to 6 rows (as
+    so few rows are cut: full tiles in the next test), ranks that do not fill a 16-row block, 1 to 16 waves per workgroup."""
     q_bit = 4
     x, _ = activation_with_outlier_channels(seed=shape[1] + len(ranks), shape=shape, frac=0.01)
     g = torch.Generator().manual_seed(7)
@@ -199,6 +199,46 @@ def test_lora_a_contraction_in_the_norm_pass(ops, dev, shape, ranks):
     again = ops.norm.rmsnorm_forward_compress(xd, wd, 1e-5, q_bit, scale_y=s_y, scale_x=s_x, outlier_idx=idx, lora_a=views)
     for xa, xb in zip(got[5], again[5]):
         assert torch.equal(xa, xb)
+
+
+def xa_operands(dev, rows, n, ranks):
+    g = torch.Generator(device=dev).manual_seed(rows + n + len(ranks))
+    rn = lambda *sh: torch.randn(*sh, generator=g, device=dev)   # noqa: E731
+    x = (rn(1, rows, n) * 2).to(BF16)
+    w = (1 + 0.1 * rn(n)).to(BF16)
+    return x, w, [(rn(r, n) / n ** 0.5).to(BF16).t() for r in ranks]
+
+
+RANKS = [(16,), (16, 16), (16, 8, 16), (16, 16, 16, 16), (40,)]
+
+
+# by size: tiles of 16 rows, or 8 past 4096 channels, and a short last one (10 and 2 rows); by the knob: the heights up to those
+@pytest.mark.parametrize("rows,n", [(4106, 512), (4106, 4096), (2058, 8192)])
+@pytest.mark.parametrize("ranks", RANKS)
+def test_lora_a_contraction_of_full_tiles(ops, dev, rows, n, ranks):
+    x, w, views = xa_operands(dev, rows, n, ranks)
+    y, _, _, _, _, xas = ops.norm.rmsnorm_forward_compress(x, w, 1e-5, 4, lora_a=views)
+    assert torch.equal(y, ops.norm.rmsnorm_forward_compress(x, w, 1e-5, 4)[0])
+    for a, xa in zip(views, xas):
+        want = (y[0].double() @ a.double()).to(BF16)
+        assert_close_bf16(xa[0].cpu(), want.cpu(), what="x@A vs float64 product")
+        assert (xa[0] == want).float().mean().item() >= 0.99
+
+
+@pytest.mark.parametrize("rows,n", [(50, 512), (4106, 1024), (50, 4096), (34, 8192)])
+@pytest.mark.parametrize("ranks", RANKS)
+def test_lora_a_contraction_at_every_strip_height(ops, dev, rows, n, ranks):
+    from hyclora_amd import _lib
+    x, w, views = xa_operands(dev, rows, n, ranks)
+    base = ops.norm.rmsnorm_forward_compress(x, w, 1e-5, 4, lora_a=views)
+    try:
+        for height in range(2, 20, 2):
+            _lib.set_tuning("norm_compress_rows_per_group", height)
+            got = ops.norm.rmsnorm_forward_compress(x, w, 1e-5, 4, lora_a=views)
+            assert torch.equal(got[0], base[0]) and torch.equal(got[1], base[1]), height
+            assert all(torch.equal(a, b) for a, b in zip(got[5], base[5])), height
+    finally:
+        _lib.set_tuning("norm_compress_rows_per_group", 0)
 
 
 def test_lora_a_contraction_limits(ops, dev):
