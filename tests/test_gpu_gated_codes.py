@@ -12,7 +12,7 @@ def bits(t):
 
 
 @pytest.mark.parametrize("q_bit", [2, 4, 8])
-@pytest.mark.parametrize("shape", [(1, 1, 32), (1, 33, 544), (3, 21, 1024), (2, 64, 512)])
+@pytest.mark.parametrize("shape", [(1, 1, 32), (1, 33, 544), (3, 21, 1024), (2, 64, 512), (1, 65541, 32)])       # the last: 8 rows a wave
 def test_against_the_separate_passes(shape, q_bit):
     import hyclora_amd  # noqa: F401
     from hyclora_amd.operators import silu_kernels as K

@@ -133,6 +133,24 @@ def test_shared_input_matches_single_calls(M, T, widths, R, q_bit):
             assert ga.t().is_contiguous() and gb.t().is_contiguous()
 
 
+@pytest.mark.parametrize("q_bit", [2, 4, 8])
+@pytest.mark.parametrize("T", [1, 300])
+def test_shared_input_with_zero_points_matches_single_calls(M, T, q_bit):
+    g = torch.Generator().manual_seed(T + q_bit)
+    K, R = 544, 16
+    x = randn(g, 1, T, K) + 0.5
+    s, z = M.cf.get_statistics_only_quant_zero_point(x, q_bit, "per-channel")
+    q = M.cf.compression_pack_quant_zp_base(x, q_bit, "per-channel", 1, 1, {"scale": s, "zero_point": z})[0]
+    z = z.to(BF16)
+    members = [(randn(g, n, K, scale=0.05), None, randn(g, R, K, scale=0.1).t(), randn(g, n, R, scale=0.1).t(), randn(g, 1, T, R), randn(g, 1, T, n))
+               for n in (512, 96, 1056)]
+    with torch.no_grad():
+        assert M.cu._lib.native().lora_products_shared([(m[2], m[3], m[4], m[5]) for m in members], None, q, s, z, q_bit) is not None
+        for (w, qs, la, lb, xa, gy), (ga, gb, (gx, mid, at)) in zip(members, M.cu.lora_backward_shared(members, None, (q, s, z, q_bit))):
+            ga1, gb1, (gx1, mid1, at1) = M.cu.lora_backward(w, qs, la, lb, None, xa, gy, x_codes=(q, s, z, q_bit), defer_input=True)
+            assert torch.equal(ga, ga1) and torch.equal(gb, gb1) and torch.equal(mid, mid1) and torch.equal(gx, gx1)
+
+
 def test_group_refusals(M):
     """What the group does not take goes the way of the single calls: ranks past 16, ranks that differ, one member, host tensors."""
     g = torch.Generator().manual_seed(2)

@@ -100,6 +100,64 @@ def test_input_gradients(M, T, outs, N, R):
             assert torch.equal(got, M.native.lora_input_grad(members, residual))
 
 
+@pytest.mark.parametrize("T", [1, 33, 200])
+@pytest.mark.parametrize("outs,N,R", [((64,), 128, 16), ((192, 64), 256, 4), ((128, 64, 320), 384, 16)])
+def test_additions_are_bf16_ones_in_order(M, T, outs, N, R):
+    """The sum of input gradients, bit for bit: the single ones added up in bf16 in their order, then the residual; and a projection's residual."""
+    g = torch.Generator().manual_seed(T + N)
+    members = [(randn(g, 1, T, k), randn(g, k, N, scale=k ** -0.5), randn(g, 1, T, R), randn(g, R, N, scale=0.1)) for k in outs]
+    res = randn(g, 1, T, N)
+    with torch.no_grad():
+        total = None
+        for m in members:
+            one = M.native.lora_input_grad([m], None)
+            total = one if total is None else total + one
+        assert torch.equal(M.native.lora_input_grad(members, None), total)
+        assert torch.equal(M.native.lora_input_grad(members, res), total + res)
+        x, w, la, lb, bias, res = project_operands(g, T, N, 64, R)
+        (bare, _, _), = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, False, None)
+        (y, _, _), = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, False, res)
+        assert torch.equal(y, res + bare)
+        (act, _, _), = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, True, None)
+        (act_res, _, _), = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, True, res)
+        assert torch.equal(act_res, res + act)
+
+
+def kinds(t):
+    """0 finite, 1 infinite, 2 negative infinite, 3 NaN"""
+    t = t.float()
+    return t.isposinf().int() + 2 * t.isneginf().int() + 3 * t.isnan().int()
+
+
+@pytest.mark.parametrize("T", [40, 200])
+def test_infinities_and_nan(M, T):
+    """They go where the library's product and the passes after it carry them, and nowhere else: rows, columns and tiles keep apart."""
+    g = torch.Generator().manual_seed(T)
+    N, K, R = 384, 256, 16
+    x, w, la, lb, bias, res = project_operands(g, T, N, K, R)
+    x[0, 1, 7], x[0, T - 1, K - 1], x[0, 9, 100] = float("nan"), float("inf"), float("-inf")
+    w[130, 5], lb[3, 200], bias[383], res[0, 20, 64] = float("inf"), float("-inf"), float("nan"), float("inf")
+    s = (torch.rand(N, generator=g) * 0.1 + 0.01).to(BF16).cuda()
+    with torch.no_grad():
+        main = x @ w.t() + bias
+        (y, xa, q), = M.native.lora_project(x, [(w, la, lb, bias, s)], 4, False, None)
+        want_q, want = M.lk.lora_add_quant(main, xa, lb, s, None, 4)
+        assert torch.equal(kinds(y), kinds(want)) and torch.equal(kinds(xa), kinds(x @ la))
+        (main_only, _, _), = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, False, None, True)
+        assert torch.equal(kinds(main_only), kinds(main)) and torch.equal(q, M.lk.lora_add_quant(main_only, xa, lb, s, None, 4)[0])
+        (y, _, _), = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, False, res)
+        assert torch.equal(kinds(y), kinds(M.lk.lora_add(main, xa, lb, residual=res)))
+        # input gradients: gy [T, N] W [N, K]
+        gy, mid, at = res, xa, la.t().contiguous()
+        gx = M.native.lora_input_grad([(gy, w, mid, at)], None)
+        assert torch.equal(kinds(gx), kinds(M.lk.lora_add(gy @ w, mid, at)))
+        # x A alone: a row's own
+        clean = torch.where(x.isfinite(), x, torch.zeros_like(x))
+        a, b = M.native.adapter_products(x, [la])[0], M.native.adapter_products(clean, [la])[0]
+        rows = x.isfinite().all(-1)
+        assert torch.equal(a[rows], b[rows]) and not a[~rows].isfinite().any()
+
+
 def test_many_tiles_and_the_library(M):
     """Tiles on every XCD, a remainder of workgroups; the library's product of these operands sums in the same order (where it takes another
     one a few results may differ by a rounding)."""
