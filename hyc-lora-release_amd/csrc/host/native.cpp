@@ -308,14 +308,17 @@ int64_t whole_rounds(int64_t rows, int64_t cols) {
 //    64 bits is 1.9e-2 of its largest entry, the oracle's 8.8e-3, the bound twice that (cosines 0.999969 and 0.999973; sums in
 //    which the terms of a channel with an outlier nearly cancel);
 //  - x W^T (4096 x 4096 18 / 22, 11008 x 4096 30 / 50): its last bits decide codes, so a step in another order has some other
-//    codes.
+//    codes, and its results move by 2.1 % instead of 0.6.
+// (Other sums in an order of their own stay inside every bound: x A and the rank-R gradients move a step's results by 0.2 % at most, through
+// the codes that a unit of x A changes now and then.  hyc_lora_gemm keeps the library's order.)
+bool few_rows_is_faster(int64_t rows, int64_t k) { return rows < 128 && k >= 4096; }
 OptT few_rows(const Tensor& x, const Tensor& w) {                  // x [.., K], w [K, N]
     if (!products_are_plain() || !plain(x) || x.dim() < 2 || x.numel() == 0 || !is_bf(w) || w.dim() != 2 || w.device() != x.device())
         return std::nullopt;
     const int64_t k = w.size(0), n = w.size(1);
     if (x.size(-1) != k || !aligned(w)) return std::nullopt;
     const int64_t rows = x.numel() / k;
-    if (w.stride(1) != 1 || w.stride(0) != n || rows >= 128 || k < 4096) return std::nullopt;
+    if (w.stride(1) != 1 || w.stride(0) != n || !few_rows_is_faster(rows, k)) return std::nullopt;
     const int64_t bytes = hyc_few_rows_workspace(rows, n, k);
     if (bytes == 0) return std::nullopt;
     auto shape = x.sizes().vec();
@@ -464,8 +467,11 @@ bool gemm_member(const Tensor& x, const Tensor& w, const Tensor& lb, const Tenso
 // [256, 4096] x 1024 46 / 23; projections [256, 3072] x 768 45 / 25, [256, 4096] x 1024 55 / 32).  It is this kernel's all the same: steps of
 // that size wait for the host, and the library's way costs a step 20 to 50 us for a gradient and 100 for a projection (whole steps, both ways
 // in turn: encoder of 768 at 32 tokens 897 / 948, of 1024 at 512 tokens 939 / 1105, decoder of 2048 at 64 tokens 1211 / 1228).  Past 4096 it
-// is more than that makes up for: [64, 8192] x 512 85 / 18.
+// is more than that makes up for: [64, 8192] x 512 85 / 18.  The results are the library's bits, but for 3 of 10000 where the library splits the contraction;
+// both are equally far from 64 bits.
 bool gemm_is_faster(int64_t n, int64_t k) { return n * k <= int64_t{1} << 22 && k <= 4096; }
+// Input gradients that few_rows takes, whose calls are as cheap for the host, are its: [96, 4096] x 1024 19 / 46
+bool gemm_is_faster_gradient(int64_t rows, int64_t n, int64_t k) { return gemm_is_faster(n, k) && !few_rows_is_faster(rows, k); }
 
 // (W, A, B, bias, steps) of projections of one x -> (y, x A, codes of the frozen part) each: bf16(main + (x A) B), main = bf16(x W^T [+
 // bias]); gelu: of that; residual: added to it; steps (all members or none): the codes of main.  main_only: y = main, for a caller that
@@ -527,7 +533,7 @@ OptT lora_input_grad(const std::vector<InputGrad>& members, const OptT& residual
         const auto& [g, w, mid, at_] = members[i];
         if (!together(first, g, residual)) return std::nullopt;
         if (!plain(g) || g.numel() != rows * g.size(-1) || w.dim() != 2 || w.size(0) != g.size(-1) || w.size(1) != n || at_.size(0) != r ||
-            !gemm_is_faster(n, w.size(0)) || !gemm_member(g, w, at_, mid, rows, n, w.size(0), std::nullopt, m[i]))
+            !gemm_is_faster_gradient(rows, n, w.size(0)) || !gemm_member(g, w, at_, mid, rows, n, w.size(0), std::nullopt, m[i]))
             return std::nullopt;
         m[i].x = g.data_ptr();
     }

@@ -12,9 +12,11 @@
 // after the product is that of lora_add.hip.
 //
 // A workgroup of 4 waves forms 128 x 128 results, 64 x 64 a wave, as products of 16x16x32 along the contraction from its start to its
-// end, which is also the order of the library's kernels for these sizes: same bits in every case compared.  The operands come through
-// LDS in tiles of 64 along the contraction (hyc_attn_tile.hpp), the copies of the next one under way; two workgroups a unit cover
-// each other's waits, and the turns are bound by the LDS reads (96 KB a turn and workgroup, 0.65 us).  (Four stages with three tiles on the
+// end, which is also the order of the library's kernels for these sizes: same bits in every case compared, but for 3 of 10000 results
+// with few tiles and a long contraction, which the library splits.  The operands come through
+// LDS in tiles of 64 along the contraction (hyc_attn_tile.hpp), the copies of the next one under way; a turn takes 0.65 us, which is its
+// LDS reads (96 KB a workgroup) where two workgroups share a unit and cover each other's waits (from 257 tiles on), and its waits where a
+// unit has one.  (Four stages with three tiles on the
 // way and one workgroup a unit: 18 against 16 us at 4096 x 768 x 768, 50 against 36 for three members.)  The product is formed transposed, so
 // that a lane holds four neighbouring columns of a row, and goes through LDS once more, rounded, into the ownership of the packed
 // codes: a lane has 8 consecutive columns of four rows.  Several projections of one x go into one launch.

@@ -190,11 +190,11 @@ def test_what_the_kernel_does_not_take(M):
     assert call(*ok()) is None                                 # gradients are to be recorded
 
 
-@pytest.mark.parametrize("rows,n,k", [(64, 2048, 2048), (64, 512, 8192), (200, 768, 3072), (1, 1024, 4096), (300, 1024, 4096), (130, 896, 4160)])
+@pytest.mark.parametrize("rows,n,k", [(64, 2048, 2048), (64, 512, 8192), (200, 768, 3072), (100, 1024, 4096), (128, 1024, 4096), (300, 1024, 4096), (130, 896, 4160)])
 @pytest.mark.parametrize("gradient", [True, False])
 def test_contractions_past_the_rule_are_the_librarys(M, rows, n, k, gradient):
     """Both sides of the rule, and that what follows it gives the projection's input gradient either way."""
-    ours = k <= 4096
+    ours = k <= 4096 and not (gradient and rows < 128 and k == 4096)          # the last: the kernel of a few rows takes it
     g = torch.Generator().manual_seed(rows + k)
     with torch.no_grad():
         if gradient:
