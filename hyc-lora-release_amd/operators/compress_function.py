@@ -391,30 +391,24 @@ def compress_attention_map(x: torch.Tensor, outlier, seg_offsets=None, compare_a
         else:
             _lib.call("hyc_sparse_count_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), scratch.data_ptr(), offsets.data_ptr(), kept, st)
 
-    def lists(room):
-        return torch.empty(room, device=x.device, dtype=torch.int64), torch.empty(room, device=x.device, dtype=BF16)
-
-    def written(room):
-        nonlocal scratch, kept
-        try:
-            idx, val = lists(room)
-        except torch.OutOfMemoryError:
-            if kept is None:
-                raise
-            scratch = kept = None
-            idx, val = lists(room)
-        if kept is None:
-            _lib.call("hyc_sparse_write_bounded", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), room, idx.data_ptr(),
-                      val.data_ptr(), st)
-        else:
-            _lib.call("hyc_sparse_write_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), kept, room, idx.data_ptr(),
-                      val.data_ptr(), st)
-        return idx, val
     if capacity is not None:
-        pending = PendingCount(offsets[-1:])            # known before the lists are written: who waits for it does not wait for those
-        return *written(int(capacity)), offsets, pending
-    nnz = int(offsets[-1].item())      # the one host sync; to_sparse() has the same one
-    return *(written(nnz) if nnz else lists(0)), offsets
+        room, pending = int(capacity), PendingCount(offsets[-1:])       # known before the lists are written: who waits for it does not wait for those
+    else:
+        room = int(offsets[-1].item())     # the one host sync; to_sparse() has the same one
+    try:
+        idx, val = torch.empty(room, device=x.device, dtype=torch.int64), torch.empty(room, device=x.device, dtype=BF16)
+    except torch.OutOfMemoryError:
+        if kept is None:
+            raise
+        scratch = kept = None
+        idx, val = torch.empty(room, device=x.device, dtype=torch.int64), torch.empty(room, device=x.device, dtype=BF16)
+    if kept is None:
+        _lib.call("hyc_sparse_write_bounded", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), room, idx.data_ptr(),
+                  val.data_ptr(), st)
+    else:
+        _lib.call("hyc_sparse_write_staged", flat.data_ptr(), n, thr.data_ptr(), int(compare_abs), offsets.data_ptr(), kept, room, idx.data_ptr(),
+                  val.data_ptr(), st)
+    return (idx, val, offsets) if capacity is None else (idx, val, offsets, pending)
 
 
 def check_map_lists(idx, val, seg_offsets, numel: int) -> None:
