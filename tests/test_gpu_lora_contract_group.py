@@ -1,6 +1,8 @@
 """The rank-R products of several projections in one launch (hyc_lora_contract_group behind lora_backward_shared) against the
 calls of the single projections, bit for bit, and the single calls at the edges of their row strips, planes and column
 blocks against float64."""
+import ctypes
+
 import pytest
 import torch
 
@@ -165,3 +167,41 @@ def test_group_refusals(M):
         host = tuple(t.cpu() for t in member(16))
         assert call([member(16), host]) is None
     assert call([member(16), member(16)]) is None                # gradients are to be recorded
+
+
+class Job(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x", "q", "scale", "zero_point", "u", "v", "p1", "p2")] + \
+               [("N", ctypes.c_int64), ("v_transposed", ctypes.c_int), ("p1_transposed", ctypes.c_int)]
+
+
+@pytest.mark.parametrize("q_bit", [0, 2, 8])
+@pytest.mark.parametrize("zero", [False, True])
+def test_jobs_with_an_input_each(M, q_bit, zero):
+    """The form of the C entry that no wrapper uses for codes: every job has its X, dense or as codes, of its own width; the bits of single calls."""
+    from hyclora_amd import _lib
+    g = torch.Generator().manual_seed(q_bit)
+    T, R, widths = 300, 12, (96, 1056, 544)
+    jobs, want, got, keep = (Job * 3)(), [], [], []
+    for job, n in zip(jobs, widths):
+        x, u = randn(g, 1, T, n), randn(g, 1, T, R)
+        out = torch.empty(n, R, dtype=BF16, device="cuda")
+        job.u, job.p1, job.N, job.p1_transposed = u.data_ptr(), out.data_ptr(), n, 1
+        if q_bit:
+            s, z = M.cf.get_statistics_only_quant_zero_point(x, q_bit, "per-channel")
+            z = z.to(BF16) if zero else None
+            q = M.cf.compression_pack_quant_zp_base(x, q_bit, "per-channel", 1, 1, {"scale": s, "zero_point": z})[0] if zero \
+                else M.cf.compression_pack_quant_base(x, q_bit, "per-channel", 1, 1, {"scale": s})[0]
+            s = s.reshape(-1).contiguous()
+            job.q, job.scale, job.zero_point = q.data_ptr(), s.data_ptr(), z.data_ptr() if zero else None
+            want.append(M.lk.lora_product_from_codes(q, s, u, z, q_bit))
+            keep += [s, z, q]
+        else:
+            job.x = x.data_ptr()
+            want.append(M.lk.lora_products(x, u)[0])
+        got.append(out)
+        keep += [x, u]
+    nbytes = max(16, sum(_lib.lib().hyc_lora_contract_workspace(T, n, R, 1, 0) for n in widths))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    _lib.call("hyc_lora_contract_group", ctypes.addressof(jobs), 3, 0, q_bit, ws.data_ptr(), nbytes, T, R, _lib.stream_of(ws))
+    for a, b in zip(got, want):
+        assert torch.equal(a.t(), b)

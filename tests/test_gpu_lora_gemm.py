@@ -1,5 +1,7 @@
 """Projections and input gradients with the product in the same kernel (hyc_lora_gemm) against float64, and against the library's product
 with this package's passes around it, at the edges of its tiles of 128 rows and columns and 64 of the contraction."""
+import ctypes
+
 import pytest
 import torch
 
@@ -210,3 +212,30 @@ def test_contractions_past_the_rule_are_the_librarys(M, rows, n, k, gradient):
             x, w, la, lb, bias, _ = project_operands(g, rows, n, k, 16)
             done = M.native.lora_project(x, [(w, la, lb, bias, None)], 0, False, None)
     assert (done is not None) == ours
+
+
+class Member(ctypes.Structure):
+    _fields_ = [(n, ctypes.c_void_p) for n in ("x", "w", "xa", "b", "bias", "residual", "scale", "q", "y")] + \
+               [("N", ctypes.c_int64), ("K", ctypes.c_int64), ("b_transposed", ctypes.c_int)]
+
+
+@pytest.mark.parametrize("T", [1, 130])
+def test_several_input_gradients_with_a_bias_each(M, T):
+    """A form of the C entry that no wrapper uses: weights as [K, N], no sum, with a bias; against the same weights as [N, K]."""
+    from hyclora_amd import _lib
+    g = torch.Generator().manual_seed(T)
+    members, keep, got, want = (Member * 2)(), [], [], []
+    for m, (n, k) in zip(members, ((128, 192), (384, 64))):
+        x, w, xa, b, bias, res = randn(g, T, k), randn(g, k, n, scale=k ** -0.5), randn(g, T, 8), randn(g, 8, n, scale=0.1), randn(g, n), randn(g, T, n)
+        y = torch.empty(T, n, dtype=BF16, device="cuda")
+        m.x, m.w, m.xa, m.b, m.bias, m.residual, m.y, m.N, m.K = *(t.data_ptr() for t in (x, w, xa, b, bias, res, y)), n, k
+        one, wt, out = (Member * 1)(), w.t().contiguous(), torch.empty_like(y)
+        ctypes.memmove(one, ctypes.addressof(members) + len(got) * ctypes.sizeof(Member), ctypes.sizeof(Member))
+        one[0].w, one[0].y = wt.data_ptr(), out.data_ptr()
+        _lib.call("hyc_lora_gemm", ctypes.addressof(one), 1, 0, 0, 0, 0, T, 8, _lib.stream_of(x))
+        keep += [x, w, xa, b, bias, res, wt]
+        got.append(y)
+        want.append(out)
+    _lib.call("hyc_lora_gemm", ctypes.addressof(members), 2, 1, 0, 0, 0, T, 8, _lib.stream_of(got[0]))
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
